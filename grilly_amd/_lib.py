@@ -41,6 +41,13 @@ class BertLayerFused(ctypes.Structure):
                                         "ws_ff1", "c_ff1", "bf_ff1", "w_ff2", "b_ff2")]
 
 
+class Ragged(ctypes.Structure):
+    _fields_ = [("offsets", c_void_p), ("positions", c_void_p), ("sequences", c_i64), ("rows", c_i64), ("longest", c_i64)]
+
+
+PACK_PREFIX, PACK_SCATTERED, PACK_OTHER_MASK, PACK_BAD_ID = 0, 1, 2, 3
+_rg = ctypes.POINTER(Ragged)
+
 # name -> (restype, argtypes); every symbol include/grilly_hip.h declares
 SIGNATURES = {
     "grl_create": (c_void_p, [c_int]),
@@ -99,6 +106,14 @@ SIGNATURES = {
     "grl_embed_layernorm": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                     c_float, c_void_p]),
     "grl_mean_pool": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_int]),
+    "grl_pack_batch": (c_int, [c_i64, c_i64, c_i64, c_void_p, c_void_p, c_int, c_void_p, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)]),
+    "grl_embed_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "grl_embed_layernorm_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64] + [c_void_p] * 6 + [c_float, c_void_p]),
+    "grl_fa2_fwd_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64] + [c_void_p] * 4 + [c_i64] * 4 + [c_float, c_int, c_int, c_float, c_float]),
+    "grl_mean_pool_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_void_p, c_i64, c_void_p, c_int]),
+    "grl_bert_layer_fwd_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayer), c_float, c_void_p, c_void_p]),
+    "grl_bert_layer_fwd_fused_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_float,
+                                        c_void_p, c_void_p, c_void_p]),
     "grl_bert_layer_workspace": (c_i64, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64]),
     "grl_bert_layer_fused_workspace": (c_i64, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64]),
     "grl_bert_layer_fwd_fused": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_void_p, c_float,

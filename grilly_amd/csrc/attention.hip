@@ -23,15 +23,17 @@
 #include <cstdlib>
 
 int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                         void* y, const float* table);
+                         void* y, const float* table, const int32_t* positions);
 int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                              void* y, const float* table);
+                              void* y, const float* table, const int32_t* positions);
 int grl_rope_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
                      const int32_t* position_ids, void* y, int style, float rope_base, float rope_scaling);
 
 struct FaArgs {
     const void* Q; const void* K; const void* V;
     const float* mask;        // (B,S) or null
+    const int32_t* offsets;   // first row of each sequence of a ragged batch (B+1 entries; S is then the longest length), or null
+    const int32_t* positions; // ragged batch: position of each row in its sequence
     void* O;
     const float2* rope;       // (S, D/2) {cos, sin} or null
     int B, S, H;
@@ -39,6 +41,18 @@ struct FaArgs {
     int causal;
     int64_t q_stride, k_stride, v_stride, o_stride;   // elements between consecutive positions
 };
+
+// Sequence b of the batch: its first row and its length.  In a ragged batch the sequences stand back to back and every one
+// has its own length (queries and keys alike); the grid is laid out for the longest, and a workgroup whose queries lie past
+// the end of its sequence has nothing to do.
+__device__ __forceinline__ void fa_sequence(const int32_t* offsets, int b, int S, int64_t& row0, int& len) {
+    if (offsets) {
+        const int o = __builtin_amdgcn_readfirstlane(offsets[b]), e = __builtin_amdgcn_readfirstlane(offsets[b + 1]);
+        row0 = o; len = e - o;
+    } else {
+        row0 = (int64_t)b * S; len = S;
+    }
+}
 
 template <int N, typename F> __device__ __forceinline__ void sfor(F&& f) {
     if constexpr (N > 0) {
@@ -127,12 +141,14 @@ __global__ __launch_bounds__(256) void fa2_fwd_kernel(FaArgs p) {
     const int b = blockIdx.z, h = blockIdx.y;
     const int qb = p.causal ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;   // heavy blocks first
     const int q0 = qb * 128;
-    const int S = p.S;
+    int64_t row0; int S;
+    fa_sequence(p.offsets, b, p.S, row0, S);
+    if (q0 >= S) return;
     const int qi = q0 + wave * 32 + li;
     const int qc = qi < S ? qi : S - 1;
-    const T* Qg = (const T*)p.Q + (int64_t)b * S * p.q_stride + h * D;
-    const T* Kg = (const T*)p.K + (int64_t)b * S * p.k_stride + h * D;
-    const T* Vg = (const T*)p.V + (int64_t)b * S * p.v_stride + h * D;
+    const T* Qg = (const T*)p.Q + row0 * p.q_stride + h * D;
+    const T* Kg = (const T*)p.K + row0 * p.k_stride + h * D;
+    const T* Vg = (const T*)p.V + row0 * p.v_stride + h * D;
 
     // ---- this lane's query, as MFMA "B" operand: slab s holds dims (2s+lg)*EPC .. +EPC-1
     u32x4 qf[NS];
@@ -180,7 +196,7 @@ __global__ __launch_bounds__(256) void fa2_fwd_kernel(FaArgs p) {
         if (tid < KT) {
             const int kk = k0 + tid;
             breg = 0.f;
-            if (p.mask && kk < S) breg = (p.mask[(int64_t)b * S + kk] - 1.0f) * 1e9f;
+            if (p.mask && kk < S) breg = (p.mask[row0 + kk] - 1.0f) * 1e9f;
             if (kk >= S) breg = -__builtin_inff();
         }
     };
@@ -300,7 +316,7 @@ __global__ __launch_bounds__(256) void fa2_fwd_kernel(FaArgs p) {
     const float l_tot = halves_sum(l_run);
     const float inv = 1.0f / fmaxf(l_tot, 1e-10f);
     if (qi < S) {
-        T* Og = (T*)p.O + ((int64_t)b * S + qi) * p.o_stride + h * D;
+        T* Og = (T*)p.O + (row0 + qi) * p.o_stride + h * D;
         sfor<DT>([&](auto idt) {
             constexpr int dt = decltype(idt)::value;
 #pragma unroll
@@ -336,6 +352,7 @@ __global__ __launch_bounds__(256) void fa2_fwd_kernel(FaArgs p) {
 struct Fa16Args {
     const uint16_t* Q; const uint16_t* K; const uint16_t* V;
     const float* mask; uint16_t* O; const float2* rope;
+    const int32_t* offsets;   // ragged batch, see FaArgs
     int B, S, H;
     float scale;
     int causal;
@@ -407,8 +424,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
     // (readfirstlane): the loop then branches on scalar conditions and keeps its counters in scalar registers.
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int li = lane & 31, lg = lane >> 5;
-    const int S = p.S;
-    const int nqb = (S + QB - 1) / QB, nbh = p.B * p.H;
+    const int nqb = (p.S + QB - 1) / QB, nbh = p.B * p.H;
     const int nwg = (int)gridDim.x, per = nwg >> 3, rem = nwg & 7, xcd = (int)blockIdx.x & 7, loc = (int)blockIdx.x >> 3;
     const int lin = (p.order & 1) ? xcd * per + (xcd < rem ? xcd : rem) + loc : (int)blockIdx.x;
     int qb, bh;
@@ -419,7 +435,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
     const int b = uni(bh / p.H), h = uni(bh % p.H);
     const int q0 = qb * QB;
     const int qw0 = q0 + wave * QW;
-    const uint16_t* Qg = p.Q + (int64_t)b * S * p.q_stride + h * D;
+    int64_t row0; int S;
+    fa_sequence(p.offsets, b, p.S, row0, S);
+    if (q0 >= S) return;
+    const uint16_t* Qg = p.Q + row0 * p.q_stride + h * D;
 
     int nkt = (S + KT - 1) / KT;
     if (p.causal) {
@@ -431,7 +450,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
     auto make_rsrc = [&](const uint16_t* base, int64_t stride) __attribute__((always_inline)) {
         int64_t bytes = (int64_t)(S - 1) * stride * 2 + RB;
         uint32_t nrec = bytes > 0xffffffffLL ? 0xffffffffu : (uint32_t)bytes;
-        return make_rsrc_words(base + (int64_t)b * S * stride + h * D, nrec);
+        return make_rsrc_words(base + row0 * stride + h * D, nrec);
     };
     // A wave's share of a tile's transfers is all K or all V (K transfers first, then V): which one is a
     // wave-uniform choice made once, so the loop issues its transfers without a branch.
@@ -441,7 +460,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
     static_assert(TPW % KVAR == 0 && TPO % KVAR == 0 && (RPI * KVAR) % 16 == 0, "swizzle period must divide the transfer split");
     const bool isv = wave * TPW >= TPO;
     const rsrc_words rsT = isv ? make_rsrc(p.V, p.v_stride) : make_rsrc(p.K, p.k_stride);
-    const rsrc_words rsM = make_rsrc_words(p.mask ? (const void*)(p.mask + (int64_t)b * S) : (const void*)p.Q, HAS_MASK ? (uint32_t)S * 4u : 0u);
+    const rsrc_words rsM = make_rsrc_words(p.mask ? (const void*)(p.mask + row0) : (const void*)p.Q, HAS_MASK ? (uint32_t)S * 4u : 0u);
     const int stride_b = uni((int)(isv ? p.v_stride : p.k_stride) * 2);
     const int inst0 = wave * TPW - (isv ? TPO : 0);
     const int t_row = lane / NCH, t_slot = lane % NCH;
@@ -861,7 +880,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
             const int qi = qw0 + 32 * u + li;
             const float inv = 1.0f / fmaxf(halves_sum(lsum[u]), 1e-10f);
             if (qi < S) {
-                uint16_t* Og = p.O + ((int64_t)b * S + qi) * p.o_stride + h * D;
+                uint16_t* Og = p.O + (row0 + qi) * p.o_stride + h * D;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -963,7 +982,7 @@ template <int D>
 static int launch_fa16(grl_ctx* c, const FaArgs& a, int rope_q) {
     Fa16Args f{};
     f.Q = (const uint16_t*)a.Q; f.K = (const uint16_t*)a.K; f.V = (const uint16_t*)a.V;
-    f.mask = a.mask; f.O = (uint16_t*)a.O; f.rope = a.rope;
+    f.mask = a.mask; f.O = (uint16_t*)a.O; f.rope = a.rope; f.offsets = a.offsets;
     f.B = a.B; f.S = a.S; f.H = a.H; f.scale = a.scale; f.causal = a.causal;
     static const int order_env = [] { const char* e = getenv("GRL_FA_ORDER"); return e ? atoi(e) : -1; }();
     // measured: causal and short sequences do best head by head on XCD-contiguous runs; long dense sequences with
@@ -1087,7 +1106,7 @@ static unsigned fa_ew_grid(int64_t n) {
 static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
                       const void* Q, const void* K, const void* V, const float* mask, void* O,
                       int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
-                      float scale, int causal, int rope, float rope_base, float rope_scaling, void* workspace);
+                      float scale, int causal, int rope, float rope_base, float rope_scaling, void* workspace, const grl_ragged* rg = nullptr);
 
 // Any head dim from 1 to 64*NAIVE_MAX and any alignment (reference backend/attention.py:403-410 reshapes with
 // whatever head_dim it is given): up to 128 through zero-padded copies and the MFMA kernels, above through the
@@ -1095,9 +1114,10 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
 static int fa2_generic(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
                        const void* Q, const void* K, const void* V, const float* mask, void* O,
                        int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
-                       float scale, int causal, int rope, float rope_base, float rope_scaling) {
-    const int64_t es = (int64_t)grl_dtype_size(dtype), rows = B * S * H;
+                       float scale, int causal, int rope, float rope_base, float rope_scaling, const grl_ragged* rg) {
+    const int64_t es = (int64_t)grl_dtype_size(dtype), rows = (rg ? rg->rows : B * S) * H;
     if (D > 128) {
+        GRL_REQUIRE(!rg, GRL_ERR_SHAPE, "%s: a ragged batch needs head_dim <= 128 (got %lld)", who, (long long)D);
         GRL_REQUIRE(rope == GRL_ROPE_NONE, GRL_ERR_SHAPE, "%s: RoPE needs head_dim <= 128 (got %lld)", who, (long long)D);
         GRL_REQUIRE((rows + 3) / 4 < (1LL << 31), GRL_ERR_SHAPE, "%s: too many queries", who);
         FaArgs a{};
@@ -1120,8 +1140,10 @@ static int fa2_generic(grl_ctx* c, const char* who, int dtype, int64_t B, int64_
     int rc = GRL_OK;
     if (rope != GRL_ROPE_NONE) {
         GRL_REQUIRE(D % 2 == 0, GRL_ERR_SHAPE, "%s: RoPE needs an even head_dim (got %lld)", who, (long long)D);
-        rc = grl_rope_strided(c, dtype, B, S, H, D, Q, q_stride, nullptr, qr.p, rope, rope_base, rope_scaling);
-        if (!rc) rc = grl_rope_strided(c, dtype, B, S, H, D, K, k_stride, nullptr, kr.p, rope, rope_base, rope_scaling);
+        const int64_t rB = rg ? 1 : B, rS = rg ? rg->rows : S;
+        const int32_t* pos = rg ? rg->positions : nullptr;
+        rc = grl_rope_strided(c, dtype, rB, rS, H, D, Q, q_stride, pos, qr.p, rope, rope_base, rope_scaling);
+        if (!rc) rc = grl_rope_strided(c, dtype, rB, rS, H, D, K, k_stride, pos, kr.p, rope, rope_base, rope_scaling);
         if (rc) return rc;
         qs = qr.p; ks = kr.p; qst = kst = H * D;
     }
@@ -1133,7 +1155,7 @@ static int fa2_generic(grl_ctx* c, const char* who, int dtype, int64_t B, int64_
     pad(qs, qst, qp.p); pad(ks, kst, kp.p); pad(V, v_stride, vp.p);
     GRL_CHECK_LAUNCH();
     rc = fa2_common(c, who, dtype, B, S, H, DP, qp.p, kp.p, vp.p, mask, op.p, H * DP, H * DP, H * DP, H * DP, scale, causal,
-                    GRL_ROPE_NONE, rope_base, rope_scaling, nullptr);
+                    GRL_ROPE_NONE, rope_base, rope_scaling, nullptr, rg);
     if (rc) return rc;
     if (dtype == GRL_F32) hipLaunchKernelGGL(unpad_heads_kernel<float>, grid, block, 0, c->stream, (const float*)op.p, (float*)O, o_stride, rows, (int)H, (int)D, (int)DP);
     else hipLaunchKernelGGL(unpad_heads_kernel<uint16_t>, grid, block, 0, c->stream, (const uint16_t*)op.p, (uint16_t*)O, o_stride, rows, (int)H, (int)D, (int)DP);
@@ -1144,7 +1166,7 @@ static int fa2_generic(grl_ctx* c, const char* who, int dtype, int64_t B, int64_
 static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
                       const void* Q, const void* K, const void* V, const float* mask, void* O,
                       int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
-                      float scale, int causal, int rope, float rope_base, float rope_scaling, void* workspace) {
+                      float scale, int causal, int rope, float rope_base, float rope_scaling, void* workspace, const grl_ragged* rg) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "%s: null context", who);
     GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "%s: bad dtype %d", who, dtype);
     GRL_REQUIRE(rope >= GRL_ROPE_NONE && rope <= GRL_ROPE_HALF, GRL_ERR_ARG, "%s: bad rope style %d", who, rope);
@@ -1161,12 +1183,15 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
                           ((q_stride | k_stride | v_stride | o_stride) * es) % 16 == 0;
     if (!((D == 32 || D == 64 || D == 128) && granular))
         return fa2_generic(c, who, dtype, B, S, H, D, Q, K, V, mask, O, q_stride, k_stride, v_stride, o_stride, scale, causal, rope,
-                           rope_base, rope_scaling);
+                           rope_base, rope_scaling, rg);
 
     FaArgs a{};
     a.Q = Q; a.K = K; a.V = V; a.mask = mask; a.O = O;
     a.B = (int)B; a.S = (int)S; a.H = (int)H; a.scale = scale; a.causal = causal ? 1 : 0;
     a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.o_stride = o_stride;
+    if (rg) { a.offsets = rg->offsets; a.positions = rg->positions; }
+    const int64_t nrows = rg ? rg->rows : B * S;
+    const int64_t rB = rg ? 1 : B, rS = rg ? nrows : S;      // how the row-wise rotation kernels see the batch
 
     GRL_REQUIRE(S * std::max(std::max(q_stride, k_stride), std::max(v_stride, o_stride)) * es < (1LL << 31), GRL_ERR_SHAPE,
                 "%s: one batch entry must span less than 2 GiB", who);
@@ -1181,19 +1206,19 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
         rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, GRL_ROPE_HALF, &tab);
         if (rc) return rc;
         a.rope = (const float2*)tab;
-        own2 = grl_malloc(c, (size_t)B * S * H * D * 2);
+        own2 = grl_malloc(c, (size_t)nrows * H * D * 2);
         if (!own2) return GRL_ERR_OOM;
-        rc = grl_rope_half_apply_table(c, dtype, B, S, H, D, K, k_stride, own2, tab);
+        rc = grl_rope_half_apply_table(c, dtype, rB, rS, H, D, K, k_stride, own2, tab, a.positions);
         a.K = own2; a.k_stride = hd;
         rope_q = 2;
     } else if (rope == GRL_ROPE_HALF) {
         // fp32: rotate Q and K once into a workspace with the standalone kernel, then run the plain kernel on
         // the rotated copies.
-        const size_t n = (size_t)B * S * H * D, bytes = n * grl_dtype_size(dtype);
+        const size_t n = (size_t)nrows * H * D, bytes = n * grl_dtype_size(dtype);
         char* ws = (char*)workspace;
         if (!ws) { own = grl_malloc(c, 2 * bytes); if (!own) return GRL_ERR_OOM; ws = (char*)own; }
-        rc = grl_rope_strided(c, dtype, B, S, H, D, Q, q_stride, nullptr, ws, GRL_ROPE_HALF, rope_base, rope_scaling);
-        if (!rc) rc = grl_rope_strided(c, dtype, B, S, H, D, K, k_stride, nullptr, ws + bytes, GRL_ROPE_HALF, rope_base, rope_scaling);
+        rc = grl_rope_strided(c, dtype, rB, rS, H, D, Q, q_stride, a.positions, ws, GRL_ROPE_HALF, rope_base, rope_scaling);
+        if (!rc) rc = grl_rope_strided(c, dtype, rB, rS, H, D, K, k_stride, a.positions, ws + bytes, GRL_ROPE_HALF, rope_base, rope_scaling);
         a.Q = ws; a.K = ws + bytes; a.q_stride = hd; a.k_stride = hd;
     } else if (rope == GRL_ROPE_INTERLEAVED) {
         // the (S, D/2) cos/sin table lives on the context and is built once per (D, base, scaling)
@@ -1203,9 +1228,9 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
         a.rope = (const float2*)tab;
         if (dtype == GRL_BF16) {
             // every K row is rotated exactly once here; the kernel rotates Q rows as it loads them
-            own2 = grl_malloc(c, (size_t)B * S * H * D * 2);
+            own2 = grl_malloc(c, (size_t)nrows * H * D * 2);
             if (!own2) return GRL_ERR_OOM;
-            rc = grl_rope_apply_table(c, dtype, B, S, H, D, K, k_stride, own2, tab);
+            rc = grl_rope_apply_table(c, dtype, rB, rS, H, D, K, k_stride, own2, tab, a.positions);
             a.K = own2; a.k_stride = hd;
         }
     }
@@ -1236,4 +1261,13 @@ extern "C" int grl_fa2_fwd_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, 
                                    float scale, int causal, int rope, float rope_base, float rope_scaling) {
     return fa2_common(c, "grl_fa2_fwd_strided", dtype, B, S, H, D, Q, K, V, mask, O, q_stride, k_stride, v_stride,
                       o_stride, scale, causal, rope, rope_base, rope_scaling, nullptr);
+}
+
+extern "C" int grl_fa2_fwd_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t H, int64_t D,
+                                  const void* Q, const void* K, const void* V, void* O,
+                                  int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                                  float scale, int causal, int rope, float rope_base, float rope_scaling) {
+    int rc = grl_check_ragged("grl_fa2_fwd_ragged", rg);
+    return rc ? rc : fa2_common(c, "grl_fa2_fwd_ragged", dtype, rg->sequences, rg->longest, H, D, Q, K, V, nullptr, O, q_stride, k_stride, v_stride,
+                                o_stride, scale, causal, rope, rope_base, rope_scaling, nullptr, rg);
 }

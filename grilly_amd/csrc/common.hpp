@@ -50,6 +50,9 @@ int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int 
 
 void grl_set_error(const char* fmt, ...);
 
+// argument check shared by the entry points on ragged batches
+int grl_check_ragged(const char* who, const grl_ragged* rg);
+
 // one lap event behind the launches enqueued so far, when a lap trace is on (and has indices left); used by the
 // entry points that launch several kernels, so that a caller can time the launches inside them
 void grl_lap_mark(grl_ctx* c);

@@ -7,6 +7,7 @@
 // last dimension :985-995).
 #include "common.hpp"
 #include <cmath>
+#include <cstring>
 
 extern "C" int64_t grl_bert_layer_workspace(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff) {
     if (!grl_valid_dtype(dtype) || B < 0 || S < 0 || H <= 0 || D <= 0 || d_ff <= 0) return -1;
@@ -17,16 +18,27 @@ extern "C" int64_t grl_bert_layer_workspace(int dtype, int64_t B, int64_t S, int
     return pad(M * 3 * d * es) + 2 * pad(M * d * es) + pad(M * d_ff * es);
 }
 
-extern "C" int grl_bert_layer_fwd(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
-                                  const grl_bert_layer* w, const float* mask, float eps, void* x, void* workspace) {
+// attention on the packed (M, 3d) projection, of a rectangular batch (rg null) or a ragged one
+static int layer_attention(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const char* qkv, const float* mask, char* attn,
+                           const grl_ragged* rg) {
+    const int64_t d = H * D, es = (int64_t)grl_dtype_size(dtype);
+    const float scale = 1.0f / sqrtf((float)D);
+    if (rg) return grl_fa2_fwd_ragged(c, dtype, rg, H, D, qkv, qkv + d * es, qkv + 2 * d * es, attn, 3 * d, 3 * d, 3 * d, d, scale, 0,
+                                      GRL_ROPE_NONE, 10000.f, 1.f);
+    return grl_fa2_fwd_strided(c, dtype, B, S, H, D, qkv, qkv + d * es, qkv + 2 * d * es, mask, attn, 3 * d, 3 * d, 3 * d, d, scale, 0,
+                               GRL_ROPE_NONE, 10000.f, 1.f);
+}
+
+static int bert_layer(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                      const grl_bert_layer* w, const float* mask, float eps, void* x, void* workspace, const grl_ragged* rg) {
     GRL_REQUIRE(c && w && x && workspace, GRL_ERR_ARG, "grl_bert_layer_fwd: null argument");
     GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_bert_layer_fwd: bad dtype %d", dtype);
     GRL_REQUIRE(B >= 0 && S >= 0 && H > 0 && d_ff > 0, GRL_ERR_SHAPE, "grl_bert_layer_fwd: bad shape");
     GRL_REQUIRE(D >= 1 && D <= 1024, GRL_ERR_SHAPE, "grl_bert_layer_fwd: head_dim must be between 1 and 1024 (got %lld)", (long long)D);
     GRL_REQUIRE(w->w_qkv && w->w_o && w->w_ff1 && w->w_ff2 && w->ln1_g && w->ln1_b && w->ln2_g && w->ln2_b,
                 GRL_ERR_ARG, "grl_bert_layer_fwd: null weight");
-    if (B == 0 || S == 0) return GRL_OK;
-    const int64_t M = B * S, d = H * D, es = (int64_t)grl_dtype_size(dtype);
+    const int64_t M = rg ? rg->rows : B * S, d = H * D, es = (int64_t)grl_dtype_size(dtype);
+    if (M == 0) return GRL_OK;
     auto pad = [](int64_t v) { return (v + 255) / 256 * 256; };
     char* qkv = (char*)workspace;
     char* attn = qkv + pad(M * 3 * d * es);
@@ -36,8 +48,7 @@ extern "C" int grl_bert_layer_fwd(grl_ctx* c, int dtype, int64_t B, int64_t S, i
     grl_lap_mark(c);
     if ((rc = grl_gemm_nt(c, dtype, dtype, M, 3 * d, d, x, w->w_qkv, w->b_qkv, qkv, GRL_EPI_NONE))) return rc;
     grl_lap_mark(c);
-    if ((rc = grl_fa2_fwd_strided(c, dtype, B, S, H, D, qkv, qkv + d * es, qkv + 2 * d * es, mask, attn,
-                                  3 * d, 3 * d, 3 * d, d, 1.0f / sqrtf((float)D), 0, GRL_ROPE_NONE, 10000.f, 1.f))) return rc;
+    if ((rc = layer_attention(c, dtype, B, S, H, D, qkv, mask, attn, rg))) return rc;
     grl_lap_mark(c);
     if ((rc = grl_gemm_nt(c, dtype, dtype, M, d, d, attn, w->w_o, w->b_o, proj, GRL_EPI_NONE))) return rc;
     grl_lap_mark(c);
@@ -52,6 +63,16 @@ extern "C" int grl_bert_layer_fwd(grl_ctx* c, int dtype, int64_t B, int64_t S, i
     return GRL_OK;
 }
 
+extern "C" int grl_bert_layer_fwd(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                                  const grl_bert_layer* w, const float* mask, float eps, void* x, void* workspace) {
+    return bert_layer(c, dtype, B, S, H, D, d_ff, w, mask, eps, x, workspace, nullptr);
+}
+extern "C" int grl_bert_layer_fwd_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t H, int64_t D, int64_t d_ff,
+                                         const grl_bert_layer* w, float eps, void* x, void* workspace) {
+    int rc = grl_check_ragged("grl_bert_layer_fwd_ragged", rg);
+    return rc ? rc : bert_layer(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, nullptr, eps, x, workspace, rg);
+}
+
 // ---- the same layer without a LayerNorm pass: the residual stream is kept as raw rows + row statistics ----------
 extern "C" int64_t grl_bert_layer_fused_workspace(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff) {
     if (!grl_valid_dtype(dtype) || B < 0 || S < 0 || H <= 0 || D <= 0 || d_ff <= 0) return -1;
@@ -62,20 +83,20 @@ extern "C" int64_t grl_bert_layer_fused_workspace(int dtype, int64_t B, int64_t 
     return pad(M * 3 * d * es) + pad(M * d * es) + pad(M * d_ff * es) + pad(M * 8) + pad(grl_gemm_nt_resln_workspace(M, d));
 }
 
-extern "C" int grl_bert_layer_fwd_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
-                                        const grl_bert_layer_fused* w, const float* mask, float eps, void* r, float* stats,
-                                        void* workspace) {
+static int bert_layer_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                            const grl_bert_layer_fused* w, const float* mask, float eps, void* r, float* stats,
+                            void* workspace, const grl_ragged* rg) {
     GRL_REQUIRE(c && w && r && stats && workspace, GRL_ERR_ARG, "grl_bert_layer_fwd_fused: null argument");
     GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_bert_layer_fwd_fused: bad dtype %d", dtype);
     GRL_REQUIRE(B >= 0 && S >= 0 && H > 0 && d_ff > 0, GRL_ERR_SHAPE, "grl_bert_layer_fwd_fused: bad shape");
     GRL_REQUIRE(D >= 1 && D <= 1024, GRL_ERR_SHAPE, "grl_bert_layer_fwd_fused: head_dim must be between 1 and 1024 (got %lld)", (long long)D);
     GRL_REQUIRE(w->ws_qkv && w->c_qkv && w->bf_qkv && w->in_g && w->in_b && w->w_o && w->ln1_g && w->ln1_b && w->ws_ff1 && w->c_ff1 &&
                 w->bf_ff1 && w->w_ff2, GRL_ERR_ARG, "grl_bert_layer_fwd_fused: null weight");
-    const int64_t M = B * S, d = H * D, es = (int64_t)grl_dtype_size(dtype), slab = 128 / es;
+    const int64_t M = rg ? rg->rows : B * S, d = H * D, es = (int64_t)grl_dtype_size(dtype), slab = 128 / es;
     GRL_REQUIRE(d % slab == 0 && d_ff % slab == 0, GRL_ERR_SHAPE,
                 "grl_bert_layer_fwd_fused: d_model (%lld) and d_ff (%lld) must be multiples of %lld; use grl_bert_layer_fwd",
                 (long long)d, (long long)d_ff, (long long)slab);
-    if (B == 0 || S == 0) return GRL_OK;
+    if (M == 0) return GRL_OK;
     auto pad = [](int64_t v) { return (v + 255) / 256 * 256; };
     char* qkv = (char*)workspace;
     char* attn = qkv + pad(M * 3 * d * es);
@@ -86,8 +107,7 @@ extern "C" int grl_bert_layer_fwd_fused(grl_ctx* c, int dtype, int64_t B, int64_
     grl_lap_mark(c);
     if ((rc = grl_ln_gemm_nt_stats(c, dtype, dtype, M, 3 * d, d, r, w->ws_qkv, w->c_qkv, w->bf_qkv, stats, qkv, GRL_EPI_NONE))) return rc;
     grl_lap_mark(c);
-    if ((rc = grl_fa2_fwd_strided(c, dtype, B, S, H, D, qkv, qkv + d * es, qkv + 2 * d * es, mask, attn,
-                                  3 * d, 3 * d, 3 * d, d, 1.0f / sqrtf((float)D), 0, GRL_ROPE_NONE, 10000.f, 1.f))) return rc;
+    if ((rc = layer_attention(c, dtype, B, S, H, D, qkv, mask, attn, rg))) return rc;
     grl_lap_mark(c);
     if ((rc = grl_gemm_nt_resln(c, dtype, M, d, d, attn, w->w_o, w->b_o, r, stats, w->in_g, w->in_b, r, eps, stats1, part))) return rc;
     grl_lap_mark(c);
@@ -96,4 +116,74 @@ extern "C" int grl_bert_layer_fwd_fused(grl_ctx* c, int dtype, int64_t B, int64_
     if ((rc = grl_gemm_nt_resln(c, dtype, M, d, d_ff, ff, w->w_ff2, w->b_ff2, r, stats1, w->ln1_g, w->ln1_b, r, eps, stats, part))) return rc;
     grl_lap_mark(c);
     return GRL_OK;
+}
+
+extern "C" int grl_bert_layer_fwd_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                                        const grl_bert_layer_fused* w, const float* mask, float eps, void* r, float* stats,
+                                        void* workspace) {
+    return bert_layer_fused(c, dtype, B, S, H, D, d_ff, w, mask, eps, r, stats, workspace, nullptr);
+}
+extern "C" int grl_bert_layer_fwd_fused_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t H, int64_t D, int64_t d_ff,
+                                               const grl_bert_layer_fused* w, float eps, void* r, float* stats, void* workspace) {
+    int rc = grl_check_ragged("grl_bert_layer_fwd_fused_ragged", rg);
+    return rc ? rc : bert_layer_fused(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, nullptr, eps, r, stats, workspace, rg);
+}
+
+// ---- a padded batch without its padding: host side --------------------------------------------------------------
+int grl_check_ragged(const char* who, const grl_ragged* rg) {
+    GRL_REQUIRE(rg && rg->offsets && rg->positions, GRL_ERR_ARG, "%s: null ragged batch", who);
+    GRL_REQUIRE(rg->sequences >= 0 && rg->rows >= 0 && rg->longest >= 0 && rg->longest <= rg->rows && rg->rows < (1LL << 31), GRL_ERR_SHAPE,
+                "%s: bad ragged batch (sequences=%lld rows=%lld longest=%lld)", who, (long long)rg->sequences, (long long)rg->rows, (long long)rg->longest);
+    return GRL_OK;
+}
+
+template <typename M>
+static int pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const M* mask, int32_t* out, int64_t* rows, int64_t* longest) {
+    int32_t* offsets = out;
+    int32_t* positions = out + (B + 1);
+    int32_t* kept = positions + B * S;
+    int64_t n = 0, most = 0;
+    bool prefix = true;
+    const int32_t top = (int32_t)vocab;
+    bool bad_id = false, bad_mask = false;
+    for (int64_t b = 0; b < B; ++b) {
+        const int64_t first = n;
+        const int64_t* row = ids + b * S;
+        offsets[b] = (int32_t)n;
+        for (int64_t s = 0; s < S; ++s) {
+            const int32_t id = (int32_t)row[s];
+            bad_id |= (uint32_t)id >= (uint32_t)top;
+            bool keep = true;
+            if (mask) {
+                const M m = mask[b * S + s];
+                keep = m != (M)0;
+                bad_mask |= keep && m != (M)1;
+            }
+            prefix &= !keep || n - first == s;
+            positions[n] = (int32_t)s;           // overwritten by the next token when this one is not kept
+            kept[n] = id;
+            n += keep;
+        }
+        if (n - first > most) most = n - first;
+    }
+    offsets[B] = (int32_t)n;
+    if (n < B * S) memmove(positions + n, kept, (size_t)n * sizeof(int32_t));
+    *rows = n; *longest = most;
+    if (bad_id) return GRL_PACK_BAD_ID;
+    if (bad_mask) return GRL_PACK_OTHER_MASK;
+    return prefix ? GRL_PACK_PREFIX : GRL_PACK_SCATTERED;
+}
+
+extern "C" int grl_pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
+                              int32_t* out, int64_t* rows, int64_t* longest) {
+    GRL_REQUIRE(B >= 0 && S >= 0 && B * S < (1LL << 31) && vocab > 0 && vocab < (1LL << 31), GRL_ERR_SHAPE, "grl_pack_batch: bad shape");
+    GRL_REQUIRE(out && rows && longest && (B * S == 0 || ids), GRL_ERR_ARG, "grl_pack_batch: null argument");
+    switch (mask ? mask_kind : 0) {
+        case 0: return pack_batch<int64_t>(B, S, vocab, ids, nullptr, out, rows, longest);
+        case 1: return pack_batch<int64_t>(B, S, vocab, ids, (const int64_t*)mask, out, rows, longest);
+        case 2: return pack_batch<float>(B, S, vocab, ids, (const float*)mask, out, rows, longest);
+        default: break;
+    }
+    grl_set_error("grl_pack_batch: mask_kind must be 0 (none), 1 (int64) or 2 (float32)");
+    return GRL_ERR_ARG;
 }

@@ -572,9 +572,9 @@ int grl_rope_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int
                      const int32_t* position_ids, void* y, int style, float rope_base, float rope_scaling);
 int grl_build_rope_table_styled(grl_ctx* c, float* tab, int S, int D, float base, float scaling, int style);
 int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                         void* y, const float* table);
+                         void* y, const float* table, const int32_t* positions);
 int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                              void* y, const float* table);
+                              void* y, const float* table, const int32_t* positions);
 
 extern "C" int grl_rope(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x,
                         const int32_t* position_ids, void* y, int style, float rope_base, float rope_scaling) {
@@ -602,8 +602,8 @@ int grl_rope_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int
             const float* tab = nullptr;
             int rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, style, &tab);
             if (rc) return rc;
-            return style == GRL_ROPE_HALF ? grl_rope_half_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab)
-                                          : grl_rope_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab);
+            return style == GRL_ROPE_HALF ? grl_rope_half_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab, nullptr)
+                                          : grl_rope_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab, nullptr);
         }
     }
     RopeFreq fr; grl_rope_freqs(&fr, (int)D, rope_base);
@@ -669,7 +669,7 @@ int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int 
 // every row read once and written once (the K pre-rotation of the fused-RoPE attention path).
 template <typename T>
 __global__ __launch_bounds__(256) void rope_table_apply_kernel(const T* __restrict__ x, int64_t x_stride, T* __restrict__ y,
-                                                              const float2* __restrict__ tab, int64_t nchunks, int S, int H, int D) {
+                                                              const float2* __restrict__ tab, const int32_t* __restrict__ positions, int64_t nchunks, int S, int H, int D) {
     constexpr int EPC = 16 / (int)sizeof(T), PPC = EPC / 2;
     const int cpr = D / EPC;                       // chunks per (position, head) row
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -677,7 +677,7 @@ __global__ __launch_bounds__(256) void rope_table_apply_kernel(const T* __restri
         const int c = (int)(i % cpr);
         const int64_t vec = i / cpr;               // (b,s,h) flat
         const int64_t bs = vec / H;
-        const int h = (int)(vec - bs * H), s = (int)(bs % S);
+        const int h = (int)(vec - bs * H), s = positions ? positions[bs] : (int)(bs % S);
         u32x4 v = *(const u32x4*)(x + bs * x_stride + (int64_t)h * D + c * EPC);
         const float2* t = tab + (int64_t)s * (D / 2) + c * PPC;
         u32x4 o;
@@ -702,13 +702,13 @@ __global__ __launch_bounds__(256) void rope_table_apply_kernel(const T* __restri
 }
 
 int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                         void* y, const float* table) {
+                         void* y, const float* table, const int32_t* positions) {
     const int64_t epc = dtype == GRL_BF16 ? 8 : 4;
     const int64_t nchunks = B * S * H * (D / epc);
     if (nchunks == 0) return GRL_OK;
     dim3 g(ew_grid(nchunks)), b(256);
-    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_table_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, nchunks, (int)S, (int)H, (int)D);
-    else hipLaunchKernelGGL(rope_table_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, nchunks, (int)S, (int)H, (int)D);
+    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_table_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
+    else hipLaunchKernelGGL(rope_table_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
 }
@@ -717,7 +717,7 @@ int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H,
 // (position, head) row and its partner chunk D/2 further on (shaders/rope.glsl:74-125 pairs d with d + D/2).
 template <typename T>
 __global__ __launch_bounds__(256) void rope_half_apply_kernel(const T* __restrict__ x, int64_t x_stride, T* __restrict__ y,
-                                                             const float2* __restrict__ tab, int64_t nchunks, int S, int H, int D) {
+                                                             const float2* __restrict__ tab, const int32_t* __restrict__ positions, int64_t nchunks, int S, int H, int D) {
     constexpr int EPC = 16 / (int)sizeof(T);
     const int half = D / 2, cph = half / EPC;      // chunks per half row
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -725,7 +725,7 @@ __global__ __launch_bounds__(256) void rope_half_apply_kernel(const T* __restric
         const int c = (int)(i % cph);
         const int64_t vec = i / cph;               // (b,s,h) flat
         const int64_t bs = vec / H;
-        const int h = (int)(vec - bs * H), s = (int)(bs % S);
+        const int h = (int)(vec - bs * H), s = positions ? positions[bs] : (int)(bs % S);
         const T* xr = x + bs * x_stride + (int64_t)h * D + c * EPC;
         const u32x4 lo = *(const u32x4*)xr, hi = *(const u32x4*)(xr + half);
         const float2* t = tab + (int64_t)s * half + c * EPC;
@@ -754,13 +754,13 @@ __global__ __launch_bounds__(256) void rope_half_apply_kernel(const T* __restric
 }
 
 int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                              void* y, const float* table) {
+                              void* y, const float* table, const int32_t* positions) {
     const int64_t epc = dtype == GRL_BF16 ? 8 : 4;
     const int64_t nchunks = B * S * H * ((D / 2) / epc);
     if (nchunks == 0) return GRL_OK;
     dim3 g(ew_grid(nchunks)), b(256);
-    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_half_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, nchunks, (int)S, (int)H, (int)D);
-    else hipLaunchKernelGGL(rope_half_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, nchunks, (int)S, (int)H, (int)D);
+    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_half_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
+    else hipLaunchKernelGGL(rope_half_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
 }
@@ -768,14 +768,14 @@ int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64
 // ------------------------------------------------------------------ embedding gather
 template <typename T>
 __global__ __launch_bounds__(256) void embed_kernel(const int32_t* __restrict__ ids, const float* __restrict__ tok,
-                                                   const float* __restrict__ pos, const float* __restrict__ typ,
+                                                   const float* __restrict__ pos, const float* __restrict__ typ, const int32_t* __restrict__ positions,
                                                    T* __restrict__ x, int64_t rows, int S, int F, int vocab) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     int id = ids[row];
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);   // the host validates; this only keeps loads in bounds
-    const int s = (int)(row % S);
+    const int s = positions ? positions[row] : (int)(row % S);
     const float* t = tok + (int64_t)id * F;
     T* o = x + row * (int64_t)F;
     if (pos && typ) {
@@ -791,7 +791,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t* __restrict__ 
 // 16-byte streaming store), eight rows per workgroup
 template <typename T>
 __global__ __launch_bounds__(512) void embed_vec_kernel(const int32_t* __restrict__ ids, const float* __restrict__ tok,
-                                                       const float* __restrict__ pos, const float* __restrict__ typ,
+                                                       const float* __restrict__ pos, const float* __restrict__ typ, const int32_t* __restrict__ positions,
                                                        T* __restrict__ x, int64_t rows, int S, int F, int vocab) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 6);
@@ -799,7 +799,7 @@ __global__ __launch_bounds__(512) void embed_vec_kernel(const int32_t* __restric
     int id = ids[row];
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);   // the host validates; this only keeps loads in bounds
     const float* t = tok + (int64_t)id * F;
-    const float* p = pos ? pos + (int64_t)(row % S) * F : nullptr;
+    const float* p = pos ? pos + (int64_t)(positions ? positions[row] : (int32_t)(row % S)) * F : nullptr;
     T* o = x + row * (int64_t)F;
     for (int f = lane * 4; f < F; f += 256) {
         f32x4 v = *(const f32x4*)(t + f);
@@ -813,26 +813,43 @@ __global__ __launch_bounds__(512) void embed_vec_kernel(const int32_t* __restric
     }
 }
 
-extern "C" int grl_embed(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, int64_t vocab, const int32_t* ids,
-                         const float* tok_emb, const float* pos_emb, const float* type_emb, void* x) {
-    GRL_REQUIRE(c && ids && tok_emb && x, GRL_ERR_ARG, "grl_embed: null argument");
-    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_embed: bad dtype %d", dtype);
-    GRL_REQUIRE(B >= 0 && S > 0 && F > 0 && vocab > 0 && S < (1LL << 31) && F < (1LL << 31) && vocab < (1LL << 31),
-                GRL_ERR_SHAPE, "grl_embed: bad shape");
-    int64_t rows = B * S;
+// positions: the row of the position table for each row (a ragged batch); null: row index modulo S
+static int embed_rows(grl_ctx* c, int dtype, int64_t rows, int64_t S, int64_t F, int64_t vocab, const int32_t* ids, const int32_t* positions,
+                      const float* tok_emb, const float* pos_emb, const float* type_emb, void* x) {
     if (rows == 0) return GRL_OK;
     if (F % 4 == 0 && aligned16(tok_emb) && aligned16(x) && (!pos_emb || aligned16(pos_emb)) && (!type_emb || aligned16(type_emb))) {
         dim3 g8((unsigned)((rows + 7) / 8)), b8(512);
-        if (dtype == GRL_F32) hipLaunchKernelGGL(embed_vec_kernel<float>, g8, b8, 0, c->stream, ids, tok_emb, pos_emb, type_emb, (float*)x, rows, (int)S, (int)F, (int)vocab);
-        else hipLaunchKernelGGL(embed_vec_kernel<uint16_t>, g8, b8, 0, c->stream, ids, tok_emb, pos_emb, type_emb, (uint16_t*)x, rows, (int)S, (int)F, (int)vocab);
+        if (dtype == GRL_F32) hipLaunchKernelGGL(embed_vec_kernel<float>, g8, b8, 0, c->stream, ids, tok_emb, pos_emb, type_emb, positions, (float*)x, rows, (int)S, (int)F, (int)vocab);
+        else hipLaunchKernelGGL(embed_vec_kernel<uint16_t>, g8, b8, 0, c->stream, ids, tok_emb, pos_emb, type_emb, positions, (uint16_t*)x, rows, (int)S, (int)F, (int)vocab);
         GRL_CHECK_LAUNCH();
         return GRL_OK;
     }
     dim3 g((unsigned)((rows + 3) / 4)), b(256);
-    if (dtype == GRL_F32) hipLaunchKernelGGL(embed_kernel<float>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, (float*)x, rows, (int)S, (int)F, (int)vocab);
-    else hipLaunchKernelGGL(embed_kernel<uint16_t>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, (uint16_t*)x, rows, (int)S, (int)F, (int)vocab);
+    if (dtype == GRL_F32) hipLaunchKernelGGL(embed_kernel<float>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, positions, (float*)x, rows, (int)S, (int)F, (int)vocab);
+    else hipLaunchKernelGGL(embed_kernel<uint16_t>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, positions, (uint16_t*)x, rows, (int)S, (int)F, (int)vocab);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
+}
+
+static int check_embed(const char* who, grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, int64_t vocab, const int32_t* ids, const float* tok_emb, const void* x) {
+    GRL_REQUIRE(c && ids && tok_emb && x, GRL_ERR_ARG, "%s: null argument", who);
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "%s: bad dtype %d", who, dtype);
+    GRL_REQUIRE(B >= 0 && S > 0 && F > 0 && vocab > 0 && S < (1LL << 31) && F < (1LL << 31) && vocab < (1LL << 31),
+                GRL_ERR_SHAPE, "%s: bad shape", who);
+    return GRL_OK;
+}
+
+extern "C" int grl_embed(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, int64_t vocab, const int32_t* ids,
+                         const float* tok_emb, const float* pos_emb, const float* type_emb, void* x) {
+    int rc = check_embed("grl_embed", c, dtype, B, S, F, vocab, ids, tok_emb, x);
+    return rc ? rc : embed_rows(c, dtype, B * S, S, F, vocab, ids, nullptr, tok_emb, pos_emb, type_emb, x);
+}
+
+extern "C" int grl_embed_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t F, int64_t vocab, const int32_t* ids,
+                                const float* tok_emb, const float* pos_emb, const float* type_emb, void* x) {
+    int rc = grl_check_ragged("grl_embed_ragged", rg);
+    if (!rc) rc = check_embed("grl_embed_ragged", c, dtype, rg->sequences, 1, F, vocab, ids, tok_emb, x);
+    return rc ? rc : embed_rows(c, dtype, rg->rows, 1, F, vocab, ids, rg->positions, tok_emb, pos_emb, type_emb, x);
 }
 
 // Embedding gather and the LayerNorm that follows it in one pass: a wave gathers its row (token + type + position, in
@@ -840,7 +857,7 @@ extern "C" int grl_embed(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F,
 // (two-pass mean / variance like layernorm_rows_kernel).  F % 4 == 0, F <= 2048, 16-byte aligned tables.
 template <typename T>
 __global__ __launch_bounds__(256) void embed_layernorm_kernel(const int32_t* __restrict__ ids, const float* __restrict__ tok,
-                                                             const float* __restrict__ pos, const float* __restrict__ typ,
+                                                             const float* __restrict__ pos, const float* __restrict__ typ, const int32_t* __restrict__ positions,
                                                              const float* __restrict__ gamma, const float* __restrict__ beta,
                                                              T* __restrict__ x, int64_t rows, int S, int F, int vocab, float eps) {
     constexpr int MAXC = 8;
@@ -850,7 +867,7 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(const int32_t* __r
     int id = ids[row];
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);   // the host validates; this only keeps loads in bounds
     const float* tr = tok + (int64_t)id * F;
-    const float* pr = pos ? pos + (int64_t)(row % S) * F : nullptr;
+    const float* pr = pos ? pos + (int64_t)(positions ? positions[row] : (int32_t)(row % S)) * F : nullptr;
     const int nch = F >> 2;
     float t[MAXC][4];
     float s = 0.f;
@@ -899,42 +916,59 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(const int32_t* __r
 extern "C" int grl_layernorm(grl_ctx* c, int dtype, int64_t rows, int64_t F, const void* x, const void* residual,
                              const float* gamma, const float* beta, float eps, void* y);
 
-extern "C" int grl_embed_layernorm(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, int64_t vocab, const int32_t* ids,
-                                   const float* tok_emb, const float* pos_emb, const float* type_emb,
-                                   const float* gamma, const float* beta, float eps, void* x) {
-    GRL_REQUIRE(c && ids && tok_emb && gamma && beta && x, GRL_ERR_ARG, "grl_embed_layernorm: null argument");
-    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_embed_layernorm: bad dtype %d", dtype);
-    GRL_REQUIRE(B >= 0 && S > 0 && F > 0 && vocab > 0 && S < (1LL << 31) && F < (1LL << 31) && vocab < (1LL << 31),
-                GRL_ERR_SHAPE, "grl_embed_layernorm: bad shape");
-    const int64_t rows = B * S;
+static int embed_layernorm_rows(grl_ctx* c, int dtype, int64_t rows, int64_t S, int64_t F, int64_t vocab, const int32_t* ids, const int32_t* positions,
+                                const float* tok_emb, const float* pos_emb, const float* type_emb,
+                                const float* gamma, const float* beta, float eps, void* x) {
     if (rows == 0) return GRL_OK;
     const bool fused = F % 4 == 0 && F <= 2048 && aligned16(tok_emb) && aligned16(x) && aligned16(gamma) && aligned16(beta) &&
                        (!pos_emb || aligned16(pos_emb)) && (!type_emb || aligned16(type_emb));
     if (!fused) {
-        int rc = grl_embed(c, dtype, B, S, F, vocab, ids, tok_emb, pos_emb, type_emb, x);
+        int rc = embed_rows(c, dtype, rows, S, F, vocab, ids, positions, tok_emb, pos_emb, type_emb, x);
         return rc ? rc : grl_layernorm(c, dtype, rows, F, x, nullptr, gamma, beta, eps, x);
     }
     dim3 g((unsigned)((rows + 3) / 4)), b(256);
-    if (dtype == GRL_F32) hipLaunchKernelGGL(embed_layernorm_kernel<float>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, gamma, beta, (float*)x, rows, (int)S, (int)F, (int)vocab, eps);
-    else hipLaunchKernelGGL(embed_layernorm_kernel<uint16_t>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, gamma, beta, (uint16_t*)x, rows, (int)S, (int)F, (int)vocab, eps);
+    if (dtype == GRL_F32) hipLaunchKernelGGL(embed_layernorm_kernel<float>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, positions, gamma, beta, (float*)x, rows, (int)S, (int)F, (int)vocab, eps);
+    else hipLaunchKernelGGL(embed_layernorm_kernel<uint16_t>, g, b, 0, c->stream, ids, tok_emb, pos_emb, type_emb, positions, gamma, beta, (uint16_t*)x, rows, (int)S, (int)F, (int)vocab, eps);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
+}
+
+extern "C" int grl_embed_layernorm(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, int64_t vocab, const int32_t* ids,
+                                   const float* tok_emb, const float* pos_emb, const float* type_emb,
+                                   const float* gamma, const float* beta, float eps, void* x) {
+    int rc = check_embed("grl_embed_layernorm", c, dtype, B, S, F, vocab, ids, tok_emb, x);
+    if (rc) return rc;
+    GRL_REQUIRE(gamma && beta, GRL_ERR_ARG, "grl_embed_layernorm: null argument");
+    return embed_layernorm_rows(c, dtype, B * S, S, F, vocab, ids, nullptr, tok_emb, pos_emb, type_emb, gamma, beta, eps, x);
+}
+
+extern "C" int grl_embed_layernorm_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t F, int64_t vocab, const int32_t* ids,
+                                          const float* tok_emb, const float* pos_emb, const float* type_emb,
+                                          const float* gamma, const float* beta, float eps, void* x) {
+    int rc = grl_check_ragged("grl_embed_layernorm_ragged", rg);
+    if (!rc) rc = check_embed("grl_embed_layernorm_ragged", c, dtype, rg->sequences, 1, F, vocab, ids, tok_emb, x);
+    if (rc) return rc;
+    GRL_REQUIRE(gamma && beta, GRL_ERR_ARG, "grl_embed_layernorm_ragged: null argument");
+    return embed_layernorm_rows(c, dtype, rg->rows, 1, F, vocab, ids, rg->positions, tok_emb, pos_emb, type_emb, gamma, beta, eps, x);
 }
 
 // ------------------------------------------------------------------ masked mean pool (+ L2 normalise)
 // grid (ceil(F/256), B).  F % 4 == 0: a lane owns 4 adjacent features (8- or 16-byte loads), the NW waves
 // of a workgroup take every NW-th position of the sequence and their partial sums meet in LDS (sixteen waves: a
 // batch of 128 sequences is only a few hundred workgroups, and the loads in flight per CU are what the rate hangs on).
+// offsets: first row of each sequence of a ragged batch, of which the first `limit` rows are averaged; null: S rows each.
 template <typename T, int NW>
-__global__ __launch_bounds__(NW * 64) void mean_pool_kernel(const T* __restrict__ x, const float* __restrict__ mask,
-                                                           float* __restrict__ out, int S, int F) {
+__global__ __launch_bounds__(NW * 64) void mean_pool_kernel(const T* __restrict__ x, const float* __restrict__ mask, const int32_t* __restrict__ offsets,
+                                                           float* __restrict__ out, int S, int F, int limit) {
     __shared__ float part[NW][256];
     __shared__ float cpart[NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int f0 = blockIdx.x * 256 + lane * 4;
     const int64_t b = blockIdx.y;
     float a[4] = {0.f, 0.f, 0.f, 0.f}, cnt = 0.f;
-    const T* xb = x + b * S * (int64_t)F + f0;
+    const int64_t row0 = offsets ? offsets[b] : b * S;
+    if (offsets) { S = offsets[b + 1] - (int)row0; S = S < limit ? S : limit; }
+    const T* xb = x + row0 * F + f0;
     const bool live = f0 < F;
 #pragma unroll 8
     for (int s = wave; s < S; s += NW) {
@@ -961,16 +995,18 @@ __global__ __launch_bounds__(NW * 64) void mean_pool_kernel(const T* __restrict_
 
 // any F: thread f sums its feature over the sequence (coalesced across f)
 template <typename T>
-__global__ __launch_bounds__(256) void mean_pool_generic_kernel(const T* __restrict__ x, const float* __restrict__ mask,
-                                                               float* __restrict__ out, int S, int F) {
+__global__ __launch_bounds__(256) void mean_pool_generic_kernel(const T* __restrict__ x, const float* __restrict__ mask, const int32_t* __restrict__ offsets,
+                                                               float* __restrict__ out, int S, int F, int limit) {
     const int f = blockIdx.x * 256 + threadIdx.x;
     const int64_t b = blockIdx.y;
     if (f >= F) return;
+    const int64_t row0 = offsets ? offsets[b] : b * S;
+    if (offsets) { S = offsets[b + 1] - (int)row0; S = S < limit ? S : limit; }
     float acc = 0.f, cnt = 0.f;
     for (int s = 0; s < S; ++s) {
         float m = mask ? mask[b * S + s] : 1.0f;
         cnt += m;
-        acc += m * elem<T>::ld(x + (b * S + s) * (int64_t)F + f);
+        acc += m * elem<T>::ld(x + (row0 + s) * (int64_t)F + f);
     }
     out[b * F + f] = acc / fmaxf(cnt, 1e-9f);
 }
@@ -987,21 +1023,18 @@ __global__ __launch_bounds__(256) void l2_normalize_kernel(float* __restrict__ v
     for (int f = threadIdx.x; f < F; f += 256) r[f] = r[f] / n;
 }
 
-extern "C" int grl_mean_pool(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, const void* x,
-                             const float* mask, float* out, int l2_normalize) {
-    GRL_REQUIRE(c && x && out, GRL_ERR_ARG, "grl_mean_pool: null argument");
-    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_mean_pool: bad dtype %d", dtype);
-    GRL_REQUIRE(B >= 0 && B < 65536 && S > 0 && F > 0 && S < (1LL << 31) && F < (1LL << 31), GRL_ERR_SHAPE, "grl_mean_pool: bad shape");
+static int mean_pool_any(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, const void* x, const float* mask, const int32_t* offsets,
+                         int limit, float* out, int l2_normalize) {
     if (B == 0) return GRL_OK;
     constexpr int PW = 16;                                  // waves per workgroup of the vector kernel
     dim3 g((unsigned)((F + 255) / 256), (unsigned)B), b(256), bv(PW * 64);
     const bool vec = F % 4 == 0 && aligned16(x);
     if (dtype == GRL_F32) {
-        if (vec) hipLaunchKernelGGL((mean_pool_kernel<float, PW>), g, bv, 0, c->stream, (const float*)x, mask, out, (int)S, (int)F);
-        else hipLaunchKernelGGL(mean_pool_generic_kernel<float>, g, b, 0, c->stream, (const float*)x, mask, out, (int)S, (int)F);
+        if (vec) hipLaunchKernelGGL((mean_pool_kernel<float, PW>), g, bv, 0, c->stream, (const float*)x, mask, offsets, out, (int)S, (int)F, limit);
+        else hipLaunchKernelGGL(mean_pool_generic_kernel<float>, g, b, 0, c->stream, (const float*)x, mask, offsets, out, (int)S, (int)F, limit);
     } else {
-        if (vec) hipLaunchKernelGGL((mean_pool_kernel<uint16_t, PW>), g, bv, 0, c->stream, (const uint16_t*)x, mask, out, (int)S, (int)F);
-        else hipLaunchKernelGGL(mean_pool_generic_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, mask, out, (int)S, (int)F);
+        if (vec) hipLaunchKernelGGL((mean_pool_kernel<uint16_t, PW>), g, bv, 0, c->stream, (const uint16_t*)x, mask, offsets, out, (int)S, (int)F, limit);
+        else hipLaunchKernelGGL(mean_pool_generic_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, mask, offsets, out, (int)S, (int)F, limit);
     }
     GRL_CHECK_LAUNCH();
     if (l2_normalize) {
@@ -1009,6 +1042,25 @@ extern "C" int grl_mean_pool(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_
         GRL_CHECK_LAUNCH();
     }
     return GRL_OK;
+}
+
+extern "C" int grl_mean_pool(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t F, const void* x,
+                             const float* mask, float* out, int l2_normalize) {
+    GRL_REQUIRE(c && x && out, GRL_ERR_ARG, "grl_mean_pool: null argument");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_mean_pool: bad dtype %d", dtype);
+    GRL_REQUIRE(B >= 0 && B < 65536 && S > 0 && F > 0 && S < (1LL << 31) && F < (1LL << 31), GRL_ERR_SHAPE, "grl_mean_pool: bad shape");
+    return mean_pool_any(c, dtype, B, S, F, x, mask, nullptr, 0, out, l2_normalize);
+}
+
+extern "C" int grl_mean_pool_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t F, const void* x, int64_t first, float* out,
+                                    int l2_normalize) {
+    int rc = grl_check_ragged("grl_mean_pool_ragged", rg);
+    if (rc) return rc;
+    GRL_REQUIRE(c && x && out, GRL_ERR_ARG, "grl_mean_pool_ragged: null argument");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_mean_pool_ragged: bad dtype %d", dtype);
+    GRL_REQUIRE(rg->sequences < 65536 && F > 0 && F < (1LL << 31) && first >= 0, GRL_ERR_SHAPE, "grl_mean_pool_ragged: bad shape");
+    return mean_pool_any(c, dtype, rg->sequences, rg->longest, F, x, nullptr, rg->offsets, first > 0 && first < rg->longest ? (int)first : (int)rg->longest,
+                         out, l2_normalize);
 }
 
 // ------------------------------------------------------------------ 2-D transpose (for gemm_nn)

@@ -63,8 +63,63 @@ def random_bert_weights(cfg, seed=0, std=0.02):
     return w
 
 
+def _token_ids(input_ids):
+    """ids as a contiguous int64 array, wrapped to 32 bits the way a cast to the kernels' int32 would"""
+    ids = np.ascontiguousarray(input_ids)
+    return ids if ids.dtype == np.int64 else ids.astype(np.int32, copy=False).astype(np.int64)
+
+
+class _Packing:
+    """What forward() makes of ids and mask in one native pass (grl_pack_batch): the real tokens' offsets, positions and
+    ids, how many there are, and whether they form a batch without padding or one whose padding can be left out."""
+    __slots__ = ("kind", "data", "B", "S", "rows", "longest")
+
+    def __init__(self, lib, input_ids, attention_mask, vocab):
+        ids = _token_ids(input_ids)
+        if ids.ndim != 2:
+            raise ValueError("input_ids must be (batch, seq_len)")
+        B, S = ids.shape
+        mask, kind = None, 0
+        if attention_mask is not None:
+            mask = np.asarray(attention_mask)
+            mask = np.ascontiguousarray(mask, dtype=np.int64 if mask.dtype == np.int64 else np.float32)
+            kind = 1 if mask.dtype == np.int64 else 2
+            if mask.shape != (B, S):
+                raise ValueError("attention_mask must be (batch, seq_len)")
+        self.B, self.S = B, S
+        self.data = np.empty(B + 1 + 2 * B * S, np.int32)
+        rows, longest = ctypes.c_int64(), ctypes.c_int64()
+        self.kind = lib.grl_pack_batch(B, S, vocab, ids.ctypes.data, mask.ctypes.data if kind else None, kind, self.data.ctypes.data,
+                                       ctypes.byref(rows), ctypes.byref(longest))
+        if self.kind == L.PACK_BAD_ID:
+            raise IndexError("token id out of range")      # numpy indexing in the reference raises IndexError
+        if self.kind < 0:
+            L.check(self.kind, "pack_batch")
+        self.rows, self.longest = rows.value, longest.value
+
+    @property
+    def full(self):
+        """no padding at all: a rectangular batch that needs no mask"""
+        return self.kind == L.PACK_PREFIX and self.rows == self.B * self.S
+
+    def ids(self):
+        return self.data[self.B + 1 + self.rows:self.B + 1 + 2 * self.rows]
+
+    def upload(self, core, dst):
+        """offsets | positions | ids to the device in one transfer -> (ragged batch, device address of the ids)"""
+        n = self.B + 1 + 2 * self.rows
+        L.check(core.lib.grl_h2d(core.ctx, dst, self.data.ctypes.data, n * 4), "upload packed batch")
+        positions = dst + 4 * (self.B + 1)
+        return L.Ragged(dst, positions, self.B, self.rows, self.longest), positions + 4 * self.rows
+
+
 class BertEncoder:
-    """fused=None (default): both LayerNorms of every layer are folded into the GEMMs around them whenever the
+    """forward(pool=True) leaves the padding of a batch out: the real tokens are stored back to back and every kernel sees
+    those rows only (no result depends on a padded position: it is masked as a key and left out of the mean).  The batch
+    keeps its rectangular form where hidden states come back (pool=False), where a mask holds other values than 0 and 1, and
+    in bf16 where tokens are masked in front of or between kept ones.
+
+    fused=None (default): both LayerNorms of every layer are folded into the GEMMs around them whenever the
     direct-to-LDS GEMM kernels take the layer's shapes (d_model and d_ff multiples of 64 in bf16, 32 in fp32) and the
     batch has at least FUSED_MIN_ROWS token rows: the residual stream then travels as raw rows plus row statistics and
     no LayerNorm pass runs over HBM between the embedding and the final LayerNorm (grl_bert_layer_fwd_fused).  Smaller
@@ -139,12 +194,13 @@ class BertEncoder:
             raise ValueError(f"sequence length {S} exceeds max_pos {cfg.max_pos}")
         es = 2 if self.code == L.GRL_BF16 else 4
         self.fused_now = self.fused and B * S >= self._fused_min_rows        # which layer form this batch runs
-        wsfn = c.lib.grl_bert_layer_fused_workspace if self.fused_now else c.lib.grl_bert_layer_workspace
-        ws = wsfn(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff)
+        ws = c.lib.grl_bert_layer_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff)
+        if self.fused_now:                   # without its padding the batch may run either form
+            ws = max(ws, c.lib.grl_bert_layer_fused_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff))
         self.x = c.alloc(B * S * cfg.d_model * es)
         self.stats = c.alloc(max(B * S, 1) * 8)        # {1/sd, mean/sd} per row of the raw residual stream (fused layers)
         self.ws = c.alloc(ws)
-        self.ids = c.alloc(B * S * 4)
+        self.ids = c.alloc((B + 1 + 2 * B * S) * 4)    # token ids, or offsets | positions | ids of the batch without its padding
         self.mask = c.alloc(B * S * 4)
         self.pooled = c.alloc(B * cfg.d_model * 4)
         self._shape = (B, S)
@@ -171,6 +227,13 @@ class BertEncoder:
             if m.shape != (B, S):
                 raise ValueError("attention_mask must be (batch, seq_len)")
             L.check(c.lib.grl_h2d(c.ctx, self.mask.ptr, m.ctypes.data, m.nbytes), "upload mask")
+
+    def _set_full(self, p):
+        """set_inputs for a batch without padding (a mask of ones changes nothing)"""
+        self.prepare(p.B, p.S)
+        ids = p.ids()
+        L.check(self.core.lib.grl_h2d(self.core.ctx, self.ids.ptr, ids.ctypes.data, ids.nbytes), "upload ids")
+        self.has_mask = False
 
     def launch(self, pool=True):
         """Enqueue one full forward on the context stream (no host synchronisation)."""
@@ -199,10 +262,44 @@ class BertEncoder:
         if pool:
             L.check(lib.grl_mean_pool(c.ctx, self.code, B, S, cfg.d_model, self.x.ptr, mask, self.pooled.ptr, 1), "mean_pool")
 
+    def _launch_packed(self, rg, ids):
+        """launch() on the batch without its padding, always pooled"""
+        cfg, c, lib = self.cfg, self.core, self.core.lib
+        r = ctypes.byref(rg)
+        if self.fused and rg.rows >= self._fused_min_rows and rg.rows > 0:
+            L.check(lib.grl_embed_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
+                                         self.x.ptr), "embedding")
+            L.check(lib.grl_ln_stats(c.ctx, self.code, rg.rows, cfg.d_model, self.x.ptr, cfg.embedding_eps, self.stats.ptr), "embedding statistics")
+            for f in self.fused_structs:
+                L.check(lib.grl_bert_layer_fwd_fused_ragged(c.ctx, self.code, r, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f), cfg.eps,
+                                                            self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layer_fwd_fused")
+            last = self.layer_structs[-1]
+            L.check(lib.grl_layernorm(c.ctx, self.code, rg.rows, cfg.d_model, self.x.ptr, None, last.ln2_g, last.ln2_b, cfg.eps,
+                                      self.x.ptr), "final layernorm")
+        else:
+            L.check(lib.grl_embed_layernorm_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
+                                                   self.emb_g.ptr, self.emb_b.ptr, cfg.embedding_eps, self.x.ptr), "embedding + layernorm")
+            for s in self.layer_structs:
+                L.check(lib.grl_bert_layer_fwd_ragged(c.ctx, self.code, r, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(s), cfg.eps,
+                                                      self.x.ptr, self.ws.ptr), "bert_layer_fwd")
+        L.check(lib.grl_mean_pool_ragged(c.ctx, self.code, r, cfg.d_model, self.x.ptr, 0, self.pooled.ptr, 1), "mean_pool")
+
     def forward(self, input_ids, attention_mask=None, pool=True):
         """pool=True -> L2-normalised mean-pooled embeddings (B, d); False -> hidden states (B,S,d)."""
-        self.set_inputs(input_ids, attention_mask)
-        self.launch(pool)
+        p = _Packing(self.core.lib, input_ids, attention_mask, self.cfg.vocab)
+        # Padding on the right leaves every key in the attention tile it has in the rectangular batch, so pooled embeddings
+        # agree with the mean of pool=False's hidden states to the last bits.  Tokens kept elsewhere move to other tiles,
+        # where bf16 rounds the softmax weights against another reference (1e-3 measured): fp32 only.
+        packs = p.kind == L.PACK_PREFIX or (p.kind == L.PACK_SCATTERED and self.code == L.GRL_F32)
+        if pool and packs and not p.full and self.cfg.head_dim <= 128:
+            self.prepare(p.B, p.S)
+            self._launch_packed(*p.upload(self.core, self.ids.ptr))
+        else:
+            if p.full:
+                self._set_full(p)
+            else:
+                self.set_inputs(input_ids, attention_mask)
+            self.launch(pool)
         B, S = self._shape
         if pool:
             return self.core.download(self.pooled, (B, self.cfg.d_model))
@@ -334,7 +431,7 @@ class PreNormEncoder:
             self.part = c.alloc(int(c.lib.grl_gemm_nt_resln_workspace(B * S, cfg.d_model)))
         self.qkv = c.alloc(3 * act)                    # packed (M, 3d): Q, K, V are its three column blocks
         self.h = c.alloc(B * S * cfg.d_ff * es)
-        self.ids = c.alloc(B * S * 4)
+        self.ids = c.alloc((B + 1 + 2 * B * S) * 4)    # token ids, or offsets | positions | ids of the batch without its padding
         self.mask = c.alloc(B * S * 4)
         first = np.zeros((B, S), np.float32)
         first[:, 0] = 1.0                              # "mean" over the first token only = that token
@@ -368,24 +465,37 @@ class PreNormEncoder:
                 raise ValueError("attention_mask must be (batch, seq_len)")
             L.check(c.lib.grl_h2d(c.ctx, self.mask.ptr, m.ctypes.data, m.nbytes), "upload mask")
 
+    _set_full = BertEncoder._set_full
+
     def launch(self, pool=True):
         """Enqueue one full forward on the context stream (no host synchronisation)."""
+        self._launch(pool, None, self.ids.ptr)
+
+    def _launch(self, pool, rg, ids):
+        """rg: the batch without its padding (pool is then True), or None for the rectangular one"""
         B, S = self._shape
         cfg, c, lib, code = self.cfg, self.core, self.core.lib, self.code
-        M, d, ff, H, D = B * S, cfg.d_model, cfg.d_ff, cfg.heads, cfg.head_dim
+        M, d, ff, H, D = B * S if rg is None else rg.rows, cfg.d_model, cfg.d_ff, cfg.heads, cfg.head_dim
         es = 2 if code == L.GRL_BF16 else 4
-        mask = self.mask.ptr if self.has_mask else None
-        L.check(lib.grl_embed_layernorm(c.ctx, code, B, S, d, cfg.vocab, self.ids.ptr, self.tok.ptr, None, None,
-                                        self.emb_g.ptr, self.emb_b.ptr, cfg.emb_eps, self.x.ptr), "embedding + layernorm")
+        if rg is None:
+            mask = self.mask.ptr if self.has_mask else None
+            L.check(lib.grl_embed_layernorm(c.ctx, code, B, S, d, cfg.vocab, ids, self.tok.ptr, None, None,
+                                            self.emb_g.ptr, self.emb_b.ptr, cfg.emb_eps, self.x.ptr), "embedding + layernorm")
+        else:
+            L.check(lib.grl_embed_layernorm_ragged(c.ctx, code, ctypes.byref(rg), d, cfg.vocab, ids, self.tok.ptr, None, None,
+                                                   self.emb_g.ptr, self.emb_b.ptr, cfg.emb_eps, self.x.ptr), "embedding + layernorm")
         for w in self.layers:
             # one GEMM with the packed weight; attention reads Q, K, V as column blocks of its output and applies
             # the rotation itself (queries as they are loaded, keys once per row from the cached table)
             L.check(lib.grl_gemm_nt(c.ctx, code, code, M, 3 * d, d, self.x.ptr, w["w_qkv"].ptr, w["b_qkv"].ptr,
                                     self.qkv.ptr, L.EPI_NONE), "q/k/v projection")
-            L.check(lib.grl_fa2_fwd_strided(c.ctx, code, B, S, H, D, self.qkv.ptr, self.qkv.ptr + d * es,
-                                            self.qkv.ptr + 2 * d * es, mask, self.att.ptr, 3 * d, 3 * d, 3 * d, d,
-                                            1.0 / float(np.sqrt(D)), 0, L.ROPE_HALF, cfg.rope_base, cfg.rope_scaling),
-                    "attention")
+            q, k, v, scale = self.qkv.ptr, self.qkv.ptr + d * es, self.qkv.ptr + 2 * d * es, 1.0 / float(np.sqrt(D))
+            if rg is None:
+                L.check(lib.grl_fa2_fwd_strided(c.ctx, code, B, S, H, D, q, k, v, mask, self.att.ptr, 3 * d, 3 * d, 3 * d, d, scale, 0,
+                                                L.ROPE_HALF, cfg.rope_base, cfg.rope_scaling), "attention")
+            else:
+                L.check(lib.grl_fa2_fwd_ragged(c.ctx, code, ctypes.byref(rg), H, D, q, k, v, self.att.ptr, 3 * d, 3 * d, 3 * d, d, scale, 0,
+                                               L.ROPE_HALF, cfg.rope_base, cfg.rope_scaling), "attention")
             # LayerNorm + dual GEMM; the dual GEMM activates its second ("up") operand: that is the first half of Wi here
             if self.stats_from_gemm:
                 L.check(lib.grl_gemm_nt_resln(c.ctx, code, M, d, d, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,
@@ -405,13 +515,24 @@ class PreNormEncoder:
         if self.final is not None:
             L.check(lib.grl_layernorm(c.ctx, code, M, d, self.x.ptr, None, self.final[0].ptr, self.final[1].ptr,
                                       cfg.final_eps, self.x.ptr), "final layernorm")
-        if pool:
+        if rg is not None:
+            L.check(lib.grl_mean_pool_ragged(c.ctx, code, ctypes.byref(rg), d, self.x.ptr, 1, self.pooled.ptr, 1), "first-token pool")
+        elif pool:
             L.check(lib.grl_mean_pool(c.ctx, code, B, S, d, self.x.ptr, self.first.ptr, self.pooled.ptr, 1), "first-token pool")
 
     def forward(self, input_ids, attention_mask=None, pool=True):
-        """pool=True -> L2-normalised first-token embeddings (B, d); False -> hidden states (B,S,d)."""
-        self.set_inputs(input_ids, attention_mask)
-        self.launch(pool)
+        """pool=True -> L2-normalised first-token embeddings (B, d); False -> hidden states (B,S,d).  Pooled batches padded
+        on the right run without their padding, as in BertEncoder (the first token has to be a real one)."""
+        p = _Packing(self.core.lib, input_ids, attention_mask, self.cfg.vocab)
+        if pool and not p.full and p.kind == L.PACK_PREFIX and (p.data[1:p.B + 1] > p.data[:p.B]).all():
+            self.prepare(p.B, p.S)
+            self._launch(True, *p.upload(self.core, self.ids.ptr))
+        else:
+            if p.full and p.S > 0:
+                self._set_full(p)
+            else:
+                self.set_inputs(input_ids, attention_mask)
+            self.launch(pool)
         B, S = self._shape
         if pool:
             return self.core.download(self.pooled, (B, self.cfg.d_model))

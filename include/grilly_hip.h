@@ -353,6 +353,43 @@ int grl_embed_layernorm(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t F
 int grl_mean_pool(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t F, const void* x,
                   const float* mask, float* out, int l2_normalize);
 
+/* ---- ragged batches: sequences of unequal length stored back to back ------------------------------------------
+ * The padding of a batch is work nobody asks for when only pooled embeddings come back: a padded position is masked out
+ * as a key and left out of the mean, so no result depends on it.  A ragged batch holds the real tokens only, sequence after
+ * sequence; row-wise kernels and GEMMs see `rows` rows, attention and pooling find their sequence through `offsets`.
+ * offsets (sequences + 1) and positions (rows; each row's position in its sequence, for the position table and the rotary
+ * angle) are device arrays; the counts are host values, longest = the longest sequence.  No counterpart in the reference,
+ * which computes the padding.  Same arithmetic as the rectangular entry points with a 0 / 1 mask. */
+typedef struct grl_ragged {
+    const int32_t* offsets;
+    const int32_t* positions;
+    int64_t sequences, rows, longest;
+} grl_ragged;
+
+/* Host side of it: token ids (B,S) int64 and a mask (mask_kind 0 none, 1 int64, 2 float32) -> out = offsets (B+1), then
+ * positions (*rows), then the kept token ids as int32 (*rows); room for B+1 + 2*B*S values.  Returns one of the following
+ * (out is good in the first two cases) or a negative grl_status. */
+enum { GRL_PACK_PREFIX = 0,      /* every sequence keeps its first tokens (padding on the right, or none) */
+       GRL_PACK_SCATTERED = 1,   /* tokens are kept elsewhere too */
+       GRL_PACK_OTHER_MASK = 2,  /* some mask value is neither 0 nor 1 */
+       GRL_PACK_BAD_ID = 3 };    /* some token id, kept or not, lies outside [0, vocab) */
+int grl_pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
+                   int32_t* out, int64_t* rows, int64_t* longest);
+int grl_embed_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t F, int64_t vocab, const int32_t* ids,
+                     const float* tok_emb, const float* pos_emb, const float* type_emb, void* x);
+int grl_embed_layernorm_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t F, int64_t vocab, const int32_t* ids,
+                               const float* tok_emb, const float* pos_emb, const float* type_emb,
+                               const float* gamma, const float* beta, float eps, void* x);
+/* grl_fa2_fwd_strided on a ragged batch: queries attend to the keys of their own sequence.  Head dims up to 128; with RoPE
+ * the rows of a sequence stand at positions 0, 1, 2 ... */
+int grl_fa2_fwd_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D,
+                       const void* Q, const void* K, const void* V, void* O,
+                       int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride,
+                       float scale, int causal, int rope, float rope_base, float rope_scaling);
+/* mean of each sequence's rows (first > 0: of its first `first` rows), zeros for an empty one; out fp32 (sequences, F) */
+int grl_mean_pool_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t F, const void* x, int64_t first,
+                         float* out, int l2_normalize);
+
 /* ---- one post-LN BERT encoder layer, device resident ----------------------------------------
  * x <- LN(x + Wo.Attn(QKV(x); mask) + bo; g1,b1,eps); x <- LN(x + W2.gelu(W1.x+b1)+b2; g2,b2,eps)
  * Replaces VulkanSentenceTransformer._forward_layer, BERT branch
@@ -372,6 +409,9 @@ int64_t grl_bert_layer_workspace(int dtype, int64_t B, int64_t S, int64_t H, int
 int grl_bert_layer_fwd(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
                        int64_t d_ff, const grl_bert_layer* w, const float* mask, float eps,
                        void* x, void* workspace);
+/* the same on a ragged batch (workspace as for B*S = rows) */
+int grl_bert_layer_fwd_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
+                              const grl_bert_layer* w, float eps, void* x, void* workspace);
 
 /* The same layer with both LayerNorms folded into the GEMMs around them: no LayerNorm pass over HBM.  The residual
  * stream travels as RAW rows r plus their statistics: on entry r holds the rows whose LayerNorm (in_g, in_b, statistics
@@ -397,6 +437,8 @@ int64_t grl_bert_layer_fused_workspace(int dtype, int64_t B, int64_t S, int64_t 
 int grl_bert_layer_fwd_fused(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
                              int64_t d_ff, const grl_bert_layer_fused* w, const float* mask, float eps,
                              void* r, float* stats, void* workspace);
+int grl_bert_layer_fwd_fused_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
+                                    const grl_bert_layer_fused* w, float eps, void* r, float* stats, void* workspace);
 
 #ifdef __cplusplus
 }
