@@ -61,6 +61,13 @@ SIGNATURES = {
     "grl_pool_trim": (c_int, [c_void_p]),
     "grl_h2d": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t]),
     "grl_d2h": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t]),
+    "grl_upload": (c_int, [c_void_p, c_int, c_i64, c_void_p, c_void_p]),
+    "grl_download": (c_int, [c_void_p, c_int, c_i64, c_void_p, c_void_p]),
+    "grl_host_linear": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 4 + [c_int, c_float, c_float]),
+    "grl_host_glu": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 8 + [c_int]),
+    "grl_host_fa2": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64] + [c_void_p] * 5 + [c_float, c_int, c_int, c_float, c_float]),
+    "grl_host_alloc": (c_void_p, [c_size_t]),
+    "grl_host_free": (None, [c_void_p]),
     "grl_d2d": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t]),
     "grl_memset": (c_int, [c_void_p, c_void_p, c_int, c_size_t]),
     "grl_sync": (c_int, [c_void_p]),

@@ -9,7 +9,7 @@ lower-triangular rule (keys after the query are excluded, shaders/attention-mask
 import numpy as np
 
 from .. import _lib as L
-from .core import dtype_code
+from .core import dtype_code, host_f32, result_array
 
 _ROPE = {None: L.ROPE_NONE, "none": L.ROPE_NONE, "interleaved": L.ROPE_INTERLEAVED, "half": L.ROPE_HALF}
 
@@ -45,19 +45,13 @@ class HipAttention:
         if rope not in _ROPE:
             raise ValueError("rope_style must be 'interleaved' or 'half'")
         c = self.core
-        es = 2 if code == L.GRL_BF16 else 4
-        dq, dk, dv = c.upload(q, code), c.upload(k, code), c.upload(v, code)
-        dm = c.upload(mask) if mask is not None else None
-        do = c.alloc(max(q.size, 1) * es)
-        try:
-            L.check(c.lib.grl_fa2_fwd(c.ctx, code, B, S, num_heads, head_dim, dq.ptr, dk.ptr, dv.ptr,
-                                      dm.ptr if dm else None, do.ptr, float(scale), int(bool(causal)), _ROPE[rope],
-                                      float(rope_base), float(rope_scaling), None), "fa2_fwd")
-            return c.download(do, (B, S, num_heads, head_dim), code)
-        finally:
-            for b in (dq, dk, dv, dm, do):
-                if b is not None:
-                    b.free()
+        q, k, v = host_f32(q), host_f32(k), host_f32(v)
+        mask = None if mask is None else host_f32(mask)
+        o = result_array(c.lib, (B, S, num_heads, head_dim))
+        L.check(c.lib.grl_host_fa2(c.ctx, code, B, S, num_heads, head_dim, q.ctypes.data, k.ctypes.data, v.ctypes.data,
+                                   None if mask is None else mask.ctypes.data, o.ctypes.data, float(scale), int(bool(causal)), _ROPE[rope],
+                                   float(rope_base), float(rope_scaling)), "fa2_fwd")
+        return o
 
     def attention_with_weights(self, queries, keys, values, scale=None, mask=None):
         """Attention that also returns the softmax weights, for key / value sequences of any length: queries

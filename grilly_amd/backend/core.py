@@ -23,6 +23,38 @@ def dtype_size(code):
     return 2 if code == L.GRL_BF16 else 4
 
 
+def host_f32(a):
+    """a C-contiguous float32 array of a's values (a itself where it is one)"""
+    return np.ascontiguousarray(a, dtype=np.float32)
+
+
+class _ResultBlock:
+    """a block of pinned memory that a result array stands in; given back when the array (and every view of it) is gone"""
+    __slots__ = ("lib", "ptr", "__array_interface__")
+
+    def __init__(self, lib, ptr, shape):
+        self.lib, self.ptr = lib, ptr
+        self.__array_interface__ = {"shape": shape, "typestr": "<f4", "data": (ptr, False), "version": 3}
+
+    def __del__(self):
+        self.lib.grl_host_free(self.ptr)
+
+
+RESULT_BLOCK_MIN = 1 << 20      # smaller results: numpy's own memory, which the allocator has at hand
+
+
+def result_array(lib, shape):
+    """uninitialised float32 array for a result: from about 1 MiB on in recycled pinned memory, as long as there is some"""
+    nbytes = 4
+    for n in shape:
+        nbytes *= int(n)
+    if nbytes >= RESULT_BLOCK_MIN:
+        ptr = lib.grl_host_alloc(nbytes)
+        if ptr:
+            return np.asarray(_ResultBlock(lib, ptr, tuple(int(n) for n in shape)))
+    return np.empty(shape, dtype=np.float32)
+
+
 class DeviceBuffer:
     """A pool-owned device allocation; returned to the pool by free() or when collected."""
     __slots__ = ("core", "ptr", "nbytes", "__weakref__")
@@ -95,15 +127,10 @@ class HipCore:
 
     def upload(self, arr, code=L.GRL_F32):
         """numpy (any dtype, any strides) -> fresh device buffer holding fp32 or bf16 values.
-        bf16 is produced on the device from the fp32 upload (round to nearest even)."""
+        bf16 is rounded (to nearest even) on the way."""
         a = np.ascontiguousarray(arr, dtype=np.float32)
-        buf = self.alloc(a.nbytes)
-        L.check(self.lib.grl_h2d(self.ctx, buf.ptr, a.ctypes.data, a.nbytes), "upload")
-        if code == L.GRL_BF16:
-            half = self.alloc(a.size * 2)
-            L.check(self.lib.grl_cast(self.ctx, L.GRL_F32, L.GRL_BF16, a.size, buf.ptr, half.ptr), "cast")
-            buf.free()
-            return half
+        buf = self.alloc(a.size * dtype_size(code))
+        L.check(self.lib.grl_upload(self.ctx, code, a.size, a.ctypes.data, buf.ptr), "upload")
         return buf
 
     def upload_raw(self, arr):
@@ -116,15 +143,8 @@ class HipCore:
     def download(self, buf, shape, code=L.GRL_F32):
         """device buffer of fp32 or bf16 values -> fresh C-contiguous float32 numpy array."""
         n = int(np.prod(shape)) if len(shape) else 1
-        out = np.empty(shape, dtype=np.float32)
-        if n == 0:
-            return out
-        if code == L.GRL_BF16:
-            with self.alloc(n * 4) as full:
-                L.check(self.lib.grl_cast(self.ctx, L.GRL_BF16, L.GRL_F32, n, buf.ptr, full.ptr), "cast")
-                L.check(self.lib.grl_d2h(self.ctx, out.ctypes.data, full.ptr, n * 4), "download")
-        else:
-            L.check(self.lib.grl_d2h(self.ctx, out.ctypes.data, buf.ptr, n * 4), "download")
+        out = result_array(self.lib, shape)
+        L.check(self.lib.grl_download(self.ctx, code, n, buf.ptr, out.ctypes.data), "download")
         return out
 
     def sync(self):

@@ -10,7 +10,7 @@ device raises.
 import numpy as np
 
 from .. import _lib as L
-from .core import dtype_code
+from .core import dtype_code, host_f32, result_array
 
 
 class _PoolView:
@@ -82,17 +82,11 @@ class HipFNN:
         if bias is not None and np.asarray(bias).size != N:
             raise ValueError(f"bias has {np.asarray(bias).size} elements, expected {N}")
         c = self.core
-        dx, dw = c.upload(x2, code), c.upload(W, code)
-        db = c.upload(np.asarray(bias).reshape(-1)) if bias is not None else None
-        dy = c.alloc(M * N * (2 if code == L.GRL_BF16 else 4))
-        try:
-            L.check(c.lib.grl_gemm_nt_act(c.ctx, code, code, M, N, K, dx.ptr, dw.ptr, db.ptr if db else None, dy.ptr, epi,
-                                          float(alpha), float(beta)), "gemm_nt")
-            return c.download(dy, (M, N), code)
-        finally:
-            for b in (dx, dw, db, dy):
-                if b is not None:
-                    b.free()
+        x2, W, b = host_f32(x2), host_f32(W), None if bias is None else host_f32(bias)
+        y = result_array(c.lib, (M, N))
+        L.check(c.lib.grl_host_linear(c.ctx, code, M, N, K, x2.ctypes.data, W.ctypes.data, None if b is None else b.ctypes.data,
+                                      y.ctypes.data, epi, float(alpha), float(beta)), "gemm_nt")
+        return y
 
     def linear(self, x, weights, bias=None, dtype="fp32"):
         """y = x.W^T + b (reference backend/fnn.py:1394-1496).  Leading dimensions of x are kept
@@ -231,26 +225,16 @@ class HipFNN:
         x2 = _as2d(x, K)
         M = x2.shape[0]
         c = self.core
-        es = 2 if code == L.GRL_BF16 else 4
-        dx, dg, du = c.upload(x2, code), c.upload(Wg, code), c.upload(Wu, code)
+        x2, Wg, Wu = host_f32(x2), host_f32(Wg), host_f32(Wu)
         both = b_gate is not None and b_up is not None
-        dbg = c.upload(np.asarray(b_gate).reshape(-1)) if both else None
-        dbu = c.upload(np.asarray(b_up).reshape(-1)) if both else None
-        dy = c.alloc(M * N * es)
-        cg = c.alloc(M * N * 4) if return_cache else None
-        cu = c.alloc(M * N * 4) if return_cache else None
-        try:
-            L.check(c.lib.grl_glu_nt(c.ctx, code, code, M, N, K, dx.ptr, dg.ptr, du.ptr,
-                                     dbg.ptr if dbg else None, dbu.ptr if dbu else None, dy.ptr,
-                                     cg.ptr if cg else None, cu.ptr if cu else None, act), "glu_nt")
-            out = c.download(dy, (M, N), code)
-            if return_cache:
-                return out, c.download(cg, (M, N)), c.download(cu, (M, N))
-            return out
-        finally:
-            for b in (dx, dg, du, dbg, dbu, dy, cg, cu):
-                if b is not None:
-                    b.free()
+        bg, bu = (host_f32(b_gate), host_f32(b_up)) if both else (None, None)
+        if both and min(bg.size, bu.size) < N:
+            raise ValueError(f"biases have {bg.size} and {bu.size} elements, expected {N}")
+        out = result_array(c.lib, (M, N))
+        cg, cu = (result_array(c.lib, (M, N)), result_array(c.lib, (M, N))) if return_cache else (None, None)
+        at = lambda a: None if a is None else a.ctypes.data
+        L.check(c.lib.grl_host_glu(c.ctx, code, M, N, K, at(x2), at(Wg), at(Wu), at(bg), at(bu), at(out), at(cg), at(cu), act), "glu_nt")
+        return (out, cg, cu) if return_cache else out
 
     # ------------------------------------------------------------------ row / element kernels
     def layernorm(self, x, gamma=None, beta=None, eps=1e-5, dtype="fp32"):

@@ -12,6 +12,14 @@
 
 // ---------------------------------------------------------------- context
 #define GRL_MAX_LAPS 256
+// several device arrays filled from one pinned slab by one kernel
+struct grl_segments {
+    struct { const void* src; void* dst; int64_t bytes; } s[8];      // all 16-byte aligned; dst blocks are whole 16-byte units
+    int count = 0;
+};
+struct grl_hostpipe;
+grl_hostpipe* grl_hostpipe_create();
+void grl_hostpipe_destroy(grl_hostpipe* h);
 struct grl_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -38,7 +46,7 @@ struct grl_ctx {
     std::mutex stage_mu;
     char* stage = nullptr;
     size_t stage_cap = 0, stage_off = 0;
-    bool stage_failed = false;          // pinned allocation refused once: stay on the blocking path
+    grl_hostpipe* hostpipe = nullptr;   // what calls on large host arrays keep (hostcall.hip)
     // shader-clock probe (grl_clock_probe_begin / _end): its own stream, so that it runs beside the work it observes
     hipStream_t probe_stream = nullptr;
     uint64_t* probe_out = nullptr;      // device: {shader cycles, 100 MHz ticks}

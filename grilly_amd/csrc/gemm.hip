@@ -89,6 +89,12 @@ extern "C" int grl_gemm_nt_act(grl_ctx* c, int in_dtype, int out_dtype, int64_t 
     return gemm_nt_act_impl(c, in_dtype, out_dtype, M, N, K, A, W, bias, C, epilogue, alpha, beta, true);
 }
 
+// a block of the rows of a larger product (hostcall.hip): the K loop is left whole, so a result does not depend on the blocks
+int grl_gemm_nt_act_block(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, void* C,
+                          int epilogue, float alpha, float beta) {
+    return gemm_nt_act_impl(c, dtype, dtype, M, N, K, A, W, bias, C, epilogue, alpha, beta, false);
+}
+
 extern "C" int grl_gemm_nt_res(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K,
                                const void* A, const void* W, const float* bias, const void* residual, void* C) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "grl_gemm_nt_res: null context");

@@ -507,6 +507,47 @@ int grl_copy_kernel_launch(grl_ctx* c, void* dst, const void* src, size_t bytes)
     return GRL_OK;
 }
 
+// any size and alignment; for the small copies to and from pinned host memory that run as kernels
+__global__ __launch_bounds__(256) void copy_bytes_kernel(const unsigned char* __restrict__ src, unsigned char* __restrict__ dst, int64_t n, bool vec) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+    const int64_t n16 = vec ? n >> 4 : 0;
+    for (int64_t k = i; k < n16; k += stride) ((u32x4*)dst)[k] = ((const u32x4*)src)[k];
+    for (int64_t k = (n16 << 4) + i; k < n; k += stride) dst[k] = src[k];
+}
+
+// a chunk from or to pinned host memory, on any stream: 64 workgroups keep PCIe busy and leave the other CUs to the work beside it
+int grl_copy_chunk_launch(hipStream_t s, void* dst, const void* src, size_t bytes) {
+    const bool vec = ((((uintptr_t)dst) | ((uintptr_t)src)) & 15u) == 0;
+    hipLaunchKernelGGL(copy_bytes_kernel, dim3(64), dim3(256), 0, s, (const unsigned char*)src, (unsigned char*)dst, (int64_t)bytes, vec);
+    GRL_CHECK_LAUNCH();
+    return GRL_OK;
+}
+
+int grl_copy_bytes_launch(grl_ctx* c, void* dst, const void* src, size_t bytes) {
+    const bool vec = ((((uintptr_t)dst) | ((uintptr_t)src)) & 15u) == 0;
+    const int64_t items = (int64_t)(vec ? (bytes + 15) / 16 : bytes), blocks = (items + 255) / 256;
+    hipLaunchKernelGGL(copy_bytes_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024)), dim3(256), 0, c->stream, (const unsigned char*)src,
+                       (unsigned char*)dst, (int64_t)bytes, vec);
+    GRL_CHECK_LAUNCH();
+    return GRL_OK;
+}
+
+__global__ __launch_bounds__(256) void copy_segments_kernel(grl_segments g) {
+    const u32x4* src = (const u32x4*)g.s[blockIdx.y].src;
+    u32x4* dst = (u32x4*)g.s[blockIdx.y].dst;
+    const int64_t n16 = (g.s[blockIdx.y].bytes + 15) >> 4, stride = (int64_t)gridDim.x * 256;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n16; k += stride) dst[k] = src[k];
+}
+
+int grl_copy_segments_launch(grl_ctx* c, const grl_segments& g) {
+    int64_t most = 0;
+    for (int i = 0; i < g.count; ++i) if (g.s[i].bytes > most) most = g.s[i].bytes;
+    const int64_t blocks = (most + 4095) / 4096;
+    hipLaunchKernelGGL(copy_segments_kernel, dim3((unsigned)(blocks < 256 ? blocks : 256), (unsigned)g.count), dim3(256), 0, c->stream, g);
+    GRL_CHECK_LAUNCH();
+    return GRL_OK;
+}
+
 // ------------------------------------------------------------------ casts
 template <typename S, typename D>
 __global__ __launch_bounds__(256) void cast_kernel(const S* __restrict__ s, D* __restrict__ d, int64_t n) {

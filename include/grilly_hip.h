@@ -97,6 +97,15 @@ int   grl_pool_trim(grl_ctx* ctx);     /* return cached blocks to the driver */
  * grl_sync replaces vkQueueWaitIdle (backend/core.py:418). */
 int grl_h2d(grl_ctx* ctx, void* dst_dev, const void* src_host, size_t bytes);
 int grl_d2h(grl_ctx* ctx, void* dst_host, const void* src_dev, size_t bytes);
+/* fp32 values on the host <-> a device array of `dtype` (bf16: rounded to nearest even on the way in), with the ordering of
+ * grl_h2d and grl_d2h. */
+int grl_upload(grl_ctx* ctx, int dtype, int64_t n, const float* src_host, void* dst_dev);
+int grl_download(grl_ctx* ctx, int dtype, int64_t n, const void* src_dev, float* dst_host);
+/* Pinned host memory for large results, recycled and bounded (512 MiB in all, NULL beyond that or when the driver refuses):
+ * results written to it leave the device in one direct transfer.  grl_host_free gives a block back for reuse.  Both belong
+ * to the process, not to a context; any thread may call them. */
+void* grl_host_alloc(size_t bytes);
+void  grl_host_free(void* ptr);
 int grl_d2d(grl_ctx* ctx, void* dst_dev, const void* src_dev, size_t bytes);
 int grl_memset(grl_ctx* ctx, void* dst_dev, int byte, size_t bytes);
 int grl_sync(grl_ctx* ctx);
@@ -249,6 +258,18 @@ int grl_fa2_fwd_strided(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H
 int grl_rope(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
              const void* x, const int32_t* position_ids, void* y,
              int style, float rope_base, float rope_scaling);
+
+/* ---- the same operators on host arrays ------------------------------------------------------------------------------
+ * fp32 arrays in host memory in, fp32 arrays in host memory out, `dtype` the storage type on the device: what the numpy
+ * methods of the package call.  Blocks until the result is there.  Large calls overlap the transfer of a block of rows
+ * (sequences, for attention) in either direction with the work on others; one large call of a context runs at a time.
+ * Arguments otherwise as grl_gemm_nt_act, grl_glu_nt and grl_fa2_fwd. */
+int grl_host_linear(grl_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, const float* x, const float* W, const float* bias,
+                    float* y, int epilogue, float alpha, float beta);
+int grl_host_glu(grl_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, const float* x, const float* W_gate, const float* W_up,
+                 const float* b_gate, const float* b_up, float* out, float* gate_cache, float* up_cache, int activation);
+int grl_host_fa2(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const float* Q, const float* K, const float* V,
+                 const float* mask, float* O, float scale, int causal, int rope, float rope_base, float rope_scaling);
 
 /* ---- bandwidth-bound row / element kernels ------------------------------------------
  * y = gamma*(t-mean)/sqrt(var+eps)+beta per row of F features, t = x (+ residual if given),
