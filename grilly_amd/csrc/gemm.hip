@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void bias_residual_kernel(OutT* C, const OutT*
 // instead of sharing it out through a pool buffer)
 static int gemm_nt_act_impl(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K,
                             const void* A, const void* W, const float* bias, void* C, int epilogue,
-                            float alpha, float beta, bool may_allocate) {
+                            float alpha, float beta, bool may_allocate, int64_t plan_rows = 0) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "grl_gemm_nt: null context");
     GRL_REQUIRE(grl_valid_dtype(in_dtype) && grl_valid_dtype(out_dtype), GRL_ERR_ARG, "grl_gemm_nt: bad dtype");
     GRL_REQUIRE(epilogue >= GRL_EPI_NONE && epilogue <= GRL_EPI_ROSWISH, GRL_ERR_ARG, "grl_gemm_nt: bad epilogue %d", epilogue);
@@ -70,7 +70,7 @@ static int gemm_nt_act_impl(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, 
     a.A = A; a.W = W; a.bias = bias; a.C = C;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
     a.act = epilogue; a.alpha = alpha; a.beta = beta;
-    a.no_alloc = !may_allocate;
+    a.no_alloc = !may_allocate; a.plan_rows = (int)plan_rows;
     const int epi = epilogue <= GRL_EPI_SILU ? epilogue : EPI_RT;
     if (K == 0) {
         int64_t total = M * N;
@@ -89,10 +89,11 @@ extern "C" int grl_gemm_nt_act(grl_ctx* c, int in_dtype, int out_dtype, int64_t 
     return gemm_nt_act_impl(c, in_dtype, out_dtype, M, N, K, A, W, bias, C, epilogue, alpha, beta, true);
 }
 
-// a block of the rows of a larger product (hostcall.hip): the K loop is left whole, so a result does not depend on the blocks
-int grl_gemm_nt_act_block(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, void* C,
-                          int epilogue, float alpha, float beta) {
-    return gemm_nt_act_impl(c, dtype, dtype, M, N, K, A, W, bias, C, epilogue, alpha, beta, false);
+// a block of the rows of a product of `rows` rows (hostcall.hip): the K loop is left whole and its slabs are added in the order of
+// the whole product, so a result does not depend on the blocks
+int grl_gemm_nt_act_block(grl_ctx* c, int dtype, int64_t rows, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias,
+                          void* C, int epilogue, float alpha, float beta) {
+    return gemm_nt_act_impl(c, dtype, dtype, M, N, K, A, W, bias, C, epilogue, alpha, beta, false, rows);
 }
 
 extern "C" int grl_gemm_nt_res(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K,
@@ -123,9 +124,9 @@ extern "C" int grl_gemm_nt(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, i
     return grl_gemm_nt_act(c, in_dtype, out_dtype, M, N, K, A, W, bias, C, epilogue, 1.0f, 1.0f);
 }
 
-extern "C" int grl_glu_nt(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K,
-                          const void* x, const void* W_gate, const void* W_up, const float* b_gate,
-                          const float* b_up, void* out, float* gate_cache, float* up_cache, int activation) {
+static int glu_nt_impl(grl_ctx* c, int in_dtype, int out_dtype, int64_t rows, int64_t M, int64_t N, int64_t K,
+                       const void* x, const void* W_gate, const void* W_up, const float* b_gate,
+                       const float* b_up, void* out, float* gate_cache, float* up_cache, int activation) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "grl_glu_nt: null context");
     GRL_REQUIRE(grl_valid_dtype(in_dtype) && grl_valid_dtype(out_dtype), GRL_ERR_ARG, "grl_glu_nt: bad dtype");
     GRL_REQUIRE(activation == GRL_EPI_SILU || activation == GRL_EPI_RELU || activation == GRL_EPI_GELU, GRL_ERR_ARG,
@@ -140,8 +141,20 @@ extern "C" int grl_glu_nt(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, in
     if (b_gate && b_up) { a.bias = b_gate; a.bias2 = b_up; }
     a.cache1 = gate_cache; a.cache2 = up_cache;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
-    a.act = activation;
+    a.act = activation; a.plan_rows = (int)rows;
     return dispatch_types(c, a, in_dtype, out_dtype, EPI_GLU);
+}
+
+extern "C" int grl_glu_nt(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K,
+                          const void* x, const void* W_gate, const void* W_up, const float* b_gate,
+                          const float* b_up, void* out, float* gate_cache, float* up_cache, int activation) {
+    return glu_nt_impl(c, in_dtype, out_dtype, 0, M, N, K, x, W_gate, W_up, b_gate, b_up, out, gate_cache, up_cache, activation);
+}
+
+// as grl_gemm_nt_act_block
+int grl_glu_nt_block(grl_ctx* c, int dtype, int64_t rows, int64_t M, int64_t N, int64_t K, const void* x, const void* W_gate, const void* W_up,
+                     const float* b_gate, const float* b_up, void* out, float* gate_cache, float* up_cache, int activation) {
+    return glu_nt_impl(c, dtype, dtype, rows, M, N, K, x, W_gate, W_up, b_gate, b_up, out, gate_cache, up_cache, activation);
 }
 
 int grl_ln_stats(grl_ctx* c, int dtype, int64_t rows, int64_t F, const void* x, float eps, float* stats);

@@ -57,6 +57,7 @@ struct GemmArgs {
     // slabs of tile x and writes its raw fp32 sums to kpart[y]; gemm_splitk_finish_kernel adds the shares and runs the epilogue
     int ksplit;              // number of shares (grid.y)
     float* kpart;            // (ksplit, M, N) fp32
+    int plan_rows;           // host side: rows of the product this launch computes a block of (0: it is the whole product), see gemm_kernel_of_block
     bool no_alloc;           // host side: the caller must not touch the buffer pool (split K takes its buffer there): no split
 };
 
@@ -106,6 +107,9 @@ __device__ __forceinline__ void glu_apply4(float (&gate)[4], float (&up)[4], con
 #pragma unroll
     for (int e = 0; e < 4; ++e) gate[e] *= up[e];
 }
+
+// at most N vector memory operations of this wave outstanding (they retire in issue order)
+template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 // ---- one 128-byte-per-row K slab on the matrix cores --------------------------------------
 template <typename T> struct MfmaSlab;
@@ -517,6 +521,190 @@ __global__ __launch_bounds__(256) void gemm_splitk_finish_kernel(GemmArgs p) {
 }
 
 // =====================================================================================
+// Small products: the four waves of a workgroup share out the K slabs of one tile.
+//
+//   Wave w multiplies slabs w, w + 4, ... of the whole BM x BN tile out of a ring of NSTG LDS stages of its own, which
+//   it fills itself (buffer_load ... lds, the image and swizzle of the kernel below): no barrier and no wait on another
+//   wave inside the K loop, a quarter of the serial chain, and NSTG slabs per wave on their way at any time.  The four
+//   partial tiles meet in LDS (each wave's goes where its ring was) and 256 threads add them in a fixed order, run the
+//   epilogue and store whole row segments.
+// =====================================================================================
+template <typename T, typename OutT, int BM, int BN, int NSTG, int EPI, bool DUAL, bool LN = false, bool SPLITK = false>
+__global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {
+    static_assert(!SPLITK || (!DUAL && !LN), "split K: plain single-weight products only (the epilogue runs in the finishing kernel)");
+    constexpr int TM = BM / 32, TN = BN / 32;
+    constexpr int BNO = DUAL ? BN / 2 : BN;
+    constexpr int STAGE = (BM + BN) * 128, RING = NSTG * STAGE;
+    constexpr int GA = BM / 8, GB = BN / 8, LPS = GA + GB;      // transfers per slab
+    static_assert(BM * BN * 4 <= RING, "a wave's partial tile takes the place of its ring");
+    static_assert(LPS * NSTG < 64, "the memory counter holds the ring");
+    static_assert(!DUAL || BN % 64 == 0, "a 32-row block holds rows of one weight");
+    __shared__ __attribute__((aligned(1024))) char lds[4 * RING];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lg = lane >> 5;
+
+    // workgroup -> tile: a contiguous run per XCD, bands of 8 tile-rows (as in the kernels above and below)
+    int m0, n0;
+    {
+        const int nb = gridDim.x, pid = blockIdx.x;
+        const int per = nb >> 3, rem = nb & 7, xcd = pid & 7, loc = pid >> 3;
+        const int npid = xcd * per + (xcd < rem ? xcd : rem) + loc;
+        const int width = 8 * p.tiles_n;
+        const int first_m = (npid / width) * 8;
+        const int gsize = p.tiles_m - first_m < 8 ? p.tiles_m - first_m : 8;
+        m0 = (first_m + (npid % width) % gsize) * BM;
+        n0 = ((npid % width) / gsize) * BNO;
+    }
+    const int rowbytes = p.K * (int)sizeof(T);
+    auto make_rsrc = [&](const void* base, int first_row, int rows_total) {
+        int64_t left = (int64_t)(rows_total - first_row) * rowbytes;
+        if (left < 0) left = 0;
+        const uint32_t nrec = left > 0xffffffffLL ? 0xffffffffu : (uint32_t)left;
+        return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)base + (int64_t)first_row * rowbytes), 0, (int)nrec, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rsA = make_rsrc(p.A, m0, p.M);
+    const __amdgpu_buffer_rsrc_t rsW = make_rsrc(p.W, n0, p.N);
+    const __amdgpu_buffer_rsrc_t rsW2 = make_rsrc(DUAL ? p.W2 : p.W, n0, p.N);
+    const int lr = lane >> 3, ls = lane & 7;
+    const int lane_off_p[2] = {lr * rowbytes + ((ls ^ lds_swz<8>(lr)) << 4), lr * rowbytes + ((ls ^ lds_swz<8>(8 + lr)) << 4)};
+    char* const ring = lds + wave * RING;
+    auto issue = [&](int kt, char* st) {
+        const int sbyte = kt * 128;
+#pragma unroll
+        for (int j = 0; j < GA; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (__attribute__((address_space(3))) void*)(st + j * 1024), 16,
+                                                     lane_off_p[j & 1] + j * 8 * rowbytes, sbyte, 0, 0);
+#pragma unroll
+        for (int j = 0; j < GB; ++j) {
+            const bool second = DUAL && j * 8 >= BNO;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(second ? rsW2 : rsW, (__attribute__((address_space(3))) void*)(st + BM * 128 + j * 1024), 16,
+                                                     lane_off_p[j & 1] + (second ? j * 8 - BNO : j * 8) * rowbytes, sbyte, 0, 0);
+        }
+    };
+
+    const int KT = p.K / (128 / (int)sizeof(T));
+    int kt0 = 0, kt1 = KT;
+    if constexpr (SPLITK) {                       // this workgroup's share of the slabs (the host leaves no share empty)
+        const int per = (KT + p.ksplit - 1) / p.ksplit;
+        kt0 = (int)blockIdx.y * per;
+        kt1 = kt0 + per < KT ? kt0 + per : KT;
+    }
+    const int mine = kt1 - kt0 > wave ? (kt1 - kt0 - wave + 3) >> 2 : 0;      // slabs of this wave
+    kt0 += wave;
+#pragma unroll
+    for (int i = 0; i < NSTG; ++i)
+        if (i < mine) issue(kt0 + 4 * i, ring + i * STAGE);
+
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+
+    char* st = ring;
+    for (int i = 0; i < mine; ++i) {
+        const int behind = mine - 1 - i;          // slabs of this wave requested after slab i
+        if (behind >= NSTG - 1) wait_vmcnt<(NSTG - 1) * LPS>();
+        else if (NSTG > 2 && behind == NSTG - 2) wait_vmcnt<(NSTG - 2) * LPS>();
+        else wait_vmcnt<0>();
+        u32x4 xf[2][TM], wf[2][TN];
+        auto load_frags = [&](int sl) {
+            const int off = li * 128 + (((2 * sl + lg) ^ lds_swz<8>(li)) << 4);      // the swizzle repeats every 16 rows
+#pragma unroll
+            for (int a = 0; a < TM; ++a) xf[sl & 1][a] = *(const u32x4*)(st + a * 4096 + off);
+#pragma unroll
+            for (int b = 0; b < TN; ++b) wf[sl & 1][b] = *(const u32x4*)(st + BM * 128 + b * 4096 + off);
+        };
+        load_frags(0);
+#pragma unroll
+        for (int sl = 0; sl < 4; ++sl) {
+            if (sl + 1 < 4) load_frags(sl + 1);
+            else {
+                // the stage has been read: request the slab that takes its place under the last products
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (i + NSTG < mine) issue(kt0 + 4 * (i + NSTG), st);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<TM>([&](auto ia) {
+                static_for<TN>([&](auto ib) {
+                    MfmaSlab<T>::run(wf[sl & 1][decltype(ib)::value], xf[sl & 1][decltype(ia)::value], acc[decltype(ia)::value][decltype(ib)::value]);
+                });
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        st += STAGE;
+        if (st == ring + RING) st = ring;
+    }
+
+    // partial tile -> LDS, fp32 rows of BN values in 16-byte chunks, chunk c of row m at slot c ^ (m mod chunks per row)
+    constexpr int CPR = BN / 4;
+    static_for<TM>([&](auto ia) {
+        static_for<TN>([&](auto ib) {
+            static_for<4>([&](auto iq) {
+                constexpr int a = decltype(ia)::value, b = decltype(ib)::value, q = decltype(iq)::value;
+                const int c = b * 8 + 2 * q + lg;
+                const f32x4 v = {acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+                *(f32x4*)(ring + (a * 32 + li) * BN * 4 + ((c ^ (li & (CPR - 1))) << 4)) = v;
+            });
+        });
+    });
+    __syncthreads();
+
+    constexpr int QPR = BNO / 4;                  // outputs per row in groups of four
+    static_assert(BM * QPR % 256 == 0 && 256 % QPR == 0, "a thread keeps its columns");
+    const int cq = tid % QPR, n = n0 + cq * 4;
+    if (n >= p.N) return;                         // N is a multiple of 4
+    auto col4 = [&](const float* v) { return v ? *(const f32x4*)(v + n) : f32x4{0.f, 0.f, 0.f, 0.f}; };
+    f32x4 b1 = {0.f, 0.f, 0.f, 0.f}, b2 = b1, c1 = b1, c2 = b1;
+    if constexpr (!SPLITK) {
+        b1 = col4(p.bias);
+        if constexpr (DUAL) b2 = col4(p.bias2);
+        if constexpr (LN) { c1 = col4(p.ln_c); if constexpr (DUAL) c2 = col4(p.ln_c2); }
+    }
+#pragma unroll
+    for (int i = 0; i < BM * QPR / 256; ++i) {
+        const int r = i * (256 / QPR) + tid / QPR, m = m0 + r;
+        if (m >= p.M) break;
+        auto total = [&](int c, float (&v)[4]) {
+            const char* at = lds + r * BN * 4 + ((c ^ (r & (CPR - 1))) << 4);
+            const f32x4 s0 = *(const f32x4*)at, s1 = *(const f32x4*)(at + RING), s2 = *(const f32x4*)(at + 2 * RING), s3 = *(const f32x4*)(at + 3 * RING);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (s0[e] + s1[e]) + (s2[e] + s3[e]);
+        };
+        const int64_t o = (int64_t)m * p.N + n;
+        float v[4];
+        total(cq, v);
+        if constexpr (SPLITK) {
+            store4<float>(p.kpart + (int64_t)blockIdx.y * p.M * p.N + o, v[0], v[1], v[2], v[3]);
+        } else {
+            float rs = 1.f, rsm = 0.f;
+            if constexpr (LN) { const f32x2_t t = *(const f32x2_t*)(p.ln_stats + 2 * (int64_t)m); rs = t[0]; rsm = t[1]; }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = LN ? v[e] * rs - rsm * c1[e] + b1[e] : v[e] + b1[e];
+            if constexpr (DUAL) {
+                float u[4];
+                total(cq + QPR, u);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u[e] = LN ? u[e] * rs - rsm * c2[e] + b2[e] : u[e] + b2[e];
+                if (p.cache1) store4<float>(p.cache1 + o, v[0], v[1], v[2], v[3]);
+                if (p.cache2) store4<float>(p.cache2 + o, u[0], u[1], u[2], u[3]);
+                glu_apply4(v, u, p);
+            } else {
+                if constexpr (EPI == EPI_GELU) gelu_fast4(v);
+                else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = epi_apply<EPI>(v[e], p);
+                if constexpr (EPI == EPI_RES) add4<OutT>((const OutT*)p.residual + o, v);
+            }
+            store4<OutT>((OutT*)p.C + o, v[0], v[1], v[2], v[3]);
+        }
+    }
+}
+
+// =====================================================================================
 // Main kernel: persistent workgroups, global -> LDS without passing through registers.
 //
 //   buffer_load_dwordx4 ... lds   writes each wave's 64 x 16 B straight into 1 KiB of LDS
@@ -541,7 +729,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_finish_kernel(GemmArgs p) {
 // (launch bounds: the four-wave workgroups of the 128 x 128 tiles run two to a CU, i.e. two waves per SIMD, like the one
 // eight-wave workgroup of the 256 x 256 tiles: the register budget is 256 per lane either way, and an instantiation that
 // would take more must spill rather than halve the occupancy)
-template <typename T, typename OutT, int BM, int BN, int WGM, int WGN, int EPI, bool DUAL, bool LN = false>
+template <typename T, typename OutT, int BM, int BN, int WGM, int WGN, int EPI, bool DUAL, bool LN = false, int NSTG = 2>
 __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm_nt_dma_kernel(GemmArgs p) {
     constexpr int NW = WGM * WGN, NT = NW * 64;
     constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -557,8 +745,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
     constexpr int CROWB = BNO * OES;                        // bytes per staged output row
     constexpr int CPR = CROWB / 16;                         // 16-byte chunks per staged row
     constexpr int RG = WGM * 32 * CROWB;                    // one staging region
-    constexpr int NREG = 2 * RG <= STAGE ? 2 : 1;
-    static_assert(RG <= STAGE && (CPR & (CPR - 1)) == 0, "output staging must fit in LDS stage 1");
+    constexpr int NREG = 2 * RG <= (NSTG - 1) * STAGE ? 2 : 1;
+    static_assert(RG <= (NSTG - 1) * STAGE && (CPR & (CPR - 1)) == 0, "output staging must fit in LDS stage 1");
     // one tile's per-column vectors, fp32: bias slice(s); with LN also the column sums c (c2) behind them and the
     // tile's BM row-statistics pairs
     constexpr int COLB = BN * 4;
@@ -566,7 +754,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
     static_assert(!(LN && RL) && !(RL && DUAL), "one set of row statistics per tile");
     constexpr int BIASB = (LN || RL) ? 2 * COLB + BM * 8 : COLB;
     static_assert(!LN || NW >= 4, "the per-tile vectors are fetched by distinct waves");
-    __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE + 2 * BIASB];
+    __shared__ __attribute__((aligned(1024))) char lds[NSTG * STAGE + 2 * BIASB];
 
     // the wave index is wave-uniform; telling the compiler so keeps everything derived from it (LDS stage addresses of
     // the transfers, the wave's tile coordinates, the branch that picks the requesting wave) in scalar registers
@@ -610,7 +798,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
 
     // the transfers of wave v's share of slab kt (v is wave-uniform; sec: v's weight rows come from W2)
     auto issue_for = [&](__amdgpu_buffer_rsrc_t rsA, __amdgpu_buffer_rsrc_t rsWv, int kt, int v, bool sec) {
-        char* st = lds + (kt & 1) * STAGE;
+        char* st = lds + (uint32_t)kt % NSTG * STAGE;
         const int sbyte = kt * 128;
         const int ar = v * GA * 8, br = v * GB * 8, bg = sec ? br - BNO : br;
 #pragma unroll
@@ -627,7 +815,10 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
     // and for its SIMD partner (waves w and w^4 share a SIMD), and the two take turns slab by slab: the
     // requesting wave sits in instruction issue while the address unit works through the queue (measured:
     // that queue is full 60 % of the time), and its partner keeps the matrix core busy meanwhile.
-    constexpr bool PAIRED = NW == 8;
+    // (not with more than three stages: a wave then has transfers of several slabs in flight, its own and its partner's in turn,
+    // and no single count to wait for)
+    constexpr bool PAIRED = NW == 8 && NSTG <= 3;
+    constexpr int LPW = GA + GB;                            // transfers of a wave per slab
     const int pw = wave ^ 4;
     const bool second_p = DUAL && (pw >= NW / 2);
     const void* Wsrc_p = second_p ? p.W2 : p.W;
@@ -641,7 +832,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
             const float* src = (w2 ? p.bias2 : p.bias) + n0t;
             int left = (p.N - n0t) * 4;
             __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, left > 0 ? left : 0, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + 2 * STAGE + buf * BIASB + (w2 ? BNO * 4 : 0)),
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + NSTG * STAGE + buf * BIASB + (w2 ? BNO * 4 : 0)),
                                                      16, lane * 16, 0, 0, 0);
         }
         if constexpr (LN) {
@@ -651,7 +842,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
                 const float* src = (w4 ? p.ln_c2 : p.ln_c) + n0t;
                 int left = (p.N - n0t) * 4;
                 __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, left > 0 ? left : 0, 0x00020000);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + 2 * STAGE + buf * BIASB + COLB + (w4 ? BNO * 4 : 0)),
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + NSTG * STAGE + buf * BIASB + COLB + (w4 ? BNO * 4 : 0)),
                                                          16, lane * 16, 0, 0, 0);
             }
         }
@@ -664,8 +855,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
                 const float* sbase = LN ? p.ln_stats : p.res_stats;
                 __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)(sbase + 2 * (int64_t)m0t), 0, left > 0 ? left : 0, 0x00020000);
 #pragma unroll
-                for (int j = 0; j < BM * 8 / 1024; ++j)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + 2 * STAGE + buf * BIASB + 2 * COLB + j * 1024),
+                for (int j = 0; j < (BM * 8 + 1023) / 1024; ++j)
+                    if (BM * 8 % 1024 == 0 || lane < BM * 8 / 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + NSTG * STAGE + buf * BIASB + 2 * COLB + j * 1024),
                                                              16, lane * 16, j * 1024, 0, 0);      // one per-lane offset for every transfer of the tile's vectors
             }
         }
@@ -712,8 +903,17 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
             rsWpn = make_rsrc(Wsrc_p, n0n, p.N);
         }
 
-        __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wave's transfers (and earlier stores) are done
-        __syncthreads();                         // ... and everybody else's; all staging reads of the last tile too
+        if constexpr (NSTG == 2) {
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's transfers (and earlier stores) are done
+            __syncthreads();                     // ... and everybody else's; all staging reads of the last tile too
+        } else {
+            // the stages behind the first are free once the last tile's staged rows have been read by everybody
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            static_for<NSTG - 2>([&](auto is) { if (decltype(is)::value + 1 < KT) issue(rsA, rsW, decltype(is)::value + 1); });
+            if (KT >= NSTG - 1) wait_vmcnt<(NSTG - 2) * LPW>();
+            else wait_vmcnt<0>();
+            asm volatile("s_barrier" ::: "memory");
+        }
         // What every accumulator block starts from: the bias of its columns when the LDS-staged epilogue follows (the first
         // MFMA of a block takes it as its C operand, so the epilogue has no bias add left), else zeros (the direct
         // epilogue adds the bias itself; the folded LayerNorm scales the sum before its bias).  Accumulator register
@@ -725,7 +925,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
 #pragma unroll
             for (int r = 0; r < 16; ++r) c0[b][r] = 0.f;
         if (BIASC && staged) {
-            const char* bl = lds + 2 * STAGE + bbuf * BIASB;
+            const char* bl = lds + NSTG * STAGE + bbuf * BIASB;
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
                 const bool up = DUAL && b >= TNO;
@@ -755,14 +955,15 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
         }
         auto k_slab = [&](int kt, auto ifirst) {
             constexpr bool FIRST = decltype(ifirst)::value;
-            if (kt + 1 < KT) {
-                if (!PAIRED) issue(rsA, rsW, kt + 1);
-                else if (((wave >> 2) & 1) == (kt & 1)) {
-                    issue_for(rsA, rsW, kt + 1, wave, second);
-                    issue_for(rsA, rsWp, kt + 1, pw, second_p);
+            const bool mine = ((wave >> 2) & 1) == (kt & 1);
+            if (kt + NSTG - 1 < KT) {
+                if (!PAIRED) issue(rsA, rsW, kt + NSTG - 1);
+                else if (mine) {
+                    issue_for(rsA, rsW, kt + NSTG - 1, wave, second);
+                    issue_for(rsA, rsWp, kt + NSTG - 1, pw, second_p);
                 }
             }
-            const char* s = lds + (kt & 1) * STAGE;
+            const char* s = lds + (uint32_t)kt % NSTG * STAGE;
             auto load_frags = [&](int sl, u32x4 (&xf)[TM], u32x4 (&wf)[TN]) {
                 const int ch = 2 * sl + lg;
 #pragma unroll
@@ -792,8 +993,22 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
                 run_mfmas(sl, xf[sl & 1], wf[sl & 1]);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_s_waitcnt(0x0f70);
-            __syncthreads();
+            if constexpr (NSTG == 2) {
+                __builtin_amdgcn_s_waitcnt(0x0f70);
+                __syncthreads();
+            } else {
+                // slab kt + 1 has landed; the slabs behind it (at most NSTG - 2 of them) stay in flight
+                const int behind = KT - 2 - kt;
+                if constexpr (PAIRED) {
+                    if (behind > 0 && mine) wait_vmcnt<2 * LPW>();      // all that is outstanding is slab kt + 2, requested above
+                    else wait_vmcnt<0>();
+                } else {
+                    if (behind >= NSTG - 2) wait_vmcnt<(NSTG - 2) * LPW>();
+                    else if (NSTG > 3 && behind == NSTG - 3) wait_vmcnt<(NSTG - 3) * LPW>();
+                    else wait_vmcnt<0>();
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
         };
         if (LN && staged) {
             // Folded LayerNorm: sum_k LN(x)[m,k] W0[n,k] = rstd_m * (acc[m,n] - mean_m * c[n]) + b'[n].  The outer product
@@ -801,7 +1016,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
             // the tile's row statistics and column sums (they arrived in LDS with the first slab).  What is left for
             // the epilogue is one multiply-add per element, the instruction count of the plain bias add.
             if constexpr (LN) {
-                const char* bl = lds + 2 * STAGE + bbuf * BIASB;
+                const char* bl = lds + NSTG * STAGE + bbuf * BIASB;
                 const float* stl = (const float*)(bl + 2 * COLB);
                 const float* cl = (const float*)(bl + COLB);
                 u32x4 xm[TM], wc[TN];
@@ -841,7 +1056,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (WGM * WGN <= 4 ? 2 : 1)) void gemm
             // ---- LDS-staged epilogue in stage 1, one 32-row band of every wave-row per pass
             constexpr int EPCO = 16 / OES;
             char* stg = lds + STAGE;
-            const char* bias_lds = lds + 2 * STAGE + bbuf * BIASB;
+            const char* bias_lds = lds + NSTG * STAGE + bbuf * BIASB;
             // bias of this lane's 4-column groups, once per tile (columns past N hold zero)
             // (the dual-weight kernel with the folded LayerNorm reads them from LDS where they are used instead: two bias
             // sets in registers next to its two accumulator sets and the row factor do not fit)
@@ -1128,7 +1343,7 @@ static inline bool prefer_big_tiles(int64_t n_big, int64_t n_small, int64_t cus,
     return !(t_small < 0.93 * t_big);
 }
 
-// Which kernel a 16-byte aligned problem gets: 1 register-staged 256 x 256 tiles, 2 register-staged 128 x 128, 3 direct-to-LDS
+// The size class of a 16-byte aligned problem (gemm_kernel() refines it): 1 register-staged 256 x 256 tiles, 2 register-staged 128 x 128, 3 direct-to-LDS
 // 256 x 256 (persistent), 4 direct-to-LDS 128 x 128, 5 register-staged 64 x 64.  The direct-to-LDS kernels need K to be a
 // whole number of 128-byte slabs.  Problems that 128 x 128 tiles would spread over a fraction of the CUs (single
 // sentences, small batches, the README-sized operators) take 64 x 64 tiles: four times the workgroups, each with a quarter
@@ -1148,6 +1363,98 @@ static inline int gemm_variant(int64_t M, int64_t N, int64_t K, size_t elem_size
     return slabs ? (big ? 3 : 4) : (big ? 1 : 2);
 }
 
+// us of an fp32 product of n tiles of `units` 32 x 32 blocks each on the CU that gets most of them: the block's matrix time on
+// one CU (0.109 us per slab) over the share of that rate a kernel reaches (lower where a CU has one workgroup only, whose
+// waits nothing fills), plus what a tile costs besides
+static inline double gemm_f32_us(int64_t n, int units, int64_t K, int64_t cus, double rate, double rate_alone, double per_tile) {
+    const int64_t most = (n + cus - 1) / cus;
+    return (double)most * (units * 0.109 * (double)(K / 32) / (most == 1 ? rate_alone : rate) + per_tile);
+}
+// the same for the kernels whose tiles hold 128 or 256 weight rows: 3, 4, 7 (numbers as below)
+static inline double gemm_f32_us_rows128(int kernel, int64_t M, int64_t N, int64_t K, int64_t cus) {
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    if (kernel == 3) return gemm_f32_us(tiles(256, 256), 64, K, cus, 0.92, 0.92, 4.0);
+    if (kernel == 4) return gemm_f32_us(tiles(128, 128), 16, K, cus, 0.91, 0.80, 2.5);
+    return gemm_f32_us(tiles(64, 128), 8, K, cus, 0.86, 0.70, 1.3);
+}
+static inline int gemm_kernel_rows128(int64_t M, int64_t N, int64_t K, int64_t cus) {
+    const double t3 = gemm_f32_us_rows128(3, M, N, K, cus), t4 = gemm_f32_us_rows128(4, M, N, K, cus), t7 = gemm_f32_us_rows128(7, M, N, K, cus);
+    return t7 < t4 ? (t7 < t3 ? 7 : 3) : (t4 < t3 ? 4 : 3);
+}
+
+// The kernel a 16-byte aligned problem really runs: gemm_variant()'s size class (1 .. 5) refined, where K is a whole number of
+// slabs and N a multiple of 4, by kernels for the sizes at which those tiles leave the chip idle:
+//   6  128 x 128 tiles, eight waves, four-stage ring, one workgroup per CU      7  64 x 128, three stages, two per CU
+//   8  64 x 64, four stages, two per CU      9 / 10  32 x 32 / 64 x 64 tiles whose K slabs the waves share out (kshare)
+//
+// bf16, kernel times in us (class kernel -> refined): what is short of work waits for memory, so the rule is the smallest tile
+// whose workgroups are all resident at once.
+//   9 up to two 32 x 32 tiles per CU: 128 x 2304 x 768 8.0 -> 4.7, 128 x 768 x 3072 10.3 -> 6.0, 250 x 768 x 768 7.8 -> 3.8; and for
+//     up to 32 rows whatever N is (there is one tile row, and the time is the weight's way through HBM)
+//   10 up to one 64 x 64 tile per CU and 12 slabs or more: 800 x 768 x 3072 19.1 -> 11.5, 2500 x 384 x 1536 15.6 -> 8.2
+//   8 up to two 64 x 64 tiles per CU: 450 x 3072 x 768 10.9 -> 8.3, 1500 x 768 x 3072 34 -> 20 (above: 800 x 3072 x 768 11.1 -> 11.6)
+//   6 up to one 128 x 128 tile per CU: 6400 x 384 x 1536 18.4 -> 15.0, 4992 x 768 x 1152 16.9 -> 15.4 (above: 2500 x 2304 x 768 13.7 -> 17.3)
+//   gated: 9 up to one tile of 32 x 32 outputs per CU (128 x 1152 x 768 12.2 -> 5.0), 10 up to two of 64 x 32 (450: 12.8 -> 10.2)
+// fp32 is bound by the matrix rate, so the rule is which kernel gives the fullest CU the least to do: tiles on that CU times
+// (matrix time of a tile / the share of the rate the kernel reaches + what a tile costs besides).  The shares and costs are
+// fitted to 100 measurements (8 ... 13000 rows, 384 ... 3072 columns) and give them within 12 %:
+//   450 x 2304 x 768 33.7 -> 22.4, 1500 x 768 x 3072 118 -> 73, 6400 x 768 x 3072 367 -> 251, 9240 x 2304 x 768 287 -> 267.
+// `in_order`: only kernels that add a product's slabs in ascending order (not 9 and 10).
+static inline int gemm_kernel(int64_t M, int64_t N, int64_t K, size_t elem_size, bool dual, int64_t cus, bool in_order = false) {
+    const int cls = gemm_variant(M, N, K, elem_size, dual, cus);
+    const int64_t bke = 128 / (int64_t)elem_size, KT = K / bke;
+    if (K % bke != 0 || N % 4 != 0) return cls;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    if (elem_size == 2) {
+        if (dual) {
+            if (in_order) return cls;
+            if (M <= 32 || tiles(32, 32) <= cus) return 9;
+            return tiles(64, 32) <= 2 * cus ? 10 : cls;
+        }
+        if (!in_order && (M <= 32 || tiles(32, 32) <= 2 * cus)) return 9;
+        if (!in_order && KT >= 12 && tiles(64, 64) <= cus) return 10;
+        if (tiles(64, 64) <= 2 * cus) return 8;
+        return tiles(128, 128) <= cus ? 6 : cls;
+    }
+    const int wide = gemm_kernel_rows128(M, dual ? 2 * N : N, K, cus);
+    auto cost = [&](int64_t n, int units, double rate, double rate_alone, double per_tile) { return gemm_f32_us(n, units, K, cus, rate, rate_alone, per_tile); };
+    if (dual && in_order) return wide;
+    if (dual) return cost(tiles(32, 32), 2, 0.79, 0.65, 3.0) < gemm_f32_us_rows128(wide, M, 2 * N, K, cus) ? 9 : wide;
+    const double t8 = cost(tiles(64, 64), 4, 0.83, 0.66, 1.0), t9 = in_order ? 1e30 : cost(tiles(32, 32), 1, 0.79, 0.65, 0.85);
+    if (std::min(t8, t9) >= gemm_f32_us_rows128(wide, M, N, K, cus)) return wide;
+    return t8 < t9 ? 8 : 9;
+}
+
+// The kernel of a block of the rows of a larger product: a result does not depend on the blocks it was computed in, so the block
+// adds its slabs in the order in which the whole product would.
+static inline int gemm_kernel_of_block(int64_t rows, int64_t M, int64_t N, int64_t K, size_t elem_size, bool dual, int64_t cus) {
+    const int whole = gemm_kernel(rows, N, K, elem_size, dual, cus);
+    return whole >= 9 ? whole : gemm_kernel(M, N, K, elem_size, dual, cus, true);
+}
+
+// shares of the K loop for kernel 9: a tile's serial chain is worth cutting where at most half of the CUs have a tile and every
+// share keeps 32 slabs (8 per wave); the second launch that adds the shares costs 3 to 5 us (128 x 768 x 3072 in fp32: 16.9 us whole)
+static inline int kshare_splits(int64_t M, int64_t N, int64_t KT, int64_t cus) {
+    const int64_t t = ((M + 31) / 32) * ((N + 31) / 32);
+    if (2 * t > cus) return 1;
+    int64_t ks = std::min<int64_t>(std::min<int64_t>(8, 2 * cus / t), KT / 32);
+    while (ks > 1 && ((KT + ks - 1) / ks) * (ks - 1) >= KT) --ks;          // no empty share
+    return ks < 1 ? 1 : (int)ks;
+}
+
+// Second launch of a split K loop: takes the shares' buffer from the pool around `first` (which launches the kernel that fills it)
+template <typename OutT, int EPI, typename F>
+static int launch_split(grl_ctx* c, GemmArgs& a, int ks, F&& first) {
+    a.ksplit = ks;
+    a.kpart = (float*)grl_malloc(c, (size_t)ks * a.M * a.N * sizeof(float));
+    if (!a.kpart) return GRL_ERR_OOM;
+    first();
+    const int64_t quads = (int64_t)a.M * a.N / 4;
+    hipLaunchKernelGGL((gemm_splitk_finish_kernel<OutT, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, c->stream, a);
+    grl_free(c, a.kpart);          // back to the pool: later users are ordered behind these launches on the stream
+    return GRL_OK;
+}
+
 template <typename T, typename OutT, int EPI, bool DUAL, bool LN = false>
 static int launch_gemm(grl_ctx* c, GemmArgs& a) {
     const int64_t epc = 16 / (int64_t)sizeof(T);
@@ -1161,8 +1468,9 @@ static int launch_gemm(grl_ctx* c, GemmArgs& a) {
         GRL_CHECK_LAUNCH();
         return GRL_OK;
     }
-    // Tile choice: gemm_variant().  GRL_GEMM_VARIANT (1..5) forces one variant, for tuning runs.
+    // Tile choice: gemm_kernel().  GRL_GEMM_VARIANT (1..10) forces one where the problem allows it, for tuning runs.
     static const int forced = [] { const char* e = getenv("GRL_GEMM_VARIANT"); return e ? atoi(e) : 0; }();
+    static const int splitk_env = [] { const char* e = getenv("GRL_GEMM_SPLITK"); return e ? atoi(e) : -1; }();
     // band height of the tile walk: rows of 8 KiB and more do better with narrow bands (measured)
     static const int group = [] { const char* e = getenv("GRL_GEMM_GROUP"); return e ? atoi(e) : 0; }();
     a.group = group > 0 ? group : (a.K * (int64_t)sizeof(T) >= 8192 ? 2 : 8);
@@ -1174,19 +1482,20 @@ static int launch_gemm(grl_ctx* c, GemmArgs& a) {
     const bool slabs = a.K % bke == 0;
     const int64_t cus = c->prop.multiProcessorCount;     // one 128 KiB-LDS workgroup per CU, two of the 64 KiB ones
     const int64_t tm = (a.M + 63) / 64, tn = (a.N + 63) / 64;      // 64 output columns per tile (with two weights: 128 LDS rows)
-    int variant = gemm_variant(a.M, a.N, a.K, sizeof(T), DUAL, cus);
-    if (forced >= 1 && forced <= 5 && (slabs || forced <= 2 || forced == 5)) variant = forced;
+    const bool fine = slabs && a.N % 4 == 0;
+    int variant = a.plan_rows > 0 ? gemm_kernel_of_block(a.plan_rows, a.M, a.N, a.K, sizeof(T), DUAL, cus) : gemm_kernel(a.M, a.N, a.K, sizeof(T), DUAL, cus);
+    if (forced >= 1 && forced <= 10 && (forced <= 2 || forced == 5 || (slabs && forced <= 4) || fine)) variant = forced;
+    constexpr bool SPLITS = !DUAL && !LN && (EPI == EPI_NONE || EPI == EPI_GELU || EPI == EPI_SILU || EPI == EPI_RT || EPI == EPI_RES);
+    constexpr bool HALF = sizeof(T) == 2;
     switch (variant) {
         case 5: {
             a.tiles_m = (int)tm; a.tiles_n = (int)tn;
-            // Few tiles and a long K (one sentence through a feed-forward block: 24 tiles, 96 slabs in fp32) leave most CUs
-            // idle behind a serial K loop whose every slab costs a memory round trip: the slabs are shared out over up to
-            // 8 workgroups per tile (16 slabs or more, at least 4 per share, at most about two workgroups per CU in all), which write raw
-            // fp32 sums to a pool buffer, and a small second kernel adds them and runs the epilogue.  GRL_GEMM_SPLITK=0
-            // switches it off, for tuning runs.
-            static const int splitk_env = [] { const char* e = getenv("GRL_GEMM_SPLITK"); return e ? atoi(e) : -1; }();
+            // Few tiles and a long K leave most CUs idle behind a serial K loop whose every slab costs a memory round trip: the
+            // slabs are shared out over up to 8 workgroups per tile (16 slabs or more, at least 4 per share, at most about two
+            // workgroups per CU in all), which write raw fp32 sums to a pool buffer, and a small second kernel adds them and
+            // runs the epilogue.  GRL_GEMM_SPLITK=0 switches it off, for tuning runs.
             int ks = 1;
-            if constexpr (!DUAL && !LN && (EPI == EPI_NONE || EPI == EPI_GELU || EPI == EPI_SILU || EPI == EPI_RT || EPI == EPI_RES)) {
+            if constexpr (SPLITS) {
                 const int64_t KT = (a.K + bke - 1) / bke, t64 = tm * tn;
                 if (splitk_env != 0 && !a.no_alloc && a.N % 4 == 0 && KT >= 16 && t64 <= cus) {
                     ks = (int)std::min<int64_t>(std::min<int64_t>(8, 2 * cus / t64), KT / 4);
@@ -1194,13 +1503,10 @@ static int launch_gemm(grl_ctx* c, GemmArgs& a) {
                     if (ks == 2 && KT < 48) ks = 1;                                      // two short halves: the second launch costs more
                 }
                 if (ks > 1) {
-                    a.ksplit = ks;
-                    a.kpart = (float*)grl_malloc(c, (size_t)ks * a.M * a.N * sizeof(float));
-                    if (!a.kpart) return GRL_ERR_OOM;
-                    hipLaunchKernelGGL((gemm_nt_kernel<T, OutT, 64, 64, 2, 2, EPI, false, false, true>), dim3((unsigned)(tm * tn), (unsigned)ks), dim3(256), 0, c->stream, a);
-                    const int64_t quads = (int64_t)a.M * a.N / 4;
-                    hipLaunchKernelGGL((gemm_splitk_finish_kernel<OutT, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, c->stream, a);
-                    grl_free(c, a.kpart);          // back to the pool: later users are ordered behind these launches on the stream
+                    const int rc = launch_split<OutT, EPI>(c, a, ks, [&] {
+                        hipLaunchKernelGGL((gemm_nt_kernel<T, OutT, 64, 64, 2, 2, EPI, false, false, true>), dim3((unsigned)(tm * tn), (unsigned)ks), dim3(256), 0, c->stream, a);
+                    });
+                    if (rc) return rc;
                     break;
                 }
             }
@@ -1219,6 +1525,49 @@ static int launch_gemm(grl_ctx* c, GemmArgs& a) {
             a.tiles_m = (int)big_m; a.tiles_n = (int)big_n;
             hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 256, 256, 2, 4, EPI, DUAL, LN>), dim3((unsigned)std::min<int64_t>(big_m * big_n, cus)), dim3(512), 0, c->stream, a);
             break;
+        case 6:
+            if constexpr (HALF && !DUAL) {
+                a.tiles_m = (int)sm; a.tiles_n = (int)sn;
+                hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 128, 128, 4, 2, EPI, DUAL, LN, 4>), dim3((unsigned)std::min<int64_t>(sm * sn, cus)), dim3(512), 0, c->stream, a);
+                break;
+            }
+        case 7:
+            if constexpr (!HALF) {
+                const int64_t t7 = (a.N + (DUAL ? 63 : 127)) / (DUAL ? 64 : 128);
+                a.tiles_m = (int)tm; a.tiles_n = (int)t7;
+                hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 64, 128, 2, 2, EPI, DUAL, LN, 3>), dim3((unsigned)std::min<int64_t>(tm * t7, 2 * cus)), dim3(256), 0, c->stream, a);
+                break;
+            }
+        case 8:
+            if constexpr (!DUAL) {
+                a.tiles_m = (int)tm; a.tiles_n = (int)tn;
+                hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 64, 64, 2, 2, EPI, DUAL, LN, 4>), dim3((unsigned)std::min<int64_t>(tm * tn, 2 * cus)), dim3(256), 0, c->stream, a);
+                break;
+            }
+        case 9: {
+            constexpr int BN9 = DUAL ? 64 : 32;
+            a.tiles_m = (a.M + 31) / 32; a.tiles_n = (a.N + 31) / 32;
+            const unsigned n9 = (unsigned)((int64_t)a.tiles_m * a.tiles_n);
+            if constexpr (SPLITS) {
+                const int ks = splitk_env != 0 && !a.no_alloc ? kshare_splits(a.M, a.N, a.K / bke, cus) : 1;
+                if (ks > 1) {
+                    const int rc = launch_split<OutT, EPI>(c, a, ks, [&] {
+                        hipLaunchKernelGGL((gemm_nt_kshare_kernel<T, OutT, 32, 32, 2, EPI, false, false, true>), dim3(n9, (unsigned)ks), dim3(256), 0, c->stream, a);
+                    });
+                    if (rc) return rc;
+                    break;
+                }
+            }
+            hipLaunchKernelGGL((gemm_nt_kshare_kernel<T, OutT, 32, BN9, 2, EPI, DUAL, LN>), dim3(n9), dim3(256), 0, c->stream, a);
+            break;
+        }
+        case 10:
+            if constexpr (HALF) {
+                constexpr int BNO10 = DUAL ? 32 : 64;
+                a.tiles_m = (int)tm; a.tiles_n = (a.N + BNO10 - 1) / BNO10;
+                hipLaunchKernelGGL((gemm_nt_kshare_kernel<T, OutT, 64, 64, 2, EPI, DUAL, LN>), dim3((unsigned)(tm * a.tiles_n)), dim3(256), 0, c->stream, a);
+                break;
+            }
         default:
             a.tiles_m = (int)sm; a.tiles_n = (int)sn;
             hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 128, 128, 2, 2, EPI, DUAL, LN>), dim3((unsigned)std::min<int64_t>(sm * sn, 2 * cus)), dim3(256), 0, c->stream, a);
@@ -1246,7 +1595,28 @@ int launch_gemm_resln(grl_ctx* c, GemmArgs& a, int* tile_cols) {
     const int64_t sm = (a.M + 127) / 128, sn = (a.N + 127) / 128;
     GRL_REQUIRE(sm * sn < (1LL << 31), GRL_ERR_SHAPE, "gemm: too many tiles");
     const int64_t cus = c->prop.multiProcessorCount;
-    if (prefer_big_tiles(big_m * big_n, sm * sn, cus, sizeof(T))) {
+    // The same refinement as gemm_kernel() for the tiles this epilogue has (a partial per 128 columns at least).  bf16, us with
+    // the merge: 64 x 128 tiles up to one per CU (2500 x 768 x 3072 41.6 -> 29.0), the four-stage ring of 128 x 128 tiles up to one
+    // per CU (4992 x 768 x 3072 42.8 -> 36.5), else the two-stage kernels.  fp32: 64 x 128 tiles, two per CU, where the fullest CU
+    // has less to do with them (9240 x 384 x 384 37.5 -> 33.5, 9240 x 384 x 1536 111 -> 102, 13000 x 384 x 1536 198 -> 161).
+    const int64_t tm = (a.M + 63) / 64;
+    const int kernel = sizeof(T) == 2 ? (tm * sn <= cus ? 7 : sm * sn <= cus ? 6 : prefer_big_tiles(big_m * big_n, sm * sn, cus, sizeof(T)) ? 3 : 4)
+                                      : gemm_kernel_rows128(a.M, a.N, a.K, cus);
+    if (kernel == 7) {
+        a.tiles_m = (int)tm; a.tiles_n = (int)sn; *tile_cols = 128;
+        hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 64, 128, 2, 2, EPI_RESLN, false, false, 3>), dim3((unsigned)std::min<int64_t>(tm * sn, 2 * cus)), dim3(256), 0, c->stream, a);
+        GRL_CHECK_LAUNCH();
+        return GRL_OK;
+    }
+    if constexpr (sizeof(T) == 2) {
+        if (kernel == 6) {
+            a.tiles_m = (int)sm; a.tiles_n = (int)sn; *tile_cols = 128;
+            hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 128, 128, 4, 2, EPI_RESLN, false, false, 4>), dim3((unsigned)std::min<int64_t>(sm * sn, cus)), dim3(512), 0, c->stream, a);
+            GRL_CHECK_LAUNCH();
+            return GRL_OK;
+        }
+    }
+    if (kernel == 3) {
         a.tiles_m = (int)big_m; a.tiles_n = (int)big_n; *tile_cols = 256;
         hipLaunchKernelGGL((gemm_nt_dma_kernel<T, OutT, 256, 256, 2, 4, EPI_RESLN, false, false>), dim3((unsigned)std::min<int64_t>(big_m * big_n, cus)), dim3(512), 0, c->stream, a);
     } else {

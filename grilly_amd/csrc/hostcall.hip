@@ -245,8 +245,10 @@ static void give_slab(grl_ctx* c, char* s) {
 
 int grl_copy_bytes_launch(grl_ctx* c, void* dst, const void* src, size_t bytes);
 int grl_copy_segments_launch(grl_ctx* c, const grl_segments& g);
-int grl_gemm_nt_act_block(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, void* C,
-                          int epilogue, float alpha, float beta);
+int grl_gemm_nt_act_block(grl_ctx* c, int dtype, int64_t rows, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias,
+                          void* C, int epilogue, float alpha, float beta);
+int grl_glu_nt_block(grl_ctx* c, int dtype, int64_t rows, int64_t M, int64_t N, int64_t K, const void* x, const void* W_gate, const void* W_up,
+                     const float* b_gate, const float* b_up, void* out, float* gate_cache, float* up_cache, int activation);
 
 // Host -> device, small: converted or copied into the staging ring, from where a copy kernel fetches it like any other kernel
 // of the stream (the copy engine would be faster from about 1 MiB on, but every hand-over to it and back costs 10 us).
@@ -465,7 +467,7 @@ extern "C" int grl_host_linear(grl_ctx* c, int dtype, int64_t M, int64_t N, int6
                       {nullptr, y, M * N, N, false}};
     if (!bias) a[1].n = 0;
     return run_on_host(c, dtype, M, true, a, 4, [&](int64_t, int64_t m, void** d) {
-        if (m < M) return grl_gemm_nt_act_block(c, dtype, m, N, K, d[2], d[0], (const float*)d[1], d[3], epilogue, alpha, beta);
+        if (m < M) return grl_gemm_nt_act_block(c, dtype, M, m, N, K, d[2], d[0], (const float*)d[1], d[3], epilogue, alpha, beta);
         return grl_gemm_nt_act(c, dtype, dtype, m, N, K, d[2], d[0], (const float*)d[1], d[3], epilogue, alpha, beta);
     });
 }
@@ -481,7 +483,7 @@ extern "C" int grl_host_glu(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t
                       {x, nullptr, M * K, K, false}, {nullptr, out, M * N, N, false},
                       {nullptr, gate_cache, gate_cache ? M * N : 0, N, true}, {nullptr, up_cache, up_cache ? M * N : 0, N, true}};
     return run_on_host(c, dtype, M, true, a, 8, [&](int64_t, int64_t m, void** d) {
-        return grl_glu_nt(c, dtype, dtype, m, N, K, d[4], d[0], d[1], (const float*)d[2], (const float*)d[3], d[5], (float*)d[6], (float*)d[7], activation);
+        return grl_glu_nt_block(c, dtype, M, m, N, K, d[4], d[0], d[1], (const float*)d[2], (const float*)d[3], d[5], (float*)d[6], (float*)d[7], activation);
     });
 }
 
