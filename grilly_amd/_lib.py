@@ -93,11 +93,15 @@ SIGNATURES = {
     "grl_fa2_fwd_strided": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64] + [c_void_p] * 5 + [c_i64] * 4 + [c_float, c_int, c_int, c_float, c_float]),
     "grl_rope": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_int, c_float, c_float]),
     "grl_ln_fold": (c_int, [c_void_p, c_int, c_i64, c_i64] + [c_void_p] * 7),
+    "grl_ln_fold_f32": (c_int, [c_void_p, c_int, c_i64, c_i64] + [c_void_p] * 7),
     "grl_ln_stats": (c_int, [c_void_p, c_int, c_i64, c_i64, c_void_p, c_float, c_void_p]),
     "grl_ln_gemm_nt": (c_int, [c_void_p, c_int, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 4 + [c_float, c_void_p, c_void_p]),
     "grl_ln_glu_nt": (c_int, [c_void_p, c_int, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 7 + [c_float, c_void_p, c_void_p, c_int]),
     "grl_ln_glu_nt_stats": (c_int, [c_void_p, c_int, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 7 + [c_void_p, c_void_p, c_int]),
     "grl_ln_gemm_nt_stats": (c_int, [c_void_p, c_int, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 6 + [c_int]),
+    "grl_ln_gemm_nt_rows": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 4 + [c_float, c_void_p, c_void_p, c_int]),
+    "grl_ln_glu_nt_rows": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 7 + [c_float, c_void_p, c_int]),
+    "grl_gemm_nt_lnres": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 8),
     "grl_gemm_nt_resln_workspace": (c_i64, [c_i64, c_i64]),
     "grl_gemm_nt_resln": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64] + [c_void_p] * 8 + [c_float, c_void_p, c_void_p]),
     "grl_layernorm": (c_int, [c_void_p, c_int, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p]),
@@ -121,6 +125,10 @@ SIGNATURES = {
     "grl_bert_layer_fwd_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayer), c_float, c_void_p, c_void_p]),
     "grl_bert_layer_fwd_fused_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_float,
                                         c_void_p, c_void_p, c_void_p]),
+    "grl_bert_layer_fwd_rows": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_void_p, c_float, c_float,
+                                c_void_p, c_void_p]),
+    "grl_bert_layer_fwd_rows_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_float, c_float,
+                                       c_void_p, c_void_p]),
     "grl_bert_layer_workspace": (c_i64, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64]),
     "grl_bert_layer_fused_workspace": (c_i64, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64]),
     "grl_bert_layer_fwd_fused": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_void_p, c_float,

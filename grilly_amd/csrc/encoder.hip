@@ -129,6 +129,54 @@ extern "C" int grl_bert_layer_fwd_fused_ragged(grl_ctx* c, int dtype, const grl_
     return rc ? rc : bert_layer_fused(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, nullptr, eps, r, stats, workspace, rg);
 }
 
+// ---- the same for few rows: five launches, no statistics pass, no partials to merge -------------------------------
+// The products that read LayerNorm(r) take its row statistics from their own operand and leave them for the residual epilogue
+// that needs them next, so between layers only the raw rows travel.  One 128-token sentence through twelve layers 768 wide in
+// bf16: 521 us with seven launches a layer (two of them LayerNorm passes of 5 us over 128 rows), 443 us with these five.  Hidden
+// states are 1 to 4 % nearer to their float64 values: a sublayer's output is rounded once, behind the residual, not before and after.
+static int bert_layer_rows(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff, const grl_bert_layer_fused* w,
+                           const float* mask, float in_eps, float eps, void* r, void* workspace, const grl_ragged* rg) {
+    GRL_REQUIRE(c && w && r && workspace, GRL_ERR_ARG, "grl_bert_layer_fwd_rows: null argument");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_bert_layer_fwd_rows: bad dtype %d", dtype);
+    GRL_REQUIRE(B >= 0 && S >= 0 && H > 0 && d_ff > 0, GRL_ERR_SHAPE, "grl_bert_layer_fwd_rows: bad shape");
+    GRL_REQUIRE(D >= 1 && D <= 1024, GRL_ERR_SHAPE, "grl_bert_layer_fwd_rows: head_dim must be between 1 and 1024 (got %lld)", (long long)D);
+    GRL_REQUIRE(w->ws_qkv && w->c_qkv && w->bf_qkv && w->in_g && w->in_b && w->w_o && w->ln1_g && w->ln1_b && w->ws_ff1 && w->c_ff1 &&
+                w->bf_ff1 && w->w_ff2, GRL_ERR_ARG, "grl_bert_layer_fwd_rows: null weight");
+    const int64_t M = rg ? rg->rows : B * S, d = H * D, es = (int64_t)grl_dtype_size(dtype), slab = 128 / es;
+    GRL_REQUIRE(d % slab == 0 && d_ff % slab == 0, GRL_ERR_SHAPE,
+                "grl_bert_layer_fwd_rows: d_model (%lld) and d_ff (%lld) must be multiples of %lld; use grl_bert_layer_fwd",
+                (long long)d, (long long)d_ff, (long long)slab);
+    if (M == 0) return GRL_OK;
+    auto pad = [](int64_t v) { return (v + 255) / 256 * 256; };
+    char* qkv = (char*)workspace;                  // the layout of the folded layer's workspace
+    char* attn = qkv + pad(M * 3 * d * es);
+    char* ff = attn + pad(M * d * es);
+    float* stats = (float*)(ff + pad(M * d_ff * es));
+    int rc;
+    grl_lap_mark(c);
+    if ((rc = grl_ln_gemm_nt_rows(c, dtype, M, 3 * d, d, r, w->ws_qkv, w->c_qkv, w->bf_qkv, in_eps, stats, qkv, GRL_EPI_NONE))) return rc;
+    grl_lap_mark(c);
+    if ((rc = layer_attention(c, dtype, B, S, H, D, qkv, mask, attn, rg))) return rc;
+    grl_lap_mark(c);
+    if ((rc = grl_gemm_nt_lnres(c, dtype, M, d, d, attn, w->w_o, w->b_o, r, stats, w->in_g, w->in_b, r))) return rc;
+    grl_lap_mark(c);
+    if ((rc = grl_ln_gemm_nt_rows(c, dtype, M, d_ff, d, r, w->ws_ff1, w->c_ff1, w->bf_ff1, eps, stats, ff, GRL_EPI_GELU))) return rc;
+    grl_lap_mark(c);
+    if ((rc = grl_gemm_nt_lnres(c, dtype, M, d, d_ff, ff, w->w_ff2, w->b_ff2, r, stats, w->ln1_g, w->ln1_b, r))) return rc;
+    grl_lap_mark(c);
+    return GRL_OK;
+}
+
+extern "C" int grl_bert_layer_fwd_rows(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                                       const grl_bert_layer_fused* w, const float* mask, float in_eps, float eps, void* r, void* workspace) {
+    return bert_layer_rows(c, dtype, B, S, H, D, d_ff, w, mask, in_eps, eps, r, workspace, nullptr);
+}
+extern "C" int grl_bert_layer_fwd_rows_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t H, int64_t D, int64_t d_ff,
+                                              const grl_bert_layer_fused* w, float in_eps, float eps, void* r, void* workspace) {
+    int rc = grl_check_ragged("grl_bert_layer_fwd_rows_ragged", rg);
+    return rc ? rc : bert_layer_rows(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, nullptr, in_eps, eps, r, workspace, rg);
+}
+
 // ---- a padded batch without its padding: host side --------------------------------------------------------------
 int grl_check_ragged(const char* who, const grl_ragged* rg) {
     GRL_REQUIRE(rg && rg->offsets && rg->positions, GRL_ERR_ARG, "%s: null ragged batch", who);

@@ -257,6 +257,63 @@ extern "C" int grl_gemm_nt_resln(grl_ctx* c, int dtype, int64_t M, int64_t N, in
     return GRL_OK;
 }
 
+// ---- products of few rows that take the row statistics of a folded LayerNorm themselves ---------------------------
+extern template int launch_gemm_rows<float>(grl_ctx*, GemmArgs&, int);
+extern template int launch_gemm_rows<uint16_t>(grl_ctx*, GemmArgs&, int);
+
+extern "C" int grl_ln_gemm_nt_rows(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* W_scaled, const float* colsum,
+                                   const float* bias_folded, float eps, float* stats_out, void* out, int epilogue) {
+    GRL_REQUIRE(c, GRL_ERR_ARG, "grl_ln_gemm_nt_rows: null context");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_ln_gemm_nt_rows: bad dtype");
+    GRL_REQUIRE(epilogue == GRL_EPI_NONE || epilogue == GRL_EPI_GELU, GRL_ERR_ARG,
+                "grl_ln_gemm_nt_rows: epilogue must be GRL_EPI_NONE or GRL_EPI_GELU (got %d)", epilogue);
+    int rc = check_dims("grl_ln_gemm_nt_rows", M, N, K);
+    if (rc) return rc;
+    if (M == 0 || N == 0) return GRL_OK;
+    GRL_REQUIRE(out && K > 0 && x && W_scaled && colsum && bias_folded, GRL_ERR_ARG, "grl_ln_gemm_nt_rows: null argument or K == 0");
+    GemmArgs a{};
+    a.A = x; a.W = W_scaled; a.bias = bias_folded; a.C = out; a.ln_c = colsum; a.stats_out = stats_out; a.eps = eps;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.act = epilogue;
+    const int epi = epilogue == GRL_EPI_GELU ? EPI_GELU : EPI_NONE;
+    return dtype == GRL_F32 ? launch_gemm_rows<float>(c, a, epi) : launch_gemm_rows<uint16_t>(c, a, epi);
+}
+
+extern "C" int grl_ln_glu_nt_rows(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* Wg_scaled, const void* Wu_scaled,
+                                  const float* colsum_gate, const float* colsum_up, const float* bias_gate_folded, const float* bias_up_folded,
+                                  float eps, void* out, int activation) {
+    GRL_REQUIRE(c, GRL_ERR_ARG, "grl_ln_glu_nt_rows: null context");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_ln_glu_nt_rows: bad dtype");
+    GRL_REQUIRE(activation == GRL_EPI_SILU || activation == GRL_EPI_RELU || activation == GRL_EPI_GELU, GRL_ERR_ARG,
+                "grl_ln_glu_nt_rows: activation must be GRL_EPI_SILU, GRL_EPI_RELU or GRL_EPI_GELU (got %d)", activation);
+    int rc = check_dims("grl_ln_glu_nt_rows", M, N, K);
+    if (rc) return rc;
+    if (M == 0 || N == 0) return GRL_OK;
+    GRL_REQUIRE(out && K > 0 && x && Wg_scaled && Wu_scaled && colsum_gate && colsum_up && bias_gate_folded && bias_up_folded, GRL_ERR_ARG,
+                "grl_ln_glu_nt_rows: null argument or K == 0");
+    GemmArgs a{};
+    a.A = x; a.W = Wg_scaled; a.W2 = Wu_scaled; a.C = out; a.bias = bias_gate_folded; a.bias2 = bias_up_folded;
+    a.ln_c = colsum_gate; a.ln_c2 = colsum_up; a.eps = eps;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.act = activation;
+    return dtype == GRL_F32 ? launch_gemm_rows<float>(c, a, EPI_GLU) : launch_gemm_rows<uint16_t>(c, a, EPI_GLU);
+}
+
+extern "C" int grl_gemm_nt_lnres(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias,
+                                 const void* R, const float* r_stats, const float* r_gamma, const float* r_beta, void* C) {
+    GRL_REQUIRE(c, GRL_ERR_ARG, "grl_gemm_nt_lnres: null context");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_gemm_nt_lnres: bad dtype");
+    int rc = check_dims("grl_gemm_nt_lnres", M, N, K);
+    if (rc) return rc;
+    if (M == 0 || N == 0) return GRL_OK;
+    GRL_REQUIRE(A && W && R && r_stats && r_gamma && r_beta && C && K > 0, GRL_ERR_ARG, "grl_gemm_nt_lnres: null argument or K == 0");
+    GemmArgs a{};
+    a.A = A; a.W = W; a.bias = bias; a.C = C; a.residual = R;
+    a.res_stats = r_stats; a.res_gamma = r_gamma; a.res_beta = r_beta;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    return dtype == GRL_F32 ? launch_gemm_rows<float>(c, a, EPI_RESLN) : launch_gemm_rows<uint16_t>(c, a, EPI_RESLN);
+}
+
 // stats == given: {1/sd, mean/sd} per row of x are the caller's (from grl_ln_stats or a GEMM epilogue); else they are computed here
 static int ln_glu_nt_impl(grl_ctx* c, const char* who, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x,
                           const void* Wg_scaled, const void* Wu_scaled, const float* colsum_gate, const float* colsum_up,

@@ -315,17 +315,18 @@ extern "C" int grl_ln_stats(grl_ctx* c, int dtype, int64_t rows, int64_t F, cons
 // Weight side of the LayerNorm-folded GEMM, once per weight: W_scaled[n,k] = gamma[k]*W[n,k] (rounded to the storage
 // type), colsum[n] = sum_k W_scaled[n,k] (of the rounded values, which is what the GEMM multiplies), bias_folded[n] =
 // bias[n] + sum_k beta[k]*W[n,k].  One wave per weight row.
-template <typename T>
-__global__ __launch_bounds__(256) void ln_fold_kernel(const T* W, const float* gamma, const float* beta, const float* bias,
+// (U: the type the weight is given in)
+template <typename T, typename U = T>
+__global__ __launch_bounds__(256) void ln_fold_kernel(const U* W, const float* gamma, const float* beta, const float* bias,
                                                       T* Ws, float* colsum, float* bias_folded, int64_t N, int K) {
     const int lane = threadIdx.x & 63;
     const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (n >= N) return;
-    const T* w = W + n * (int64_t)K;
+    const U* w = W + n * (int64_t)K;
     T* ws = Ws + n * (int64_t)K;
     float cs = 0.f, ds = 0.f;
     for (int k = lane; k < K; k += 64) {
-        const float wv = elem<T>::ld(w + k);
+        const float wv = elem<U>::ld(w + k);
         elem<T>::st(ws + k, gamma[k] * wv);
         cs += elem<T>::ld(ws + k);          // the value as stored
         ds += beta[k] * wv;
@@ -344,6 +345,21 @@ extern "C" int grl_ln_fold(grl_ctx* c, int dtype, int64_t N, int64_t K, const vo
     dim3 grid((unsigned)((N + 3) / 4)), block(256);
     if (dtype == GRL_F32) hipLaunchKernelGGL(ln_fold_kernel<float>, grid, block, 0, c->stream, (const float*)W, gamma, beta, bias, (float*)W_scaled, colsum, bias_folded, N, (int)K);
     else hipLaunchKernelGGL(ln_fold_kernel<uint16_t>, grid, block, 0, c->stream, (const uint16_t*)W, gamma, beta, bias, (uint16_t*)W_scaled, colsum, bias_folded, N, (int)K);
+    GRL_CHECK_LAUNCH();
+    return GRL_OK;
+}
+
+// the same from an fp32 weight: gamma*W is rounded to bf16 once.  Folding a weight that already is bf16 rounds it twice, which is
+// most of what a folded layer is further off than one with LayerNorm passes.
+extern "C" int grl_ln_fold_f32(grl_ctx* c, int dtype, int64_t N, int64_t K, const float* W, const float* gamma, const float* beta,
+                               const float* bias, void* W_scaled, float* colsum, float* bias_folded) {
+    if (dtype != GRL_BF16) return grl_ln_fold(c, dtype, N, K, W, gamma, beta, bias, W_scaled, colsum, bias_folded);
+    GRL_REQUIRE(c, GRL_ERR_ARG, "grl_ln_fold_f32: null context");
+    GRL_REQUIRE(N >= 0 && K > 0 && K < (1LL << 31) && N < (1LL << 31), GRL_ERR_SHAPE, "grl_ln_fold_f32: bad shape N=%lld K=%lld", (long long)N, (long long)K);
+    if (N == 0) return GRL_OK;
+    GRL_REQUIRE(W && gamma && beta && W_scaled && colsum && bias_folded, GRL_ERR_ARG, "grl_ln_fold_f32: null argument");
+    hipLaunchKernelGGL((ln_fold_kernel<uint16_t, float>), dim3((unsigned)((N + 3) / 4)), dim3(256), 0, c->stream, W, gamma, beta, bias, (uint16_t*)W_scaled,
+                       colsum, bias_folded, N, (int)K);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
 }

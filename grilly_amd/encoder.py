@@ -121,15 +121,20 @@ class BertEncoder:
 
     fused=None (default): both LayerNorms of every layer are folded into the GEMMs around them whenever the
     direct-to-LDS GEMM kernels take the layer's shapes (d_model and d_ff multiples of 64 in bf16, 32 in fp32) and the
-    batch has at least FUSED_MIN_ROWS token rows: the residual stream then travels as raw rows plus row statistics and
-    no LayerNorm pass runs over HBM between the embedding and the final LayerNorm (grl_bert_layer_fwd_fused).  Smaller
+    batch has at least FUSED_MIN_ROWS token rows, or in bf16 few enough for the form without statistics passes: the residual stream then travels as raw rows plus row statistics and
+    no LayerNorm pass runs over HBM between the embedding and the final LayerNorm (grl_bert_layer_fwd_fused).  Other
     batches run the seven-launch layer with its two LayerNorm passes (grl_bert_layer_fwd): a handful of token rows
-    make a handful of tiles, the plain GEMMs then take 64 x 64 tiles while the fused layer's residual GEMM has none
-    below 128 x 128, and the LayerNorm passes it saves cost next to nothing there (one sentence of 32 tokens in fp32:
-    1.9 against 4.5 ms; level at 4096 rows; the fused layer 4 - 7 % ahead at 8192 - 16384 rows in bf16).  Both weight
+    make a handful of tiles, the plain GEMMs then take tiles down to 32 x 32 while the fused layer's residual GEMM has none
+    below 64 x 128, and the LayerNorm passes it saves cost next to nothing there (level at 4096 rows; the fused layer 4 - 7 %
+    ahead at 8192 - 16384 rows in bf16).  Both weight
     sets stay resident.  fused=False always takes the seven-launch layer;
     fused=True always the fused one, and raises for shapes it does not take."""
     FUSED_MIN_ROWS = 8192
+    # bf16: up to this many values of a layer's widest activation (rows x d_ff) a layer runs as five launches without a LayerNorm
+    # pass (grl_bert_layer_fwd_rows).  us per forward, seven launches -> five: d_ff 3072 / 768 wide / 12 layers: 16 rows 412 -> 360,
+    # 128 rows 521 -> 443, 384 rows 613 -> 573, 560 rows 664 -> 676; 1536 / 384 / 6 layers: 100 rows 207 -> 179, 768 rows 280 -> 255,
+    # 1280 rows 277 -> 287.  In fp32 the two forms are within 4 % of each other from 128 rows on and the seven launches ahead below.
+    ROWS_MAX_OUTPUTS = 5 << 18
 
     def __init__(self, core, cfg, weights, dtype="fp32", fused=None):
         self.core = core.core if hasattr(core, "core") else core
@@ -157,6 +162,8 @@ class BertEncoder:
             raise ValueError(f"the fused layer needs d_model and d_ff to be multiples of {slab} in {dtype}")
         self.fused = eligible if fused is None else bool(fused)
         self._fused_min_rows = self.FUSED_MIN_ROWS if fused is None else 0
+        few = fused is None and self.fused and self.code == L.GRL_BF16
+        self._rows_max = self.ROWS_MAX_OUTPUTS // cfg.d_ff if few else 0
         self.fused_structs = []
         if self.fused:
             # every GEMM that reads a LayerNorm's output gets that norm folded into its weight (once, here):
@@ -164,17 +171,19 @@ class BertEncoder:
             d, ff = cfg.d_model, cfg.d_ff
             es = 2 if self.code == L.GRL_BF16 else 4
 
-            def fold(w_ptr, b_ptr, g_ptr, bt_ptr, n, k):
+            def fold(w, b_ptr, g_ptr, bt_ptr, n, k):
+                raw = c.upload(w)
                 ws, cs, bf = self._own(c.alloc(n * k * es)), self._own(c.alloc(n * 4)), self._own(c.alloc(n * 4))
-                L.check(c.lib.grl_ln_fold(c.ctx, self.code, n, k, w_ptr, g_ptr, bt_ptr, b_ptr, ws.ptr, cs.ptr, bf.ptr), "fold layernorm")
+                L.check(c.lib.grl_ln_fold_f32(c.ctx, self.code, n, k, raw.ptr, g_ptr, bt_ptr, b_ptr, ws.ptr, cs.ptr, bf.ptr), "fold layernorm")
+                raw.free()
                 return ws.ptr, cs.ptr, bf.ptr
             in_g, in_b = self.emb_g.ptr, self.emb_b.ptr
-            for s in self.layer_structs:
+            for s, lw in zip(self.layer_structs, weights["layers"]):
                 f = L.BertLayerFused()
-                f.ws_qkv, f.c_qkv, f.bf_qkv = fold(s.w_qkv, s.b_qkv, in_g, in_b, 3 * d, d)
+                f.ws_qkv, f.c_qkv, f.bf_qkv = fold(lw["w_qkv"], s.b_qkv, in_g, in_b, 3 * d, d)
                 f.in_g, f.in_b = in_g, in_b
                 f.w_o, f.b_o, f.ln1_g, f.ln1_b = s.w_o, s.b_o, s.ln1_g, s.ln1_b
-                f.ws_ff1, f.c_ff1, f.bf_ff1 = fold(s.w_ff1, s.b_ff1, s.ln1_g, s.ln1_b, ff, d)
+                f.ws_ff1, f.c_ff1, f.bf_ff1 = fold(lw["w_ff1"], s.b_ff1, s.ln1_g, s.ln1_b, ff, d)
                 f.w_ff2, f.b_ff2 = s.w_ff2, s.b_ff2
                 self.fused_structs.append(f)
                 in_g, in_b = s.ln2_g, s.ln2_b
@@ -195,7 +204,7 @@ class BertEncoder:
         es = 2 if self.code == L.GRL_BF16 else 4
         self.fused_now = self.fused and B * S >= self._fused_min_rows        # which layer form this batch runs
         ws = c.lib.grl_bert_layer_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff)
-        if self.fused_now:                   # without its padding the batch may run either form
+        if self.fused:                       # without its padding the batch may run any form
             ws = max(ws, c.lib.grl_bert_layer_fused_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff))
         self.x = c.alloc(B * S * cfg.d_model * es)
         self.stats = c.alloc(max(B * S, 1) * 8)        # {1/sd, mean/sd} per row of the raw residual stream (fused layers)
@@ -240,7 +249,16 @@ class BertEncoder:
         B, S = self._shape
         cfg, c, lib = self.cfg, self.core, self.core.lib
         mask = self.mask.ptr if self.has_mask else None
-        if self.fused_now and B * S > 0:
+        if 0 < B * S <= self._rows_max:
+            L.check(lib.grl_embed(c.ctx, self.code, B, S, cfg.d_model, cfg.vocab, self.ids.ptr, self.tok.ptr, self.pos.ptr,
+                                  self.typ.ptr, self.x.ptr), "embedding")
+            in_eps = cfg.embedding_eps
+            for f in self.fused_structs:
+                L.check(lib.grl_bert_layer_fwd_rows(c.ctx, self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f), mask,
+                                                    in_eps, cfg.eps, self.x.ptr, self.ws.ptr), "bert_layer_fwd_rows")
+                in_eps = cfg.eps
+            self._last_layernorm(B * S)
+        elif self.fused_now and B * S > 0:
             # raw embedding rows + their statistics; every layer consumes and produces (raw rows, statistics); the last
             # layer's second LayerNorm is the one pass that writes normalised rows
             L.check(lib.grl_embed(c.ctx, self.code, B, S, cfg.d_model, cfg.vocab, self.ids.ptr, self.tok.ptr, self.pos.ptr,
@@ -249,9 +267,7 @@ class BertEncoder:
             for f in self.fused_structs:
                 L.check(lib.grl_bert_layer_fwd_fused(c.ctx, self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f),
                                                      mask, cfg.eps, self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layer_fwd_fused")
-            last = self.layer_structs[-1]
-            L.check(lib.grl_layernorm(c.ctx, self.code, B * S, cfg.d_model, self.x.ptr, None, last.ln2_g, last.ln2_b, cfg.eps,
-                                      self.x.ptr), "final layernorm")
+            self._last_layernorm(B * S)
         else:
             L.check(lib.grl_embed_layernorm(c.ctx, self.code, B, S, cfg.d_model, cfg.vocab, self.ids.ptr, self.tok.ptr,
                                             self.pos.ptr, self.typ.ptr, self.emb_g.ptr, self.emb_b.ptr, cfg.embedding_eps,
@@ -262,20 +278,33 @@ class BertEncoder:
         if pool:
             L.check(lib.grl_mean_pool(c.ctx, self.code, B, S, cfg.d_model, self.x.ptr, mask, self.pooled.ptr, 1), "mean_pool")
 
+    def _last_layernorm(self, rows):
+        """raw rows -> the last layer's normalised ones"""
+        c, last = self.core, self.layer_structs[-1]
+        L.check(c.lib.grl_layernorm(c.ctx, self.code, rows, self.cfg.d_model, self.x.ptr, None, last.ln2_g, last.ln2_b, self.cfg.eps,
+                                    self.x.ptr), "final layernorm")
+
     def _launch_packed(self, rg, ids):
         """launch() on the batch without its padding, always pooled"""
         cfg, c, lib = self.cfg, self.core, self.core.lib
         r = ctypes.byref(rg)
-        if self.fused and rg.rows >= self._fused_min_rows and rg.rows > 0:
+        if 0 < rg.rows <= self._rows_max:
+            L.check(lib.grl_embed_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
+                                         self.x.ptr), "embedding")
+            in_eps = cfg.embedding_eps
+            for f in self.fused_structs:
+                L.check(lib.grl_bert_layer_fwd_rows_ragged(c.ctx, self.code, r, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f), in_eps,
+                                                           cfg.eps, self.x.ptr, self.ws.ptr), "bert_layer_fwd_rows")
+                in_eps = cfg.eps
+            self._last_layernorm(rg.rows)
+        elif self.fused and rg.rows >= self._fused_min_rows and rg.rows > 0:
             L.check(lib.grl_embed_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
                                          self.x.ptr), "embedding")
             L.check(lib.grl_ln_stats(c.ctx, self.code, rg.rows, cfg.d_model, self.x.ptr, cfg.embedding_eps, self.stats.ptr), "embedding statistics")
             for f in self.fused_structs:
                 L.check(lib.grl_bert_layer_fwd_fused_ragged(c.ctx, self.code, r, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f), cfg.eps,
                                                             self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layer_fwd_fused")
-            last = self.layer_structs[-1]
-            L.check(lib.grl_layernorm(c.ctx, self.code, rg.rows, cfg.d_model, self.x.ptr, None, last.ln2_g, last.ln2_b, cfg.eps,
-                                      self.x.ptr), "final layernorm")
+            self._last_layernorm(rg.rows)
         else:
             L.check(lib.grl_embed_layernorm_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
                                                    self.emb_g.ptr, self.emb_b.ptr, cfg.embedding_eps, self.x.ptr), "embedding + layernorm")
@@ -373,6 +402,12 @@ class PreNormEncoder:
         if not isinstance(self.core, HipCore):
             raise TypeError("PreNormEncoder needs a Compute() backend or its HipCore")
         self._stats_from_gemm = stats_from_gemm        # None: wherever the kernel takes the width
+        # Few rows (rows x d_ff up to this): the gated GEMM takes the statistics of its rows itself.  us per forward of 22 layers,
+        # 768 wide, d_ff 1152: bf16 20 rows 824 -> 678, 512 rows 1169 -> 1082, 768 rows 1186 -> 1196; fp32 20 rows 1630 -> 1084,
+        # 896 rows 3327 -> 2829, 1280 rows 3915 -> 3744, 2048 rows 5629 -> 5651
+        half = dtype_code(dtype) == L.GRL_BF16
+        takes = cfg.d_model % (64 if half else 32) == 0 and cfg.d_ff % 4 == 0
+        self._own_max = (5 << 17 if half else 7 << 18) if stats_from_gemm is None and takes else 0
         if cfg.head_dim * cfg.heads != cfg.d_model or cfg.head_dim % 2 or cfg.head_dim > 128:
             raise ValueError("d_model must be heads*head_dim with an even head_dim up to 128 (rotary positions)")
         self.cfg, self.dtype, self.code = cfg, dtype, dtype_code(dtype)
@@ -393,10 +428,10 @@ class PreNormEncoder:
             entry.update({k: vec(lw[k]) for k in ("b_qkv", "b_o", "b_ff2")})
             g, bt = c.upload(np.asarray(lw["ffn_ln_g"], np.float32).reshape(-1)), c.upload(np.asarray(lw["ffn_ln_b"], np.float32).reshape(-1))
             for name in ("gate", "in"):
-                raw = c.upload(lw["w_ff_" + name], self.code)
+                raw = c.upload(lw["w_ff_" + name])
                 b = c.upload(np.asarray(lw["b_ff_" + name], np.float32).reshape(-1))
                 ws, cs, bf = self._own(c.alloc(ff * d * es)), self._own(c.alloc(ff * 4)), self._own(c.alloc(ff * 4))
-                L.check(c.lib.grl_ln_fold(c.ctx, self.code, ff, d, raw.ptr, g.ptr, bt.ptr, b.ptr, ws.ptr, cs.ptr, bf.ptr), "fold mlp layernorm")
+                L.check(c.lib.grl_ln_fold_f32(c.ctx, self.code, ff, d, raw.ptr, g.ptr, bt.ptr, b.ptr, ws.ptr, cs.ptr, bf.ptr), "fold mlp layernorm")
                 entry["ws_" + name], entry["cs_" + name], entry["bf_" + name] = ws, cs, bf
                 raw.free(); b.free()
             g.free(); bt.free()
@@ -477,6 +512,7 @@ class PreNormEncoder:
         cfg, c, lib, code = self.cfg, self.core, self.core.lib, self.code
         M, d, ff, H, D = B * S if rg is None else rg.rows, cfg.d_model, cfg.d_ff, cfg.heads, cfg.head_dim
         es = 2 if code == L.GRL_BF16 else 4
+        own_stats = 0 < M * ff <= self._own_max
         if rg is None:
             mask = self.mask.ptr if self.has_mask else None
             L.check(lib.grl_embed_layernorm(c.ctx, code, B, S, d, cfg.vocab, ids, self.tok.ptr, None, None,
@@ -497,7 +533,13 @@ class PreNormEncoder:
                 L.check(lib.grl_fa2_fwd_ragged(c.ctx, code, ctypes.byref(rg), H, D, q, k, v, self.att.ptr, 3 * d, 3 * d, 3 * d, d, scale, 0,
                                                L.ROPE_HALF, cfg.rope_base, cfg.rope_scaling), "attention")
             # LayerNorm + dual GEMM; the dual GEMM activates its second ("up") operand: that is the first half of Wi here
-            if self.stats_from_gemm:
+            if own_stats:
+                L.check(lib.grl_gemm_nt_res(c.ctx, code, code, M, d, d, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,
+                                            self.x.ptr), "output projection + residual")
+                L.check(lib.grl_ln_glu_nt_rows(c.ctx, code, M, ff, d, self.x.ptr, w["ws_gate"].ptr, w["ws_in"].ptr, w["cs_gate"].ptr,
+                                               w["cs_in"].ptr, w["bf_gate"].ptr, w["bf_in"].ptr, cfg.eps, self.h.ptr, L.EPI_GELU),
+                        "mlp layernorm + geglu")
+            elif self.stats_from_gemm:
                 L.check(lib.grl_gemm_nt_resln(c.ctx, code, M, d, d, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,
                                               self.ident_stats.ptr, self.ones.ptr, self.zeros.ptr, self.x.ptr, cfg.eps,
                                               self.stats.ptr, self.part.ptr), "output projection + residual + row statistics")

@@ -294,6 +294,9 @@ int grl_layernorm(grl_ctx* ctx, int dtype, int64_t rows, int64_t F, const void* 
  * LN(x), both weights folded with the same gamma / beta.  Statistics as grl_layernorm (biased variance, two passes). */
 int grl_ln_fold(grl_ctx* ctx, int dtype, int64_t N, int64_t K, const void* W, const float* gamma, const float* beta,
                 const float* bias /* (N) or NULL */, void* W_scaled, float* colsum, float* bias_folded);
+/* the same from an fp32 weight, rounded to the storage type once (after the scaling) */
+int grl_ln_fold_f32(grl_ctx* ctx, int dtype, int64_t N, int64_t K, const float* W, const float* gamma, const float* beta,
+                    const float* bias /* (N) or NULL */, void* W_scaled, float* colsum, float* bias_folded);
 int grl_ln_stats(grl_ctx* ctx, int dtype, int64_t rows, int64_t F, const void* x, float eps, float* stats);
 int grl_ln_gemm_nt(grl_ctx* ctx, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x,
                    const void* W_scaled, const float* colsum, const float* bias_folded /* (N) or NULL */, float eps,
@@ -328,10 +331,24 @@ int grl_gemm_nt_resln(grl_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, 
                       const float* bias, const void* R, const float* r_stats, const float* r_gamma, const float* r_beta,
                       void* C, float eps, float* stats_out, void* workspace);
 
+/* The products of an encoder layer of few rows, which then needs no LayerNorm pass and no statistics pass:
+ * grl_ln_gemm_nt_rows / grl_ln_glu_nt_rows are grl_ln_gemm_nt_stats / grl_ln_glu_nt_stats with the row statistics taken inside
+ * the product (the workgroups read their rows whole); stats_out, if not NULL, receives them: (M, 2) floats {1/sd, mean/sd}.
+ * grl_gemm_nt_lnres is grl_gemm_nt_resln without statistics of its result: C = A.W^T + bias + LayerNorm(R), C may be R.
+ * Same arguments otherwise; operands 16-byte aligned, K a multiple of 64 (bf16) / 32 (fp32), N a multiple of 4, else GRL_ERR_SHAPE.
+ * Any M, but made for the sizes where 32 x 32 tiles fit the chip a few times over. */
+int grl_ln_gemm_nt_rows(grl_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* W_scaled, const float* colsum,
+                        const float* bias_folded, float eps, float* stats_out, void* out, int epilogue);
+int grl_ln_glu_nt_rows(grl_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* Wg_scaled, const void* Wu_scaled,
+                       const float* colsum_gate, const float* colsum_up, const float* bias_gate_folded, const float* bias_up_folded,
+                       float eps, void* out, int activation);
+int grl_gemm_nt_lnres(grl_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias,
+                      const void* R, const float* r_stats, const float* r_gamma, const float* r_beta, void* C);
+
 /* out = a + b.  Replaces VulkanFNN.residual (shaders/fnn-residual.glsl:25-34).
  * grl_add, grl_gelu, grl_silu and grl_relu may run in place (out == a, out == b, y == x).
  * Every other entry point of this header needs its outputs distinct from its inputs unless its own
- * comment says otherwise (grl_gemm_nt_res, grl_gemm_nt_resln: C may be the residual; grl_bert_layer_fwd, grl_bert_layer_fwd_fused: x / r is
+ * comment says otherwise (grl_gemm_nt_res, grl_gemm_nt_resln, grl_gemm_nt_lnres: C may be the residual; grl_bert_layer_fwd, grl_bert_layer_fwd_fused: x / r is
  * updated in place). */
 int grl_add(grl_ctx* ctx, int dtype, int64_t n, const void* a, const void* b, void* out);
 /* Replaces VulkanFNN.activation_gelu (backend/fnn.py:285-342, shaders/activation-gelu.glsl:23-53). */
@@ -461,6 +478,13 @@ int grl_bert_layer_fwd_fused(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int6
                              void* r, float* stats, void* workspace);
 int grl_bert_layer_fwd_fused_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
                                     const grl_bert_layer_fused* w, float eps, void* r, float* stats, void* workspace);
+/* The folded layer for few rows in five launches (grl_ln_gemm_nt_rows, attention, grl_gemm_nt_lnres, grl_ln_gemm_nt_rows,
+ * grl_gemm_nt_lnres): only the raw rows r travel between layers.  in_eps: of the LayerNorm that turns r into the layer's input,
+ * eps: of ln1.  workspace: grl_bert_layer_fused_workspace bytes. */
+int grl_bert_layer_fwd_rows(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                            const grl_bert_layer_fused* w, const float* mask, float in_eps, float eps, void* r, void* workspace);
+int grl_bert_layer_fwd_rows_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
+                                   const grl_bert_layer_fused* w, float in_eps, float eps, void* r, void* workspace);
 
 #ifdef __cplusplus
 }

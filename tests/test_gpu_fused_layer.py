@@ -306,3 +306,70 @@ def test_resln_and_given_statistics_gemms_randomized(backend):
             if not inplace:
                 dC.free()
     print("worst", worst)
+
+
+# rows around the 32-row tiles, one row, slab counts that leave waves of a workgroup without one
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("M,K,N", [(1, 64, 4), (33, 128, 100), (128, 768, 768), (95, 320, 260)])
+def test_products_of_few_rows(backend, dtype, M, K, N):
+    """grl_ln_gemm_nt_rows / grl_ln_glu_nt_rows / grl_gemm_nt_lnres: folded LayerNorm with the kernel's own row statistics."""
+    c, code = backend.core, _code(dtype)
+    rng = np.random.default_rng(M + K + N)
+    tol, es, eps = (TOL_BF16 if dtype == "bf16" else TOL_F32), (2 if dtype == "bf16" else 4), 1e-5
+    x = _q(dtype, (rng.standard_normal((M, K)) * (0.5 + rng.random((M, 1))) + rng.standard_normal((M, 1))).astype(np.float32))
+    Ws = [(rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32) for _ in range(2)]
+    b = rng.standard_normal(N).astype(np.float32)
+    g, bt = (1 + 0.2 * rng.standard_normal(K)).astype(np.float32), (0.3 * rng.standard_normal(K)).astype(np.float32)
+    bufs = [c.upload(x, code), c.upload(b), c.upload(g), c.upload(bt), c.alloc(M * N * es), c.alloc(M * 8)]
+    dx, db, dg, dbt, out, st = bufs
+    folded = []
+    try:
+        for W in Ws:
+            raw = c.upload(W)
+            f = [c.alloc(N * K * es), c.alloc(N * 4), c.alloc(N * 4)]
+            bufs += [raw] + f
+            L.check(c.lib.grl_ln_fold_f32(c.ctx, code, N, K, raw.ptr, dg.ptr, dbt.ptr, db.ptr, f[0].ptr, f[1].ptr, f[2].ptr), "fold")
+            folded.append(f)
+        (w, cs, bf), (w2, cs2, bf2) = folded
+        ln = O.truth_layernorm(x, g, bt, eps)
+        pre, pre2 = O.truth_linear(ln, Ws[0], b), O.truth_linear(ln, Ws[1], b)
+        for epi, ref in ((L.EPI_NONE, pre), (L.EPI_GELU, O.truth_gelu(pre))):
+            L.check(c.lib.grl_ln_gemm_nt_rows(c.ctx, code, M, N, K, dx.ptr, w.ptr, cs.ptr, bf.ptr, eps, st.ptr, out.ptr, epi), "rows")
+            assert O.max_rel(c.download(out, (M, N), code), ref) < tol
+            # single-pass moments in fp32: a few ulp times 1 + (mean/sd)^2, here at most about 30
+            np.testing.assert_allclose(c.download(st, (M, 2)), _stats(x, eps), rtol=2e-4, atol=2e-5)
+        L.check(c.lib.grl_ln_glu_nt_rows(c.ctx, code, M, N, K, dx.ptr, w.ptr, w2.ptr, cs.ptr, cs2.ptr, bf.ptr, bf2.ptr, eps, out.ptr, L.EPI_GELU), "glu")
+        assert O.max_rel(c.download(out, (M, N), code), pre * O.truth_gelu(pre2)) < tol
+        # residual: LayerNorm(R) with given statistics, in place
+        R = _q(dtype, (2 * rng.standard_normal((M, N)) + 1).astype(np.float32))
+        g2, bt2 = (1 + 0.2 * rng.standard_normal(N)).astype(np.float32), (0.3 * rng.standard_normal(N)).astype(np.float32)
+        dR, ds, dg2, dbt2, dw = more = [c.upload(R, code), c.upload(_stats(R, eps).astype(np.float32)), c.upload(g2), c.upload(bt2), c.upload(Ws[0], code)]
+        bufs += more
+        L.check(c.lib.grl_gemm_nt_lnres(c.ctx, code, M, N, K, dx.ptr, dw.ptr, db.ptr, dR.ptr, ds.ptr, dg2.ptr, dbt2.ptr, dR.ptr), "lnres")
+        ref = O.truth_linear(x, _q(dtype, Ws[0]), b) + O.truth_layernorm(R, g2, bt2, eps)
+        assert O.max_rel(c.download(dR, (M, N), code), ref) < tol
+        assert c.lib.grl_gemm_nt_lnres(c.ctx, code, M, N, K + 8, dx.ptr, dw.ptr, db.ptr, dR.ptr, ds.ptr, dg2.ptr, dbt2.ptr, dR.ptr) == L.ERR_SHAPE
+    finally:
+        for t in bufs:
+            t.free()
+
+
+@pytest.mark.parametrize("pad", [False, True])
+@pytest.mark.parametrize("B,S", [(1, 1), (1, 37), (3, 50)])
+def test_encoder_of_few_rows_equals_the_seven_launch_one(backend, pad, B, S):
+    """The form small bf16 batches run against the oracle's float64 layers (one rounding of every stored activation)."""
+    cfg = EncoderConfig(layers=2, d_model=128, heads=2, d_ff=256, vocab=100, max_pos=64, eps=1e-5, emb_eps=1e-3)
+    w = random_bert_weights(cfg, seed=5)
+    rng = np.random.default_rng(B + S)
+    for lw in w["layers"]:
+        for k in ("ln1_g", "ln2_g"):
+            lw[k] = (1 + 0.2 * rng.standard_normal(lw[k].shape)).astype(np.float32)
+        for k in ("ln1_b", "ln2_b", "b_qkv", "b_o", "b_ff1", "b_ff2"):
+            lw[k] = (0.2 * rng.standard_normal(lw[k].shape)).astype(np.float32)
+    ids = rng.integers(0, 100, (B, S))
+    mask = (np.arange(S)[None] < np.maximum(1, S - 7 * np.arange(B))[:, None]).astype(np.int64) if pad else None
+    few, plain = BertEncoder(backend, cfg, w, dtype="bf16"), BertEncoder(backend, cfg, w, dtype="bf16", fused=False)
+    assert few._rows_max >= B * S
+    for pool in (True, False):
+        a, b = few.forward(ids, mask, pool=pool), plain.forward(ids, mask, pool=pool)
+        assert np.isfinite(a).all() and O.max_rel(a, b) < TOL_BF16
