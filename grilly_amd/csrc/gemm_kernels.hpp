@@ -534,7 +534,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_finish_kernel(GemmArgs p) {
 // OWN (with LN): the statistics of the tile's rows come from the operand fragments themselves: every workgroup reads its rows
 // whole, so it sums them and their squares on the way (two v_dot2 per two bf16 values, under the wait for the next slab), and the
 // tiles of the first column write them out for a later residual epilogue.  No statistics pass, no LayerNorm pass: the kernel
-// takes 6.2 us at 128 x 2304 x 768 in bf16, the plain one 5.4 behind a LayerNorm of 5.0.
+// takes 5.7 us at 128 x 2304 x 768 in bf16, the plain one 5.4 behind a LayerNorm of 5.0.
 // EPI_RESLN here adds LayerNorm(residual) like the kernels below and leaves the statistics of the result to its OWN consumer.
 template <typename T, typename OutT, int BM, int BN, int NSTG, int EPI, bool DUAL, bool LN = false, bool SPLITK = false, bool OWN = false>
 __global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {
@@ -599,6 +599,34 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {
         kt0 = (int)blockIdx.y * per;
         kt1 = kt0 + per < KT ? kt0 + per : KT;
     }
+    // What the epilogue needs besides the sums, requested in front of the first slab (raw: a conversion here would wait for it):
+    // behind the loop it is a memory round trip of its own (us at 128 rows: EPI_RESLN 6.8 -> 6.0, own statistics 6.2 -> 5.7)
+    constexpr int QPR = BNO / 4;                  // outputs per row in groups of four
+    constexpr int ITERS = BM * QPR / 256;
+    static_assert(BM * QPR % 256 == 0 && 256 % QPR == 0, "a thread keeps its columns");
+    typedef typename std::conditional<sizeof(OutT) == 2, u32x2, u32x4>::type quad_t;
+    const int cq = tid % QPR, n = n0 + cq * 4;    // N is a multiple of 4
+    auto col4 = [&](const float* v) { return v && n < p.N ? *(const f32x4*)(v + n) : f32x4{0.f, 0.f, 0.f, 0.f}; };
+    f32x4 b1 = {0.f, 0.f, 0.f, 0.f}, b2 = b1, c1 = b1, c2 = b1, g1 = b1, bt1 = b1;
+    quad_t resq[(EPI == EPI_RES || EPI == EPI_RESLN) ? ITERS : 1];
+    f32x2_t rst[((LN && !OWN) || EPI == EPI_RESLN) ? ITERS : 1];
+    if constexpr (!SPLITK) {
+        b1 = col4(p.bias);
+        if constexpr (DUAL) b2 = col4(p.bias2);
+        if constexpr (LN) { c1 = col4(p.ln_c); if constexpr (DUAL) c2 = col4(p.ln_c2); }
+        if constexpr (EPI == EPI_RESLN) { g1 = col4(p.res_gamma); bt1 = col4(p.res_beta); }
+#pragma unroll
+        for (int i = 0; i < ITERS; ++i) {
+            const int m = m0 + i * (256 / QPR) + tid / QPR;
+            if constexpr ((LN && !OWN) || EPI == EPI_RESLN)
+                rst[i] = m < p.M ? *(const f32x2_t*)((LN ? p.ln_stats : p.res_stats) + 2 * (int64_t)m) : f32x2_t{0.f, 0.f};
+            if constexpr (EPI == EPI_RES || EPI == EPI_RESLN) {
+                resq[i] = quad_t{};
+                if (m < p.M && n < p.N) resq[i] = *(const quad_t*)((const OutT*)p.residual + (int64_t)m * p.N + n);
+            }
+        }
+    }
+
     const int mine = kt1 - kt0 > wave ? (kt1 - kt0 - wave + 3) >> 2 : 0;      // slabs of this wave
     kt0 += wave;
 #pragma unroll
@@ -670,26 +698,10 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {
     if constexpr (OWN) moments[wave * 2 + lg][li] = mom;
     __syncthreads();
 
-    constexpr int QPR = BNO / 4;                  // outputs per row in groups of four
-    static_assert(BM * QPR % 256 == 0 && 256 % QPR == 0, "a thread keeps its columns");
-    const int cq = tid % QPR, n = n0 + cq * 4;
-    if (n >= p.N) return;                         // N is a multiple of 4
-    auto col4 = [&](const float* v) { return v ? *(const f32x4*)(v + n) : f32x4{0.f, 0.f, 0.f, 0.f}; };
-    f32x4 b1 = {0.f, 0.f, 0.f, 0.f}, b2 = b1, c1 = b1, c2 = b1;
-    f32x4 g1 = b1;
-    if constexpr (!SPLITK) {
-        b1 = col4(p.bias);
-        if constexpr (EPI == EPI_RESLN) {         // the beta of the residual's LayerNorm is a per-column constant like the bias
-            g1 = col4(p.res_gamma);
-            const f32x4 bt = col4(p.res_beta);
+    if (n >= p.N) return;
+    if constexpr (EPI == EPI_RESLN) b1 += bt1;     // the beta of the residual's LayerNorm is a per-column constant like the bias
 #pragma unroll
-            for (int e = 0; e < 4; ++e) b1[e] += bt[e];
-        }
-        if constexpr (DUAL) b2 = col4(p.bias2);
-        if constexpr (LN) { c1 = col4(p.ln_c); if constexpr (DUAL) c2 = col4(p.ln_c2); }
-    }
-#pragma unroll
-    for (int i = 0; i < BM * QPR / 256; ++i) {
+    for (int i = 0; i < ITERS; ++i) {
         const int r = i * (256 / QPR) + tid / QPR, m = m0 + r;
         if (m >= p.M) break;
         auto total = [&](int c, float (&v)[4]) {
@@ -714,8 +726,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {
                 rs = 1.0f / sd; rsm = mean / sd;
                 if (p.stats_out && n == 0) *(f32x2_t*)(p.stats_out + 2 * (int64_t)m) = f32x2_t{rs, rsm};
             } else if constexpr (LN) {
-                const f32x2_t t = *(const f32x2_t*)(p.ln_stats + 2 * (int64_t)m);
-                rs = t[0]; rsm = t[1];
+                rs = rst[i][0]; rsm = rst[i][1];
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = LN ? v[e] * rs - rsm * c1[e] + b1[e] : v[e] + b1[e];
@@ -732,13 +743,12 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {
                 else
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = epi_apply<EPI>(v[e], p);
-                if constexpr (EPI == EPI_RES) add4<OutT>((const OutT*)p.residual + o, v);
+                if constexpr (EPI == EPI_RES) add4<OutT>((const OutT*)&resq[i], v);
                 if constexpr (EPI == EPI_RESLN) {
-                    const f32x2_t t = *(const f32x2_t*)(p.res_stats + 2 * (int64_t)m);
                     float x[4] = {0.f, 0.f, 0.f, 0.f};
-                    add4<OutT>((const OutT*)p.residual + o, x);
+                    add4<OutT>((const OutT*)&resq[i], x);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = fmaf(fmaf(x[e], t[0], -t[1]), g1[e], v[e]);
+                    for (int e = 0; e < 4; ++e) v[e] = fmaf(fmaf(x[e], rst[i][0], -rst[i][1]), g1[e], v[e]);
                 }
             }
             store4<OutT>((OutT*)p.C + o, v[0], v[1], v[2], v[3]);
