@@ -209,14 +209,15 @@ class BertEncoder:
         self.x = c.alloc(B * S * cfg.d_model * es)
         self.stats = c.alloc(max(B * S, 1) * 8)        # {1/sd, mean/sd} per row of the raw residual stream (fused layers)
         self.ws = c.alloc(ws)
-        self.ids = c.alloc((B + 1 + 2 * B * S) * 4)    # token ids, or offsets | positions | ids of the batch without its padding
+        self.ids = c.alloc(B * S * 4)
+        self.packed = c.alloc((B + 1 + 2 * B * S) * 4) # offsets | positions | ids of the batch without its padding
         self.mask = c.alloc(B * S * 4)
         self.pooled = c.alloc(B * cfg.d_model * 4)
         self._shape = (B, S)
 
     def release_activations(self):
         if self._shape is not None:
-            for b in (self.x, self.stats, self.ws, self.ids, self.mask, self.pooled):
+            for b in (self.x, self.stats, self.ws, self.ids, self.packed, self.mask, self.pooled):
                 b.free()
             self._shape = None
 
@@ -245,7 +246,8 @@ class BertEncoder:
         self.has_mask = False
 
     def launch(self, pool=True):
-        """Enqueue one full forward on the context stream (no host synchronisation)."""
+        """Enqueue one full forward of the batch that set_inputs() or forward() had last, in its rectangular form, on the
+        context stream (no host synchronisation); its hidden states are left in x as (B, S, d)."""
         B, S = self._shape
         cfg, c, lib = self.cfg, self.core, self.core.lib
         mask = self.mask.ptr if self.has_mask else None
@@ -322,7 +324,8 @@ class BertEncoder:
         packs = p.kind == L.PACK_PREFIX or (p.kind == L.PACK_SCATTERED and self.code == L.GRL_F32)
         if pool and packs and not p.full and self.cfg.head_dim <= 128:
             self.prepare(p.B, p.S)
-            self._launch_packed(*p.upload(self.core, self.ids.ptr))
+            self._launch_packed(*p.upload(self.core, self.packed.ptr))
+            self.set_inputs(input_ids, attention_mask)      # what a launch() from here on reads; uploaded while the layers run
         else:
             if p.full:
                 self._set_full(p)
@@ -466,7 +469,8 @@ class PreNormEncoder:
             self.part = c.alloc(int(c.lib.grl_gemm_nt_resln_workspace(B * S, cfg.d_model)))
         self.qkv = c.alloc(3 * act)                    # packed (M, 3d): Q, K, V are its three column blocks
         self.h = c.alloc(B * S * cfg.d_ff * es)
-        self.ids = c.alloc((B + 1 + 2 * B * S) * 4)    # token ids, or offsets | positions | ids of the batch without its padding
+        self.ids = c.alloc(B * S * 4)
+        self.packed = c.alloc((B + 1 + 2 * B * S) * 4) # offsets | positions | ids of the batch without its padding
         self.mask = c.alloc(B * S * 4)
         first = np.zeros((B, S), np.float32)
         first[:, 0] = 1.0                              # "mean" over the first token only = that token
@@ -476,7 +480,7 @@ class PreNormEncoder:
 
     def release_activations(self):
         if self._shape is not None:
-            for b in (self.x, self.qkv, self.att, self.stats, self.h, self.ids, self.mask, self.first, self.pooled):
+            for b in (self.x, self.qkv, self.att, self.stats, self.h, self.ids, self.packed, self.mask, self.first, self.pooled):
                 b.free()
             if self.stats_from_gemm:
                 for b in (self.ident_stats, self.ones, self.zeros, self.part):
@@ -503,7 +507,7 @@ class PreNormEncoder:
     _set_full = BertEncoder._set_full
 
     def launch(self, pool=True):
-        """Enqueue one full forward on the context stream (no host synchronisation)."""
+        """Enqueue one full forward of the batch that set_inputs() or forward() had last (as in BertEncoder)."""
         self._launch(pool, None, self.ids.ptr)
 
     def _launch(self, pool, rg, ids):
@@ -568,7 +572,8 @@ class PreNormEncoder:
         p = _Packing(self.core.lib, input_ids, attention_mask, self.cfg.vocab)
         if pool and not p.full and p.kind == L.PACK_PREFIX and (p.data[1:p.B + 1] > p.data[:p.B]).all():
             self.prepare(p.B, p.S)
-            self._launch(True, *p.upload(self.core, self.ids.ptr))
+            self._launch(True, *p.upload(self.core, self.packed.ptr))
+            self.set_inputs(input_ids, attention_mask)      # as in BertEncoder
         else:
             if p.full and p.S > 0:
                 self._set_full(p)

@@ -124,3 +124,36 @@ def test_pooled_forward_without_padding(backend, dtype, arch, fused, form):
     assert O.max_rel(got, want) < (1e-5 if dtype == "fp32" else 7e-3)
     # a mask of ones is the same batch as no mask, bit for bit
     np.testing.assert_array_equal(enc.forward(ids, np.ones((B, S), np.int64)), enc.forward(ids, None))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("arch", ["bert", "prenorm"])
+@pytest.mark.parametrize("form", ["right", "left", "holes", "soft", "none"])
+def test_launch_after_a_pooled_forward(backend, dtype, arch, form):
+    """launch() runs the batch that forward() had last, whatever form that forward took: the same kernels on the same inputs
+    as after set_inputs(), so the same bits.  The batch before has the same shape and another mask, or none."""
+    B, S = 6, 75
+    rng = np.random.default_rng(12)
+    if arch == "bert":
+        cfg = EncoderConfig(layers=2, d_model=128, heads=2, d_ff=256, vocab=300, max_pos=S)
+        enc = BertEncoder(backend, cfg, random_bert_weights(cfg, seed=3, std=0.08), dtype=dtype)
+    else:
+        cfg = PreNormEncoderConfig(layers=2, d_model=128, heads=2, d_ff=192, vocab=300)
+        enc = PreNormEncoder(backend, cfg, random_prenorm_weights(cfg, seed=3, std=0.08), dtype=dtype)
+    masks = _masks(rng, B, S)
+    mask = masks.get(form)
+    ids, before = rng.integers(0, 300, (2, B, S))
+
+    def launched():
+        enc.launch(True)
+        return backend.core.download(enc.pooled, (B, cfg.d_model)), backend.core.download(enc.x, (B, S, cfg.d_model), enc.code)
+
+    enc.set_inputs(ids, mask)
+    want = launched()
+    for earlier in (None, masks["right"][::-1].copy()):
+        enc.forward(before, earlier)
+        enc.forward(ids, mask)
+        for _ in range(2):
+            for got, w in zip(launched(), want):
+                np.testing.assert_array_equal(got, w)
