@@ -68,6 +68,7 @@ SIGNATURES = {
     "grl_host_fa2": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64] + [c_void_p] * 5 + [c_float, c_int, c_int, c_float, c_float]),
     "grl_host_alloc": (c_void_p, [c_size_t]),
     "grl_host_free": (None, [c_void_p]),
+    "grl_numpy_handler": (c_void_p, []),
     "grl_d2d": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t]),
     "grl_memset": (c_int, [c_void_p, c_void_p, c_int, c_size_t]),
     "grl_sync": (c_int, [c_void_p]),

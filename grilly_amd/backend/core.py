@@ -5,6 +5,8 @@ One HipCore = one gfx950 device + one HIP stream + one caching buffer pool, all 
 libgrilly_hip.so.  numpy arrays are copied in and out; nothing here computes.
 """
 import ctypes
+import functools
+
 import numpy as np
 
 from .. import _lib as L
@@ -28,31 +30,40 @@ def host_f32(a):
     return np.ascontiguousarray(a, dtype=np.float32)
 
 
-class _ResultBlock:
-    """a block of pinned memory that a result array stands in; given back when the array (and every view of it) is gone"""
-    __slots__ = ("lib", "ptr", "__array_interface__")
-
-    def __init__(self, lib, ptr, shape):
-        self.lib, self.ptr = lib, ptr
-        self.__array_interface__ = {"shape": shape, "typestr": "<f4", "data": (ptr, False), "version": 3}
-
-    def __del__(self):
-        self.lib.grl_host_free(self.ptr)
+RECYCLED_MIN = 32 << 20         # smaller results: the C library recycles their memory itself
 
 
-RESULT_BLOCK_MIN = 1 << 20      # smaller results: numpy's own memory, which the allocator has at hand
+@functools.lru_cache(maxsize=None)
+def _result_allocator(lib):
+    """(numpy's PyDataMem_SetHandler, the library's allocator as numpy takes one), or None where numpy has no such interface
+    (before 1.22)"""
+    api = getattr(getattr(np, "_core", None) or np.core, "_multiarray_umath")._ARRAY_API
+    pointer, new = ctypes.pythonapi.PyCapsule_GetPointer, ctypes.pythonapi.PyCapsule_New
+    pointer.restype, pointer.argtypes = ctypes.c_void_p, [ctypes.py_object, ctypes.c_char_p]
+    new.restype, new.argtypes = ctypes.py_object, [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_void_p]
+    table = ctypes.cast(pointer(api, None), ctypes.POINTER(ctypes.c_void_p))
+    # slots of numpy's C interface (numpy/__multiarray_api.h): PyArray_GetNDArrayCFeatureVersion, PyDataMem_SetHandler
+    if ctypes.PYFUNCTYPE(ctypes.c_uint)(table[211])() < 0x0F:
+        return None
+    set_handler = ctypes.PYFUNCTYPE(ctypes.py_object, ctypes.py_object)(table[304])
+    return set_handler, new(lib.grl_numpy_handler(), b"mem_handler", None)
 
 
 def result_array(lib, shape):
-    """uninitialised float32 array for a result: from about 1 MiB on in recycled pinned memory, as long as there is some"""
+    """uninitialised float32 array for a result, numpy's own in every respect; a large one stands in recycled memory, whose
+    pages the process has already.  numpy keeps its allocator in a context variable, so no other thread or task sees it."""
     nbytes = 4
     for n in shape:
         nbytes *= int(n)
-    if nbytes >= RESULT_BLOCK_MIN:
-        ptr = lib.grl_host_alloc(nbytes)
-        if ptr:
-            return np.asarray(_ResultBlock(lib, ptr, tuple(int(n) for n in shape)))
-    return np.empty(shape, dtype=np.float32)
+    recycled = _result_allocator(lib) if nbytes >= RECYCLED_MIN else None
+    if recycled is None:
+        return np.empty(shape, dtype=np.float32)
+    set_handler, handler = recycled
+    usual = set_handler(handler)
+    try:
+        return np.empty(shape, dtype=np.float32)
+    finally:
+        set_handler(usual)
 
 
 class DeviceBuffer:

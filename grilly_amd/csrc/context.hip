@@ -1,5 +1,6 @@
 // Context, caching device-buffer pool, copies and the event stopwatch.
 #include "common.hpp"
+#include "hostcopy.hpp"
 #include <cstring>
 
 static thread_local char g_err[512] = "";
@@ -69,6 +70,7 @@ extern "C" void grl_destroy(grl_ctx* c) {
     grl_hostpipe_destroy(c->hostpipe);
     hipStreamDestroy(c->stream);
     delete c;
+    grl_host_trim();
 }
 
 extern "C" void* grl_stream(grl_ctx* c) { return c ? (void*)c->stream : nullptr; }
@@ -168,6 +170,7 @@ extern "C" int grl_pool_trim(grl_ctx* c) {
         kv.second.clear();
     }
     c->stats.bytes_cached = 0;
+    grl_host_trim();
     return GRL_OK;
 }
 

@@ -7,8 +7,8 @@
 //     its result straight into pinned memory;
 //   * large calls are cut into blocks of rows (sequences, for attention).  Blocks come in and are computed on the context's
 //     stream and leave on a second one, so both directions of PCIe are busy at once.  They come in through a ring of pinned
-//     chunks that a few host threads fill (hostcopy.cpp); results go straight into a recycled pinned block, or through a second
-//     ring into ordinary memory.  bf16 operands are converted by those threads, so half the bytes cross PCIe.
+//     chunks that a few host threads fill (hostcopy.cpp), and results leave through a second one that those threads empty.
+//     bf16 operands are converted by those threads, so half the bytes cross PCIe.
 #include "common.hpp"
 #include "hostcopy.hpp"
 #include <algorithm>
@@ -20,68 +20,14 @@ namespace {
 constexpr size_t SLAB = 2u << 20;                    // pinned slab of a small call
 // Rings of pinned chunks, 16 MiB per direction.  Chunks move by copy kernels: the copy engines need 10 us from one transfer
 // to the next (1 MiB: 37 GB/s, 512 KiB with an event behind each: 19 GB/s), kernels 2 us.
-constexpr size_t CHUNK = 1u << 20, SLOTS = 16;
+constexpr size_t CHUNK = 2u << 20, SLOTS = 8;
 constexpr size_t CHUNK_MIN = 256u << 10;
 constexpr size_t BLOCK = 8u << 20;                   // bytes moved per block of a large call: tying the two streams together costs 15 us a block
+constexpr size_t PAST_CACHES = 4u << 20;             // results from this size on are copied to the caller past the caches (4, 8, 16 MiB: level or ahead)
 constexpr size_t DIRECT = 64u << 10;                 // results up to this size are written into pinned memory by the operator's kernel
 constexpr int MAXBLOCKS = 8;
 
-// ---- memory for large results --------------------------------------------------------------------------------------
-// A fresh numpy array costs a page fault and the zeroing of every page before the result can be copied into it: 10 GB/s
-// against the 56 GB/s at which the result arrives.  Large results therefore live in pinned blocks that the copy engine writes
-// directly and that come back here when the array is collected.  At most RESULT_MAX of them exist, in use or waiting; beyond
-// that (a program that keeps its results) the caller gets ordinary memory.  A block outlives the context that filled it.
-constexpr size_t RESULT_MAX = 512u << 20;
-struct Results {
-    std::mutex mu;
-    std::map<char*, size_t> live, idle;
-    size_t total = 0;
-    static Results& get() { static Results* r = new Results(); return *r; }
-    void* take(size_t bytes) {
-        bytes = (bytes + (1u << 20) - 1) >> 20 << 20;
-        std::lock_guard<std::mutex> lk(mu);
-        auto best = idle.end();
-        for (auto it = idle.begin(); it != idle.end(); ++it)
-            if (it->second >= bytes && it->second <= bytes + bytes / 4 && (best == idle.end() || it->second < best->second)) best = it;
-        if (best != idle.end()) {
-            char* p = best->first;
-            live[p] = best->second;
-            idle.erase(best);
-            return p;
-        }
-        while (total + bytes > RESULT_MAX && !idle.empty()) {
-            hipHostFree(idle.begin()->first);
-            total -= idle.begin()->second;
-            idle.erase(idle.begin());
-        }
-        void* p = nullptr;
-        if (total + bytes > RESULT_MAX) return nullptr;
-        if (hipHostMalloc(&p, bytes, hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-        grl_host_touch(p, bytes);          // once per block: the process maps these pages one fault at a time
-        total += bytes;
-        live[(char*)p] = bytes;
-        return p;
-    }
-    void give(void* p) {
-        std::lock_guard<std::mutex> lk(mu);
-        auto it = live.find((char*)p);
-        if (it == live.end()) return;
-        idle[it->first] = it->second;
-        live.erase(it);
-    }
-    bool holds(const void* p, size_t bytes) {
-        std::lock_guard<std::mutex> lk(mu);
-        auto it = live.upper_bound((char*)p);
-        if (it == live.begin()) return false;
-        --it;
-        return (const char*)p + bytes <= it->first + it->second;
-    }
-};
-
 }  // namespace
-
-extern "C" void* grl_host_alloc(size_t bytes) { return bytes ? Results::get().take(bytes) : nullptr; }
-extern "C" void grl_host_free(void* p) { if (p) Results::get().give(p); }
 
 struct grl_hostpipe {
     std::mutex mu;                       // one large call of a context at a time
@@ -147,21 +93,14 @@ static int send(grl_hostpipe* h, hipStream_t s, int kind, void* dst, const void*
     return GRL_OK;
 }
 
-// Results on their way out.  fp32 into a result block: one transfer, enqueued at once.  bf16 (widened by the host threads, so
-// that half the bytes cross PCIe) and ordinary memory: chunks are requested as far ahead as the ring has room, and copied to
-// the caller in order.
+// Results on their way out: chunks are requested as far ahead as the ring has room, and copied to the caller in order (bf16
+// widened by the host threads, so that half the bytes cross PCIe).
 struct Outflow {
     grl_hostpipe* h; hipStream_t s;
+    bool past;                            // copied to the caller past the caches
     struct Piece { int kind; char* dst; const char* src; size_t n; hipEvent_t after; };
     std::vector<Piece> pieces;
     size_t asked = 0, taken = 0;          // pieces requested from the device, pieces delivered
-    bool straight = false;                // some transfer goes into a result block
-    int add_straight(void* dst, const void* src, size_t bytes, hipEvent_t after) {
-        if (after) GRL_CHECK_HIP(hipStreamWaitEvent(s, after, 0));
-        GRL_CHECK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-        straight = true;
-        return GRL_OK;
-    }
     void add(int kind, void* dst, const void* src, size_t n, hipEvent_t after) {
         const size_t es = kind == GRL_COPY_BF16_F32 ? 2 : 4, ed = 4;
         const size_t chunk = std::min(CHUNK, std::max(CHUNK_MIN, (n * es / 2 + 4095) / 4096 * 4096)) / es;
@@ -180,10 +119,7 @@ struct Outflow {
                 GRL_CHECK_HIP(hipEventRecord(h->down_done[asked % SLOTS], s));
                 ++asked;
             }
-            if (taken == asked) {
-                if (finish && straight) GRL_CHECK_HIP(hipStreamSynchronize(s));
-                return GRL_OK;
-            }
+            if (taken == asked) return GRL_OK;
             const hipEvent_t e = h->down_done[taken % SLOTS];
             if (finish) GRL_CHECK_HIP(hipEventSynchronize(e));
             else {
@@ -192,7 +128,7 @@ struct Outflow {
                 GRL_CHECK_HIP(q);
             }
             const Piece& p = pieces[taken];
-            grl_host_copy(p.kind, p.dst, h->ring_down + (taken % SLOTS) * CHUNK, p.n);
+            grl_host_copy(p.kind, p.dst, h->ring_down + (taken % SLOTS) * CHUNK, p.n, past);
             ++taken;
         }
     }
@@ -210,11 +146,8 @@ static int transfer_out(grl_ctx* c, int kind, void* dst, const void* src, size_t
     std::lock_guard<std::mutex> lk(h->mu);
     int rc = pipe_ready(c, h);
     if (rc) return rc;
-    Outflow o{h, c->stream};
-    if (kind == GRL_COPY_F32 && Results::get().holds(dst, n * 4)) {
-        rc = o.add_straight(dst, src, n * 4, nullptr);
-        if (rc) return rc;
-    } else o.add(kind, dst, src, n, nullptr);
+    Outflow o{h, c->stream, n * 4 >= PAST_CACHES};
+    o.add(kind, dst, src, n, nullptr);
     rc = o.pump(true);
     if (rc) hipStreamSynchronize(c->stream);        // nothing may still be writing into the ring
     return rc;
@@ -396,8 +329,9 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
     if (rows) step = step > 256 ? (step + 255) / 256 * 256 : (step + 15) / 16 * 16;
 
     std::vector<void*> owned;
-    bool straight[8] = {};
-    Outflow o{h, h->down};
+    size_t results = 0;
+    for (int i = 0; i < count; ++i) if (arrays[i].out) results += (size_t)arrays[i].n * 4;
+    Outflow o{h, h->down, results >= PAST_CACHES};
     auto body = [&]() -> int {
         for (int i = 0; i < count; ++i) {
             dev[i] = nullptr;
@@ -405,7 +339,6 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
             dev[i] = grl_malloc(c, std::max<size_t>(dsize(arrays[i]), 1));
             if (!dev[i]) return GRL_ERR_OOM;
             owned.push_back(dev[i]);
-            straight[i] = arrays[i].out && (dtype == GRL_F32 || arrays[i].f32) && Results::get().holds(arrays[i].out, (size_t)arrays[i].n * 4);
         }
         auto meanwhile = [&]() { return o.pump(false); };
         auto send_part = [&](int i, int64_t first, int64_t n) {
@@ -427,14 +360,9 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
             int r = op(u, m, part);
             if (r) return r;
             GRL_CHECK_HIP(hipEventRecord(h->out[b], c->stream));
-            const hipEvent_t after = h->out[b];      // for every output: chunks are requested later, whole transfers at once
             for (int i = 0; i < count; ++i) {
                 const HostArray& a = arrays[i];
-                if (!a.out) continue;
-                if (straight[i]) {
-                    r = o.add_straight(a.out + u * a.per_unit, part[i], (size_t)(m * a.per_unit) * 4, after);
-                    if (r) return r;
-                } else o.add(dtype == GRL_BF16 && !a.f32 ? GRL_COPY_BF16_F32 : GRL_COPY_F32, a.out + u * a.per_unit, part[i], (size_t)(m * a.per_unit), after);
+                if (a.out) o.add(dtype == GRL_BF16 && !a.f32 ? GRL_COPY_BF16_F32 : GRL_COPY_F32, a.out + u * a.per_unit, part[i], (size_t)(m * a.per_unit), h->out[b]);
             }
             if ((r = o.pump(false))) return r;
         }

@@ -5,12 +5,17 @@
 // 27.8 / 13.3, 4 threads 87.9 / 38.6, 8 threads 119.6 / 51.5 GB/s into pinned / fresh memory).  Conversions to and from bf16
 // ride along: half the bytes cross PCIe and no cast kernel runs.
 #include "hostcopy.hpp"
+#include "../../include/grilly_hip.h"
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <mutex>
+#include <pthread.h>
 #include <sched.h>
+#include <sys/mman.h>
 #include <thread>
 #include <unistd.h>
 #include <immintrin.h>
@@ -31,12 +36,38 @@ GRL_CLONES void from_bf16(uint32_t* __restrict d, const uint16_t* __restrict s, 
     for (size_t i = 0; i < n; ++i) d[i] = (uint32_t)s[i] << 16;
 }
 
-constexpr int TOUCH = -1;
+// float results past the caches: a store that misses reads its line first, so a result much larger than they are costs three
+// passes over memory the ordinary way and two this way (49 MiB into pages already mapped: 890 -> 600 us beside the transfers,
+// widened from bf16 690 -> 420).
+void stream(float* d, const float* s, size_t n) {
+    size_t i = 0;
+    for (; i < n && ((uintptr_t)(d + i) & 15u); ++i) d[i] = s[i];
+    for (; i + 8 <= n; i += 8) {
+        const __m128i a = _mm_loadu_si128((const __m128i*)(s + i)), b = _mm_loadu_si128((const __m128i*)(s + i + 4));
+        _mm_stream_si128((__m128i*)(d + i), a);
+        _mm_stream_si128((__m128i*)(d + i + 4), b);
+    }
+    for (; i < n; ++i) d[i] = s[i];
+    _mm_sfence();
+}
+void stream(uint32_t* d, const uint16_t* s, size_t n) {
+    const __m128i zero = _mm_setzero_si128();
+    size_t i = 0;
+    for (; i < n && ((uintptr_t)(d + i) & 15u); ++i) d[i] = (uint32_t)s[i] << 16;
+    for (; i + 8 <= n; i += 8) {
+        const __m128i a = _mm_loadu_si128((const __m128i*)(s + i));
+        _mm_stream_si128((__m128i*)(d + i), _mm_unpacklo_epi16(zero, a));
+        _mm_stream_si128((__m128i*)(d + i + 4), _mm_unpackhi_epi16(zero, a));
+    }
+    for (; i < n; ++i) d[i] = (uint32_t)s[i] << 16;
+    _mm_sfence();
+}
 
-void copy_range(int kind, void* dst, const void* src, size_t a, size_t b) {
+void copy_range(int kind, bool past, void* dst, const void* src, size_t a, size_t b) {
+    if (past && kind == GRL_COPY_F32) { stream((float*)dst + a, (const float*)src + a, b - a); return; }
+    if (past && kind == GRL_COPY_BF16_F32) { stream((uint32_t*)dst + a, (const uint16_t*)src + a, b - a); return; }
     if (kind == GRL_COPY_F32) memcpy((float*)dst + a, (const float*)src + a, (b - a) * sizeof(float));
     else if (kind == GRL_COPY_F32_BF16) to_bf16((uint16_t*)dst + a, (const uint32_t*)src + a, b - a);
-    else if (kind == TOUCH) for (size_t i = a * 4; i < b * 4; i += 4096) ((volatile char*)dst)[i] = 0;
     else from_bf16((uint32_t*)dst + a, (const uint16_t*)src + a, b - a);
 }
 
@@ -45,12 +76,12 @@ void copy_range(int kind, void* dst, const void* src, size_t a, size_t b) {
 class Crew {
 public:
     static Crew& get() { static Crew* c = new Crew(); return *c; }      // never destroyed: its threads sleep until the process ends
-    void copy(int kind, void* dst, const void* src, size_t n) {
+    void copy(int kind, void* dst, const void* src, size_t n, bool past) {
         constexpr size_t PIECE = 16 * 1024;                              // values
         // too small to share, a forked child (the threads stayed in the parent), or another thread's job is on: alone
-        if (n < 4 * PIECE || workers_ == 0 || getpid() != pid_ || !turn_.try_lock()) { copy_range(kind, dst, src, 0, n); return; }
+        if (n < 4 * PIECE || workers_ == 0 || getpid() != pid_ || !turn_.try_lock()) { copy_range(kind, past, dst, src, 0, n); return; }
         const size_t pieces = (n + PIECE - 1) / PIECE;
-        kind_ = kind; dst_ = dst; src_ = src; n_ = n; piece_ = PIECE;
+        kind_ = kind; past_ = past; dst_ = dst; src_ = src; n_ = n; piece_ = PIECE;
         next_.store(0, std::memory_order_relaxed);
         pieces_ = pieces;
         open_.store(true);
@@ -80,7 +111,7 @@ private:
     void work() {
         for (size_t i; (i = next_.fetch_add(1, std::memory_order_relaxed)) < pieces_;) {
             const size_t a = i * piece_, b = a + piece_ < n_ ? a + piece_ : n_;
-            copy_range(kind_, dst_, src_, a, b);
+            copy_range(kind_, past_, dst_, src_, a, b);
         }
     }
     void loop() {
@@ -105,12 +136,115 @@ private:
     std::atomic<bool> open_{false};
     size_t pieces_ = 0, n_ = 0, piece_ = 0;
     int kind_ = 0, workers_ = 0;
+    bool past_ = false;
     void* dst_ = nullptr;
     const void* src_ = nullptr;
     pid_t pid_ = 0;
 };
 
+// ---- memory for large results
+// The C library maps every block above 32 MiB afresh and unmaps it when it is freed, so a result of that size pays a fault and
+// the zeroing of every page: the 48 MiB result of a 4000 x 3072 x 768 product took 4.1 ms of numpy call in such memory, 1.7 ms
+// in pages the process has already (24 MiB results: 0.60 ms both ways).  Freed blocks are kept here and handed out again, up
+// to IDLE_MAX of them waiting.  They are ordinary private pages: a forked child has its own copy of them.
+class Results {
+public:
+    static Results& get() { static Results* r = new Results(); return *r; }     // never destroyed: arrays may outlive everything else
+    void* take(size_t bytes) {
+        const size_t len = (std::max<size_t>(bytes, 1) + PAGE - 1) / PAGE * PAGE;
+        if (len < bytes) return nullptr;
+        std::lock_guard<std::mutex> lk(mu_);
+        auto best = idle_.end();
+        for (auto it = idle_.begin(); it != idle_.end(); ++it)
+            if (it->second >= len && it->second <= len + len / 4 && (best == idle_.end() || it->second < best->second)) best = it;
+        if (best != idle_.end()) {
+            void* p = best->first;
+            live_[p] = best->second;
+            waiting_ -= best->second;
+            idle_.erase(best);
+            return p;
+        }
+        void* p = mmap(nullptr, len, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+        if (p == MAP_FAILED) return nullptr;
+        madvise(p, len, MADV_HUGEPAGE);
+        live_[p] = len;
+        return p;
+    }
+    size_t size(void* p) {
+        std::lock_guard<std::mutex> lk(mu_);
+        auto it = live_.find(p);
+        return it == live_.end() ? 0 : it->second;
+    }
+    void give(void* p) {
+        std::lock_guard<std::mutex> lk(mu_);
+        auto it = live_.find(p);
+        if (it == live_.end()) return;
+        const size_t len = it->second;
+        live_.erase(it);
+        drop_to(len > IDLE_MAX ? IDLE_MAX : IDLE_MAX - len);
+        if (len > IDLE_MAX) { munmap(p, len); return; }
+        idle_[p] = len;
+        waiting_ += len;
+    }
+    void trim() {
+        std::lock_guard<std::mutex> lk(mu_);
+        drop_to(0);
+    }
+
+private:
+    static constexpr size_t PAGE = 4096, IDLE_MAX = 512u << 20;
+    // a child forked while another thread is in here would find the lock taken for ever
+    Results() { pthread_atfork([] { get().mu_.lock(); }, [] { get().mu_.unlock(); }, [] { get().mu_.unlock(); }); }
+    void drop_to(size_t most) {
+        while (waiting_ > most) {
+            munmap(idle_.begin()->first, idle_.begin()->second);
+            waiting_ -= idle_.begin()->second;
+            idle_.erase(idle_.begin());
+        }
+    }
+    std::mutex mu_;
+    std::map<void*, size_t> live_, idle_;
+    size_t waiting_ = 0;
+};
+
+void* result_realloc(void*, void* p, size_t bytes) {
+    const size_t old = p ? Results::get().size(p) : 0;
+    if (p && bytes <= old && bytes >= old / 2) return p;
+    void* q = Results::get().take(bytes);
+    if (q && p) {
+        memcpy(q, p, std::min(old, bytes));
+        Results::get().give(p);
+    }
+    return q;
+}
+void* result_calloc(void*, size_t n, size_t each) {
+    size_t bytes;
+    if (__builtin_mul_overflow(n, each, &bytes)) return nullptr;
+    void* p = Results::get().take(bytes);
+    if (p) memset(p, 0, bytes);
+    return p;
+}
+
+// numpy's public allocator interface, version 1: PyDataMem_Handler of numpy/ndarraytypes.h
+struct NumpyHandler {
+    char name[127];
+    uint8_t version;
+    struct {
+        void* ctx;
+        void* (*malloc)(void*, size_t);
+        void* (*calloc)(void*, size_t, size_t);
+        void* (*realloc)(void*, void*, size_t);
+        void (*free)(void*, void*, size_t);
+    } allocator;
+};
+const NumpyHandler numpy_handler = {"grilly_results", 1, {nullptr, [](void*, size_t n) { return Results::get().take(n); }, result_calloc, result_realloc,
+                                                          [](void*, void* p, size_t) { if (p) Results::get().give(p); }}};
+
 }  // namespace
 
-void grl_host_touch(void* p, size_t bytes) { Crew::get().copy(TOUCH, p, p, bytes / 4); }
-void grl_host_copy(int kind, void* dst, const void* src, size_t n) { Crew::get().copy(kind, dst, src, n); }
+void grl_host_copy(int kind, void* dst, const void* src, size_t n, bool past_caches) { Crew::get().copy(kind, dst, src, n, past_caches); }
+void grl_host_trim() { Results::get().trim(); }
+
+extern "C" void* grl_host_alloc(size_t bytes) { return bytes ? Results::get().take(bytes) : nullptr; }
+extern "C" void grl_host_free(void* p) { if (p) Results::get().give(p); }
+extern "C" const void* grl_numpy_handler(void) { return &numpy_handler; }

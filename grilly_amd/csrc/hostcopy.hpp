@@ -5,7 +5,7 @@
 enum { GRL_COPY_F32 = 0,          // float -> float
        GRL_COPY_F32_BF16 = 1,     // float -> bf16 bits, round to nearest even, NaN stays NaN (as f32_to_bf16_bits on the device)
        GRL_COPY_BF16_F32 = 2 };   // bf16 bits -> float
-// n values from src to dst; returns when they are there
-void grl_host_copy(int kind, void* dst, const void* src, size_t n);
-// writes one byte of every 4 KiB page, so that the process has all of them mapped
-void grl_host_touch(void* p, size_t bytes);
+// n values from src to dst; returns when they are there.  past_caches: float values are stored without reading their lines first
+void grl_host_copy(int kind, void* dst, const void* src, size_t n, bool past_caches = false);
+// unmaps the result memory that no array stands in
+void grl_host_trim();

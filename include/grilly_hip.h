@@ -88,7 +88,7 @@ void*       grl_stream(grl_ctx* ctx);
 void* grl_malloc(grl_ctx* ctx, size_t bytes);
 int   grl_free(grl_ctx* ctx, void* ptr);
 int   grl_pool_get_stats(grl_ctx* ctx, grl_pool_stats* out);
-int   grl_pool_trim(grl_ctx* ctx);     /* return cached blocks to the driver */
+int   grl_pool_trim(grl_ctx* ctx);     /* return cached blocks to the driver, and waiting result memory to the system */
 
 /* Host <-> device copies, replacing _upload_buffer / _download_buffer (backend/core.py:345-360).  grl_h2d returns when
  * the host buffer has been consumed (the caller may reuse it at once); the transfer itself is ordered on the context
@@ -101,11 +101,13 @@ int grl_d2h(grl_ctx* ctx, void* dst_host, const void* src_dev, size_t bytes);
  * grl_h2d and grl_d2h. */
 int grl_upload(grl_ctx* ctx, int dtype, int64_t n, const float* src_host, void* dst_dev);
 int grl_download(grl_ctx* ctx, int dtype, int64_t n, const void* src_dev, float* dst_host);
-/* Pinned host memory for large results, recycled and bounded (512 MiB in all, NULL beyond that or when the driver refuses):
- * results written to it leave the device in one direct transfer.  grl_host_free gives a block back for reuse.  Both belong
- * to the process, not to a context; any thread may call them. */
+/* Host memory for large results: ordinary pages, recycled so that they need not be faulted in for every call.  grl_host_free
+ * gives a block back for reuse; up to 512 MiB wait for the next call, grl_pool_trim and grl_destroy return them.  They belong
+ * to the process, not to a context; any thread may call them.  grl_numpy_handler is the same memory as numpy's allocator
+ * interface (PyDataMem_Handler, version 1). */
 void* grl_host_alloc(size_t bytes);
 void  grl_host_free(void* ptr);
+const void* grl_numpy_handler(void);
 int grl_d2d(grl_ctx* ctx, void* dst_dev, const void* src_dev, size_t bytes);
 int grl_memset(grl_ctx* ctx, void* dst_dev, int byte, size_t bytes);
 int grl_sync(grl_ctx* ctx);

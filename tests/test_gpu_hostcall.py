@@ -1,5 +1,6 @@
 """Operators on host arrays: the sizes where the path changes (one pinned slab / rings and blocks, results written in place /
-copied back / in recycled pinned memory), transfers of odd byte counts, results that are kept, and calls from several threads."""
+copied back in one piece or in chunks), transfers of odd byte counts, results that are kept, and calls from several threads."""
+import os
 import threading
 
 import numpy as np
@@ -76,8 +77,8 @@ def test_bf16_transfers_round_to_nearest_even(backend, n):
 
 
 def test_kept_results_stay_what_they_were(backend):
-    """Results of a program that keeps them are its own: more of them than there is recycled memory for (512 MiB), views that
-    outlive their array, and none changed by later calls."""
+    """Results of a program that keeps them are its own: more of them than wait for reuse (512 MiB), views that outlive their
+    array, and none changed by later calls."""
     n = 1 << 24                                      # 64 MiB each
     kept = []
     for i in range(10):
@@ -110,3 +111,35 @@ def test_large_calls_from_several_threads(backend):
     for t in threads:
         t.join(timeout=100)
     assert not errors and not any(t.is_alive() for t in threads)
+
+
+def test_results_are_the_callers_own(backend):
+    """A large result is an array like any other: numpy owns and resizes it, a forked child reads it and has its own copy of
+    it, and a program that trims gets the memory of collected results back."""
+    n = 3 << 22                                      # 48 MiB
+    def result(v):
+        return backend.fnn.residual(np.full(n, v, np.float32), np.full(n, 0.5, np.float32))
+
+    y = result(3)
+    assert y.flags.owndata and y.base is None
+    for size in (n // 3, n):
+        y.resize(size, refcheck=False)
+        assert y.shape == (size,) and (y[:n // 3] == 3.5).all()
+    y = result(4)
+    child = os.fork()
+    if child == 0:
+        good = bool((y == 4.5).all())
+        y[:] = 7.0
+        z = np.empty(n, np.float32)
+        z[:] = y
+        os._exit(0 if good and (z == 7.0).all() else 1)
+    assert os.waitpid(child, 0)[1] == 0
+    assert (y == 4.5).all()
+
+    def resident():
+        return int(open("/proc/self/statm").read().split()[1]) * 4096
+
+    del y
+    before = resident()
+    L.check(backend.core.lib.grl_pool_trim(backend.core.ctx))
+    assert resident() <= before - n * 4
