@@ -12,6 +12,7 @@
 #include "common.hpp"
 #include "hostcopy.hpp"
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <functional>
 
@@ -30,6 +31,7 @@ constexpr int MAXBLOCKS = 8;
 }  // namespace
 
 struct grl_hostpipe {
+    std::atomic<bool> refused{false};    // pinned memory was refused once: what needs more of it runs on the runtime's own copies
     std::mutex mu;                       // one large call of a context at a time
     std::mutex slab_mu;
     std::vector<char*> slabs;            // free slabs of small calls (at most as many as calls have run at once)
@@ -56,18 +58,50 @@ void grl_hostpipe_destroy(grl_hostpipe* h) {
     delete h;
 }
 
-// streams, rings and events of the large calls, on first use (under h->mu)
+// pinned memory, or nullptr where the driver refuses it (a limit of the container, a full host): that is no error
+static char* pinned(grl_ctx* c, size_t bytes) {
+    void* p = nullptr;
+    if (c->hostpipe->refused) return nullptr;
+    if (hipSetDevice(c->device) == hipSuccess && hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess && p) return (char*)p;
+    (void)hipGetLastError();
+    c->hostpipe->refused = true;
+    return nullptr;
+}
+
+// streams, rings and events of the large calls, on first use (under h->mu); h->ready stays false where pinned memory is refused
 static int pipe_ready(grl_ctx* c, grl_hostpipe* h) {
     if (h->ready) return GRL_OK;
-    GRL_CHECK_HIP(hipSetDevice(c->device));
+    if (!h->ring_up && !(h->ring_up = pinned(c, CHUNK * SLOTS))) return GRL_OK;
+    if (!h->ring_down && !(h->ring_down = pinned(c, CHUNK * SLOTS))) return GRL_OK;
     if (!h->down) GRL_CHECK_HIP(hipStreamCreateWithFlags(&h->down, hipStreamNonBlocking));
-    if (!h->ring_up) GRL_CHECK_HIP(hipHostMalloc((void**)&h->ring_up, CHUNK * SLOTS, hipHostMallocDefault));
-    if (!h->ring_down) GRL_CHECK_HIP(hipHostMalloc((void**)&h->ring_down, CHUNK * SLOTS, hipHostMallocDefault));
     auto event = [](hipEvent_t& e) { return e ? hipSuccess : hipEventCreateWithFlags(&e, hipEventDisableTiming); };
     for (auto& e : h->up_done) GRL_CHECK_HIP(event(e));
     for (auto& e : h->down_done) GRL_CHECK_HIP(event(e));
     for (auto& e : h->out) GRL_CHECK_HIP(event(e));
     h->ready = true;
+    return GRL_OK;
+}
+
+// Without pinned memory: the runtime's copies of pageable memory, one at a time and waited for.  n values (kind
+// GRL_COPY_F32_BF16 / GRL_COPY_BF16_F32, converted through a buffer) or, for GRL_COPY_F32, n bytes.
+static int plain_in(grl_ctx* c, int kind, void* dst, const void* src, size_t n) {
+    std::vector<uint16_t> half;
+    if (kind == GRL_COPY_F32_BF16) {
+        half.resize(n);
+        grl_host_copy(kind, half.data(), src, n);
+        src = half.data();
+        n *= 2;
+    }
+    GRL_CHECK_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c->stream));
+    GRL_CHECK_HIP(hipStreamSynchronize(c->stream));
+    return GRL_OK;
+}
+static int plain_out(grl_ctx* c, int kind, void* dst, const void* src, size_t n) {
+    std::vector<uint16_t> half(kind == GRL_COPY_BF16_F32 ? n : 0);
+    const bool widen = !half.empty();
+    GRL_CHECK_HIP(hipMemcpyAsync(widen ? (void*)half.data() : dst, src, widen ? n * 2 : n, hipMemcpyDeviceToHost, c->stream));
+    GRL_CHECK_HIP(hipStreamSynchronize(c->stream));
+    if (widen) grl_host_copy(kind, dst, half.data(), n);
     return GRL_OK;
 }
 
@@ -139,13 +173,16 @@ static int transfer_in(grl_ctx* c, int kind, void* dst, const void* src, size_t 
     grl_hostpipe* h = c->hostpipe;
     std::lock_guard<std::mutex> lk(h->mu);
     int rc = pipe_ready(c, h);
-    return rc ? rc : send(h, c->stream, kind, dst, src, n, nullptr);
+    if (rc) return rc;
+    if (!h->ready) return plain_in(c, kind, dst, src, kind == GRL_COPY_F32 ? n * 4 : n);
+    return send(h, c->stream, kind, dst, src, n, nullptr);
 }
 static int transfer_out(grl_ctx* c, int kind, void* dst, const void* src, size_t n) {
     grl_hostpipe* h = c->hostpipe;
     std::lock_guard<std::mutex> lk(h->mu);
     int rc = pipe_ready(c, h);
     if (rc) return rc;
+    if (!h->ready) return plain_out(c, kind, dst, src, kind == GRL_COPY_F32 ? n * 4 : n);
     Outflow o{h, c->stream, n * 4 >= PAST_CACHES};
     o.add(kind, dst, src, n, nullptr);
     rc = o.pump(true);
@@ -153,6 +190,7 @@ static int transfer_out(grl_ctx* c, int kind, void* dst, const void* src, size_t
     return rc;
 }
 
+// nullptr: pinned memory is refused
 static char* take_slab(grl_ctx* c) {
     grl_hostpipe* h = c->hostpipe;
     char* s = nullptr;
@@ -163,13 +201,7 @@ static char* take_slab(grl_ctx* c) {
     std::lock_guard<std::mutex> pool(c->mu);          // a slab is a pool block too, as far as the statistics go
     if (s) { c->stats.hits++; return s; }
     c->stats.misses++;
-    void* p = nullptr;
-    if (hipSetDevice(c->device) != hipSuccess || hipHostMalloc(&p, SLAB, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        grl_set_error("pinned host memory: hipHostMalloc(%zu) failed", SLAB);
-        return nullptr;
-    }
-    return (char*)p;
+    return pinned(c, SLAB);
 }
 static void give_slab(grl_ctx* c, char* s) {
     std::lock_guard<std::mutex> lk(c->hostpipe->slab_mu);
@@ -190,8 +222,7 @@ constexpr size_t STAGE_RING = 4u << 20, SMALL_COPY = 256u << 10;
 static int stage_in(grl_ctx* c, int kind, void* dst, const void* src, size_t bytes, size_t n) {
     std::lock_guard<std::mutex> lk(c->stage_mu);
     if (!c->stage) {
-        GRL_CHECK_HIP(hipSetDevice(c->device));
-        GRL_CHECK_HIP(hipHostMalloc((void**)&c->stage, STAGE_RING, hipHostMallocDefault));
+        if (!(c->stage = pinned(c, STAGE_RING))) return plain_in(c, kind, dst, src, kind == GRL_COPY_F32 ? bytes : n);
         c->stage_cap = STAGE_RING;
     }
     if (c->stage_off + bytes > c->stage_cap) {
@@ -209,7 +240,7 @@ static int stage_in(grl_ctx* c, int kind, void* dst, const void* src, size_t byt
 // device -> host, small: a copy kernel writes into a pinned slab
 static int slab_out(grl_ctx* c, int kind, void* dst, const void* src, size_t bytes, size_t n) {
     char* slab = take_slab(c);
-    if (!slab) return GRL_ERR_OOM;
+    if (!slab) return plain_out(c, kind, dst, src, kind == GRL_COPY_F32 ? bytes : n);
     int rc = grl_copy_bytes_launch(c, slab, src, bytes);
     const hipError_t e = hipStreamSynchronize(c->stream);
     if (!rc && e != hipSuccess) { grl_set_error("grl_d2h: %s", hipGetErrorString(e)); rc = GRL_ERR_HIP; }
@@ -267,6 +298,27 @@ struct HostArray {
     bool f32;                         // keeps 32 bits on the device whatever the storage type (biases, masks, caches)
 };
 
+// run_on_host without pinned memory: everything in, the whole operator, everything out
+int run_plain(grl_ctx* c, int dtype, int64_t units, HostArray* arrays, int count, const std::function<int(int64_t, int64_t, void**)>& op) {
+    void* dev[8] = {};
+    auto half = [&](const HostArray& a) { return dtype == GRL_BF16 && !a.f32; };
+    int rc = GRL_OK;
+    for (int i = 0; i < count && !rc; ++i) {
+        const HostArray& a = arrays[i];
+        if (!a.in && !a.out) continue;
+        dev[i] = grl_malloc(c, std::max<size_t>((size_t)a.n * (half(a) ? 2 : 4), 1));
+        if (!dev[i]) rc = GRL_ERR_OOM;
+        else if (a.in && a.n) rc = plain_in(c, half(a) ? GRL_COPY_F32_BF16 : GRL_COPY_F32, dev[i], a.in, (size_t)a.n * (half(a) ? 1 : 4));
+    }
+    if (!rc) rc = op(0, units, dev);
+    for (int i = 0; i < count && !rc; ++i) {
+        const HostArray& a = arrays[i];
+        if (a.out && a.n) rc = plain_out(c, half(a) ? GRL_COPY_BF16_F32 : GRL_COPY_F32, a.out, dev[i], (size_t)a.n * (half(a) ? 1 : 4));
+    }
+    for (void* p : dev) grl_free(c, p);
+    return rc;
+}
+
 // Runs op(first unit, units, device pointers of the arrays at `first unit`) over `units` rows (rows == true) or sequences.
 int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arrays, int count, const std::function<int(int64_t, int64_t, void**)>& op) {
     grl_hostpipe* h = c->hostpipe;
@@ -279,7 +331,7 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
 
     if (ins + outs <= SLAB) {
         char* slab = take_slab(c);
-        if (!slab) return GRL_ERR_OOM;
+        if (!slab) return run_plain(c, dtype, units, arrays, count, op);
         const bool direct = outs <= DIRECT;
         grl_segments seg;
         void* owned[8] = {};
@@ -319,6 +371,7 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
     std::lock_guard<std::mutex> lk(h->mu);
     int rc = pipe_ready(c, h);
     if (rc) return rc;
+    if (!h->ready) return run_plain(c, dtype, units, arrays, count, op);
     // Blocks: enough of them that transfers in, work and transfers out overlap.
     size_t moving = 0;
     for (int i = 0; i < count; ++i) if (arrays[i].per_unit) moving += dsize(arrays[i]);
