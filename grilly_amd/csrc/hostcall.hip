@@ -2,9 +2,9 @@
 //
 // Bound: PCIe (56.7 GB/s each way measured, 48 + 48 with both directions busy), for small calls the latencies of launch and
 // wait (11 us for an empty kernel).  So:
-//   * small calls (2 MiB in and out together) never touch the copy engines, whose hand-over to the compute queue costs 10 us
-//     each way: inputs are packed into one pinned slab, one copy kernel brings them in, and the operator's own kernel writes
-//     its result straight into pinned memory;
+//   * small calls (5 MiB in and out together) never touch the copy engines, whose hand-over to the compute queue costs 10 us
+//     each way, and no events: inputs are copied into one pinned slab, from where a kernel per MiB fetches them while the next
+//     are copied; results up to 64 KiB are written straight into the slab by the operator's kernel, larger ones by a copy kernel;
 //   * large calls are cut into blocks of rows (sequences, for attention).  Blocks come in and are computed on the context's
 //     stream and leave on a second one, so both directions of PCIe are busy at once.  They come in through a ring of pinned
 //     chunks that a few host threads fill (hostcopy.cpp), and results leave through a second one that those threads empty.
@@ -18,12 +18,20 @@
 
 namespace {
 
-constexpr size_t SLAB = 2u << 20;                    // pinned slab of a small call
+// Pinned slabs of small calls, and what counts as small.  us per fp32 call as a slab / through the rings, once the helper threads
+// are awake: linear with 1 MiB of weights 2.5 MiB 113 / 140, 3.5 MiB 141 / 160, 4.5 MiB 168 / 189, 5.5 MiB 203 / 208; attention
+// 3.5 MiB 138 / 159, 4.5 MiB 160 / 182, 5.5 MiB 189 / 202; linear with 256 columns 3.5 MiB 140 / 150, 5.5 MiB 198 / 196, 7.5 MiB
+// 276 / 243: where the result is most of it, the rings overlap its copies and the slab does not.
+constexpr size_t SLAB = 2u << 20, SLAB_MAX = 5u << 20;
+constexpr size_t SLAB_PART = 1u << 20;               // of a slab's inputs, fetched by the device while the next are copied (512 KiB: 3 - 5 % slower)
 // Rings of pinned chunks, 16 MiB per direction.  Chunks move by copy kernels: the copy engines need 10 us from one transfer
 // to the next (1 MiB: 37 GB/s, 512 KiB with an event behind each: 19 GB/s), kernels 2 us.
 constexpr size_t CHUNK = 2u << 20, SLOTS = 8;
 constexpr size_t CHUNK_MIN = 256u << 10;
-constexpr size_t BLOCK = 8u << 20;                   // bytes moved per block of a large call: tying the two streams together costs 15 us a block
+// Bytes moved per block of a large call: tying the two streams together costs 15 us a block, and a block of few sequences leaves
+// CUs idle.  Half of it: attention 12 MiB 334 -> 420 us, 20 MiB 530 -> 683, linear with 256 columns 12 MiB 344 -> 361.  Up to
+// 16 MiB there is one block: nothing but the host's own copies overlaps the transfers there.
+constexpr size_t BLOCK = 8u << 20;
 constexpr size_t PAST_CACHES = 4u << 20;             // results from this size on are copied to the caller past the caches (4, 8, 16 MiB: level or ahead)
 constexpr size_t DIRECT = 64u << 10;                 // results up to this size are written into pinned memory by the operator's kernel
 constexpr int MAXBLOCKS = 8;
@@ -34,7 +42,8 @@ struct grl_hostpipe {
     std::atomic<bool> refused{false};    // pinned memory was refused once: what needs more of it runs on the runtime's own copies
     std::mutex mu;                       // one large call of a context at a time
     std::mutex slab_mu;
-    std::vector<char*> slabs;            // free slabs of small calls (at most as many as calls have run at once)
+    struct slab { char* p; size_t cap; };
+    std::vector<slab> slabs;             // free slabs of small calls (at most as many as calls have run at once)
     hipStream_t down = nullptr;
     char* ring_up = nullptr; char* ring_down = nullptr;
     hipEvent_t up_done[SLOTS] = {}, down_done[SLOTS] = {};
@@ -48,7 +57,7 @@ grl_hostpipe* grl_hostpipe_create() { return new grl_hostpipe(); }
 
 void grl_hostpipe_destroy(grl_hostpipe* h) {
     if (!h) return;
-    for (char* s : h->slabs) hipHostFree(s);
+    for (auto& s : h->slabs) hipHostFree(s.p);
     if (h->down) { hipStreamSynchronize(h->down); hipStreamDestroy(h->down); }
     if (h->ring_up) hipHostFree(h->ring_up);
     if (h->ring_down) hipHostFree(h->ring_down);
@@ -190,20 +199,28 @@ static int transfer_out(grl_ctx* c, int kind, void* dst, const void* src, size_t
     return rc;
 }
 
-// nullptr: pinned memory is refused
-static char* take_slab(grl_ctx* c) {
+// the smallest free slab of at least `need` bytes, or a new one; p is nullptr where pinned memory is refused
+static grl_hostpipe::slab take_slab(grl_ctx* c, size_t need) {
     grl_hostpipe* h = c->hostpipe;
-    char* s = nullptr;
+    grl_hostpipe::slab s = {nullptr, SLAB};
     {
         std::lock_guard<std::mutex> lk(h->slab_mu);
-        if (!h->slabs.empty()) { s = h->slabs.back(); h->slabs.pop_back(); }
+        size_t best = h->slabs.size();
+        for (size_t i = 0; i < h->slabs.size(); ++i)
+            if (h->slabs[i].cap >= need && (best == h->slabs.size() || h->slabs[i].cap < h->slabs[best].cap)) best = i;
+        if (best < h->slabs.size()) {
+            s = h->slabs[best];
+            h->slabs.erase(h->slabs.begin() + (long)best);
+        }
     }
     std::lock_guard<std::mutex> pool(c->mu);          // a slab is a pool block too, as far as the statistics go
-    if (s) { c->stats.hits++; return s; }
+    if (s.p) { c->stats.hits++; return s; }
     c->stats.misses++;
-    return pinned(c, SLAB);
+    while (s.cap < need) s.cap *= 2;
+    s.p = pinned(c, s.cap);
+    return s;
 }
-static void give_slab(grl_ctx* c, char* s) {
+static void give_slab(grl_ctx* c, grl_hostpipe::slab s) {
     std::lock_guard<std::mutex> lk(c->hostpipe->slab_mu);
     c->hostpipe->slabs.push_back(s);
 }
@@ -239,14 +256,14 @@ static int stage_in(grl_ctx* c, int kind, void* dst, const void* src, size_t byt
 
 // device -> host, small: a copy kernel writes into a pinned slab
 static int slab_out(grl_ctx* c, int kind, void* dst, const void* src, size_t bytes, size_t n) {
-    char* slab = take_slab(c);
-    if (!slab) return plain_out(c, kind, dst, src, kind == GRL_COPY_F32 ? bytes : n);
-    int rc = grl_copy_bytes_launch(c, slab, src, bytes);
+    const auto slab = take_slab(c, bytes);
+    if (!slab.p) return plain_out(c, kind, dst, src, kind == GRL_COPY_F32 ? bytes : n);
+    int rc = grl_copy_bytes_launch(c, slab.p, src, bytes);
     const hipError_t e = hipStreamSynchronize(c->stream);
     if (!rc && e != hipSuccess) { grl_set_error("grl_d2h: %s", hipGetErrorString(e)); rc = GRL_ERR_HIP; }
     if (!rc) {
-        if (kind == GRL_COPY_F32) memcpy(dst, slab, bytes);
-        else grl_host_copy(kind, dst, slab, n);
+        if (kind == GRL_COPY_F32) memcpy(dst, slab.p, bytes);
+        else grl_host_copy(kind, dst, slab.p, n);
     }
     give_slab(c, slab);
     return rc;
@@ -329,40 +346,55 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
     void* dev[8];
     GRL_REQUIRE(count <= 8, GRL_ERR_ARG, "run_on_host: too many arrays");
 
-    if (ins + outs <= SLAB) {
-        char* slab = take_slab(c);
-        if (!slab) return run_plain(c, dtype, units, arrays, count, op);
+    const grl_host_calling calling;
+    if (ins + outs <= SLAB_MAX) {
+        const auto slab = take_slab(c, ins + outs);
+        if (!slab.p) return run_plain(c, dtype, units, arrays, count, op);
         const bool direct = outs <= DIRECT;
-        grl_segments seg;
+        grl_segments seg, back;
         void* owned[8] = {};
-        int rc = GRL_OK;
-        size_t at = 0, oat = ins;
         char* res[8] = {};
-        grl_segments back;
+        int rc = GRL_OK;
+        size_t at = 0, oat = ins, held = 0;
+        // pieces that lie in the slab, on their way to the device
+        auto fetch = [&]() {
+            const int r = seg.count ? grl_copy_segments_launch(c, seg) : GRL_OK;
+            seg.count = 0;
+            held = 0;
+            return r;
+        };
         for (int i = 0; i < count && !rc; ++i) {
             const HostArray& a = arrays[i];
             if (a.in) {
-                grl_host_copy(dtype == GRL_BF16 && !a.f32 ? GRL_COPY_F32_BF16 : GRL_COPY_F32, slab + at, a.in, (size_t)a.n);
                 dev[i] = owned[i] = grl_malloc(c, dsize(a));          // (pool blocks are at least 256 bytes, in powers of two)
                 if (!dev[i]) { rc = GRL_ERR_OOM; break; }
-                seg.s[seg.count].src = slab + at; seg.s[seg.count].dst = dev[i]; seg.s[seg.count++].bytes = (int64_t)dsize(a);
+                const bool half = dtype == GRL_BF16 && !a.f32;
+                const size_t es = half ? 2 : 4, part = SLAB_PART / es;
+                for (size_t v = 0; v < (size_t)a.n && !rc; v += part) {
+                    const size_t m = std::min(part, (size_t)a.n - v);
+                    grl_host_copy(half ? GRL_COPY_F32_BF16 : GRL_COPY_F32, slab.p + at + v * es, a.in + v, m);
+                    auto& s = seg.s[seg.count++];
+                    s.src = slab.p + at + v * es; s.dst = (char*)dev[i] + v * es; s.bytes = (int64_t)(m * es);
+                    if ((held += m * es) >= SLAB_PART || seg.count == 8) rc = fetch();
+                }
                 at += pad(dsize(a));
             } else if (a.out) {
-                res[i] = slab + oat;
+                res[i] = slab.p + oat;
                 dev[i] = direct ? res[i] : (owned[i] = grl_malloc(c, dsize(a)));
                 if (!dev[i]) { rc = GRL_ERR_OOM; break; }
                 if (!direct) { back.s[back.count].src = dev[i]; back.s[back.count].dst = res[i]; back.s[back.count++].bytes = (int64_t)dsize(a); }
                 oat += pad(dsize(a));
             } else dev[i] = nullptr;
         }
-        if (!rc && seg.count) rc = grl_copy_segments_launch(c, seg);
+        if (!rc) rc = fetch();
         if (!rc) rc = op(0, units, dev);
         if (!rc && back.count) rc = grl_copy_segments_launch(c, back);
         const hipError_t e = hipStreamSynchronize(c->stream);          // also on failure: kernels may still read the slab
         if (!rc && e != hipSuccess) { grl_set_error("operator on host arrays: %s", hipGetErrorString(e)); rc = GRL_ERR_HIP; }
         for (int i = 0; i < count && !rc; ++i)
             if (arrays[i].out)
-                grl_host_copy(dtype == GRL_BF16 && !arrays[i].f32 ? GRL_COPY_BF16_F32 : GRL_COPY_F32, arrays[i].out, res[i], (size_t)arrays[i].n);
+                grl_host_copy(dtype == GRL_BF16 && !arrays[i].f32 ? GRL_COPY_BF16_F32 : GRL_COPY_F32, arrays[i].out, res[i], (size_t)arrays[i].n,
+                              (size_t)arrays[i].n * 4 >= PAST_CACHES);
         for (void* p : owned) grl_free(c, p);
         give_slab(c, slab);
         return rc;
@@ -372,7 +404,7 @@ int run_on_host(grl_ctx* c, int dtype, int64_t units, bool rows, HostArray* arra
     int rc = pipe_ready(c, h);
     if (rc) return rc;
     if (!h->ready) return run_plain(c, dtype, units, arrays, count, op);
-    // Blocks: enough of them that transfers in, work and transfers out overlap.
+    // from two blocks on, transfers in, work and transfers out overlap
     size_t moving = 0;
     for (int i = 0; i < count; ++i) if (arrays[i].per_unit) moving += dsize(arrays[i]);
     int64_t blocks = std::min<int64_t>(std::min<int64_t>(MAXBLOCKS, (int64_t)(moving / BLOCK)), units);

@@ -13,13 +13,15 @@ from grilly_amd import _lib as L
 pytestmark = pytest.mark.gpu
 
 
-# (M, K, N): 64 KiB of results in place and just above; 2 MiB of slab and just above; several blocks of rows with a ragged last
+# (M, K, N): 64 KiB of results in place and just above; 2 MiB and just above; several blocks of rows with a ragged last
 # one; rows that are no multiple of 16 bytes; one row of a wide product; more blocks than there are rows for
+# and, around the 5 MiB up to which a call is one slab: inputs of several parts with a ragged last one, odd widths, one row more
+SLAB_SHAPES = [(900, 384, 517), (3, 1100, 1101), (520, 1025, 300), (2431, 256, 256), (2432, 256, 256), (1250, 384, 700)]
 SHAPES = [(128, 64, 128), (130, 64, 128), (700, 384, 128), (710, 384, 128), (9001, 256, 640), (4099, 40, 1030), (1, 2048, 4096), (17, 4096, 24000)]
 
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
-@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("M,K,N", SHAPES + SLAB_SHAPES)
 def test_linear_on_host_arrays(backend, dtype, M, K, N):
     rng = np.random.default_rng(M + N)
     x = rng.standard_normal((M, K), dtype=np.float32)
@@ -37,7 +39,7 @@ def test_linear_on_host_arrays(backend, dtype, M, K, N):
 
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
-@pytest.mark.parametrize("B,S,masked", [(3, 40, True), (40, 128, True), (37, 200, False), (1, 2100, False)])
+@pytest.mark.parametrize("B,S,masked", [(3, 40, True), (12, 100, True), (40, 128, True), (37, 200, False), (1, 2100, False)])
 def test_attention_on_host_arrays(backend, dtype, B, S, masked):
     H, D = 4, 64
     rng = np.random.default_rng(B + S)
