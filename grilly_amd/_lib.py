@@ -119,6 +119,7 @@ SIGNATURES = {
                                     c_float, c_void_p]),
     "grl_mean_pool": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_int]),
     "grl_pack_batch": (c_int, [c_i64, c_i64, c_i64, c_void_p, c_void_p, c_int, c_void_p, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)]),
+    "grl_pack_inputs": (c_int, [c_i64, c_i64, c_i64, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)]),
     "grl_embed_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "grl_embed_layernorm_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64] + [c_void_p] * 6 + [c_float, c_void_p]),
     "grl_fa2_fwd_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64] + [c_void_p] * 4 + [c_i64] * 4 + [c_float, c_int, c_int, c_float, c_float]),

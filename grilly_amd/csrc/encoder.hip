@@ -186,7 +186,8 @@ int grl_check_ragged(const char* who, const grl_ragged* rg) {
 }
 
 template <typename M>
-static int pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const M* mask, int32_t* out, int64_t* rows, int64_t* longest) {
+static int pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const M* mask, int32_t* all_ids, float* all_mask, int32_t* out,
+                      int64_t* rows, int64_t* longest) {
     int32_t* offsets = out;
     int32_t* positions = out + (B + 1);
     int32_t* kept = positions + B * S;
@@ -206,7 +207,9 @@ static int pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, c
                 const M m = mask[b * S + s];
                 keep = m != (M)0;
                 bad_mask |= keep && m != (M)1;
+                if (all_mask) all_mask[b * S + s] = (float)m;
             }
+            if (all_ids) all_ids[b * S + s] = id;
             prefix &= !keep || n - first == s;
             positions[n] = (int32_t)s;           // overwritten by the next token when this one is not kept
             kept[n] = id;
@@ -222,16 +225,21 @@ static int pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, c
     return prefix ? GRL_PACK_PREFIX : GRL_PACK_SCATTERED;
 }
 
-extern "C" int grl_pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
-                              int32_t* out, int64_t* rows, int64_t* longest) {
+extern "C" int grl_pack_inputs(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
+                               int32_t* all_ids, float* all_mask, int32_t* out, int64_t* rows, int64_t* longest) {
     GRL_REQUIRE(B >= 0 && S >= 0 && B * S < (1LL << 31) && vocab > 0 && vocab < (1LL << 31), GRL_ERR_SHAPE, "grl_pack_batch: bad shape");
     GRL_REQUIRE(out && rows && longest && (B * S == 0 || ids), GRL_ERR_ARG, "grl_pack_batch: null argument");
     switch (mask ? mask_kind : 0) {
-        case 0: return pack_batch<int64_t>(B, S, vocab, ids, nullptr, out, rows, longest);
-        case 1: return pack_batch<int64_t>(B, S, vocab, ids, (const int64_t*)mask, out, rows, longest);
-        case 2: return pack_batch<float>(B, S, vocab, ids, (const float*)mask, out, rows, longest);
+        case 0: return pack_batch<int64_t>(B, S, vocab, ids, nullptr, all_ids, nullptr, out, rows, longest);
+        case 1: return pack_batch<int64_t>(B, S, vocab, ids, (const int64_t*)mask, all_ids, all_mask, out, rows, longest);
+        case 2: return pack_batch<float>(B, S, vocab, ids, (const float*)mask, all_ids, all_mask, out, rows, longest);
         default: break;
     }
     grl_set_error("grl_pack_batch: mask_kind must be 0 (none), 1 (int64) or 2 (float32)");
     return GRL_ERR_ARG;
+}
+
+extern "C" int grl_pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
+                              int32_t* out, int64_t* rows, int64_t* longest) {
+    return grl_pack_inputs(B, S, vocab, ids, mask, mask_kind, nullptr, nullptr, out, rows, longest);
 }

@@ -69,10 +69,39 @@ def _token_ids(input_ids):
     return ids if ids.dtype == np.int64 else ids.astype(np.int32, copy=False).astype(np.int64)
 
 
+class _Slice:
+    """a part of a device buffer"""
+    __slots__ = ("ptr", "nbytes")
+
+    def __init__(self, ptr, nbytes):
+        self.ptr, self.nbytes = ptr, nbytes
+
+
+class _Inputs:
+    """Device memory for one batch's ids and mask, and behind them for the same batch without its padding: what forward()
+    sends there in one transfer leaves launch() everything it reads."""
+    __slots__ = ("buffer", "ids", "mask", "packed")
+
+    def __init__(self, core, B, S):
+        n = 4 * _Inputs.plane(B * S)
+        self.buffer = core.alloc(2 * n + 4 * (B + 1 + 2 * B * S))
+        self.ids, self.mask = _Slice(self.buffer.ptr, 4 * B * S), _Slice(self.buffer.ptr + n, 4 * B * S)
+        self.packed = _Slice(self.buffer.ptr + 2 * n, 4 * (B + 1 + 2 * B * S))
+
+    @staticmethod
+    def plane(n):
+        """values from the ids to the mask and from there to the packed batch: whole 256-byte units"""
+        return (n + 63) // 64 * 64
+
+    def free(self):
+        self.buffer.free()
+
+
 class _Packing:
-    """What forward() makes of ids and mask in one native pass (grl_pack_batch): the real tokens' offsets, positions and
-    ids, how many there are, and whether they form a batch without padding or one whose padding can be left out."""
-    __slots__ = ("kind", "data", "B", "S", "rows", "longest")
+    """What forward() makes of ids and mask in one native pass (grl_pack_inputs): both as the kernels take them, the real
+    tokens' offsets, positions and ids, how many there are, and whether they form a batch without padding or one whose
+    padding can be left out."""
+    __slots__ = ("kind", "data", "packed", "B", "S", "rows", "longest")
 
     def __init__(self, lib, input_ids, attention_mask, vocab):
         ids = _token_ids(input_ids)
@@ -87,14 +116,17 @@ class _Packing:
             if mask.shape != (B, S):
                 raise ValueError("attention_mask must be (batch, seq_len)")
         self.B, self.S = B, S
-        self.data = np.empty(B + 1 + 2 * B * S, np.int32)
+        plane = _Inputs.plane(B * S)
+        self.data = np.empty(2 * plane + B + 1 + 2 * B * S, np.int32)
+        self.packed = self.data[2 * plane:]
         rows, longest = ctypes.c_int64(), ctypes.c_int64()
-        self.kind = lib.grl_pack_batch(B, S, vocab, ids.ctypes.data, mask.ctypes.data if kind else None, kind, self.data.ctypes.data,
-                                       ctypes.byref(rows), ctypes.byref(longest))
+        at = self.data.ctypes.data
+        self.kind = lib.grl_pack_inputs(B, S, vocab, ids.ctypes.data, mask.ctypes.data if kind else None, kind, at, at + 4 * plane,
+                                        at + 8 * plane, ctypes.byref(rows), ctypes.byref(longest))
         if self.kind == L.PACK_BAD_ID:
             raise IndexError("token id out of range")      # numpy indexing in the reference raises IndexError
         if self.kind < 0:
-            L.check(self.kind, "pack_batch")
+            L.check(self.kind, "pack_inputs")
         self.rows, self.longest = rows.value, longest.value
 
     @property
@@ -102,15 +134,17 @@ class _Packing:
         """no padding at all: a rectangular batch that needs no mask"""
         return self.kind == L.PACK_PREFIX and self.rows == self.B * self.S
 
-    def ids(self):
-        return self.data[self.B + 1 + self.rows:self.B + 1 + 2 * self.rows]
+    def upload_full(self, core, inputs):
+        """the ids of a batch without padding (a mask of ones changes nothing)"""
+        L.check(core.lib.grl_h2d(core.ctx, inputs.ids.ptr, self.data.ctypes.data, 4 * self.B * self.S), "upload ids")
 
-    def upload(self, core, dst):
-        """offsets | positions | ids to the device in one transfer -> (ragged batch, device address of the ids)"""
-        n = self.B + 1 + 2 * self.rows
-        L.check(core.lib.grl_h2d(core.ctx, dst, self.data.ctypes.data, n * 4), "upload packed batch")
-        positions = dst + 4 * (self.B + 1)
-        return L.Ragged(dst, positions, self.B, self.rows, self.longest), positions + 4 * self.rows
+    def upload(self, core, inputs):
+        """ids, mask and offsets | positions | ids of the batch without its padding, in one transfer -> (ragged batch, device
+        address of the latter ids)"""
+        n = self.data.size - self.packed.size + self.B + 1 + 2 * self.rows
+        L.check(core.lib.grl_h2d(core.ctx, inputs.ids.ptr, self.data.ctypes.data, n * 4), "upload batch")
+        positions = inputs.packed.ptr + 4 * (self.B + 1)
+        return L.Ragged(inputs.packed.ptr, positions, self.B, self.rows, self.longest), positions + 4 * self.rows
 
 
 class BertEncoder:
@@ -209,15 +243,14 @@ class BertEncoder:
         self.x = c.alloc(B * S * cfg.d_model * es)
         self.stats = c.alloc(max(B * S, 1) * 8)        # {1/sd, mean/sd} per row of the raw residual stream (fused layers)
         self.ws = c.alloc(ws)
-        self.ids = c.alloc(B * S * 4)
-        self.packed = c.alloc((B + 1 + 2 * B * S) * 4) # offsets | positions | ids of the batch without its padding
-        self.mask = c.alloc(B * S * 4)
+        self.inputs = _Inputs(c, B, S)
+        self.ids, self.mask = self.inputs.ids, self.inputs.mask
         self.pooled = c.alloc(B * cfg.d_model * 4)
         self._shape = (B, S)
 
     def release_activations(self):
         if self._shape is not None:
-            for b in (self.x, self.stats, self.ws, self.ids, self.packed, self.mask, self.pooled):
+            for b in (self.x, self.stats, self.ws, self.inputs, self.pooled):
                 b.free()
             self._shape = None
 
@@ -239,11 +272,16 @@ class BertEncoder:
             L.check(c.lib.grl_h2d(c.ctx, self.mask.ptr, m.ctypes.data, m.nbytes), "upload mask")
 
     def _set_full(self, p):
-        """set_inputs for a batch without padding (a mask of ones changes nothing)"""
+        """set_inputs for a batch without padding"""
         self.prepare(p.B, p.S)
-        ids = p.ids()
-        L.check(self.core.lib.grl_h2d(self.core.ctx, self.ids.ptr, ids.ctypes.data, ids.nbytes), "upload ids")
+        p.upload_full(self.core, self.inputs)
         self.has_mask = False
+
+    def _set_packed(self, p):
+        """set_inputs for a batch that runs without its padding -> what upload() returns"""
+        self.prepare(p.B, p.S)
+        self.has_mask = True
+        return p.upload(self.core, self.inputs)
 
     def launch(self, pool=True):
         """Enqueue one full forward of the batch that set_inputs() or forward() had last, in its rectangular form, on the
@@ -323,9 +361,7 @@ class BertEncoder:
         # where bf16 rounds the softmax weights against another reference (1e-3 measured): fp32 only.
         packs = p.kind == L.PACK_PREFIX or (p.kind == L.PACK_SCATTERED and self.code == L.GRL_F32)
         if pool and packs and not p.full and self.cfg.head_dim <= 128:
-            self.prepare(p.B, p.S)
-            self._launch_packed(*p.upload(self.core, self.packed.ptr))
-            self.set_inputs(input_ids, attention_mask)      # what a launch() from here on reads; uploaded while the layers run
+            self._launch_packed(*self._set_packed(p))
         else:
             if p.full:
                 self._set_full(p)
@@ -469,9 +505,8 @@ class PreNormEncoder:
             self.part = c.alloc(int(c.lib.grl_gemm_nt_resln_workspace(B * S, cfg.d_model)))
         self.qkv = c.alloc(3 * act)                    # packed (M, 3d): Q, K, V are its three column blocks
         self.h = c.alloc(B * S * cfg.d_ff * es)
-        self.ids = c.alloc(B * S * 4)
-        self.packed = c.alloc((B + 1 + 2 * B * S) * 4) # offsets | positions | ids of the batch without its padding
-        self.mask = c.alloc(B * S * 4)
+        self.inputs = _Inputs(c, B, S)
+        self.ids, self.mask = self.inputs.ids, self.inputs.mask
         first = np.zeros((B, S), np.float32)
         first[:, 0] = 1.0                              # "mean" over the first token only = that token
         self.first = c.upload_raw(first)
@@ -480,7 +515,7 @@ class PreNormEncoder:
 
     def release_activations(self):
         if self._shape is not None:
-            for b in (self.x, self.qkv, self.att, self.stats, self.h, self.ids, self.packed, self.mask, self.first, self.pooled):
+            for b in (self.x, self.qkv, self.att, self.stats, self.h, self.inputs, self.first, self.pooled):
                 b.free()
             if self.stats_from_gemm:
                 for b in (self.ident_stats, self.ones, self.zeros, self.part):
@@ -504,7 +539,7 @@ class PreNormEncoder:
                 raise ValueError("attention_mask must be (batch, seq_len)")
             L.check(c.lib.grl_h2d(c.ctx, self.mask.ptr, m.ctypes.data, m.nbytes), "upload mask")
 
-    _set_full = BertEncoder._set_full
+    _set_full, _set_packed = BertEncoder._set_full, BertEncoder._set_packed
 
     def launch(self, pool=True):
         """Enqueue one full forward of the batch that set_inputs() or forward() had last (as in BertEncoder)."""
@@ -570,10 +605,8 @@ class PreNormEncoder:
         """pool=True -> L2-normalised first-token embeddings (B, d); False -> hidden states (B,S,d).  Pooled batches padded
         on the right run without their padding, as in BertEncoder (the first token has to be a real one)."""
         p = _Packing(self.core.lib, input_ids, attention_mask, self.cfg.vocab)
-        if pool and not p.full and p.kind == L.PACK_PREFIX and (p.data[1:p.B + 1] > p.data[:p.B]).all():
-            self.prepare(p.B, p.S)
-            self._launch(True, *p.upload(self.core, self.packed.ptr))
-            self.set_inputs(input_ids, attention_mask)      # as in BertEncoder
+        if pool and not p.full and p.kind == L.PACK_PREFIX and (p.packed[1:p.B + 1] > p.packed[:p.B]).all():
+            self._launch(True, *self._set_packed(p))
         else:
             if p.full and p.S > 0:
                 self._set_full(p)

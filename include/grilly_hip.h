@@ -416,6 +416,9 @@ enum { GRL_PACK_PREFIX = 0,      /* every sequence keeps its first tokens (paddi
        GRL_PACK_BAD_ID = 3 };    /* some token id, kept or not, lies outside [0, vocab) */
 int grl_pack_batch(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
                    int32_t* out, int64_t* rows, int64_t* longest);
+/* the same, and the whole batch as the rectangular entry points take it: ids as int32, the mask (if there is one) as float32 */
+int grl_pack_inputs(int64_t B, int64_t S, int64_t vocab, const int64_t* ids, const void* mask, int mask_kind,
+                    int32_t* all_ids, float* all_mask, int32_t* out, int64_t* rows, int64_t* longest);
 int grl_embed_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t F, int64_t vocab, const int32_t* ids,
                      const float* tok_emb, const float* pos_emb, const float* type_emb, void* x);
 int grl_embed_layernorm_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t F, int64_t vocab, const int32_t* ids,
