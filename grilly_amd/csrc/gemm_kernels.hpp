@@ -535,6 +535,8 @@ __global__ __launch_bounds__(256) void gemm_splitk_finish_kernel(GemmArgs p) {
 // whole, so it sums them and their squares on the way (two v_dot2 per two bf16 values, under the wait for the next slab), and the
 // tiles of the first column write them out for a later residual epilogue.  No statistics pass, no LayerNorm pass: the kernel
 // takes 5.7 us at 128 x 2304 x 768 in bf16, the plain one 5.4 behind a LayerNorm of 5.0.
+// One pass in fp32 (mean of the squares minus square of the mean): good to K / 8 * 2^-24 * (1 + (mean/sd)^2), like the merged
+// statistics of ln_stats_merge_kernel.  bf16 rows that far from zero have lost their spread to their storage long before.
 // EPI_RESLN here adds LayerNorm(residual) like the kernels below and leaves the statistics of the result to its OWN consumer.
 template <typename T, typename OutT, int BM, int BN, int NSTG, int EPI, bool DUAL, bool LN = false, bool SPLITK = false, bool OWN = false>
 __global__ __launch_bounds__(256, 1) void gemm_nt_kshare_kernel(GemmArgs p) {

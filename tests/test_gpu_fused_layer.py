@@ -354,6 +354,41 @@ def test_products_of_few_rows(backend, dtype, M, K, N):
             t.free()
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("M,K,N,spreads", [(33, 768, 768, 6), (128, 768, 768, 30), (128, 3072, 768, 30)])
+def test_products_of_few_rows_far_from_zero(backend, dtype, M, K, N, spreads):
+    """Rows whose mean is many spreads away from zero, where the kernel's single pass over them (mean of the squares minus
+    square of the mean) cancels.  Each of eight partial sums adds K / 8 terms, each addition good to 2^-24: the two moments are
+    off by at most K / 8 * 2^-24, and the variance, 1 + (mean/sd)^2 times smaller than they are, by that factor more; half of it
+    comes through to 1/sd, and mean/sd carries the mean's own share besides.  The product sums K / 4 terms per wave whose running
+    sums are mean/sd times the result's size.  The bf16 rows themselves hold their spread to 2^-9 * mean/sd only (6 % at thirty
+    spreads): there the cancellation is far below what the storage has rounded away."""
+    c, code = backend.core, _code(dtype)
+    rng = np.random.default_rng(M + K + spreads)
+    es, eps = (2 if dtype == "bf16" else 4), 1e-5
+    side = np.where(rng.random((M, 1)) < 0.5, -1.0, 1.0)
+    x = _q(dtype, ((rng.standard_normal((M, K)) + spreads * side) * (0.5 + rng.random((M, 1)))).astype(np.float32))
+    W = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    g, bt = (1 + 0.2 * rng.standard_normal(K)).astype(np.float32), (0.3 * rng.standard_normal(K)).astype(np.float32)
+    want = _stats(x, eps)
+    far = np.abs(want[:, 1]).max()
+    moments = K / 8 * 2.0 ** -24 * (1 + far ** 2)
+    product = K / 4 * 2.0 ** -24 * far
+    bufs = [c.upload(x, code), c.upload(W), c.upload(b), c.upload(g), c.upload(bt), c.alloc(N * K * es), c.alloc(N * 4), c.alloc(N * 4),
+            c.alloc(M * N * es), c.alloc(M * 8)]
+    dx, raw, db, dg, dbt, w, cs, bf, out, st = bufs
+    try:
+        L.check(c.lib.grl_ln_fold_f32(c.ctx, code, N, K, raw.ptr, dg.ptr, dbt.ptr, db.ptr, w.ptr, cs.ptr, bf.ptr), "fold")
+        L.check(c.lib.grl_ln_gemm_nt_rows(c.ctx, code, M, N, K, dx.ptr, w.ptr, cs.ptr, bf.ptr, eps, st.ptr, out.ptr, L.EPI_NONE), "rows")
+        np.testing.assert_allclose(c.download(st, (M, 2)), want, rtol=moments)
+        ref = O.truth_linear(O.truth_layernorm(x, g, bt, eps), W, b)
+        assert O.max_rel(c.download(out, (M, N), code), ref) < (TOL_BF16 if dtype == "bf16" else TOL_F32) + moments + product
+    finally:
+        for t in bufs:
+            t.free()
+
+
 @pytest.mark.parametrize("pad", [False, True])
 @pytest.mark.parametrize("B,S", [(1, 1), (1, 37), (3, 50)])
 def test_encoder_of_few_rows_equals_the_seven_launch_one(backend, pad, B, S):
