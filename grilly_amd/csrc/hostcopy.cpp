@@ -8,6 +8,7 @@
 #include "../../include/grilly_hip.h"
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
@@ -81,7 +82,12 @@ public:
     void copy(int kind, void* dst, const void* src, size_t n, bool past) {
         constexpr size_t PIECE = 16 * 1024;                              // values
         // too small to share, a forked child (the threads stayed in the parent), or another thread's job is on: alone
-        if (n < 4 * PIECE || workers_ == 0 || getpid() != pid_ || !turn_.try_lock()) { copy_range(kind, past, dst, src, 0, n); return; }
+        // or the CPUs have turned out to be taken
+        const int64_t begin = now();
+        if (n < 4 * PIECE || workers_ == 0 || begin < alone_until_.load(std::memory_order_relaxed) || getpid() != pid_ || !turn_.try_lock()) {
+            copy_range(kind, past, dst, src, 0, n);
+            return;
+        }
         const size_t pieces = (n + PIECE - 1) / PIECE;
         kind_ = kind; past_ = past; dst_ = dst; src_ = src; n_ = n; piece_ = PIECE;
         next_.store(0, std::memory_order_relaxed);
@@ -97,6 +103,7 @@ public:
         // job closed and touches nothing of it, so there is no waiting for sleepers.
         open_.store(false);
         while (inside_.load() != 0) _mm_pause();
+        judge(begin, now(), n);
         turn_.unlock();
     }
 
@@ -111,6 +118,22 @@ private:
         workers_ = cpus / 2 - 1;
         workers_ = workers_ < 0 ? 0 : workers_ > 7 ? 7 : workers_;
         for (int i = 0; i < workers_; ++i) std::thread([this] { loop(); }).detach();
+    }
+    static int64_t now() { return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
+    // Where every CPU already runs a thread (the threads of a BLAS or an OpenMP runtime spin for 1 - 200 ms behind each of its calls),
+    // helpers do harm: one that loses its CPU in the middle of a piece, or takes the caller's, holds the call up for time slices of
+    // some milliseconds.  A job that takes far longer than its bytes is the sign of it.  After two of them within 20 ms the caller
+    // copies alone for 20 ms, and twice as long each time it happens again soon after.  Mean us per call with a 1024-cube product of
+    // numpy before each, always with helpers / with this: attention 32 x 64 x 8 x 64 1445 - 1840 / 540 - 660, in bf16
+    // 1090 - 1560 / 390 - 480, fused_linear_gelu 4000 x 3072 x 768 3600 - 4500 / 2300 - 2600.
+    void judge(int64_t begin, int64_t end, size_t n) {
+        constexpr int64_t SLACK = 300000, FIRST = 20000000, LONGEST = 640000000;        // ns
+        if (end - begin <= SLACK + (int64_t)n) return;                                  // 4 GB/s, a quarter of what one thread moves
+        const bool soon = begin - alone_until_.load(std::memory_order_relaxed) < 2 * pause_, twice = begin - stalled_ < FIRST;
+        stalled_ = end;
+        if (!soon && !twice) return;
+        pause_ = soon ? std::min(2 * pause_, LONGEST) : FIRST;
+        alone_until_.store(end + pause_, std::memory_order_relaxed);
     }
     void work() {
         for (size_t i; (i = next_.fetch_add(1, std::memory_order_relaxed)) < pieces_;) {
@@ -139,6 +162,8 @@ private:
     std::atomic<size_t> next_{0};
     std::atomic<int> inside_{0}, calls_{0};
     std::atomic<bool> open_{false};
+    std::atomic<int64_t> alone_until_{0};
+    int64_t pause_ = 0, stalled_ = -1000000000;
     size_t pieces_ = 0, n_ = 0, piece_ = 0;
     int kind_ = 0, workers_ = 0;
     bool past_ = false;
