@@ -68,3 +68,34 @@ def test_scales(backend, scale):
         y = backend.attention.flash_attention2(q, k, v, 2, 64, scale=scale, causal=causal)
         ref = exact(q, k, v, scale, causal)
         assert np.linalg.norm(y - ref) < 1e-6 * np.linalg.norm(ref)
+
+
+def clear_rows(q, k, scale, gap):
+    """Queries whose best key is ahead of the second by more than `gap`: the output is that key's value."""
+    s = np.einsum("bqhd,bkhd->bqhk", q.astype(np.float64), k.astype(np.float64)) * scale
+    top = np.sort(s, -1)
+    return top[..., -1] - top[..., -2] > gap
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("mag", [900.0, 2e4, 5e4])
+def test_large_scores(backend, D, mag):
+    """Scores of 2^20 and far beyond, where a unit in the last place is many powers of two of a weight: the largest weight is 1 all the
+    same, with and without a mask that excludes nothing.  (Products round to 2^-24 of about mag^2 each: the best key is told from
+    the second where 1e-4 of that lies between them.)"""
+    S, H = 70, 3
+    q, k, v = qkv(D, 2, S, H, D)
+    q, k = q * np.float32(mag), k * np.float32(mag)
+    clear = clear_rows(q, k, D ** -0.5, 1e-4 * mag * mag)
+    assert clear.mean() > 0.9
+    ref = exact(q, k, v, D ** -0.5)
+    for mask in (None, np.ones((2, S), np.float32)):
+        y = backend.attention.flash_attention2(q, k, v, H, D, mask=mask)
+        np.testing.assert_allclose(y[clear], ref[clear], rtol=1e-6, atol=1e-7)
+    k[0, 3, 0, 0] = np.inf                        # head 0 of batch entry 0 once more with the fp32 instruction
+    q[0, :, 0, 0] = -np.abs(q[0, :, 0, 0])        # a score of -infinity: no weight
+    y, kk = backend.attention.flash_attention2(q, k, v, H, D), k.copy()
+    kk[0, 3, 0, 0] = 1e30
+    clear = clear_rows(q, kk, D ** -0.5, 1e-4 * mag * mag)
+    ref = exact(q, kk, v, D ** -0.5)
+    np.testing.assert_allclose(y[clear], ref[clear], rtol=1e-6, atol=1e-7)
