@@ -99,3 +99,13 @@ def test_large_scores(backend, D, mag):
     clear = clear_rows(q, kk, D ** -0.5, 1e-4 * mag * mag)
     ref = exact(q, kk, v, D ** -0.5)
     np.testing.assert_allclose(y[clear], ref[clear], rtol=1e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("scale", [0.0, 1e-38, -3e-39])
+def test_scales_next_to_zero_with_large_products(backend, scale):
+    q, k, v = qkv(7, 1, 70, 2, 64)
+    q, k = q * np.float32(2.0 ** 62), k * np.float32(2.0 ** 60)      # products around 1e38
+    for causal in (False, True):
+        y = backend.attention.flash_attention2(q, k, v, 2, 64, scale=scale, causal=causal)
+        ref = exact(q, k, v, np.float64(np.float32(scale)), causal)
+        assert np.linalg.norm(y - ref) < 1e-5 * np.linalg.norm(ref)      # (a scale below the normal numbers has few bits)
