@@ -109,6 +109,20 @@ def test_small_and_large_values(backend):
         np.testing.assert_array_equal(run(backend, x * s, W * t, b * (s * t)), y * (s * t))
 
 
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_one_term(backend, M, K, N):
+    """A sum of one product (a row selector, a diagonal scaling).  The largest of its six plane products comes last, so the sum is rounded
+    at its own size once (measured: to within a unit in the last place, 2^-23), and what is left out is at most 2^-24: m and l are
+    up to 2^-8 and 2^-17 of an operand.  Measured 1.5e-7; with the largest product third, 2.8e-7."""
+    rng = np.random.default_rng(M + K + N)
+    x, W = np.zeros((M, K), np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    at, val = rng.integers(0, K, M), rng.standard_normal(M).astype(np.float32)
+    x[np.arange(M), at] = val
+    y = run(backend, x, W, np.zeros(N, np.float32))
+    ref = W.astype(np.float64).T[at] * val[:, None].astype(np.float64)
+    assert (np.abs(y - ref) / np.maximum(np.abs(ref), 1e-30)).max() < 3 * 2.0 ** -24
+
+
 def test_shares_of_k_take_nothing_from_the_pool_under_capture(backend):
     """A captured graph would keep the address of the shares after the pool has given it away: a product that runs in shares of K
     otherwise is recorded without them, and its replays give what new inputs ask for."""
