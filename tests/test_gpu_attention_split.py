@@ -109,3 +109,35 @@ def test_scales_next_to_zero_with_large_products(backend, scale):
         y = backend.attention.flash_attention2(q, k, v, 2, 64, scale=scale, causal=causal)
         ref = exact(q, k, v, np.float64(np.float32(scale)), causal)
         assert np.linalg.norm(y - ref) < 1e-5 * np.linalg.norm(ref)      # (a scale below the normal numbers has few bits)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("eq,ek,ev", [(-118, 116, 0), (116, -118, 0), (-125, 124, 0), (0, 0, -112), (0, 0, -120), (-60, 60, -118), (0, 0, 100)])
+def test_operands_far_below_one(backend, D, eq, ek, ev):
+    """Operands near the smallest normal number, with partners that bring the products back to ordinary size: the bound of
+    test_error_against_float64."""
+    S, H = 129, 2
+    q, k, v = qkv(D - ev - 2 * eq, 2, S, H, D) if ev + 2 * eq < D else qkv(D + 400, 2, S, H, D)
+    sq, sk, sv = (np.float32(2.0 ** e) for e in (eq, ek, ev))
+    q, k, v = q * sq, k * sk, v * sv
+    bound = 2.0 ** -24 * (6 + np.sqrt(6 * D / 16) + np.sqrt(6 * S / 16))
+    for causal in (False, True):
+        y = backend.attention.flash_attention2(q, k, v, H, D, causal=causal).astype(np.float64) / np.float64(sv)
+        ref = exact(q, k, v, D ** -0.5, causal) / np.float64(sv)
+        assert np.linalg.norm(y - ref) < bound * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_tiny_weight_of_a_large_value(backend, D):
+    """A weight of 2^-122 on a value of 2^110, beside one of 1 on a value of 2^-20.  The products are exact, the score is -85: its weight
+    is off by 85 * 2^-24 and the exponent's rounding."""
+    S, H = 40, 2
+    rng = np.random.default_rng(D)
+    q, k, v = np.zeros((1, S, H, D), np.float32), np.zeros((1, S, H, D), np.float32), rng.standard_normal((1, S, H, D)).astype(np.float32)
+    q[..., 0], k[..., 0] = 1.0, -2000.0
+    k[0, 0, :, 0] = 0.0
+    k[0, 33, :, 0] = -85.0
+    v[0, 0] *= np.float32(2.0 ** -20)
+    v[0, 33] *= np.float32(2.0 ** 110)
+    y, ref = backend.attention.flash_attention2(q, k, v, H, D, scale=1.0), exact(q, k, v, 1.0)
+    assert np.linalg.norm(y - ref) < 4 * 85 * 2.0 ** -24 * np.linalg.norm(ref)

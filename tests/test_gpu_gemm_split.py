@@ -123,6 +123,18 @@ def test_one_term(backend, M, K, N):
     assert (np.abs(y - ref) / np.maximum(np.abs(ref), 1e-30)).max() < 3 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("M,K,N", [(1500, 384, 384), (1499, 160, 1152), (1500, 768, 2304), (1499, 3040, 764), (2001, 768, 3068), (3000, 768, 2304), (3000, 768, 2303), (6400, 768, 2304)])
+@pytest.mark.parametrize("ex,ew", [(-112, 100), (100, -112), (-120, 124), (-125, 60), (60, -125), (-118, 0), (0, -118), (-70, -45)])
+def test_operands_far_below_one(backend, M, K, N, ex, ew):
+    """Operands near the smallest normal number: every bit of theirs counts as it does elsewhere (the bound of test_error_against_float64)."""
+    rng = np.random.default_rng(M + K + N)
+    x, W = rng.standard_normal((M, K)).astype(np.float32) * np.float32(2.0 ** ex), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32) * np.float32(2.0 ** ew)
+    y = run(backend, x, W, np.zeros(N, np.float32)).astype(np.float64)
+    rows = slice(0, 257)
+    ref = x[rows].astype(np.float64) @ W.T.astype(np.float64)
+    assert rel(y[rows], ref) < 2.0 ** -24 * (1 + np.sqrt(6 * K / 16))
+
+
 def test_shares_of_k_take_nothing_from_the_pool_under_capture(backend):
     """A captured graph would keep the address of the shares after the pool has given it away: a product that runs in shares of K
     otherwise is recorded without them, and its replays give what new inputs ask for."""
