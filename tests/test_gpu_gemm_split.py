@@ -109,6 +109,37 @@ def test_small_and_large_values(backend):
         np.testing.assert_array_equal(run(backend, x * s, W * t, b * (s * t)), y * (s * t))
 
 
+# where the 32 x 32 tiles' four sums on the fp32 instruction were the fastest before the split operands, and more than one 128 x 128
+# tile per CU all the same; plain and gated
+FOUR_SUMS = [(2722, 3072, 2304, False), (8251, 3072, 768, False), (2722, 4096, 3072, False), (6400, 4096, 1024, False), (800, 2048, 8192, False),
+             (800, 8192, 4096, True), (6400, 11008, 512, True)]
+
+
+@pytest.mark.parametrize("M,K,N,gated", FOUR_SUMS)
+def test_four_sums_where_four_were(backend, M, K, N, gated):
+    """R = 6 K / 16 roundings walk along one sum whose size grows with the root of its length: an error of e sqrt(R / 2), e = 0.41 * 2^-24
+    the mean rounding; along four sums of a quarter each it is e sqrt(R / 8).  Measured at K = 768: 4.2e-7 and 2.0e-7, i.e. e = 0.30 and
+    0.28 times 2^-24 sqrt(R).  The bound lies between the two."""
+    rng = np.random.default_rng(M + K + N)
+    x, W = rng.standard_normal((M, K)).astype(np.float32), (rng.standard_normal((2 if gated else 1, N, K)) / np.sqrt(K)).astype(np.float32)
+    bound = 2.0 ** -24 * 0.29 * np.sqrt(6 * K / 16)
+    rows = slice(0, 257)                          # (float64 in full would take a minute)
+    ref = [x[rows].astype(np.float64) @ w.T.astype(np.float64) for w in W]
+    if not gated:
+        y = run(backend, x, W[0], np.zeros(N, np.float32))
+        assert rel(y[rows], ref[0]) < bound
+        return
+    c = backend.core
+    bufs = [c.upload(x), c.upload(W[0]), c.upload(W[1]), c.alloc(M * N * 4)]
+    try:
+        L.check(c.lib.grl_glu_nt(c.ctx, L.GRL_F32, L.GRL_F32, M, N, K, *(t.ptr for t in bufs[:3]), None, None, bufs[3].ptr, None, None, L.EPI_RELU), "glu_nt")
+        y = c.download(bufs[3], (M, N))
+    finally:
+        for t in bufs:
+            t.free()
+    assert rel(y[rows], ref[0] * np.maximum(ref[1], 0)) < 1.5 * bound      # two independent sums: sqrt(2)
+
+
 @pytest.mark.parametrize("M,K,N", SHAPES)
 def test_one_term(backend, M, K, N):
     """A sum of one product (a row selector, a diagonal scaling).  The largest of its six plane products comes last, so the sum is rounded
