@@ -166,30 +166,33 @@ def test_operands_far_below_one(backend, M, K, N, ex, ew):
     assert rel(y[rows], ref) < 2.0 ** -24 * (1 + np.sqrt(6 * K / 16))
 
 
-def test_shares_of_k_take_nothing_from_the_pool_under_capture(backend):
+@pytest.mark.parametrize("M,K,N,dtype", [(1499, 3040, 764, "fp32"), (128, 3072, 768, "fp32"), (128, 4096, 768, "bf16"),      # 128 x 128 and 32 x 32 tiles
+                                         (100, 1000, 256, "fp32"), (100, 2056, 256, "bf16")])                          # the register-staged 64 x 64 tiles
+def test_shares_of_k_take_nothing_from_the_pool_under_capture(backend, M, K, N, dtype):
     """A captured graph would keep the address of the shares after the pool has given it away: a product that runs in shares of K
     otherwise is recorded without them, and its replays give what new inputs ask for."""
-    c, (M, K, N) = backend.core, (1499, 3040, 764)
-    rng = np.random.default_rng(8)
-    W, b = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
-    dx, dw, db, dy = bufs = [c.alloc(M * K * 4), c.upload(W), c.upload(b), c.alloc(M * N * 4)]
+    c, rng = backend.core, np.random.default_rng(8)
+    code, q = (L.GRL_BF16, lambda a: O.bf16_round(a.astype(np.float32))) if dtype == "bf16" else (L.GRL_F32, lambda a: a.astype(np.float32))
+    W, b = q(rng.standard_normal((N, K)) / np.sqrt(K)), rng.standard_normal(N).astype(np.float32)
+    inputs = [q(np.random.default_rng(seed).standard_normal((M, K))) for seed in range(3)]
+    dx, dw, db, dy, *dxs = bufs = [c.upload(inputs[0], code), c.upload(W, code), c.upload(b), c.alloc(M * N * 4)] + [c.upload(x, code) for x in inputs]
+    product = lambda x: c.lib.grl_gemm_nt(c.ctx, code, L.GRL_F32, M, N, K, x.ptr, dw.ptr, db.ptr, dy.ptr, L.EPI_NONE)
     stream, graph, run_it = ctypes.c_void_p(c.lib.grl_stream(c.ctx)), ctypes.c_void_p(), ctypes.c_void_p()
     hip = lambda name, *args: L.check(getattr(c.lib, name)(*args), name)
     try:
         before = c.pool_stats()
         hip("hipStreamBeginCapture", stream, 2)          # relaxed: an allocation would go through
-        rc = c.lib.grl_gemm_nt(c.ctx, L.GRL_F32, L.GRL_F32, M, N, K, dx.ptr, dw.ptr, db.ptr, dy.ptr, L.EPI_NONE)
+        rc = product(dx)
         hip("hipStreamEndCapture", stream, ctypes.byref(graph))
         L.check(rc, "gemm_nt")
         assert c.pool_stats() == before
         hip("hipGraphInstantiate", ctypes.byref(run_it), graph, None, None, ctypes.c_size_t(0))
-        for seed in range(3):
-            x = np.random.default_rng(seed).standard_normal((M, K)).astype(np.float32)
-            L.check(c.lib.grl_h2d(c.ctx, dx.ptr, x.ctypes.data, M * K * 4), "h2d")
+        for x, d in zip(inputs, dxs):
+            hip("hipMemcpyAsync", ctypes.c_void_p(dx.ptr), ctypes.c_void_p(d.ptr), ctypes.c_size_t(x.size * (2 if dtype == "bf16" else 4)), 3, stream)
             hip("hipGraphLaunch", run_it, stream)
             ref = x.astype(np.float64) @ W.T.astype(np.float64) + b
-            assert rel(c.download(dy, (M, N)), ref) < 2.0 ** -24 * (1 + np.sqrt(6 * K / 16))
-            run(backend, x, W, b)                        # eager work between the replays takes and returns the pool's blocks
+            assert rel(c.download(dy, (M, N)), ref) < 2.0 ** -24 * (1 + np.sqrt(K))      # bf16 products are exact; up to K roundings
+            L.check(product(dxs[0]), "gemm_nt")          # eager work between the replays takes and returns the pool's blocks
     finally:
         if run_it:
             c.lib.hipGraphExecDestroy(run_it)
