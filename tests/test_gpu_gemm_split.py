@@ -117,9 +117,9 @@ FOUR_SUMS = [(2722, 3072, 2304, False), (8251, 3072, 768, False), (2722, 4096, 3
 
 @pytest.mark.parametrize("M,K,N,gated", FOUR_SUMS)
 def test_four_sums_where_four_were(backend, M, K, N, gated):
-    """R = 6 K / 16 roundings walk along one sum whose size grows with the root of its length: an error of e sqrt(R / 2), e = 0.41 * 2^-24
-    the mean rounding; along four sums of a quarter each it is e sqrt(R / 8).  Measured at K = 768: 4.2e-7 and 2.0e-7, i.e. e = 0.30 and
-    0.28 times 2^-24 sqrt(R).  The bound lies between the two."""
+    """R = 6 K / 16 roundings walk along one sum whose size grows with the root of its length: an error of e sqrt(R / 2); along four sums of
+    a quarter each it is e sqrt(R / 8), half of it.  Measured at K = 768: 4.2e-7 and 2.0e-7, i.e. 0.42 and 0.20 times 2^-24 sqrt(R).  The
+    bound lies between the two."""
     rng = np.random.default_rng(M + K + N)
     x, W = rng.standard_normal((M, K)).astype(np.float32), (rng.standard_normal((2 if gated else 1, N, K)) / np.sqrt(K)).astype(np.float32)
     bound = 2.0 ** -24 * 0.29 * np.sqrt(6 * K / 16)
@@ -155,15 +155,16 @@ def test_one_term(backend, M, K, N):
 
 
 @pytest.mark.parametrize("M,K,N", [(1500, 384, 384), (1499, 160, 1152), (1500, 768, 2304), (1499, 3040, 764), (2001, 768, 3068), (3000, 768, 2304), (3000, 768, 2303), (6400, 768, 2304)])
-@pytest.mark.parametrize("ex,ew", [(-112, 100), (100, -112), (-120, 124), (-125, 60), (60, -125), (-118, 0), (0, -118), (-70, -45)])
+@pytest.mark.parametrize("ex,ew", [(-112, 100), (100, -112), (-120, 124), (-125, 60), (60, -125), (-118, 0), (0, -118), (-70, -45), (60, 40), (110, -120)])
 def test_operands_far_below_one(backend, M, K, N, ex, ew):
-    """Operands near the smallest normal number: every bit of theirs counts as it does elsewhere (the bound of test_error_against_float64)."""
+    """Operands near the smallest normal number: every bit of theirs counts as it does elsewhere (the bound of test_error_against_float64).
+    The last two overflow at the size that operands are split at and are formed with the fp32 instruction (one rounding per product)."""
     rng = np.random.default_rng(M + K + N)
     x, W = rng.standard_normal((M, K)).astype(np.float32) * np.float32(2.0 ** ex), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32) * np.float32(2.0 ** ew)
     y = run(backend, x, W, np.zeros(N, np.float32)).astype(np.float64)
     rows = slice(0, 257)
     ref = x[rows].astype(np.float64) @ W.T.astype(np.float64)
-    assert rel(y[rows], ref) < 2.0 ** -24 * (1 + np.sqrt(6 * K / 16))
+    assert rel(y[rows], ref) < 2.0 ** -24 * (1 + np.sqrt(K if ex + ew >= 80 or ex > 104 else 6 * K / 16))
 
 
 @pytest.mark.parametrize("M,K,N,dtype", [(1499, 3040, 764, "fp32"), (128, 3072, 768, "fp32"), (128, 4096, 768, "bf16"),      # 128 x 128 and 32 x 32 tiles
