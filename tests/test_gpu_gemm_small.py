@@ -76,7 +76,7 @@ def test_layernormed_residual(backend, dtype, M, K, N):
 
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
-@pytest.mark.parametrize("M,K,N", [(3000, 768, 768), (700, 768, 768), (4000, 256, 1024)])
+@pytest.mark.parametrize("M,K,N", [(3000, 768, 768), (700, 768, 768), (4000, 256, 1024), (16384, 128, 2048)])
 def test_blocks_of_a_host_call_add_in_the_order_of_the_whole_product(backend, dtype, M, K, N):
     c, code = backend.core, CODE[dtype]
     rng = np.random.default_rng(M + N)
