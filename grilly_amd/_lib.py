@@ -135,6 +135,12 @@ SIGNATURES = {
     "grl_bert_layer_fused_workspace": (c_i64, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64]),
     "grl_bert_layer_fwd_fused": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_void_p, c_float,
                                  c_void_p, c_void_p, c_void_p]),
+    "grl_bert_layers_fused_workspace": (c_i64, [c_int, c_i64, c_i64, c_i64, c_i64, c_i64]),
+    "grl_bert_layers_fwd_fused": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_i64, c_void_p, c_float,
+                                  c_void_p, c_void_p, c_void_p]),
+    "grl_bert_layers_fwd_fused_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_i64, c_float,
+                                         c_void_p, c_void_p, c_void_p]),
+    "grl_resln_ln_glu": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64] + [c_void_p] * 14 + [c_float, c_void_p, c_void_p, c_void_p, c_int]),
     "grl_bert_layer_fwd": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayer), c_void_p, c_float, c_void_p, c_void_p]),
 }
 

@@ -83,15 +83,19 @@ extern "C" int64_t grl_bert_layer_fused_workspace(int dtype, int64_t B, int64_t 
     return pad(M * 3 * d * es) + pad(M * d * es) + pad(M * d_ff * es) + pad(M * 8) + pad(grl_gemm_nt_resln_workspace(M, d));
 }
 
-static int bert_layer_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
-                            const grl_bert_layer_fused* w, const float* mask, float eps, void* r, float* stats,
-                            void* workspace, const grl_ragged* rg) {
-    GRL_REQUIRE(c && w && r && stats && workspace, GRL_ERR_ARG, "grl_bert_layer_fwd_fused: null argument");
+// `layers` layers, the first of which finds the statistics of r in stats.  Between them, and inside each, the statistics stay the partials
+// that the residual products leave; with `last_merged` those of the final r are merged into stats (workspace: as of one layer then;
+// else grl_bert_layers_fused_workspace, as the partials that a layer starts from live beside those of its middle).
+static int bert_layers_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                             const grl_bert_layer_fused* w, int64_t layers, bool last_merged, const float* mask, float eps, void* r, float* stats,
+                             void* workspace, const grl_ragged* rg) {
+    GRL_REQUIRE(c && w && r && stats && workspace && layers >= 0, GRL_ERR_ARG, "grl_bert_layer_fwd_fused: null argument");
     GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_bert_layer_fwd_fused: bad dtype %d", dtype);
     GRL_REQUIRE(B >= 0 && S >= 0 && H > 0 && d_ff > 0, GRL_ERR_SHAPE, "grl_bert_layer_fwd_fused: bad shape");
     GRL_REQUIRE(D >= 1 && D <= 1024, GRL_ERR_SHAPE, "grl_bert_layer_fwd_fused: head_dim must be between 1 and 1024 (got %lld)", (long long)D);
-    GRL_REQUIRE(w->ws_qkv && w->c_qkv && w->bf_qkv && w->in_g && w->in_b && w->w_o && w->ln1_g && w->ln1_b && w->ws_ff1 && w->c_ff1 &&
-                w->bf_ff1 && w->w_ff2, GRL_ERR_ARG, "grl_bert_layer_fwd_fused: null weight");
+    for (int64_t l = 0; l < layers; ++l)
+        GRL_REQUIRE(w[l].ws_qkv && w[l].c_qkv && w[l].bf_qkv && w[l].in_g && w[l].in_b && w[l].w_o && w[l].ln1_g && w[l].ln1_b && w[l].ws_ff1 && w[l].c_ff1 &&
+                    w[l].bf_ff1 && w[l].w_ff2, GRL_ERR_ARG, "grl_bert_layer_fwd_fused: null weight");
     const int64_t M = rg ? rg->rows : B * S, d = H * D, es = (int64_t)grl_dtype_size(dtype), slab = 128 / es;
     GRL_REQUIRE(d % slab == 0 && d_ff % slab == 0, GRL_ERR_SHAPE,
                 "grl_bert_layer_fwd_fused: d_model (%lld) and d_ff (%lld) must be multiples of %lld; use grl_bert_layer_fwd",
@@ -103,30 +107,68 @@ static int bert_layer_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t
     char* ff = attn + pad(M * d * es);
     float* stats1 = (float*)(ff + pad(M * d_ff * es));
     char* part = (char*)stats1 + pad(M * 8);
-    int rc;
-    grl_lap_mark(c);
-    if ((rc = grl_ln_gemm_nt_stats(c, dtype, dtype, M, 3 * d, d, r, w->ws_qkv, w->c_qkv, w->bf_qkv, stats, qkv, GRL_EPI_NONE))) return rc;
-    grl_lap_mark(c);
-    if ((rc = layer_attention(c, dtype, B, S, H, D, qkv, mask, attn, rg))) return rc;
-    grl_lap_mark(c);
-    if ((rc = grl_gemm_nt_resln(c, dtype, M, d, d, attn, w->w_o, w->b_o, r, stats, w->in_g, w->in_b, r, eps, stats1, part))) return rc;
-    grl_lap_mark(c);
-    if ((rc = grl_ln_gemm_nt_stats(c, dtype, dtype, M, d_ff, d, r, w->ws_ff1, w->c_ff1, w->bf_ff1, stats1, ff, GRL_EPI_GELU))) return rc;
-    grl_lap_mark(c);
-    if ((rc = grl_gemm_nt_resln(c, dtype, M, d, d_ff, ff, w->w_ff2, w->b_ff2, r, stats1, w->ln1_g, w->ln1_b, r, eps, stats, part))) return rc;
-    grl_lap_mark(c);
+    char* part_next = part + pad(grl_gemm_nt_resln_workspace(M, d));
+    grl_row_stats in = {stats, nullptr, 0, eps}, mid{};
+    for (int64_t l = 0; l < layers; ++l, ++w) {
+        int rc;
+        grl_lap_mark(c);
+        if ((rc = grl_ln_gemm_nt_from(c, dtype, M, 3 * d, d, r, w->ws_qkv, w->c_qkv, w->bf_qkv, in, stats, qkv, GRL_EPI_NONE))) return rc;
+        grl_lap_mark(c);
+        if ((rc = layer_attention(c, dtype, B, S, H, D, qkv, mask, attn, rg))) return rc;
+        grl_lap_mark(c);
+        if ((rc = grl_gemm_nt_resln_parts(c, dtype, M, d, d, attn, w->w_o, w->b_o, r, in, w->in_g, w->in_b, r, eps, stats1, part, &mid))) return rc;
+        grl_lap_mark(c);
+        if ((rc = grl_ln_gemm_nt_from(c, dtype, M, d_ff, d, r, w->ws_ff1, w->c_ff1, w->bf_ff1, mid, stats1, ff, GRL_EPI_GELU))) return rc;
+        grl_lap_mark(c);
+        // (the partials that the layer started from have been read by now)
+        if (last_merged && l == layers - 1) {
+            if (mid.nparts) {      // the one partials' buffer of a single layer is read and written by this product: other rows, other tiles
+                if ((rc = grl_merge_row_stats(c, mid.parts, stats1, M, d, mid.nparts, eps))) return rc;
+                mid = {stats1, nullptr, 0, eps};
+            }
+            rc = grl_gemm_nt_resln(c, dtype, M, d, d_ff, ff, w->w_ff2, w->b_ff2, r, mid.stats, w->ln1_g, w->ln1_b, r, eps, stats, part);
+        } else rc = grl_gemm_nt_resln_parts(c, dtype, M, d, d_ff, ff, w->w_ff2, w->b_ff2, r, mid, w->ln1_g, w->ln1_b, r, eps, stats, part_next, &in);
+        if (rc) return rc;
+        grl_lap_mark(c);
+    }
     return GRL_OK;
 }
 
 extern "C" int grl_bert_layer_fwd_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
                                         const grl_bert_layer_fused* w, const float* mask, float eps, void* r, float* stats,
                                         void* workspace) {
-    return bert_layer_fused(c, dtype, B, S, H, D, d_ff, w, mask, eps, r, stats, workspace, nullptr);
+    return bert_layers_fused(c, dtype, B, S, H, D, d_ff, w, 1, true, mask, eps, r, stats, workspace, nullptr);
 }
 extern "C" int grl_bert_layer_fwd_fused_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t H, int64_t D, int64_t d_ff,
                                                const grl_bert_layer_fused* w, float eps, void* r, float* stats, void* workspace) {
     int rc = grl_check_ragged("grl_bert_layer_fwd_fused_ragged", rg);
-    return rc ? rc : bert_layer_fused(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, nullptr, eps, r, stats, workspace, rg);
+    return rc ? rc : bert_layers_fused(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, 1, true, nullptr, eps, r, stats, workspace, rg);
+}
+
+extern "C" int64_t grl_bert_layers_fused_workspace(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff) {
+    const int64_t one = grl_bert_layer_fused_workspace(dtype, B, S, H, D, d_ff);
+    return one < 0 ? one : one + (grl_gemm_nt_resln_workspace(B * S, H * D) + 255) / 256 * 256;
+}
+extern "C" int grl_bert_layers_fwd_fused(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff,
+                                         const grl_bert_layer_fused* w, int64_t layers, const float* mask, float eps, void* r, float* stats,
+                                         void* workspace) {
+    return bert_layers_fused(c, dtype, B, S, H, D, d_ff, w, layers, false, mask, eps, r, stats, workspace, nullptr);
+}
+extern "C" int grl_bert_layers_fwd_fused_ragged(grl_ctx* c, int dtype, const grl_ragged* rg, int64_t H, int64_t D, int64_t d_ff,
+                                                const grl_bert_layer_fused* w, int64_t layers, float eps, void* r, float* stats, void* workspace) {
+    int rc = grl_check_ragged("grl_bert_layers_fwd_fused_ragged", rg);
+    return rc ? rc : bert_layers_fused(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, layers, false, nullptr, eps, r, stats, workspace, rg);
+}
+
+// ---- the two products around the LayerNorm of a gated MLP ---------------------------------------------------------
+extern "C" int grl_resln_ln_glu(grl_ctx* c, int dtype, int64_t M, int64_t d, int64_t K, int64_t d_ff, const void* A, const void* W, const float* bias,
+                                const void* R, const float* r_stats, const float* r_gamma, const float* r_beta, void* C, const void* Wg_scaled,
+                                const void* Wu_scaled, const float* colsum_gate, const float* colsum_up, const float* bias_gate_folded,
+                                const float* bias_up_folded, float eps, float* stats, void* workspace, void* out, int activation) {
+    grl_row_stats rows{};
+    const int rc = grl_gemm_nt_resln_parts(c, dtype, M, d, K, A, W, bias, R, grl_row_stats{r_stats, nullptr, 0, 0.f}, r_gamma, r_beta, C, eps, stats, workspace, &rows);
+    if (rc || M == 0 || d == 0) return rc;
+    return grl_ln_glu_nt_from(c, dtype, M, d_ff, d, C, Wg_scaled, Wu_scaled, colsum_gate, colsum_up, bias_gate_folded, bias_up_folded, rows, stats, out, activation);
 }
 
 // ---- the same for few rows: five launches, no statistics pass, no partials to merge -------------------------------

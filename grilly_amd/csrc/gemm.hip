@@ -180,9 +180,8 @@ extern "C" int grl_ln_gemm_nt(grl_ctx* c, int in_dtype, int out_dtype, int64_t M
 }
 
 // the same with the row statistics given (computed earlier, e.g. by the GEMM that produced x) and a choice of epilogue
-extern "C" int grl_ln_gemm_nt_stats(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x,
-                                    const void* W_scaled, const float* colsum, const float* bias_folded,
-                                    const float* stats, void* out, int epilogue) {
+static int ln_gemm_nt_impl(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* W_scaled,
+                           const float* colsum, const float* bias_folded, const grl_row_stats& rows, float* merged, void* out, int epilogue) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "grl_ln_gemm_nt_stats: null context");
     GRL_REQUIRE(grl_valid_dtype(in_dtype) && grl_valid_dtype(out_dtype), GRL_ERR_ARG, "grl_ln_gemm_nt_stats: bad dtype");
     GRL_REQUIRE(epilogue == GRL_EPI_NONE || epilogue == GRL_EPI_GELU, GRL_ERR_ARG,
@@ -190,13 +189,24 @@ extern "C" int grl_ln_gemm_nt_stats(grl_ctx* c, int in_dtype, int out_dtype, int
     int rc = check_dims("grl_ln_gemm_nt_stats", M, N, K);
     if (rc) return rc;
     if (M == 0 || N == 0) return GRL_OK;
-    GRL_REQUIRE(out && K > 0 && x && W_scaled && colsum && bias_folded && stats, GRL_ERR_ARG, "grl_ln_gemm_nt_stats: null argument or K == 0");
+    GRL_REQUIRE(out && K > 0 && x && W_scaled && colsum && bias_folded && (rows.stats || (rows.nparts && merged)), GRL_ERR_ARG,
+                "grl_ln_gemm_nt_stats: null argument or K == 0");
     GemmArgs a{};
     a.A = x; a.W = W_scaled; a.bias = bias_folded; a.C = out;
-    a.ln_stats = stats; a.ln_c = colsum;
+    a.ln_stats = rows.stats; a.ln_c = colsum;
+    a.parts = rows.parts; a.nparts = rows.nparts; a.eps = rows.eps; a.merged = merged;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
     a.act = epilogue;
     return dispatch_types_ln(c, a, in_dtype, out_dtype, epilogue == GRL_EPI_GELU ? EPI_GELU : EPI_NONE);
+}
+extern "C" int grl_ln_gemm_nt_stats(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x,
+                                    const void* W_scaled, const float* colsum, const float* bias_folded,
+                                    const float* stats, void* out, int epilogue) {
+    return ln_gemm_nt_impl(c, in_dtype, out_dtype, M, N, K, x, W_scaled, colsum, bias_folded, grl_row_stats{stats, nullptr, 0, 0.f}, nullptr, out, epilogue);
+}
+int grl_ln_gemm_nt_from(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* W_scaled, const float* colsum,
+                        const float* bias_folded, const grl_row_stats& rows, float* merged, void* out, int epilogue) {
+    return ln_gemm_nt_impl(c, dtype, dtype, M, N, K, x, W_scaled, colsum, bias_folded, rows, merged, out, epilogue);
 }
 
 // which kernel / tile size grl_gemm_nt and its siblings pick for a 16-byte aligned problem (pure host arithmetic)
@@ -227,34 +237,57 @@ __global__ __launch_bounds__(256) void ln_stats_merge_kernel(const float* __rest
     *(float2*)(stats + 2 * (int64_t)m) = make_float2(1.0f / sd, mean / sd);
 }
 
+int grl_merge_row_stats(grl_ctx* c, const float* parts, float* stats, int64_t M, int64_t N, int nparts, float eps) {
+    hipLaunchKernelGGL(ln_stats_merge_kernel, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, c->stream, parts, stats, (int)M, (int)N, nparts, eps);
+    GRL_CHECK_LAUNCH();
+    return GRL_OK;
+}
+
 extern "C" int64_t grl_gemm_nt_resln_workspace(int64_t M, int64_t N) {
     if (M < 0 || N < 0) return -1;
     return ((N + 127) / 128) * M * 8 + 256;          // one {sum, sum of squares} pair per row and 128-column tile (the narrowest tile)
 }
 
-extern "C" int grl_gemm_nt_resln(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W,
-                                 const float* bias, const void* R, const float* r_stats, const float* r_gamma,
-                                 const float* r_beta, void* C, float eps, float* stats_out, void* workspace) {
+// out == nullptr: the statistics are merged into stats_out.  Else they may stay partials, which spares a launch of 4 to 5 us: the products
+// that read them merge those of a tile's rows when they start it, under 1 % of its time.
+static int resln(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, const void* R,
+                 const grl_row_stats& r_stats, const float* r_gamma, const float* r_beta, void* C, float eps, float* stats_out,
+                 void* workspace, grl_row_stats* out) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "grl_gemm_nt_resln: null context");
     GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_gemm_nt_resln: bad dtype");
     int rc = check_dims("grl_gemm_nt_resln", M, N, K);
     if (rc) return rc;
     if (M == 0 || N == 0) return GRL_OK;
-    GRL_REQUIRE(A && W && R && r_stats && r_gamma && r_beta && C && stats_out && workspace && K > 0, GRL_ERR_ARG,
+    GRL_REQUIRE(A && W && R && (r_stats.stats || r_stats.nparts) && r_gamma && r_beta && C && stats_out && workspace && K > 0, GRL_ERR_ARG,
                 "grl_gemm_nt_resln: null argument or K == 0");
     GRL_REQUIRE((((uintptr_t)workspace) & 15u) == 0 && (((uintptr_t)stats_out) & 15u) == 0, GRL_ERR_ARG, "grl_gemm_nt_resln: workspace and stats_out must be 16-byte aligned");
     GemmArgs a{};
     a.A = A; a.W = W; a.bias = bias; a.C = C; a.residual = R;
-    a.res_stats = r_stats; a.res_gamma = r_gamma; a.res_beta = r_beta; a.part_out = (float*)workspace;
+    a.res_stats = r_stats.stats; a.res_gamma = r_gamma; a.res_beta = r_beta; a.part_out = (float*)workspace;
+    a.parts = r_stats.parts; a.nparts = r_stats.nparts; a.eps = r_stats.eps;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
     int tile_cols = 0;
     rc = dtype == GRL_F32 ? launch_gemm_resln<float, float>(c, a, &tile_cols) : launch_gemm_resln<uint16_t, uint16_t>(c, a, &tile_cols);
     if (rc) return rc;
     const int nparts = (int)((N + tile_cols - 1) / tile_cols);
-    hipLaunchKernelGGL(ln_stats_merge_kernel, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, c->stream, (const float*)workspace, stats_out,
-                       (int)M, (int)N, nparts, eps);
-    GRL_CHECK_LAUNCH();
-    return GRL_OK;
+    if (out && nparts <= GRL_MAX_PARTS) {
+        *out = {nullptr, (const float*)workspace, nparts, eps};
+        return GRL_OK;
+    }
+    if (out) *out = {stats_out, nullptr, 0, eps};
+    return grl_merge_row_stats(c, (const float*)workspace, stats_out, M, N, nparts, eps);
+}
+
+extern "C" int grl_gemm_nt_resln(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W,
+                                 const float* bias, const void* R, const float* r_stats, const float* r_gamma,
+                                 const float* r_beta, void* C, float eps, float* stats_out, void* workspace) {
+    return resln(c, dtype, M, N, K, A, W, bias, R, grl_row_stats{r_stats, nullptr, 0, 0.f}, r_gamma, r_beta, C, eps, stats_out, workspace, nullptr);
+}
+
+int grl_gemm_nt_resln_parts(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, const void* R,
+                            const grl_row_stats& r_stats, const float* r_gamma, const float* r_beta, void* C, float eps, float* stats_out,
+                            void* workspace, grl_row_stats* out) {
+    return resln(c, dtype, M, N, K, A, W, bias, R, r_stats, r_gamma, r_beta, C, eps, stats_out, workspace, out);
 }
 
 // ---- products of few rows that take the row statistics of a folded LayerNorm themselves ---------------------------
@@ -318,7 +351,7 @@ extern "C" int grl_gemm_nt_lnres(grl_ctx* c, int dtype, int64_t M, int64_t N, in
 static int ln_glu_nt_impl(grl_ctx* c, const char* who, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x,
                           const void* Wg_scaled, const void* Wu_scaled, const float* colsum_gate, const float* colsum_up,
                           const float* bias_gate_folded, const float* bias_up_folded, bool given, float eps, float* stats,
-                          void* out, int activation) {
+                          void* out, int activation, const grl_row_stats* rows = nullptr) {
     GRL_REQUIRE(c, GRL_ERR_ARG, "%s: null context", who);
     GRL_REQUIRE(grl_valid_dtype(in_dtype) && grl_valid_dtype(out_dtype), GRL_ERR_ARG, "%s: bad dtype", who);
     GRL_REQUIRE(activation == GRL_EPI_SILU || activation == GRL_EPI_RELU || activation == GRL_EPI_GELU, GRL_ERR_ARG,
@@ -336,6 +369,10 @@ static int ln_glu_nt_impl(grl_ctx* c, const char* who, int in_dtype, int out_dty
     a.A = x; a.W = Wg_scaled; a.W2 = Wu_scaled; a.C = out;
     a.bias = bias_gate_folded; a.bias2 = bias_up_folded;
     a.ln_stats = stats; a.ln_c = colsum_gate; a.ln_c2 = colsum_up;
+    if (rows) {
+        a.ln_stats = rows->stats; a.merged = stats;
+        a.parts = rows->parts; a.nparts = rows->nparts; a.eps = rows->eps;
+    }
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
     a.act = activation;
     return dispatch_types_ln(c, a, in_dtype, out_dtype, EPI_GLU);
@@ -347,6 +384,12 @@ extern "C" int grl_ln_glu_nt(grl_ctx* c, int in_dtype, int out_dtype, int64_t M,
                              void* out, int activation) {
     return ln_glu_nt_impl(c, "grl_ln_glu_nt", in_dtype, out_dtype, M, N, K, x, Wg_scaled, Wu_scaled, colsum_gate, colsum_up,
                           bias_gate_folded, bias_up_folded, false, eps, stats, out, activation);
+}
+int grl_ln_glu_nt_from(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* x, const void* Wg_scaled, const void* Wu_scaled,
+                       const float* colsum_gate, const float* colsum_up, const float* bias_gate_folded, const float* bias_up_folded,
+                       const grl_row_stats& rows, float* merged, void* out, int activation) {
+    return ln_glu_nt_impl(c, "grl_ln_glu_nt_stats", dtype, dtype, M, N, K, x, Wg_scaled, Wu_scaled, colsum_gate, colsum_up,
+                          bias_gate_folded, bias_up_folded, true, 0.f, merged, out, activation, &rows);
 }
 extern "C" int grl_ln_glu_nt_stats(grl_ctx* c, int in_dtype, int out_dtype, int64_t M, int64_t N, int64_t K, const void* x,
                                    const void* Wg_scaled, const void* Wu_scaled, const float* colsum_gate, const float* colsum_up,

@@ -221,6 +221,7 @@ class BertEncoder:
                 f.w_ff2, f.b_ff2 = s.w_ff2, s.b_ff2
                 self.fused_structs.append(f)
                 in_g, in_b = s.ln2_g, s.ln2_b
+            self._fused_array = (L.BertLayerFused * len(self.fused_structs))(*self.fused_structs)
         self._shape = None
 
     def _own(self, buf):
@@ -239,7 +240,7 @@ class BertEncoder:
         self.fused_now = self.fused and B * S >= self._fused_min_rows        # which layer form this batch runs
         ws = c.lib.grl_bert_layer_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff)
         if self.fused:                       # without its padding the batch may run any form
-            ws = max(ws, c.lib.grl_bert_layer_fused_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff))
+            ws = max(ws, c.lib.grl_bert_layers_fused_workspace(self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff))
         self.x = c.alloc(B * S * cfg.d_model * es)
         self.stats = c.alloc(max(B * S, 1) * 8)        # {1/sd, mean/sd} per row of the raw residual stream (fused layers)
         self.ws = c.alloc(ws)
@@ -299,14 +300,13 @@ class BertEncoder:
                 in_eps = cfg.eps
             self._last_layernorm(B * S)
         elif self.fused_now and B * S > 0:
-            # raw embedding rows + their statistics; every layer consumes and produces (raw rows, statistics); the last
-            # layer's second LayerNorm is the one pass that writes normalised rows
+            # raw embedding rows + their statistics; the layers pass raw rows and row statistics on; the last layer's second
+            # LayerNorm is the one pass that writes normalised rows
             L.check(lib.grl_embed(c.ctx, self.code, B, S, cfg.d_model, cfg.vocab, self.ids.ptr, self.tok.ptr, self.pos.ptr,
                                   self.typ.ptr, self.x.ptr), "embedding")
             L.check(lib.grl_ln_stats(c.ctx, self.code, B * S, cfg.d_model, self.x.ptr, cfg.embedding_eps, self.stats.ptr), "embedding statistics")
-            for f in self.fused_structs:
-                L.check(lib.grl_bert_layer_fwd_fused(c.ctx, self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f),
-                                                     mask, cfg.eps, self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layer_fwd_fused")
+            L.check(lib.grl_bert_layers_fwd_fused(c.ctx, self.code, B, S, cfg.heads, cfg.head_dim, cfg.d_ff, self._fused_array, cfg.layers,
+                                                  mask, cfg.eps, self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layers_fwd_fused")
             self._last_layernorm(B * S)
         else:
             L.check(lib.grl_embed_layernorm(c.ctx, self.code, B, S, cfg.d_model, cfg.vocab, self.ids.ptr, self.tok.ptr,
@@ -341,9 +341,8 @@ class BertEncoder:
             L.check(lib.grl_embed_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
                                          self.x.ptr), "embedding")
             L.check(lib.grl_ln_stats(c.ctx, self.code, rg.rows, cfg.d_model, self.x.ptr, cfg.embedding_eps, self.stats.ptr), "embedding statistics")
-            for f in self.fused_structs:
-                L.check(lib.grl_bert_layer_fwd_fused_ragged(c.ctx, self.code, r, cfg.heads, cfg.head_dim, cfg.d_ff, ctypes.byref(f), cfg.eps,
-                                                            self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layer_fwd_fused")
+            L.check(lib.grl_bert_layers_fwd_fused_ragged(c.ctx, self.code, r, cfg.heads, cfg.head_dim, cfg.d_ff, self._fused_array, cfg.layers,
+                                                         cfg.eps, self.x.ptr, self.stats.ptr, self.ws.ptr), "bert_layers_fwd_fused")
             self._last_layernorm(rg.rows)
         else:
             L.check(lib.grl_embed_layernorm_ragged(c.ctx, self.code, r, cfg.d_model, cfg.vocab, ids, self.tok.ptr, self.pos.ptr, self.typ.ptr,
@@ -579,12 +578,10 @@ class PreNormEncoder:
                                                w["cs_in"].ptr, w["bf_gate"].ptr, w["bf_in"].ptr, cfg.eps, self.h.ptr, L.EPI_GELU),
                         "mlp layernorm + geglu")
             elif self.stats_from_gemm:
-                L.check(lib.grl_gemm_nt_resln(c.ctx, code, M, d, d, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,
-                                              self.ident_stats.ptr, self.ones.ptr, self.zeros.ptr, self.x.ptr, cfg.eps,
-                                              self.stats.ptr, self.part.ptr), "output projection + residual + row statistics")
-                L.check(lib.grl_ln_glu_nt_stats(c.ctx, code, code, M, ff, d, self.x.ptr, w["ws_gate"].ptr, w["ws_in"].ptr,
-                                                w["cs_gate"].ptr, w["cs_in"].ptr, w["bf_gate"].ptr, w["bf_in"].ptr,
-                                                self.stats.ptr, self.h.ptr, L.EPI_GELU), "mlp layernorm + geglu")
+                L.check(lib.grl_resln_ln_glu(c.ctx, code, M, d, d, ff, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,
+                                             self.ident_stats.ptr, self.ones.ptr, self.zeros.ptr, self.x.ptr, w["ws_gate"].ptr, w["ws_in"].ptr,
+                                             w["cs_gate"].ptr, w["cs_in"].ptr, w["bf_gate"].ptr, w["bf_in"].ptr, cfg.eps, self.stats.ptr,
+                                             self.part.ptr, self.h.ptr, L.EPI_GELU), "output projection + residual, mlp layernorm + geglu")
             else:
                 L.check(lib.grl_gemm_nt_res(c.ctx, code, code, M, d, d, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,
                                             self.x.ptr), "output projection + residual")

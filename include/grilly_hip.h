@@ -483,6 +483,21 @@ int grl_bert_layer_fwd_fused(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int6
                              void* r, float* stats, void* workspace);
 int grl_bert_layer_fwd_fused_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
                                     const grl_bert_layer_fused* w, float eps, void* r, float* stats, void* workspace);
+/* `layers` such layers one behind the other.  The row statistics between the products stay the partial sums that the residual products
+ * leave, which the products that read them merge, so no launch between the products is left.  stats: those of r on entry, scratch
+ * afterwards (the output is raw rows for a grl_layernorm).  workspace: grl_bert_layers_fused_workspace bytes. */
+int64_t grl_bert_layers_fused_workspace(int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff);
+int grl_bert_layers_fwd_fused(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, int64_t d_ff, const grl_bert_layer_fused* w,
+                              int64_t layers, const float* mask, float eps, void* r, float* stats, void* workspace);
+int grl_bert_layers_fwd_fused_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
+                                     const grl_bert_layer_fused* w, int64_t layers, float eps, void* r, float* stats, void* workspace);
+/* grl_gemm_nt_resln (C = A.W^T + bias + LayerNorm(R), d columns), then grl_ln_glu_nt_stats on its rows (d_ff outputs): the block in front
+ * of a gated MLP, utils/vulkan_sentence_transformer.py:893-927, in two launches.  stats: (M, 2) floats of scratch, 16-byte aligned;
+ * workspace: grl_gemm_nt_resln_workspace(M, d) bytes. */
+int grl_resln_ln_glu(grl_ctx* ctx, int dtype, int64_t M, int64_t d, int64_t K, int64_t d_ff, const void* A, const void* W, const float* bias,
+                     const void* R, const float* r_stats, const float* r_gamma, const float* r_beta, void* C, const void* Wg_scaled,
+                     const void* Wu_scaled, const float* colsum_gate, const float* colsum_up, const float* bias_gate_folded,
+                     const float* bias_up_folded, float eps, float* stats, void* workspace, void* out, int activation);
 /* The folded layer for few rows in five launches (grl_ln_gemm_nt_rows, attention, grl_gemm_nt_lnres, grl_ln_gemm_nt_rows,
  * grl_gemm_nt_lnres): only the raw rows r travel between layers.  in_eps: of the LayerNorm that turns r into the layer's input,
  * eps: of ln1.  workspace: grl_bert_layer_fused_workspace bytes. */
