@@ -54,7 +54,8 @@ def test_pack_batch_refusals():
 
 
 # edges of the 32-query waves, 64- and 128-key tiles and 128- / 256-query workgroups, an empty and a one-token sequence
-LENGTHS = {"short": [1, 32, 0, 33, 64, 65, 127, 129], "long": [1025, 3, 256, 1200]}
+# and enough sequences (of two heads each, no whole turn of eight) that their heads are dealt out
+LENGTHS = {"short": [1, 32, 0, 33, 64, 65, 127, 129], "long": [1025, 3, 256, 1200], "many": [(37 * i * i + 11 * i) % 290 for i in range(35)]}
 
 
 @pytest.mark.gpu
