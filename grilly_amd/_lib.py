@@ -140,6 +140,7 @@ SIGNATURES = {
                                   c_void_p, c_void_p, c_void_p]),
     "grl_bert_layers_fwd_fused_ragged": (c_int, [c_void_p, c_int, _rg, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayerFused), c_i64, c_float,
                                          c_void_p, c_void_p, c_void_p]),
+    "grl_rotary_attention": (c_int, [c_void_p, c_int, c_i64, c_i64, _rg, c_i64, c_i64] + [c_void_p] * 6 + [c_float, c_float]),
     "grl_resln_ln_glu": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64] + [c_void_p] * 14 + [c_float, c_void_p, c_void_p, c_void_p, c_int]),
     "grl_bert_layer_fwd": (c_int, [c_void_p, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(BertLayer), c_void_p, c_float, c_void_p, c_void_p]),
 }

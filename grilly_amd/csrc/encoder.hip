@@ -160,6 +160,34 @@ extern "C" int grl_bert_layers_fwd_fused_ragged(grl_ctx* c, int dtype, const grl
     return rc ? rc : bert_layers_fused(c, dtype, rg->sequences, rg->longest, H, D, d_ff, w, layers, false, nullptr, eps, r, stats, workspace, rg);
 }
 
+// ---- projection and attention with rotary positions ---------------------------------------------------------------
+extern "C" int grl_rotary_attention(grl_ctx* c, int dtype, int64_t B, int64_t S, const grl_ragged* rg, int64_t H, int64_t D, const void* x,
+                                    const void* w_qkv, const float* b_qkv, const float* mask, void* qkv, void* out, float rope_base, float rope_scaling) {
+    GRL_REQUIRE(c && x && w_qkv && qkv && out, GRL_ERR_ARG, "grl_rotary_attention: null argument");
+    GRL_REQUIRE(grl_valid_dtype(dtype), GRL_ERR_ARG, "grl_rotary_attention: bad dtype %d", dtype);
+    GRL_REQUIRE(B >= 0 && S >= 0 && H > 0 && D >= 2 && D <= 128 && D % 2 == 0, GRL_ERR_SHAPE, "grl_rotary_attention: bad shape");
+    GRL_REQUIRE(rope_base > 0.f && rope_scaling != 0.f, GRL_ERR_ARG, "grl_rotary_attention: bad rope base/scaling");
+    if (rg) {
+        const int rc = grl_check_ragged("grl_rotary_attention", rg);
+        if (rc) return rc;
+    }
+    const int64_t M = rg ? rg->rows : B * S, longest = rg ? rg->longest : S, d = H * D, es = (int64_t)grl_dtype_size(dtype);
+    if (M == 0) return GRL_OK;
+    char* q = (char*)qkv;
+    int rope = GRL_ROPE_HALF, rc;
+    if (dtype == GRL_BF16 && D == 64 && M < (1LL << 31) && 3 * d < (1LL << 31)) {
+        const float* table = nullptr;
+        if ((rc = grl_rope_table_get(c, (int)longest, (int)D, rope_base, rope_scaling, GRL_ROPE_HALF, &table))) return rc;
+        bool taken = false;
+        if ((rc = grl_gemm_nt_rope_bf16(c, M, 3 * d, d, x, w_qkv, b_qkv, qkv, 2 * d, table, rg ? rg->positions : nullptr, S, &taken))) return rc;
+        if (taken) rope = GRL_ROPE_NONE;
+    }
+    if (rope == GRL_ROPE_HALF && (rc = grl_gemm_nt(c, dtype, dtype, M, 3 * d, d, x, w_qkv, b_qkv, qkv, GRL_EPI_NONE))) return rc;
+    const float scale = (float)(1.0 / sqrt((double)D));
+    if (rg) return grl_fa2_fwd_ragged(c, dtype, rg, H, D, q, q + d * es, q + 2 * d * es, out, 3 * d, 3 * d, 3 * d, d, scale, 0, rope, rope_base, rope_scaling);
+    return grl_fa2_fwd_strided(c, dtype, B, S, H, D, q, q + d * es, q + 2 * d * es, mask, out, 3 * d, 3 * d, 3 * d, d, scale, 0, rope, rope_base, rope_scaling);
+}
+
 // ---- the two products around the LayerNorm of a gated MLP ---------------------------------------------------------
 extern "C" int grl_resln_ln_glu(grl_ctx* c, int dtype, int64_t M, int64_t d, int64_t K, int64_t d_ff, const void* A, const void* W, const float* bias,
                                 const void* R, const float* r_stats, const float* r_gamma, const float* r_beta, void* C, const void* Wg_scaled,

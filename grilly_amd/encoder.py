@@ -563,17 +563,11 @@ class PreNormEncoder:
             L.check(lib.grl_embed_layernorm_ragged(c.ctx, code, ctypes.byref(rg), d, cfg.vocab, ids, self.tok.ptr, None, None,
                                                    self.emb_g.ptr, self.emb_b.ptr, cfg.emb_eps, self.x.ptr), "embedding + layernorm")
         for w in self.layers:
-            # one GEMM with the packed weight; attention reads Q, K, V as column blocks of its output and applies
-            # the rotation itself (queries as they are loaded, keys once per row from the cached table)
-            L.check(lib.grl_gemm_nt(c.ctx, code, code, M, 3 * d, d, self.x.ptr, w["w_qkv"].ptr, w["b_qkv"].ptr,
-                                    self.qkv.ptr, L.EPI_NONE), "q/k/v projection")
-            q, k, v, scale = self.qkv.ptr, self.qkv.ptr + d * es, self.qkv.ptr + 2 * d * es, 1.0 / float(np.sqrt(D))
-            if rg is None:
-                L.check(lib.grl_fa2_fwd_strided(c.ctx, code, B, S, H, D, q, k, v, mask, self.att.ptr, 3 * d, 3 * d, 3 * d, d, scale, 0,
-                                                L.ROPE_HALF, cfg.rope_base, cfg.rope_scaling), "attention")
-            else:
-                L.check(lib.grl_fa2_fwd_ragged(c.ctx, code, ctypes.byref(rg), H, D, q, k, v, self.att.ptr, 3 * d, 3 * d, 3 * d, d, scale, 0,
-                                               L.ROPE_HALF, cfg.rope_base, cfg.rope_scaling), "attention")
+            # one GEMM with the packed weight, rotating queries and keys on its way out where its kernel can; attention reads Q, K, V
+            # as column blocks of its output
+            L.check(lib.grl_rotary_attention(c.ctx, code, B, S, None if rg is None else ctypes.byref(rg), H, D, self.x.ptr, w["w_qkv"].ptr,
+                                             w["b_qkv"].ptr, mask if rg is None else None, self.qkv.ptr, self.att.ptr, cfg.rope_base,
+                                             cfg.rope_scaling), "q/k/v projection, attention")
             # LayerNorm + dual GEMM; the dual GEMM activates its second ("up") operand: that is the first half of Wi here
             if own_stats:
                 L.check(lib.grl_gemm_nt_res(c.ctx, code, code, M, d, d, self.att.ptr, w["w_o"].ptr, w["b_o"].ptr, self.x.ptr,

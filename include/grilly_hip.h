@@ -491,6 +491,13 @@ int grl_bert_layers_fwd_fused(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int
                               int64_t layers, const float* mask, float eps, void* r, float* stats, void* workspace);
 int grl_bert_layers_fwd_fused_ragged(grl_ctx* ctx, int dtype, const grl_ragged* batch, int64_t H, int64_t D, int64_t d_ff,
                                      const grl_bert_layer_fused* w, int64_t layers, float eps, void* r, float* stats, void* workspace);
+/* Self-attention with rotary positions from the rows x (B*S, or those of a ragged batch; d = H*D) on: qkv = x.Wqkv^T + b (rows of 3*d), the
+ * halves of each head of Q and K rotated as pairs (GRL_ROPE_HALF), out = attention.  Replaces the projection, rotation and attention
+ * of utils/vulkan_sentence_transformer.py:806-891.  In bf16 with D = 64 the rotation runs in the projection's epilogue wherever its
+ * kernel has one, and Q and K stand in qkv rotated; else attention rotates and they stand as projected.  mask: (B, S) or NULL, of a
+ * rectangular batch. */
+int grl_rotary_attention(grl_ctx* ctx, int dtype, int64_t B, int64_t S, const grl_ragged* batch, int64_t H, int64_t D, const void* x,
+                         const void* w_qkv, const float* b_qkv, const float* mask, void* qkv, void* out, float rope_base, float rope_scaling);
 /* grl_gemm_nt_resln (C = A.W^T + bias + LayerNorm(R), d columns), then grl_ln_glu_nt_stats on its rows (d_ff outputs): the block in front
  * of a gated MLP, utils/vulkan_sentence_transformer.py:893-927, in two launches.  stats: (M, 2) floats of scratch, 16-byte aligned;
  * workspace: grl_gemm_nt_resln_workspace(M, d) bytes. */

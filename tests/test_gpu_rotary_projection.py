@@ -1,0 +1,49 @@
+"""GPU parity of grl_rotary_attention: the projection whose epilogue rotates queries and keys (128 x 128 tiles on four and eight waves,
+256 x 256 tiles, ragged last tiles) and the products that leave the rotation to attention, on rectangular and ragged batches, against the
+float64 oracle of projection, rotation and attention on whole sequences.  Tolerances: max|y-ref|/max|ref| <= 1e-4 (fp32), 2e-2 (bf16)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import TOL_F32, TOL_BF16
+from oracle import oracle_np as O
+from grilly_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+# rows 12*S*... : 1500 -> kernel 6, 3000 -> kernel 4, 5390 -> kernel 3 at 768 columns; few rows and other head dims rotate in attention
+@pytest.mark.parametrize("dtype,B,S,H,D", [("bf16", 2, 50, 12, 64), ("bf16", 15, 100, 12, 64), ("bf16", 30, 100, 12, 64), ("bf16", 55, 98, 12, 64),
+                                           ("bf16", 30, 100, 6, 128), ("bf16", 30, 100, 12, 32), ("bf16", 3, 700, 10, 64), ("fp32", 30, 100, 6, 64)])
+@pytest.mark.parametrize("ragged", [False, True])
+def test_rotary_attention(backend, dtype, B, S, H, D, ragged):
+    c, code, d = backend.core, (L.GRL_BF16 if dtype == "bf16" else L.GRL_F32), H * D
+    rng = np.random.default_rng(B + S + D)
+    q = (lambda a: O.bf16_round(a)) if dtype == "bf16" else (lambda a: a)
+    n = rng.integers(1, S + 1, B) if ragged else np.full(B, S)
+    n[0] = S
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    M = int(off[-1])
+    x = q(rng.standard_normal((M, d), dtype=np.float32))
+    w = q((rng.standard_normal((3 * d, d)) / np.sqrt(d)).astype(np.float32))
+    b = rng.standard_normal(3 * d).astype(np.float32)
+    dx, dw, db = c.upload(x, code), c.upload(w, code), c.upload(b)
+    do, dp = c.upload_raw(off), c.upload_raw(np.concatenate([np.arange(k) for k in n]).astype(np.int32))
+    guard = np.full(M * d + 64, 7.0, np.float32)
+    qkv, out = c.alloc(M * 3 * d * 4), c.upload(guard, code)
+    try:
+        rg = L.Ragged(do.ptr, dp.ptr, B, M, S)
+        L.check(c.lib.grl_rotary_attention(c.ctx, code, B, S, ctypes.byref(rg) if ragged else None, H, D, dx.ptr, dw.ptr, db.ptr, None, qkv.ptr, out.ptr,
+                                           10000.0, 1.0), "rotary_attention")
+        got = c.download(out, (M * d + 64,), code)
+        assert (got[M * d:] == 7.0).all() and np.isfinite(got).all()
+        got = got[:M * d].reshape(M, H, D)
+        for s in sorted({0, 1, B // 2, B - 1}):
+            rows = slice(off[s], off[s + 1])
+            parts = O.truth_linear(x[rows], w, b).reshape(n[s], 3, H, D)
+            ref = O.truth_attention(parts[None, :, 0], parts[None, :, 1], parts[None, :, 2], rope="half")
+            assert O.max_rel(got[None, rows], ref) < (TOL_F32 if dtype == "fp32" else TOL_BF16), (s, n[s])
+    finally:
+        for t in (dx, dw, db, do, dp, qkv, out):
+            t.free()
