@@ -290,15 +290,16 @@ int grl_gemm_nt_resln_parts(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t
     return resln(c, dtype, M, N, K, A, W, bias, R, r_stats, r_gamma, r_beta, C, eps, stats_out, workspace, out);
 }
 
-// ---- C = A.W^T + bias, then columns 0 .. rotated as heads of 64 rotated by each row's position (bf16) ---------------
+// ---- C = A.W^T + bias, then columns 0 .. rotated as heads of 64 rotated by each row's position ----------------------
+extern template int launch_gemm_rope<float>(grl_ctx*, GemmArgs&, bool*);
 extern template int launch_gemm_rope<uint16_t>(grl_ctx*, GemmArgs&, bool*);
-int grl_gemm_nt_rope_bf16(grl_ctx* c, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, void* C, int64_t rotated,
-                          const float* table, const int32_t* positions, int64_t S, bool* taken) {
+int grl_gemm_nt_rope(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, void* C, int64_t rotated,
+                     const float* table, const int32_t* positions, int64_t S, bool* taken) {
     GemmArgs a{};
     a.A = A; a.W = W; a.bias = bias; a.C = C;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
     a.rope = (const float2*)table; a.rope_pos = positions; a.rope_S = (int)S; a.rope_cols = (int)rotated;
-    return launch_gemm_rope<uint16_t>(c, a, taken);
+    return dtype == GRL_F32 ? launch_gemm_rope<float>(c, a, taken) : launch_gemm_rope<uint16_t>(c, a, taken);
 }
 
 // ---- products of few rows that take the row statistics of a folded LayerNorm themselves ---------------------------
