@@ -170,9 +170,9 @@ class BertEncoder:
     FUSED_MIN_VALUES = {L.GRL_BF16: 2 << 20, L.GRL_F32: 3 << 20}      # rows x d_model
     # bf16: up to this many values of a layer's widest activation (rows x d_ff) a layer runs as five launches without a LayerNorm
     # pass (grl_bert_layer_fwd_rows).  us per forward, seven launches -> five: d_ff 3072 / 768 wide / 12 layers: 128 rows 517 -> 399,
-    # 320 rows 536 -> 455, 512 rows 642 -> 600, 768 rows 730 -> 726; 1536 / 384 / 6 layers: 256 rows 227 -> 196, 768 rows 267 -> 258,
-    # 1024 rows level, 1280 rows 291 -> 301.  In fp32 the two forms are within 4 % of each other from 128 rows on and the seven launches ahead below.
-    ROWS_MAX_OUTPUTS = 3 << 19
+    # 320 rows 536 -> 449, 512 rows 642 -> 560, 640 rows 667 -> 584, 768 rows 732 -> 692; 1536 / 384 / 6 layers: 256 rows 227 -> 196,
+    # 768 rows 267 -> 250, 1280 rows 294 -> 271, 1536 rows 331 -> 324.  In fp32 the two forms are within 4 % of each other from 128 rows on and the seven launches ahead below.
+    ROWS_MAX_OUTPUTS = 9 << 18
 
     def __init__(self, core, cfg, weights, dtype="fp32", fused=None):
         self.core = core.core if hasattr(core, "core") else core
@@ -445,7 +445,7 @@ class PreNormEncoder:
             raise TypeError("PreNormEncoder needs a Compute() backend or its HipCore")
         self._stats_from_gemm = stats_from_gemm        # None: wherever the kernel takes the width
         # Few rows (rows x d_ff up to this): the gated GEMM takes the statistics of its rows itself.  us per forward of 22 layers,
-        # 768 wide, d_ff 1152: bf16 128 rows 796 -> 637, 640 rows 1117 -> 1008, 896 rows 1164 -> 1077, 1024 rows 1214 -> 1202; fp32 20 rows 1630 -> 1084,
+        # 768 wide, d_ff 1152: bf16 128 rows 796 -> 637, 640 rows 1117 -> 896, 896 rows 1164 -> 972; fp32 20 rows 1630 -> 1084,
         # 896 rows 3327 -> 2829, 1280 rows 3915 -> 3744, 2048 rows 5629 -> 5651
         half = dtype_code(dtype) == L.GRL_BF16
         takes = cfg.d_model % (64 if half else 32) == 0 and cfg.d_ff % 4 == 0
