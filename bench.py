@@ -93,7 +93,7 @@ def median(v):
 def forward_kernel_times(backend, enc, cfg, forwards=8):
     """Durations of the layer's launches INSIDE whole forwards: the layer entry points record a lap event at entry and after
     each of their kernels (grl_timer_lap_trace), `forwards` forwards run back to back behind two untimed ones, and every
-    interval is attributed to the launch it follows (a residual-type GEMM's interval includes its 3-5 us moment merge).
+    interval is attributed to the launch it follows.
     Returns {launch name: {ms (mean), median_ms, n}} and "layer_ms": what the kernels do under the forward's sustained
     load, next to the back-to-back table of kernel_table()."""
     from grilly_amd import _lib as L
@@ -780,7 +780,7 @@ def main():
                                          "power limit the launches run at shader_clock_ghz (probe kernel beside the forward, or beside the "
                                          "back-to-back launches), and frac_at_measured_clock is the same achieved rate against the peak at that clock",
                            "note": "achieved / frac / avg_launch_ms: the kernel's launches inside whole forwards (lap events between the "
-                                   "layer's launches; a launch's interval includes its 3-5 us moment-merge kernel), i.e. under the sustained "
+                                   "layer's launches), i.e. under the sustained "
                                    "load of the timed region; back_to_back: the same launches in a table of their own (`kernels`), where "
                                    "the board often holds a higher clock because the load comes in bursts of a few milliseconds between "
                                    "host-side checks.  Both move with the box (up to 20 % between boxes)."}
