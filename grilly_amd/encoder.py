@@ -155,19 +155,21 @@ class BertEncoder:
 
     fused=None (default): both LayerNorms of every layer are folded into the GEMMs around them whenever the
     direct-to-LDS GEMM kernels take the layer's shapes (d_model and d_ff multiples of 64 in bf16, 32 in fp32) and the
-    hidden states hold at least FUSED_MIN_VALUES values, or in bf16 few enough for the form without statistics passes: the residual stream
-    then travels as raw rows plus row statistics and no LayerNorm pass runs over HBM between the embedding and the final LayerNorm
+    batch has at least FUSED_MIN_ROWS token rows (fp32: or FUSED_MIN_VALUES_F32 hidden values), or in bf16 few enough for the form without
+    statistics passes: the residual stream then travels as raw rows plus row statistics and no LayerNorm pass runs over HBM between the embedding and the final LayerNorm
     (grl_bert_layers_fwd_fused).  Other batches run the seven-launch layer with its two LayerNorm passes (grl_bert_layer_fwd): a
     handful of token rows make a handful of tiles, the plain GEMMs then take tiles down to 32 x 32 while the fused layer's residual
     GEMM has none below 64 x 128, and the LayerNorm passes it saves cost next to nothing there.  Both weight
     sets stay resident.  fused=False always takes the seven-launch layer;
     fused=True always the fused one, and raises for shapes it does not take."""
-    # us per forward, seven launches a layer -> fused: bf16 768 wide, 12 layers: 1024 rows 761 -> 839, 1536 rows 919 -> 884, 4096 rows
-    # 1473 -> 1403; 384 wide, 6 layers: 2048 rows 338 -> 352, 3072 rows 380 -> 364, 6400 rows 502 -> 466.  fp32 768 wide: 2048 rows
-    # 2856 -> 3048, 4096 rows level, 6400 rows 7153 -> 6911; 384 wide: 4096 rows 942 -> 951, 6400 rows level.  The bf16 line stands above the
-    # crossover: pooled embeddings and the mean of the hidden states agree to the last bits where a batch and the same batch without its
-    # padding run one form, and so the small ones do.
-    FUSED_MIN_VALUES = {L.GRL_BF16: 2 << 20, L.GRL_F32: 3 << 20}      # rows x d_model
+    # us per forward, seven launches a layer -> fused: fp32 768 wide, 12 layers: 2048 rows 2856 -> 3048, 4096 rows level, 6400 rows
+    # 7153 -> 6911; 384 wide, 6 layers: 4096 rows 942 -> 951, 6400 rows level; 128 wide, 4 layers, 20000 rows 453 -> 432.  In fp32 hidden
+    # states are nearer to float64 with it (768 wide, 4400 rows: 7.35e-7 against 7.50e-7).  In bf16 they are not: the residual product's sum
+    # is rounded before the residual is added, and the raw row once more in front of the last LayerNorm (twelve seeds each: 768 wide,
+    # 2880 rows 8.86e-3 against 8.81e-3, 384 wide, 6400 rows 6.335e-3 against 6.327e-3).  So the bf16 line stands where the time saved is
+    # more than a few per cent, not at the crossover (768 wide: 1536 rows 919 -> 884 us, 4096 rows 1473 -> 1403).
+    FUSED_MIN_ROWS = 8192
+    FUSED_MIN_VALUES_F32 = 3 << 20          # or, in fp32, so many values of the hidden states (rows x d_model)
     # bf16: up to this many values of a layer's widest activation (rows x d_ff) a layer runs as five launches without a LayerNorm
     # pass (grl_bert_layer_fwd_rows).  us per forward, seven launches -> five: d_ff 3072 / 768 wide / 12 layers: 128 rows 517 -> 399,
     # 320 rows 536 -> 449, 512 rows 642 -> 560, 640 rows 667 -> 584, 768 rows 732 -> 692; 1536 / 384 / 6 layers: 256 rows 227 -> 196,
@@ -199,7 +201,7 @@ class BertEncoder:
         if fused and not eligible:
             raise ValueError(f"the fused layer needs d_model and d_ff to be multiples of {slab} in {dtype}")
         self.fused = eligible if fused is None else bool(fused)
-        self._fused_min_rows = -(-self.FUSED_MIN_VALUES[self.code] // cfg.d_model) if fused is None else 0
+        self._fused_min_rows = self.fused_min_rows(cfg.d_model, self.code) if fused is None else 0
         few = fused is None and self.fused and self.code == L.GRL_BF16
         self._rows_max = self.ROWS_MAX_OUTPUTS // cfg.d_ff if few else 0
         self.fused_structs = []
@@ -227,6 +229,11 @@ class BertEncoder:
                 in_g, in_b = s.ln2_g, s.ln2_b
             self._fused_array = (L.BertLayerFused * len(self.fused_structs))(*self.fused_structs)
         self._shape = None
+
+    @classmethod
+    def fused_min_rows(cls, d_model, code):
+        """token rows from which a batch runs the fused layers by default"""
+        return cls.FUSED_MIN_ROWS if code == L.GRL_BF16 else min(cls.FUSED_MIN_ROWS, -(-cls.FUSED_MIN_VALUES_F32 // d_model))
 
     def _own(self, buf):
         self._keep.append(buf)
