@@ -170,11 +170,13 @@ class BertEncoder:
     # more than a few per cent, not at the crossover (768 wide: 1536 rows 919 -> 884 us, 4096 rows 1473 -> 1403).
     FUSED_MIN_ROWS = 8192
     FUSED_MIN_VALUES_F32 = 3 << 20          # or, in fp32, so many values of the hidden states (rows x d_model)
-    # bf16: up to this many values of a layer's widest activation (rows x d_ff) a layer runs as five launches without a LayerNorm
-    # pass (grl_bert_layer_fwd_rows).  us per forward, seven launches -> five: d_ff 3072 / 768 wide / 12 layers: 128 rows 517 -> 399,
-    # 320 rows 536 -> 449, 512 rows 642 -> 560, 640 rows 667 -> 584, 768 rows 732 -> 692; 1536 / 384 / 6 layers: 256 rows 227 -> 196,
-    # 768 rows 267 -> 250, 1280 rows 294 -> 271, 1536 rows 331 -> 324.  In fp32 the two forms are within 4 % of each other from 128 rows on and the seven launches ahead below.
-    ROWS_MAX_OUTPUTS = 9 << 18
+    # bf16: up to so many values a layer runs as five launches without a LayerNorm pass (grl_bert_layer_fwd_rows): rows x the widest
+    # activation (3 d_model or d_ff) up to the first, or rows x d_ff up to the second.  us per forward, seven launches -> five: d_ff 3072 /
+    # 768 wide / 12 layers: 128 rows 517 -> 399, 320 rows 536 -> 449, 512 rows 642 -> 560, 640 rows 667 -> 584, 768 rows 732 -> 692;
+    # 1536 / 384 / 6 layers: 256 rows 227 -> 196, 768 rows 267 -> 250, 1280 rows 294 -> 271, 1536 rows 331 -> 324.  Where d_ff is narrow the
+    # QKV product is on far more 32 x 32 tiles than there are CUs (4 layers: 768 / 768 wide, 2560 rows 298 -> 336; 1536 / 768, 1500 rows
+    # 293 -> 311; 256 / 256, 6000 rows 218 -> 253).  In fp32 the two forms are within 4 % of each other from 128 rows on and the seven launches ahead below.
+    ROWS_MAX_OUTPUTS, ROWS_MAX_FF = 9 << 18, 5 << 18
 
     def __init__(self, core, cfg, weights, dtype="fp32", fused=None):
         self.core = core.core if hasattr(core, "core") else core
@@ -203,7 +205,7 @@ class BertEncoder:
         self.fused = eligible if fused is None else bool(fused)
         self._fused_min_rows = self.fused_min_rows(cfg.d_model, self.code) if fused is None else 0
         few = fused is None and self.fused and self.code == L.GRL_BF16
-        self._rows_max = self.ROWS_MAX_OUTPUTS // cfg.d_ff if few else 0
+        self._rows_max = self.rows_max(cfg.d_model, cfg.d_ff) if few else 0
         self.fused_structs = []
         if self.fused:
             # every GEMM that reads a LayerNorm's output gets that norm folded into its weight (once, here):
@@ -234,6 +236,11 @@ class BertEncoder:
     def fused_min_rows(cls, d_model, code):
         """token rows from which a batch runs the fused layers by default"""
         return cls.FUSED_MIN_ROWS if code == L.GRL_BF16 else min(cls.FUSED_MIN_ROWS, -(-cls.FUSED_MIN_VALUES_F32 // d_model))
+
+    @classmethod
+    def rows_max(cls, d_model, d_ff):
+        """token rows up to which a bf16 batch runs the five-launch layers by default"""
+        return max(cls.ROWS_MAX_OUTPUTS // max(3 * d_model, d_ff), cls.ROWS_MAX_FF // d_ff)
 
     def _own(self, buf):
         self._keep.append(buf)

@@ -14,6 +14,12 @@ def test_fused_lines():
         assert rows <= 8192 and (rows == 8192 or (rows - 1) * d < 3 << 20 <= rows * d)
 
 
+def test_five_launch_line_looks_at_the_widest_product():
+    for d, ff, rows in ((768, 3072, 768), (384, 1536, 1536), (768, 768, 1706), (256, 256, 5120), (768, 1536, 1024), (1024, 1024, 1280)):
+        assert BertEncoder.rows_max(d, ff) == rows
+        assert rows * max(3 * d, ff) <= 9 << 18 or rows * ff <= 5 << 18
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,B,S,heads", [("bf16", 30, 100, 12), ("bf16", 63, 130, 6), ("fp32", 30, 100, 12), ("fp32", 64, 127, 2)])
 def test_batches_below_the_fused_line(backend, dtype, B, S, heads):
