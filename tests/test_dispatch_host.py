@@ -1,0 +1,36 @@
+"""The launchers' host rules, compiled from the kernels' headers by the host pass alone (no GPU, no device code)."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "grilly_amd", "csrc")
+SOURCE = r"""
+#include "gemm_kernels.hpp"
+extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
+extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    at = tmp_path_factory.mktemp("rules")
+    (at / "rules.hip").write_text(SOURCE)
+    subprocess.run(["hipcc", "-std=c++17", "-O0", "--offload-host-only", "-shared", "-fPIC", "-Wno-unused-result", "-I", CSRC,
+                    "-o", str(at / "rules.so"), str(at / "rules.hip")], check=True, timeout=100)
+    return ctypes.CDLL(str(at / "rules.so"))
+
+
+@pytest.mark.parametrize("elem_size", [2, 4])
+@pytest.mark.parametrize("dual", [0, 1])
+def test_partials_go_to_kernels_that_merge_them(rules, elem_size, dual):
+    """The shared-K kernels (9, 10) and the register-staged ones (1, 2, 5) read merged statistics from memory: no number may end in one of
+    them and count as a kernel that takes partials."""
+    has = {1, 2, 3, 4, 5, 9} | ({6, 7, 8} if elem_size == 2 and not dual else {6, 7} if elem_size == 4 else set())
+    has |= {10} if elem_size == 2 else {11}
+    has |= {8} if elem_size == 4 and not dual else set()
+    for variant in range(1, 12):
+        kernel = rules.kernel_run(variant, elem_size, dual)
+        assert kernel in has and (variant not in has or kernel == variant)
+        assert rules.takes_partials(kernel) == (kernel in (3, 4, 6, 7, 8))

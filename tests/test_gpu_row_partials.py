@@ -5,10 +5,14 @@ four and eight waves, 256 x 256, and the small ones that take none) with ragged 
 The sums are the same in the same order, so what differs is at most the rounding of a quotient: 2^-23 of a statistic, which can move a
 stored value by one unit of its type (bf16 2^-8, fp32 2^-23) and that unit through the rest: 2-norms agree to 4e-3 and 4e-6."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
+from conftest import ROOT
 from grilly_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +76,23 @@ def test_gated_block(backend, dtype, M, d, ff):
     near(c.download(o1, (M, ff), code), c.download(o2, (M, ff), code), dtype)
     for t in (A, W, R, Wg, Wu, b, g, bt, cg, cu, bg, bu, st, C1, C2, o1, o2, stats, ws):
         t.free()
+
+
+FORCED = """
+import sys
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+import grilly_amd, test_gpu_row_partials as t
+backend = grilly_amd.Compute()
+for dtype in ("fp32", "bf16"):
+    for shape in ((130, 384, 96), (1401, 768, 200)):
+        print(dtype, shape, flush=True)
+        t.test_gated_block(backend, dtype, *shape)
+print("passed")
+"""
+
+
+@pytest.mark.parametrize("variant", [6, 7, 8])
+def test_gated_block_with_a_forced_kernel(variant):
+    """GRL_GEMM_VARIANT may name a kernel that a two-weight product does not have: the one that runs in its place takes no partials."""
+    child = subprocess.run([sys.executable, "-c", FORCED, ROOT], capture_output=True, text=True, timeout=100, env=dict(os.environ, GRL_GEMM_VARIANT=str(variant)))
+    assert child.returncode == 0 and "passed" in child.stdout, child.stdout + child.stderr
