@@ -147,12 +147,9 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int li = lane & 31, lg = lane >> 5;
     const int nqb = (p.S + QB - 1) / QB, nbh = p.B * p.H;
-    const int nwg = (int)gridDim.x, per = nwg >> 3, rem = nwg & 7, xcd = (int)blockIdx.x & 7, loc = (int)blockIdx.x >> 3;
-    int lin = (p.order & 1) ? xcd * per + (xcd < rem ? xcd : rem) + loc : (int)blockIdx.x;
-    // Heads dealt out in turn, as far as they make whole turns of eight; the rest keep their ids.  Not compiled in where nothing asks
-    // for it: causal rotary attention of 4 x 8192 x 32 x 128 was 0.5 to 0.8 % slower with these lines in its kernel.
-    if constexpr (ROPE_Q == 0 && !HAS_MASK)
-        if ((p.order & 4) && (int)blockIdx.x < (nbh & ~7) * nqb) lin = (loc / nqb * 8 + xcd) * nqb + loc % nqb;
+    // Dealt-out heads are not compiled in where nothing asks for them: causal rotary attention of 4 x 8192 x 32 x 128 was 0.5 to 0.8 %
+    // slower with those lines in its kernel.
+    const int lin = fa_place<ROPE_Q == 0 && !HAS_MASK>(p.order, (int)blockIdx.x, (int)gridDim.x, nqb, nbh);
     int qb, bh;
     if (p.order & 2) { qb = nqb - 1 - lin / nbh; bh = lin % nbh; }
     else if (p.causal) { bh = lin / nqb; qb = nqb - 1 - lin % nqb; }
@@ -718,7 +715,7 @@ static int launch_fa16(grl_ctx* c, const FaArgs& a, int rope_q) {
     // up to 384 long, 12 heads: 30.9 -> 28.5 us; 32 up to 300: 20.0 -> 19.7).  A rectangular batch with a mask is level to 5 %
     // slower (32 x 200), and with few heads a turn is too coarse.  Only where the kernel does not rotate: see there.
     const bool deal = a.offsets && !a.mask && rope_q == 0 && (int64_t)a.B * a.H >= 64 && a.S <= 1024;
-    f.order = order_env >= 0 ? order_env : deal ? 4 : ((a.causal || a.S <= 1024) ? 1 : 0);
+    f.order = order_env >= 0 ? fa_order_checked(order_env) : deal ? 4 : ((a.causal || a.S <= 1024) ? 1 : 0);
     f.q_stride = a.q_stride; f.k_stride = a.k_stride; f.v_stride = a.v_stride; f.o_stride = a.o_stride;
     // GRL_FA_CFG forces a configuration, for tuning runs:
     //   1: 8 waves, 64-key tiles, deep ring   2: 8 waves, 128-key tiles   3: 4 waves, 64-key tiles, 4 stages (head dims up to 64)

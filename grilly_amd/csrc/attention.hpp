@@ -16,6 +16,19 @@ struct FaArgs {
     int64_t q_stride, k_stride, v_stride, o_stride;   // elements between consecutive positions
 };
 
+// Workgroup numbering of the bf16 kernel, bits: 1 XCD-contiguous runs of ids, 2 the heaviest query blocks of all heads first, 4 heads dealt out to
+// the XCDs in turn (in place of 1: mixed, some heads would be computed twice and others never).
+static inline int fa_order_checked(int order) { return order & 4 ? order & 6 : order & 3; }
+// Where workgroup `id` of nwg = nqb * nbh stands in the walk.  DEAL: the heads that make whole turns of eight are dealt out, the query blocks
+// of one head next to each other on one XCD; the rest keep their ids.
+template <bool DEAL> __host__ __device__ __forceinline__ int fa_place(int order, int id, int nwg, int nqb, int nbh) {
+    const int per = nwg >> 3, rem = nwg & 7, xcd = id & 7, loc = id >> 3;
+    int lin = (order & 1) ? xcd * per + (xcd < rem ? xcd : rem) + loc : id;
+    if constexpr (DEAL)
+        if ((order & 4) && id < (nbh & ~7) * nqb) lin = (loc / nqb * 8 + xcd) * nqb + loc % nqb;
+    return lin;
+}
+
 // Sequence b of the batch: its first row and its length.  In a ragged batch the sequences stand back to back and every one
 // has its own length (queries and keys alike); the grid is laid out for the longest, and a workgroup whose queries lie past
 // the end of its sequence has nothing to do.

@@ -8,8 +8,13 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "grilly_amd", "csrc")
 SOURCE = r"""
 #include "gemm_kernels.hpp"
+#include "attention.hpp"
 extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
+extern "C" int order_checked(int order) { return fa_order_checked(order); }
+extern "C" int place(int deal, int order, int id, int nwg, int nqb, int nbh) {
+    return deal ? fa_place<true>(order, id, nwg, nqb, nbh) : fa_place<false>(order, id, nwg, nqb, nbh);
+}
 """
 
 
@@ -34,3 +39,14 @@ def test_partials_go_to_kernels_that_merge_them(rules, elem_size, dual):
         kernel = rules.kernel_run(variant, elem_size, dual)
         assert kernel in has and (variant not in has or kernel == variant)
         assert rules.takes_partials(kernel) == (kernel in (3, 4, 6, 7, 8))
+
+
+@pytest.mark.parametrize("order", range(8))
+def test_every_attention_block_is_computed_once(rules, order):
+    """whatever GRL_FA_ORDER says, in the kernels with and without the dealt-out map"""
+    order = rules.order_checked(order)
+    for deal in (0, 1):
+        for nbh in (1, 7, 8, 9, 24, 70):
+            for nqb in (1, 2, 3, 8):
+                n = nbh * nqb
+                assert sorted(rules.place(deal, order, i, n, nqb, nbh) for i in range(n)) == list(range(n))
