@@ -708,14 +708,7 @@ static int launch_fa16(grl_ctx* c, const FaArgs& a, int rope_q) {
     f.mask = a.mask; f.O = (uint16_t*)a.O; f.rope = a.rope; f.offsets = a.offsets;
     f.B = a.B; f.S = a.S; f.H = a.H; f.scale = a.scale; f.causal = a.causal;
     static const int order_env = [] { const char* e = getenv("GRL_FA_ORDER"); return e ? atoi(e) : -1; }();
-    // measured: causal and short sequences do best head by head on XCD-contiguous runs; long dense sequences with
-    // the plain id order (32 CUs of an XCD streaming the same K/V tiles in lockstep miss L2 together)
-    // Ragged batches: heads dealt out to the XCDs in turn, the query blocks of one head still next to each other on one XCD.  A
-    // contiguous run per XCD gives an XCD six sequences of a batch of 48, and the launch lasts as long as the longest six (48 sequences
-    // up to 384 long, 12 heads: 30.9 -> 28.5 us; 32 up to 300: 20.0 -> 19.7).  A rectangular batch with a mask is level to 5 %
-    // slower (32 x 200), and with few heads a turn is too coarse.  Only where the kernel does not rotate: see there.
-    const bool deal = a.offsets && !a.mask && rope_q == 0 && (int64_t)a.B * a.H >= 64 && a.S <= 1024;
-    f.order = order_env >= 0 ? fa_order_checked(order_env) : deal ? 4 : ((a.causal || a.S <= 1024) ? 1 : 0);
+    f.order = order_env >= 0 ? fa_order_checked(order_env) : fa_order(a.causal, a.S, a.offsets && !a.mask && rope_q == 0, (int64_t)a.B * a.H, D);
     f.q_stride = a.q_stride; f.k_stride = a.k_stride; f.v_stride = a.v_stride; f.o_stride = a.o_stride;
     // GRL_FA_CFG forces a configuration, for tuning runs:
     //   1: 8 waves, 64-key tiles, deep ring   2: 8 waves, 128-key tiles   3: 4 waves, 64-key tiles, 4 stages (head dims up to 64)

@@ -19,6 +19,17 @@ struct FaArgs {
 // Workgroup numbering of the bf16 kernel, bits: 1 XCD-contiguous runs of ids, 2 the heaviest query blocks of all heads first, 4 heads dealt out to
 // the XCDs in turn (in place of 1: mixed, some heads would be computed twice and others never).
 static inline int fa_order_checked(int order) { return order & 4 ? order & 6 : order & 3; }
+// Measured: causal and short sequences do best head by head on XCD-contiguous runs; long dense sequences with the plain id order (32 CUs of
+// an XCD streaming the same K/V tiles in lockstep miss L2 together).
+// Ragged batches (without mask and rotation: see the kernel): heads dealt out.  A contiguous run per XCD gives an XCD six sequences of a
+// batch of 48, and the launch lasts as long as the longest six (48 sequences up to 384 long, 12 heads: 30.9 -> 28.5 us; 32 up to 300:
+// 20.0 -> 19.7; 16 to 128 sequences of 16 to 900 tokens, 4 to 16 heads: 4 % on the mean at head dim 64, 3 % at 128).  Not at head dim 32: two heads
+// share every 128-byte line of K and V, which then goes to two XCDs (64 sequences 2 % slower on the mean, 128 sequences 8 %, of equal
+// length up to 46 %).  A rectangular batch with a mask is level to 5 % slower (32 x 200), and with few heads a turn is too coarse.
+static inline int fa_order(bool causal, int64_t S, bool ragged, int64_t heads, int D) {
+    if (ragged && D >= 64 && heads >= 64 && S <= 1024) return 4;
+    return causal || S <= 1024 ? 1 : 0;
+}
 // Where workgroup `id` of nwg = nqb * nbh stands in the walk.  DEAL: the heads that make whole turns of eight are dealt out, the query blocks
 // of one head next to each other on one XCD; the rest keep their ids.
 template <bool DEAL> __host__ __device__ __forceinline__ int fa_place(int order, int id, int nwg, int nqb, int nbh) {

@@ -12,6 +12,7 @@ SOURCE = r"""
 extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
 extern "C" int order_checked(int order) { return fa_order_checked(order); }
+extern "C" int order(int causal, int S, int ragged, int heads, int D) { return fa_order(causal, S, ragged, heads, D); }
 extern "C" int place(int deal, int order, int id, int nwg, int nqb, int nbh) {
     return deal ? fa_place<true>(order, id, nwg, nqb, nbh) : fa_place<false>(order, id, nwg, nqb, nbh);
 }
@@ -50,3 +51,9 @@ def test_every_attention_block_is_computed_once(rules, order):
             for nqb in (1, 2, 3, 8):
                 n = nbh * nqb
                 assert sorted(rules.place(deal, order, i, n, nqb, nbh) for i in range(n)) == list(range(n))
+
+
+def test_heads_that_share_lines_are_not_dealt_out(rules):
+    """head dim 32: two heads in every 128-byte line, which dealing out would send to two XCDs"""
+    assert [rules.order(0, 256, 1, 1536, D) for D in (32, 64, 128)] == [1, 4, 4]
+    assert rules.order(0, 1025, 1, 1536, 64) == 0 and rules.order(1, 4096, 0, 64, 128) == 1
