@@ -10,6 +10,7 @@ SOURCE = r"""
 #include "gemm_kernels.hpp"
 #include "attention.hpp"
 extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
+extern "C" int kernel(long long M, long long N, long long K, int elem_size, int dual) { return gemm_kernel(M, N, K, elem_size, dual, 256); }
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
 extern "C" int order_checked(int order) { return fa_order_checked(order); }
 extern "C" int order(int causal, int S, int ragged, int heads, int D) { return fa_order(causal, S, ragged, heads, D); }
@@ -25,7 +26,9 @@ def rules(tmp_path_factory):
     (at / "rules.hip").write_text(SOURCE)
     subprocess.run(["hipcc", "-std=c++17", "-O0", "--offload-host-only", "-shared", "-fPIC", "-Wno-unused-result", "-I", CSRC,
                     "-o", str(at / "rules.so"), str(at / "rules.hip")], check=True, timeout=100)
-    return ctypes.CDLL(str(at / "rules.so"))
+    lib = ctypes.CDLL(str(at / "rules.so"))
+    lib.kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
+    return lib
 
 
 @pytest.mark.parametrize("elem_size", [2, 4])
@@ -57,3 +60,10 @@ def test_heads_that_share_lines_are_not_dealt_out(rules):
     """head dim 32: two heads in every 128-byte line, which dealing out would send to two XCDs"""
     assert [rules.order(0, 256, 1, 1536, D) for D in (32, 64, 128)] == [1, 4, 4]
     assert rules.order(0, 1025, 1, 1536, 64) == 0 and rules.order(1, 4096, 0, 64, 128) == 1
+
+
+def test_two_shared_tiles_per_unit_need_a_long_sum(rules):
+    """bf16: between 257 and 512 tiles of 64 x 64 the shared-K kernel is ahead everywhere from 96 slabs on only"""
+    for M, N in ((2100, 512), (2600, 512), (1088, 1152), (2000, 768), (512, 4096)):
+        assert [rules.kernel(M, N, K, 2, 0) for K in (3072, 5120, 6080, 6144, 11008)] == [8, 8, 8, 10, 10]
+    assert rules.kernel(800, 768, 768, 2, 0) == 10

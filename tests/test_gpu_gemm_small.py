@@ -19,7 +19,7 @@ CODE = {"fp32": L.GRL_F32, "bf16": L.GRL_BF16}
 
 # (M, slabs of 128 bytes, N)
 PLAIN = [(1, 1, 4), (33, 5, 36), (128, 12, 2304), (250, 48, 768), (30, 70, 100),          # 32 x 32 tiles (the last: split K in fp32)
-         (800, 12, 768), (777, 13, 780),                                                  # bf16: 64 x 64 shared K
+         (800, 12, 768), (777, 13, 780), (1990, 97, 764),                                 # bf16: 64 x 64 shared K, one and two per compute unit
          (450, 1, 3072), (449, 2, 3004), (449, 3, 3072), (450, 13, 3072),                 # 64 x 64 ring around its four stages
          (1500, 1, 2304), (1499, 2, 2300), (1500, 3, 2304), (1500, 4, 2304), (1500, 5, 2304),   # bf16: 128 x 128 ring
          (3000, 1, 1152), (2999, 2, 1148), (3000, 3, 1152), (3000, 12, 1152)]             # fp32: 64 x 128 ring
