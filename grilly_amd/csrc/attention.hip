@@ -17,9 +17,9 @@
 #include <cstdlib>
 
 int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                         void* y, const float* table, const int32_t* positions);
+                         void* y, const float* table, const int32_t* positions, int table_S);
 int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                              void* y, const float* table, const int32_t* positions);
+                              void* y, const float* table, const int32_t* positions, int table_S);
 int grl_rope_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
                      const int32_t* position_ids, void* y, int style, float rope_base, float rope_scaling);
 
@@ -915,12 +915,13 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
         // bf16: the kernel rotates the query rows as it loads them (both halves of a pair are chunks of the same
         // lane); every K row is rotated exactly once here, from the table kept on the context
         const float* tab = nullptr;
-        rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, GRL_ROPE_HALF, &tab);
+        int tab_S = 0;
+        rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, GRL_ROPE_HALF, &tab, &tab_S);
         if (rc) return rc;
         a.rope = (const float2*)tab;
         own2 = grl_malloc(c, (size_t)nrows * H * D * 2);
         if (!own2) return GRL_ERR_OOM;
-        rc = grl_rope_half_apply_table(c, dtype, rB, rS, H, D, K, k_stride, own2, tab, a.positions);
+        rc = grl_rope_half_apply_table(c, dtype, rB, rS, H, D, K, k_stride, own2, tab, a.positions, tab_S);
         a.K = own2; a.k_stride = hd;
         rope_q = 2;
     } else if (rope == GRL_ROPE_HALF) {
@@ -935,14 +936,15 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
     } else if (rope == GRL_ROPE_INTERLEAVED) {
         // the (S, D/2) cos/sin table lives on the context and is built once per (D, base, scaling)
         const float* tab = nullptr;
-        rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, GRL_ROPE_INTERLEAVED, &tab);
+        int tab_S = 0;
+        rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, GRL_ROPE_INTERLEAVED, &tab, &tab_S);
         if (rc) return rc;
         a.rope = (const float2*)tab;
         if (dtype == GRL_BF16) {
             // every K row is rotated exactly once here; the kernel rotates Q rows as it loads them
             own2 = grl_malloc(c, (size_t)nrows * H * D * 2);
             if (!own2) return GRL_ERR_OOM;
-            rc = grl_rope_apply_table(c, dtype, rB, rS, H, D, K, k_stride, own2, tab, a.positions);
+            rc = grl_rope_apply_table(c, dtype, rB, rS, H, D, K, k_stride, own2, tab, a.positions, tab_S);
             a.K = own2; a.k_stride = hd;
         }
     }

@@ -176,10 +176,9 @@ extern "C" int grl_rotary_attention(grl_ctx* c, int dtype, int64_t B, int64_t S,
     char* q = (char*)qkv;
     int rope = GRL_ROPE_HALF, rc;
     if (D == 64 && M < (1LL << 31) && 3 * d < (1LL << 31)) {
-        const float* table = nullptr;
-        if ((rc = grl_rope_table_get(c, (int)longest, (int)D, rope_base, rope_scaling, GRL_ROPE_HALF, &table))) return rc;
         bool taken = false;
-        if ((rc = grl_gemm_nt_rope(c, dtype, M, 3 * d, d, x, w_qkv, b_qkv, qkv, 2 * d, table, rg ? rg->positions : nullptr, S, &taken))) return rc;
+        if ((rc = grl_gemm_nt_rope(c, dtype, M, 3 * d, d, x, w_qkv, b_qkv, qkv, 2 * d, rg ? rg->positions : nullptr, longest, rope_base, rope_scaling, &taken)))
+            return rc;
         if (taken) rope = GRL_ROPE_NONE;
     }
     if (rope == GRL_ROPE_HALF && (rc = grl_gemm_nt(c, dtype, dtype, M, 3 * d, d, x, w_qkv, b_qkv, qkv, GRL_EPI_NONE))) return rc;

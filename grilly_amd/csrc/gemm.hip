@@ -291,15 +291,22 @@ int grl_gemm_nt_resln_parts(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t
 }
 
 // ---- C = A.W^T + bias, then columns 0 .. rotated as heads of 64 rotated by each row's position ----------------------
-extern template int launch_gemm_rope<float>(grl_ctx*, GemmArgs&, bool*);
-extern template int launch_gemm_rope<uint16_t>(grl_ctx*, GemmArgs&, bool*);
+extern template int launch_gemm_rope<float>(grl_ctx*, GemmArgs&, int);
+extern template int launch_gemm_rope<uint16_t>(grl_ctx*, GemmArgs&, int);
 int grl_gemm_nt_rope(grl_ctx* c, int dtype, int64_t M, int64_t N, int64_t K, const void* A, const void* W, const float* bias, void* C, int64_t rotated,
-                     const float* table, const int32_t* positions, int64_t S, bool* taken) {
+                     const int32_t* positions, int64_t S, float rope_base, float rope_scaling, bool* taken) {
+    const bool aligned = ((((uintptr_t)A) | ((uintptr_t)W) | ((uintptr_t)C) | ((uintptr_t)bias)) & 15u) == 0;
+    const int kernel = aligned ? gemm_rope_kernel(M, N, K, rotated, grl_dtype_size(dtype), c->prop.multiProcessorCount) : 0;
+    *taken = kernel != 0;
+    if (!kernel) return GRL_OK;
+    const float* table = nullptr;
+    int held = 0;
+    if (const int rc = grl_rope_table_get(c, (int)S, 64, rope_base, rope_scaling, GRL_ROPE_HALF, &table, &held)) return rc;
     GemmArgs a{};
     a.A = A; a.W = W; a.bias = bias; a.C = C;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
-    a.rope = (const float2*)table; a.rope_pos = positions; a.rope_S = (int)S; a.rope_cols = (int)rotated;
-    return dtype == GRL_F32 ? launch_gemm_rope<float>(c, a, taken) : launch_gemm_rope<uint16_t>(c, a, taken);
+    a.rope = (const float2*)table; a.rope_pos = positions; a.rope_S = positions ? held : (int)S; a.rope_cols = (int)rotated;
+    return dtype == GRL_F32 ? launch_gemm_rope<float>(c, a, kernel) : launch_gemm_rope<uint16_t>(c, a, kernel);
 }
 
 // ---- products of few rows that take the row statistics of a folded LayerNorm themselves ---------------------------

@@ -5,4 +5,4 @@ template int dispatch_epi<float, float>(grl_ctx*, GemmArgs&, int);
 template int dispatch_epi_ln<float, float>(grl_ctx*, GemmArgs&, int);
 template int launch_gemm_resln<float, float>(grl_ctx*, GemmArgs&, int*);
 template int launch_gemm_rows<float>(grl_ctx*, GemmArgs&, int);
-template int launch_gemm_rope<float>(grl_ctx*, GemmArgs&, bool*);
+template int launch_gemm_rope<float>(grl_ctx*, GemmArgs&, int);

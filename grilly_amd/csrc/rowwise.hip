@@ -631,9 +631,9 @@ int grl_rope_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int
                      const int32_t* position_ids, void* y, int style, float rope_base, float rope_scaling);
 int grl_build_rope_table_styled(grl_ctx* c, float* tab, int S, int D, float base, float scaling, int style);
 int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                         void* y, const float* table, const int32_t* positions);
+                         void* y, const float* table, const int32_t* positions, int table_S);
 int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                              void* y, const float* table, const int32_t* positions);
+                              void* y, const float* table, const int32_t* positions, int table_S);
 
 extern "C" int grl_rope(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x,
                         const int32_t* position_ids, void* y, int style, float rope_base, float rope_scaling) {
@@ -661,8 +661,8 @@ int grl_rope_strided(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int
             const float* tab = nullptr;
             int rc = grl_rope_table_get(c, (int)S, (int)D, rope_base, rope_scaling, style, &tab);
             if (rc) return rc;
-            return style == GRL_ROPE_HALF ? grl_rope_half_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab, nullptr)
-                                          : grl_rope_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab, nullptr);
+            return style == GRL_ROPE_HALF ? grl_rope_half_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab, nullptr, 0)
+                                          : grl_rope_apply_table(c, dtype, B, S, H, D, x, x_stride, y, tab, nullptr, 0);
         }
     }
     RopeFreq fr; grl_rope_freqs(&fr, (int)D, rope_base);
@@ -695,10 +695,14 @@ int grl_build_rope_table(grl_ctx* c, float* tab, int S, int D, float base, float
     return grl_build_rope_table_styled(c, tab, S, D, base, scaling, GRL_ROPE_INTERLEAVED);
 }
 
-int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int style, const float** out) {
+int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int style, const float** out, int* positions) {
     std::lock_guard<std::mutex> lk(c->tab_mu);
     for (auto& t : c->rope_tables)
-        if (t.D == D && t.style == style && t.base == base && t.scaling == scaling && t.S >= S) { *out = (const float*)t.dev; return GRL_OK; }
+        if (t.D == D && t.style == style && t.base == base && t.scaling == scaling && t.S >= S) {
+            *out = (const float*)t.dev;
+            if (positions) *positions = t.S;
+            return GRL_OK;
+        }
     // Not there (or too short): build one.  The pointer handed out leaves this function without any hold on the
     // table (another thread of the same context may be between its lookup and its launch), so a table is NEVER
     // freed while the context lives: a superseded one moves to the retired list and keeps its memory until
@@ -721,6 +725,7 @@ int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int 
     if (rc) { grl_free(c, dev); return rc; }
     c->rope_tables.push_back({(int)cap, D, style, base, scaling, dev});
     *out = (const float*)dev;
+    if (positions) *positions = (int)cap;
     return GRL_OK;
 }
 
@@ -728,7 +733,7 @@ int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int 
 // every row read once and written once (the K pre-rotation of the fused-RoPE attention path).
 template <typename T>
 __global__ __launch_bounds__(256) void rope_table_apply_kernel(const T* __restrict__ x, int64_t x_stride, T* __restrict__ y,
-                                                              const float2* __restrict__ tab, const int32_t* __restrict__ positions, int64_t nchunks, int S, int H, int D) {
+                                                              const float2* __restrict__ tab, const int32_t* __restrict__ positions, int64_t nchunks, int S, int H, int D, int table_S) {
     constexpr int EPC = 16 / (int)sizeof(T), PPC = EPC / 2;
     const int cpr = D / EPC;                       // chunks per (position, head) row
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -736,7 +741,7 @@ __global__ __launch_bounds__(256) void rope_table_apply_kernel(const T* __restri
         const int c = (int)(i % cpr);
         const int64_t vec = i / cpr;               // (b,s,h) flat
         const int64_t bs = vec / H;
-        const int h = (int)(vec - bs * H), s = positions ? positions[bs] : (int)(bs % S);
+        const int h = (int)(vec - bs * H), s = positions ? (int)min((uint32_t)positions[bs], (uint32_t)(table_S - 1)) : (int)(bs % S);
         u32x4 v = *(const u32x4*)(x + bs * x_stride + (int64_t)h * D + c * EPC);
         const float2* t = tab + (int64_t)s * (D / 2) + c * PPC;
         u32x4 o;
@@ -761,13 +766,13 @@ __global__ __launch_bounds__(256) void rope_table_apply_kernel(const T* __restri
 }
 
 int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                         void* y, const float* table, const int32_t* positions) {
+                         void* y, const float* table, const int32_t* positions, int table_S) {
     const int64_t epc = dtype == GRL_BF16 ? 8 : 4;
     const int64_t nchunks = B * S * H * (D / epc);
     if (nchunks == 0) return GRL_OK;
     dim3 g(ew_grid(nchunks)), b(256);
-    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_table_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
-    else hipLaunchKernelGGL(rope_table_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
+    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_table_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D, table_S);
+    else hipLaunchKernelGGL(rope_table_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D, table_S);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
 }
@@ -776,7 +781,7 @@ int grl_rope_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H,
 // (position, head) row and its partner chunk D/2 further on (shaders/rope.glsl:74-125 pairs d with d + D/2).
 template <typename T>
 __global__ __launch_bounds__(256) void rope_half_apply_kernel(const T* __restrict__ x, int64_t x_stride, T* __restrict__ y,
-                                                             const float2* __restrict__ tab, const int32_t* __restrict__ positions, int64_t nchunks, int S, int H, int D) {
+                                                             const float2* __restrict__ tab, const int32_t* __restrict__ positions, int64_t nchunks, int S, int H, int D, int table_S) {
     constexpr int EPC = 16 / (int)sizeof(T);
     const int half = D / 2, cph = half / EPC;      // chunks per half row
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -784,7 +789,7 @@ __global__ __launch_bounds__(256) void rope_half_apply_kernel(const T* __restric
         const int c = (int)(i % cph);
         const int64_t vec = i / cph;               // (b,s,h) flat
         const int64_t bs = vec / H;
-        const int h = (int)(vec - bs * H), s = positions ? positions[bs] : (int)(bs % S);
+        const int h = (int)(vec - bs * H), s = positions ? (int)min((uint32_t)positions[bs], (uint32_t)(table_S - 1)) : (int)(bs % S);
         const T* xr = x + bs * x_stride + (int64_t)h * D + c * EPC;
         const u32x4 lo = *(const u32x4*)xr, hi = *(const u32x4*)(xr + half);
         const float2* t = tab + (int64_t)s * half + c * EPC;
@@ -813,13 +818,13 @@ __global__ __launch_bounds__(256) void rope_half_apply_kernel(const T* __restric
 }
 
 int grl_rope_half_apply_table(grl_ctx* c, int dtype, int64_t B, int64_t S, int64_t H, int64_t D, const void* x, int64_t x_stride,
-                              void* y, const float* table, const int32_t* positions) {
+                              void* y, const float* table, const int32_t* positions, int table_S) {
     const int64_t epc = dtype == GRL_BF16 ? 8 : 4;
     const int64_t nchunks = B * S * H * ((D / 2) / epc);
     if (nchunks == 0) return GRL_OK;
     dim3 g(ew_grid(nchunks)), b(256);
-    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_half_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
-    else hipLaunchKernelGGL(rope_half_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D);
+    if (dtype == GRL_F32) hipLaunchKernelGGL(rope_half_apply_kernel<float>, g, b, 0, c->stream, (const float*)x, x_stride, (float*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D, table_S);
+    else hipLaunchKernelGGL(rope_half_apply_kernel<uint16_t>, g, b, 0, c->stream, (const uint16_t*)x, x_stride, (uint16_t*)y, (const float2*)table, positions, nchunks, (int)S, (int)H, (int)D, table_S);
     GRL_CHECK_LAUNCH();
     return GRL_OK;
 }

@@ -493,8 +493,9 @@ int grl_bert_layers_fwd_fused_ragged(grl_ctx* ctx, int dtype, const grl_ragged* 
                                      const grl_bert_layer_fused* w, int64_t layers, float eps, void* r, float* stats, void* workspace);
 /* Self-attention with rotary positions from the rows x (B*S, or those of a ragged batch; d = H*D) on: qkv = x.Wqkv^T + b (rows of 3*d), the
  * halves of each head of Q and K rotated as pairs (GRL_ROPE_HALF), out = attention.  Replaces the projection, rotation and attention
- * of utils/vulkan_sentence_transformer.py:806-891.  In bf16 with D = 64 the rotation runs in the projection's epilogue wherever its
- * kernel has one, and Q and K stand in qkv rotated; else attention rotates and they stand as projected.  mask: (B, S) or NULL, of a
+ * of utils/vulkan_sentence_transformer.py:806-891.  With D = 64 the rotation runs in the projection's epilogue wherever its kernel has
+ * one (bf16: nearly all; fp32: those of few rows), and Q and K stand in qkv rotated; else attention rotates and they stand as projected.
+ * As in grl_fa2_fwd_ragged the rows of a sequence stand at positions 0, 1, 2 ... (a batch of GRL_PACK_PREFIX).  mask: (B, S) or NULL, of a
  * rectangular batch. */
 int grl_rotary_attention(grl_ctx* ctx, int dtype, int64_t B, int64_t S, const grl_ragged* batch, int64_t H, int64_t D, const void* x,
                          const void* w_qkv, const float* b_qkv, const float* mask, void* qkv, void* out, float rope_base, float rope_scaling);

@@ -11,6 +11,7 @@ SOURCE = r"""
 #include "attention.hpp"
 extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
 extern "C" int kernel(long long M, long long N, long long K, int elem_size, int dual) { return gemm_kernel(M, N, K, elem_size, dual, 256); }
+extern "C" int rope_kernel(long long M, long long N, long long K, int elem_size) { return gemm_rope_kernel(M, N, K, 2 * N / 3, elem_size, 256); }
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
 extern "C" int order_checked(int order) { return fa_order_checked(order); }
 extern "C" int order(int causal, int S, int ragged, int heads, int D) { return fa_order(causal, S, ragged, heads, D); }
@@ -28,6 +29,7 @@ def rules(tmp_path_factory):
                     "-o", str(at / "rules.so"), str(at / "rules.hip")], check=True, timeout=100)
     lib = ctypes.CDLL(str(at / "rules.so"))
     lib.kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
+    lib.rope_kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     return lib
 
 
@@ -67,3 +69,10 @@ def test_two_shared_tiles_per_unit_need_a_long_sum(rules):
     for M, N in ((2100, 512), (2600, 512), (1088, 1152), (2000, 768), (512, 4096)):
         assert [rules.kernel(M, N, K, 2, 0) for K in (3072, 5120, 6080, 6144, 11008)] == [8, 8, 8, 10, 10]
     assert rules.kernel(800, 768, 768, 2, 0) == 10
+
+
+def test_rotary_products(rules):
+    """which kernel rotates in its epilogue; 0: none, and no table is fetched for it"""
+    assert [rules.rope_kernel(M, 2304, 768, 2) for M in (16, 100, 400, 810, 1500, 3000, 5390, 65536)] == [9, 9, 10, 7, 6, 4, 3, 3]
+    assert [rules.rope_kernel(M, 2304, 768, 4) for M in (27, 300, 3000, 65536)] == [9, 9, 0, 0]
+    assert rules.rope_kernel(100, 2304, 776, 2) == 0 and rules.rope_kernel(100, 96, 768, 2) == 0

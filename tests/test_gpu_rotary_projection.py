@@ -51,3 +51,69 @@ def test_rotary_attention(backend, dtype, B, S, H, D, ragged):
     finally:
         for t in (dx, dw, db, do, dp, qkv, out):
             t.free()
+
+
+# (rows, head dim): products that rotate on tiles of 32 (100), 128 on eight waves (1500) and four (3000), 256 (5400); at head dim 32 a pass over the keys
+@pytest.mark.parametrize("dtype,n,D", [("bf16", 50, 64), ("bf16", 750, 64), ("bf16", 1500, 64), ("bf16", 2700, 64), ("fp32", 50, 64), ("bf16", 50, 32)])
+def test_positions_behind_the_table(backend, dtype, n, D):
+    """Rows have to stand at positions 0, 1, 2 ...; others read nothing behind the table, whose last position (a power of two, 1024 at least) they take."""
+    c, code, H = backend.core, (L.GRL_BF16 if dtype == "bf16" else L.GRL_F32), 12 * 64 // D
+    base = 9000.0 + n + D + 7 * code          # a table of its own, no longer than it has to be
+    d, M, end = H * D, 2 * n, max(1024, 1 << (n - 1).bit_length())
+    rng = np.random.default_rng(n)
+    bufs = dx, dw, db, do = [c.upload(rng.standard_normal((M, d), dtype=np.float32), code), c.upload((rng.standard_normal((3 * d, d)) / 30).astype(np.float32), code),
+                             c.upload(rng.standard_normal(3 * d).astype(np.float32)), c.upload_raw(np.array([0, n, M], np.int32))]
+    pos = np.concatenate([np.arange(n), np.arange(n) * 3 + end - n]).astype(np.int32)
+    pos[-1] = 2 ** 31 - 1
+    qkv, out = c.alloc(M * 3 * d * 4), c.alloc(M * d * 4)
+    got = []
+    for p in (np.minimum(pos, end - 1), pos):
+        dp = c.upload_raw(p)
+        L.check(c.lib.grl_rotary_attention(c.ctx, code, 0, 0, ctypes.byref(L.Ragged(do.ptr, dp.ptr, 2, M, n)), H, D, dx.ptr, dw.ptr, db.ptr, None, qkv.ptr, out.ptr,
+                                           base, 1.0), "rotary_attention")
+        got.append(c.download(out, (M, d), code))
+        dp.free()
+    np.testing.assert_array_equal(got[0], got[1])
+    for t in bufs + [qkv, out]:
+        t.free()
+
+
+def test_no_table_where_nothing_reads_one(backend):
+    """fp32 products of many rows leave the rotation to kernels that form their angles themselves (ragged batches)"""
+    c, B, S, H, D = backend.core, 30, 100, 6, 64
+    d, M = H * D, 3000
+    bufs = dx, dw, do, dp, qkv, out = [c.alloc(M * d * 4), c.alloc(3 * d * d * 4), c.upload_raw(np.arange(0, M + 1, S, dtype=np.int32)),
+                                       c.upload_raw(np.tile(np.arange(S, dtype=np.int32), B)), c.alloc(M * 3 * d * 4), c.alloc(M * d * 4)]
+    for t in (dx, dw):
+        L.check(c.lib.grl_memset(c.ctx, t.ptr, 0, t.nbytes), "memset")
+    def in_use():
+        stats = L.PoolStats()
+        L.check(c.lib.grl_pool_get_stats(c.ctx, ctypes.byref(stats)), "pool")
+        return stats.bytes_in_use
+    before = in_use()
+    L.check(c.lib.grl_rotary_attention(c.ctx, L.GRL_F32, B, S, ctypes.byref(L.Ragged(do.ptr, dp.ptr, B, M, S)), H, D, dx.ptr, dw.ptr, None, None, qkv.ptr, out.ptr,
+                                       9998.0, 1.0), "rotary_attention")
+    assert in_use() == before
+    for t in bufs:
+        t.free()
+
+
+@pytest.mark.parametrize("dtype,B,S,D", [("bf16", 2, 50, 64), ("bf16", 15, 100, 64), ("bf16", 55, 98, 64), ("bf16", 5, 80, 32), ("fp32", 2, 50, 64), ("fp32", 30, 100, 64)])
+def test_key_mask(backend, dtype, B, S, D):
+    c, code, H = backend.core, (L.GRL_BF16 if dtype == "bf16" else L.GRL_F32), 12 * 64 // D
+    d, M = H * D, B * S
+    rng = np.random.default_rng(B * S)
+    q = (lambda a: O.bf16_round(a)) if dtype == "bf16" else (lambda a: a)
+    x, w, b = q(rng.standard_normal((M, d), dtype=np.float32)), q((rng.standard_normal((3 * d, d)) / np.sqrt(d)).astype(np.float32)), rng.standard_normal(3 * d).astype(np.float32)
+    mask = (rng.random((B, S)) < 0.7).astype(np.float32)
+    mask[-1] = np.arange(S) >= S // 2          # padding on the left
+    mask[:, -1] = 1.0
+    bufs = dx, dw, db, dm, qkv, out = [c.upload(x, code), c.upload(w, code), c.upload(b), c.upload(mask), c.alloc(M * 3 * d * 4), c.alloc(M * d * 4)]
+    L.check(c.lib.grl_rotary_attention(c.ctx, code, B, S, None, H, D, dx.ptr, dw.ptr, db.ptr, dm.ptr, qkv.ptr, out.ptr, 10000.0, 1.0), "rotary_attention")
+    got = c.download(out, (B, S, H, D), code)
+    for s in sorted({0, B // 2, B - 1}):
+        parts = O.truth_linear(x[s * S:(s + 1) * S], w, b).reshape(S, 3, H, D)
+        ref = O.truth_attention(parts[None, :, 0], parts[None, :, 1], parts[None, :, 2], mask=mask[s:s + 1], rope="half")
+        assert O.max_rel(got[s:s + 1], ref) < (TOL_F32 if dtype == "fp32" else TOL_BF16)
+    for t in bufs:
+        t.free()
