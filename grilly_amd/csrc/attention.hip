@@ -200,11 +200,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
         const int so = kt * soff_tile + soff_w;
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         ::"s"(lds_t + ST * TILE + j * 1024), "v"(voffT[j % KVAR]), "s"(rsT), "s"(so + j * soff_step) : "memory");
-        if constexpr (HAS_MASK)
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         ::"s"(lds0 + OFF_M + ST * 1024), "v"(lane * 16), "s"(rsM), "s"(kt * KT * 4) : "memory");
+            dma16(rsT, lds_t + ST * TILE + j * 1024, voffT[j % KVAR], so + j * soff_step);
+        if constexpr (HAS_MASK) dma16(rsM, lds0 + OFF_M + ST * 1024, lane * 16, kt * KT * 4);
     };
     // the stage a runtime tile index lives in (prologue only; the loop knows its stage at compile time)
     auto issue_rt = [&](int kt) __attribute__((always_inline)) { issue(kt, kt % NSTG); };
