@@ -567,7 +567,6 @@ class PreNormEncoder:
         B, S = self._shape
         cfg, c, lib, code = self.cfg, self.core, self.core.lib, self.code
         M, d, ff, H, D = B * S if rg is None else rg.rows, cfg.d_model, cfg.d_ff, cfg.heads, cfg.head_dim
-        es = 2 if code == L.GRL_BF16 else 4
         own_stats = 0 < M * ff <= self._own_max
         if rg is None:
             mask = self.mask.ptr if self.has_mask else None
