@@ -41,6 +41,13 @@ def test_every_transfer_has_its_destination(code):
         assert any(re.match(r"s_\w+ m0,", l) for l in code[first + 1:last]), code
 
 
+def test_a_wait_state_follows_the_write_of_m0(code):
+    """as the compiler arranges it for its own transfers"""
+    for i, l in enumerate(code):
+        if re.match(r"s_\w+ m0,", l):
+            assert not code[i + 1].endswith(" lds"), code[i:i + 2]
+
+
 def test_one_place_writes_m0():
     text = "".join(open(f).read() for pattern in ("*.hip", "*.hpp") for f in glob.glob(os.path.join(CSRC, pattern)))
     assert len(re.findall(r"s_mov_b32 m0", text)) == 1
