@@ -12,6 +12,7 @@ SOURCE = r"""
 extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
 extern "C" int kernel(long long M, long long N, long long K, int elem_size, int dual) { return gemm_kernel(M, N, K, elem_size, dual, 256); }
 extern "C" int rope_kernel(long long M, long long N, long long K, int elem_size) { return gemm_rope_kernel(M, N, K, 2 * N / 3, elem_size, 256); }
+extern "C" int resln_kernel(long long M, long long N, long long K, int elem_size) { return gemm_resln_kernel(M, N, K, elem_size, 256); }
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
 extern "C" int order_checked(int order) { return fa_order_checked(order); }
 extern "C" int order(int causal, int S, int ragged, int heads, int D) { return fa_order(causal, S, ragged, heads, D); }
@@ -29,7 +30,7 @@ def rules(tmp_path_factory):
                     "-o", str(at / "rules.so"), str(at / "rules.hip")], check=True, timeout=100)
     lib = ctypes.CDLL(str(at / "rules.so"))
     lib.kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
-    lib.rope_kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
+    lib.rope_kernel.argtypes = lib.resln_kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     return lib
 
 
@@ -76,3 +77,16 @@ def test_rotary_products(rules):
     assert [rules.rope_kernel(M, 2304, 768, 2) for M in (16, 100, 400, 810, 1500, 3000, 5390, 65536)] == [9, 9, 10, 7, 6, 4, 3, 3]
     assert [rules.rope_kernel(M, 2304, 768, 4) for M in (27, 300, 3000, 65536)] == [9, 9, 0, 0]
     assert rules.rope_kernel(100, 2304, 776, 2) == 0 and rules.rope_kernel(100, 96, 768, 2) == 0
+
+
+def test_sizes_of_the_row_partials_tests(rules):
+    """test_gpu_row_partials names the bf16 kernel that writes the partials and the one that merges them; both as the launchers choose."""
+    from test_gpu_row_partials import GATED, LAYERS
+    for M, d, ff, writes, reads in GATED:
+        assert rules.resln_kernel(M, d, d, 2) == writes and rules.kernel(M, ff, d, 2, 1) == reads, (M, d)
+    for B, S, heads, ff, kernels in LAYERS:
+        M, d = B * S, 64 * heads
+        assert (rules.resln_kernel(M, d, d, 2), rules.resln_kernel(M, d, ff, 2), rules.kernel(M, 3 * d, d, 2, 0), rules.kernel(M, ff, d, 2, 0)) == kernels, (M, d)
+    assert {g[3] for g in GATED} == {3, 4, 6, 7} and {k for l in LAYERS for k in l[4]} >= {3, 4, 6, 7, 8}
+    odd = [(M, d, w) for M, d, _, w, _ in GATED if M % 2 and 128 < d <= (1536 if w == 3 else 768)]      # two to six partials
+    assert {w for _, _, w in odd} == {3, 4, 6, 7}

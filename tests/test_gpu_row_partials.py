@@ -1,7 +1,8 @@
 """GPU parity of row statistics that stay partial sums between products: several folded layers in one call against the same layers one
 call each (which merge them in a launch of their own), and the gated MLP block against its two products.  Widths give 1 to 6 partials, and
-7 and more, which are merged in any case; row counts reach every kernel that writes or reads them (64 x 64 and 64 x 128 tiles, 128 x 128 on
-four and eight waves, 256 x 256, and the small ones that take none) with ragged last tiles.
+7 and more, which are merged in any case; row counts, odd ones among them, reach every kernel that writes or reads them in bf16 (64 x 64 and
+64 x 128 tiles, 128 x 128 on four and eight waves, 256 x 256 with more than one tile per workgroup, and the small ones that take none) with
+ragged last tiles.  The kernels' numbers stand beside the sizes; test_dispatch_host.py holds them against the launchers' rules.
 The sums are the same in the same order, so what differs is at most the rounding of a quotient: 2^-23 of a statistic, which can move a
 stored value by one unit of its type (bf16 2^-8, fp32 2^-23) and that unit through the rest: 2-norms agree to 4e-3 and 4e-6."""
 import ctypes
@@ -26,9 +27,14 @@ def near(a, b, dtype):
     assert np.linalg.norm(a - b) <= NEAR[dtype] * np.linalg.norm(b)
 
 
+# (sequences, length, heads of 64, d_ff, bf16 kernels of out-proj, FFN2 (these write partials), QKV, FFN1 (these read them))
+LAYERS = [(1, 1, 2, 64, (7, 7, 9, 9)), (3, 43, 2, 192, (7, 7, 9, 9)), (5, 60, 6, 256, (7, 7, 9, 9)), (20, 65, 12, 192, (7, 7, 6, 9)), (21, 120, 12, 448, (7, 7, 4, 8)),
+          (70, 128, 6, 1536, (6, 6, 4, 3)), (90, 160, 12, 256, (4, 4, 4, 6)), (9, 100, 14, 128, (7, 7, 6, 9)), (13, 100, 16, 128, (7, 7, 4, 9)),
+          (19, 67, 12, 192, (7, 7, 6, 9)), (73, 73, 12, 256, (6, 6, 4, 8)), (85, 511, 12, 768, (3, 3, 3, 3))]
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
-@pytest.mark.parametrize("B,S,heads,ff", [(1, 1, 2, 64), (3, 43, 2, 192), (5, 60, 6, 256), (20, 65, 12, 192), (21, 120, 12, 448), (70, 128, 6, 1536), (90, 160, 12, 256),
-                                          (9, 100, 14, 128), (13, 100, 16, 128)])
+@pytest.mark.parametrize("B,S,heads,ff", [l[:4] for l in LAYERS])
 def test_layers_in_one_call(backend, dtype, B, S, heads, ff):
     import grilly_amd
     c, d = backend.core, 64 * heads
@@ -55,8 +61,14 @@ def test_layers_in_one_call(backend, dtype, B, S, heads, ff):
     enc.release_activations()
 
 
+# (rows, d_model, d_ff, bf16 kernels of the product that writes partials and of the gated one)
+GATED = [(1, 64, 64, 7, 9), (130, 384, 96, 7, 9), (1400, 768, 200, 7, 10), (3100, 768, 1152, 6, 4), (7300, 640, 1152, 4, 4), (26000, 768, 1152, 4, 3), (900, 960, 128, 7, 9),
+         (2501, 384, 384, 7, 10), (2501, 768, 384, 7, 10), (9001, 384, 384, 6, 4), (5001, 768, 384, 6, 4), (11001, 384, 384, 4, 4), (7301, 768, 384, 4, 4),
+         (43435, 768, 384, 3, 3), (32695, 1024, 512, 3, 3)]
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
-@pytest.mark.parametrize("M,d,ff", [(1, 64, 64), (130, 384, 96), (1400, 768, 200), (3100, 768, 1152), (7300, 640, 1152), (26000, 768, 1152), (900, 960, 128)])
+@pytest.mark.parametrize("M,d,ff", [g[:3] for g in GATED])
 def test_gated_block(backend, dtype, M, d, ff):
     c, code, lib = backend.core, (L.GRL_BF16 if dtype == "bf16" else L.GRL_F32), backend.core.lib
     rng = np.random.default_rng(M + d)
