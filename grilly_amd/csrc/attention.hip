@@ -200,8 +200,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
         const int so = kt * soff_tile + soff_w;
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
-            dma16(rsT, lds_t + ST * TILE + j * 1024, voffT[j % KVAR], so + j * soff_step);
-        if constexpr (HAS_MASK) dma16(rsM, lds0 + OFF_M + ST * 1024, lane * 16, kt * KT * 4);
+            dma16(rsT, lds_t + ST * TILE + j * 1024, voffT[j % KVAR], so, j * soff_step);
+        if constexpr (HAS_MASK) dma16(rsM, lds0 + OFF_M + ST * 1024, lane * 16, kt * KT * 4, 0);
     };
     // the stage a runtime tile index lives in (prologue only; the loop knows its stage at compile time)
     auto issue_rt = [&](int kt) __attribute__((always_inline)) { issue(kt, kt % NSTG); };

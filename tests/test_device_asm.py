@@ -14,7 +14,7 @@ __global__ void transfers(const void* p, int* out, int n) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, n, 0x00020000);
     auto own = [&](int at) { __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)lds, 16, threadIdx.x * 16, at, 0, 0); };
     own(4096);
-    dma16(make_rsrc_words(p, n), 1024, threadIdx.x * 16, n);
+    dma16(make_rsrc_words(p, n), 1024, threadIdx.x * 16, n, 64);
     own(8192);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
