@@ -711,7 +711,11 @@ int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int 
     int64_t cap = 1024;
     while (cap < S) cap *= 2;
     if (cap * (D / 2) >= (1LL << 31)) cap = S;
-    for (size_t i = 0; i < c->rope_tables.size(); ++i) {
+    // A stream under capture only records the launch that fills the table.  Its replays fill it, so the table is that graph's (kept until
+    // grl_destroy), and no other call may find it.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool recorded = hipStreamIsCapturing(c->stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
+    for (size_t i = 0; i < c->rope_tables.size() && !recorded; ++i) {
         auto& t = c->rope_tables[i];
         if ((t.D == D && t.style == style && t.base == base && t.scaling == scaling) || c->rope_tables.size() >= 16) {
             c->retired_tables.push_back(t.dev);
@@ -723,7 +727,8 @@ int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int 
     if (!dev) return GRL_ERR_OOM;
     int rc = grl_build_rope_table_styled(c, (float*)dev, (int)cap, D, base, scaling, style);
     if (rc) { grl_free(c, dev); return rc; }
-    c->rope_tables.push_back({(int)cap, D, style, base, scaling, dev});
+    if (recorded) c->retired_tables.push_back(dev);
+    else c->rope_tables.push_back({(int)cap, D, style, base, scaling, dev});
     *out = (const float*)dev;
     if (positions) *positions = (int)cap;
     return GRL_OK;

@@ -117,3 +117,39 @@ def test_key_mask(backend, dtype, B, S, D):
         assert O.max_rel(got[s:s + 1], ref) < (TOL_F32 if dtype == "fp32" else TOL_BF16)
     for t in bufs:
         t.free()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+def test_a_table_first_needed_under_capture(backend, dtype):
+    """The launch that fills the cos/sin table is only recorded then: calls in front of the first replay do not use that table."""
+    c, code, B, S, H, D = backend.core, (L.GRL_BF16 if dtype == "bf16" else L.GRL_F32), 2, 50, 12, 64
+    d, M, base = H * D, B * S, 7001.0 + 8 * code                  # a base that nothing else uses
+    rng = np.random.default_rng(6)
+    q = (lambda a: O.bf16_round(a)) if dtype == "bf16" else (lambda a: a)
+    x, w, b = q(rng.standard_normal((M, d), dtype=np.float32)), q((rng.standard_normal((3 * d, d)) / np.sqrt(d)).astype(np.float32)), rng.standard_normal(3 * d).astype(np.float32)
+    bufs = dx, dw, db, do, dp, qkv, out = [c.upload(x, code), c.upload(w, code), c.upload(b), c.upload_raw(np.arange(0, M + 1, S, dtype=np.int32)),
+                                           c.upload_raw(np.tile(np.arange(S, dtype=np.int32), B)), c.alloc(M * 3 * d * 4), c.alloc(M * d * 4)]
+    rg = L.Ragged(do.ptr, dp.ptr, B, M, S)
+    run = lambda: c.lib.grl_rotary_attention(c.ctx, code, 0, 0, ctypes.byref(rg), H, D, dx.ptr, dw.ptr, db.ptr, None, qkv.ptr, out.ptr, base, 1.0)
+    parts = O.truth_linear(x, w, b).reshape(B, S, 3, H, D)
+    ref = O.truth_attention(parts[:, :, 0], parts[:, :, 1], parts[:, :, 2], rope="half", base=base)
+    stream, graph, replay = ctypes.c_void_p(c.lib.grl_stream(c.ctx)), ctypes.c_void_p(), ctypes.c_void_p()
+    hip = lambda name, *args: L.check(getattr(c.lib, name)(*args), name)
+    try:
+        hip("hipStreamBeginCapture", stream, 2)          # relaxed: the table's allocation goes through
+        rc = run()
+        hip("hipStreamEndCapture", stream, ctypes.byref(graph))
+        L.check(rc, "rotary_attention")
+        hip("hipGraphInstantiate", ctypes.byref(replay), graph, None, None, ctypes.c_size_t(0))
+        for _ in range(3):
+            for launch in (lambda: L.check(run(), "rotary_attention"), lambda: hip("hipGraphLaunch", replay, stream)):
+                L.check(c.lib.grl_memset(c.ctx, out.ptr, 0, out.nbytes), "memset")
+                launch()
+                assert O.max_rel(c.download(out, (B, S, H, D), code), ref) < (TOL_F32 if dtype == "fp32" else TOL_BF16)
+    finally:
+        if replay:
+            c.lib.hipGraphExecDestroy(replay)
+        if graph:
+            c.lib.hipGraphDestroy(graph)
+        for t in bufs:
+            t.free()
