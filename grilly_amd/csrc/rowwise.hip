@@ -697,40 +697,49 @@ int grl_build_rope_table(grl_ctx* c, float* tab, int S, int D, float base, float
 
 int grl_rope_table_get(grl_ctx* c, int S, int D, float base, float scaling, int style, const float** out, int* positions) {
     std::lock_guard<std::mutex> lk(c->tab_mu);
-    for (auto& t : c->rope_tables)
-        if (t.D == D && t.style == style && t.base == base && t.scaling == scaling && t.S >= S) {
-            *out = (const float*)t.dev;
-            if (positions) *positions = t.S;
-            return GRL_OK;
-        }
-    // Not there (or too short): build one.  The pointer handed out leaves this function without any hold on the
-    // table (another thread of the same context may be between its lookup and its launch), so a table is NEVER
-    // freed while the context lives: a superseded one moves to the retired list and keeps its memory until
-    // grl_destroy.  Lengths are rounded up to a power of two (at least 1024 positions), so one kind of table is
-    // rebuilt at most once per doubling of the sequence length and the retired ones add up to less than the live one.
-    int64_t cap = 1024;
-    while (cap < S) cap *= 2;
-    if (cap * (D / 2) >= (1LL << 31)) cap = S;
-    // A stream under capture only records the launch that fills the table.  Its replays fill it, so the table is that graph's (kept until
-    // grl_destroy), and no other call may find it.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool recorded = hipStreamIsCapturing(c->stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
-    for (size_t i = 0; i < c->rope_tables.size() && !recorded; ++i) {
-        auto& t = c->rope_tables[i];
-        if ((t.D == D && t.style == style && t.base == base && t.scaling == scaling) || c->rope_tables.size() >= 16) {
-            c->retired_tables.push_back(t.dev);
-            c->rope_tables.erase(c->rope_tables.begin() + i);
-            break;
+    auto same = [&](const grl_ctx::rope_table& t) { return t.D == D && t.style == style && t.base == base && t.scaling == scaling; };
+    size_t at = 0;
+    while (at < c->rope_tables.size() && !(same(c->rope_tables[at]) && c->rope_tables[at].S >= S)) ++at;
+    if (at == c->rope_tables.size() || c->rope_tables[at].capture) {
+        // A stream under capture only records the launch that fills a table: its values are there for what the same capture records behind it, and
+        // for nobody else.  Any other call fills the table once more, with the same values, so graphs that share it do not mind.
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        const bool recorded = hipStreamGetCaptureInfo(c->stream, &status, &id) == hipSuccess && status != hipStreamCaptureStatusNone;
+        const unsigned long long capture = recorded ? id + 1 : 0;
+        if (at < c->rope_tables.size()) {
+            auto& t = c->rope_tables[at];
+            if (t.capture != capture) {
+                const int rc = grl_build_rope_table_styled(c, (float*)t.dev, t.S, D, base, scaling, style);
+                if (rc) return rc;
+                t.capture = capture;
+            }
+        } else {
+            // Not there (or too short): build one.  The pointer handed out leaves this function without any hold on the
+            // table (another thread of the same context may be between its lookup and its launch), so a table is NEVER
+            // freed while the context lives: a superseded one moves to the retired list and keeps its memory until
+            // grl_destroy.  Lengths are rounded up to a power of two (at least 1024 positions), so one kind of table is
+            // rebuilt at most once per doubling of the sequence length and the retired ones add up to less than the live one.
+            int64_t cap = 1024;
+            while (cap < S) cap *= 2;
+            if (cap * (D / 2) >= (1LL << 31)) cap = S;
+            for (size_t i = 0; i < c->rope_tables.size(); ++i) {
+                if (same(c->rope_tables[i]) || c->rope_tables.size() >= 16) {
+                    c->retired_tables.push_back(c->rope_tables[i].dev);
+                    c->rope_tables.erase(c->rope_tables.begin() + i);
+                    break;
+                }
+            }
+            void* dev = grl_malloc(c, (size_t)cap * (D / 2) * sizeof(float2));
+            if (!dev) return GRL_ERR_OOM;
+            int rc = grl_build_rope_table_styled(c, (float*)dev, (int)cap, D, base, scaling, style);
+            if (rc) { grl_free(c, dev); return rc; }
+            at = c->rope_tables.size();
+            c->rope_tables.push_back({(int)cap, D, style, base, scaling, dev, capture});
         }
     }
-    void* dev = grl_malloc(c, (size_t)cap * (D / 2) * sizeof(float2));
-    if (!dev) return GRL_ERR_OOM;
-    int rc = grl_build_rope_table_styled(c, (float*)dev, (int)cap, D, base, scaling, style);
-    if (rc) { grl_free(c, dev); return rc; }
-    if (recorded) c->retired_tables.push_back(dev);
-    else c->rope_tables.push_back({(int)cap, D, style, base, scaling, dev});
-    *out = (const float*)dev;
-    if (positions) *positions = (int)cap;
+    *out = (const float*)c->rope_tables[at].dev;
+    if (positions) *positions = c->rope_tables[at].S;
     return GRL_OK;
 }
 

@@ -153,3 +153,58 @@ def test_a_table_first_needed_under_capture(backend, dtype):
             c.lib.hipGraphDestroy(graph)
         for t in bufs:
             t.free()
+
+
+def test_captures_share_one_table(backend):
+    """Each capture records the filling once, into the same memory, and a call outside fills it again; all replays and calls agree."""
+    c, code, B, S, H, D = backend.core, L.GRL_BF16, 2, 50, 12, 64
+    d, M, base = H * D, B * S, 7103.0                            # a base that nothing else uses
+    rng = np.random.default_rng(7)
+    bufs = dx, dw, do, dp, qkv, out = [c.upload(rng.standard_normal((M, d), dtype=np.float32), code), c.upload((rng.standard_normal((3 * d, d)) / 28).astype(np.float32), code),
+                                       c.upload_raw(np.arange(0, M + 1, S, dtype=np.int32)), c.upload_raw(np.tile(np.arange(S, dtype=np.int32), B)),
+                                       c.alloc(M * 3 * d * 2), c.alloc(M * d * 2)]
+    rg = L.Ragged(do.ptr, dp.ptr, B, M, S)
+    run = lambda: L.check(c.lib.grl_rotary_attention(c.ctx, code, 0, 0, ctypes.byref(rg), H, D, dx.ptr, dw.ptr, None, None, qkv.ptr, out.ptr, base, 1.0), "rotary_attention")
+    stream, graphs, replays = ctypes.c_void_p(c.lib.grl_stream(c.ctx)), [], []
+    hip = lambda name, *args: L.check(getattr(c.lib, name)(*args), name)
+
+    def in_use():
+        stats = L.PoolStats()
+        L.check(c.lib.grl_pool_get_stats(c.ctx, ctypes.byref(stats)), "pool")
+        return stats.bytes_in_use
+
+    def nodes(graph):
+        n = ctypes.c_size_t()
+        hip("hipGraphGetNodes", graph, None, ctypes.byref(n))
+        return n.value
+    try:
+        before = in_use()
+        for calls in (3, 1):
+            graph, replay = ctypes.c_void_p(), ctypes.c_void_p()
+            hip("hipStreamBeginCapture", stream, 2)              # relaxed: the table's allocation goes through
+            try:
+                for _ in range(calls):
+                    run()
+            finally:
+                hip("hipStreamEndCapture", stream, ctypes.byref(graph))
+            graphs.append(graph)
+            hip("hipGraphInstantiate", ctypes.byref(replay), graph, None, None, ctypes.c_size_t(0))
+            replays.append(replay)
+        assert in_use() - before == 1024 * (D // 2) * 8
+        assert (nodes(graphs[0]) - 1) == 3 * (nodes(graphs[1]) - 1)
+        got = []
+        for launch in [lambda r=r: hip("hipGraphLaunch", r, stream) for r in reversed(replays)] + [run] + [lambda r=r: hip("hipGraphLaunch", r, stream) for r in replays]:
+            L.check(c.lib.grl_memset(c.ctx, out.ptr, 0, out.nbytes), "memset")
+            launch()
+            got.append(c.download(out, (M, d), code))
+        assert np.isfinite(got[0]).all() and np.abs(got[0]).max() > 0
+        for g in got[1:]:
+            np.testing.assert_array_equal(g, got[0])
+        assert in_use() - before == 1024 * (D // 2) * 8
+    finally:
+        for r in replays:
+            c.lib.hipGraphExecDestroy(r)
+        for g in graphs:
+            c.lib.hipGraphDestroy(g)
+        for t in bufs:
+            t.free()
