@@ -237,7 +237,8 @@ int grl_swiglu_nt(grl_ctx* ctx, int in_dtype, int out_dtype, int64_t M, int64_t 
  * from the pool, larger ones a one-wave-per-query kernel; RoPE needs an even D up to 128.
  * GRL_ROPE_HALF uses the (d, d+D/2) pairing of shaders/rope.glsl:74-125 and, on the direct path, a workspace of
  * 2*B*S*H*D elements (NULL = pool).  The cos/sin table of the rotation is built once per (D, base, scaling,
- * pairing) and kept on the context. */
+ * pairing) and kept on the context; first needed under stream capture, it is filled by every replay of that graph, and
+ * once more by the first call or capture behind it. */
 int grl_fa2_fwd(grl_ctx* ctx, int dtype, int64_t B, int64_t S, int64_t H, int64_t D,
                 const void* Q, const void* K, const void* V, const float* mask, void* O,
                 float scale, int causal, int rope, float rope_base, float rope_scaling,
