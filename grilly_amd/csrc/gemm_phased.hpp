@@ -1,0 +1,451 @@
+// bf16 products on 256 x 256 tiles (with two weights: 256 x 128 outputs): persistent workgroups of eight waves, one per CU, whose K steps
+// run in phases (included by gemm_kernels.hpp).
+//
+// A step is 64 k.  Its operands lie in one of two LDS stages of four halves, 128 rows each: A0, A1, B0, B1; half q holds the q-th 64
+// activation rows of both wave rows, or the q-th 32 weight rows of the four wave columns (two weights: half 0 is the gate's, half 1 the
+// up weight's).  A wave owns 128 x 64 of the tile and does a step in two phases: a memory part (fragment reads, transfers, a counted wait)
+// and a matrix part of 32 instructions, a barrier behind each.  Waves 4 to 7 run one part behind waves 0 to 3, so that of the two waves of a
+// SIMD one multiplies while the other reads.
+//
+//   memory part 0: reads B0, A0, B1 of step t;  requests A1 of step t + 1;          matrix part 0: rows of A0
+//   memory part 1: reads A1 of step t;          requests B0, A0, B1 of step t + 2;  matrix part 1: rows of A1
+//
+// A memory part ends when its reads are back, so a half is requested again one part after its last read, and is due six parts later: 64 to
+// 96 KiB are in flight all the time.  The cursor runs on into the next tile, so nothing drains between tiles: the epilogue stands between
+// the last matrix part and the next tile's first memory part, and only A1 of the last step's stage is not being refilled then.  There,
+// in the 2 KiB that its own transfers will fill, every wave turns 16 output rows at a time into 16-byte pieces of 128-byte rows: no barrier
+// in the epilogue, and the stores stand behind the transfers of two steps in the memory counter.
+//
+// Bound: the board's power limit on real operands (with all-zero ones the same launches are 20 to 25 % faster: a step of 2048 matrix cycles
+// takes 2340 at 2.4 GHz), then the output stores, which all CUs issue at once: without them 65536 x 2304 x 768 takes 163 us instead of
+// 184, 65536 x 768 x 768 with LayerNormed residual 75 instead of 88.
+// us, four phases of 16 instructions with an epilogue staged by the whole workgroup (four barriers, the stages drained for it) -> this:
+// 65536 x 2304 x 768 195.6 -> 187.6, 65536 x 2304 x 384 112.6 -> 105.7, folded 65536 x 3072 x 768 with GELU 301 -> 292, 65536 x 768 x 768 with
+// LayerNormed residual 93.1 -> 90.3, 8192 x 8192 x 8192 764 -> 739, gated 16384 x 11008 x 4096 2115 -> 2066; 65536 x 768 x 3072 level.
+// Without the stagger 27 % slower (four phases).  Tried and dropped: workgroups that start up to 3 us apart, so that their stores
+// do not meet (65536 x 2304 x 768 184 -> 185; x 384 109 -> 106), stores that stay in the caches (188.7 -> 199.8), no wave priorities (level).
+#pragma once
+
+template <typename OutT, int EPI, bool DUAL, bool LN = false>
+__global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
+    constexpr int BM = 256, BN = 256, BNO = DUAL ? BN / 2 : BN, WNO = BNO / 4, TNO = WNO / 32;
+    constexpr int HALFB = 128 * 128, STAGE = 4 * HALFB;
+    constexpr int OES = (int)sizeof(OutT), EPCO = 16 / OES;
+    constexpr bool RL = EPI == EPI_RESLN;                   // LayerNorm(residual) formed in the epilogue + row statistics out
+    constexpr bool HASRES = EPI == EPI_RES || RL, ROWS = LN || RL;
+    // one tile's vectors, fp32: bias slice(s); with row statistics also the column sums c (c2), or the residual norm's beta, and the
+    // tile's 256 row-statistics pairs.  Two buffers, alternating per tile.
+    constexpr int VECS = 2 * STAGE, COLB = BN * 4, BIASB = ROWS ? 2 * COLB + BM * 8 : COLB;
+    constexpr int PARTS_AT = VECS + 2 * BIASB, SUMS_AT = PARTS_AT + (ROWS ? GRL_MAX_PARTS * BM * 8 : 0);
+    __shared__ __attribute__((aligned(1024))) char lds[SUMS_AT + (RL ? 4 * BM * 8 : 0)];
+    static_assert(!(LN && RL) && !(RL && DUAL) && !(HASRES && DUAL), "one set of row statistics per tile");
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 2, wn = wave & 3, l4 = lane & 15, lq = lane >> 4;
+    const bool behind = wave >= 4;                           // the waves that run one part behind
+    const int ntiles = p.tiles_m * p.tiles_n;
+    const int64_t rowbytes = (int64_t)p.K * 2;
+    const int KT = p.K / 64;                                 // the host launches this kernel with two steps or more
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
+
+    auto tile_of = [&](int pid, int& m0, int& n0) {          // as in gemm_nt_dma_kernel
+        const int per = ntiles >> 3, rem = ntiles & 7, xcd = pid & 7, loc = pid >> 3;
+        const int npid = xcd * per + (xcd < rem ? xcd : rem) + loc;
+        const int width = p.group * p.tiles_n;
+        const int first_m = (npid / width) * p.group;
+        const int gsize = p.tiles_m - first_m < p.group ? p.tiles_m - first_m : p.group;
+        m0 = (first_m + (npid % width) % gsize) * BM;
+        n0 = ((npid % width) / gsize) * BNO;
+    };
+    auto rsrc_of = [&](const void* base, int first_row, int rows_total) {
+        int64_t left = (int64_t)(rows_total - first_row) * rowbytes;
+        if (left < 0) left = 0;
+        return make_rsrc_words((const char*)base + (int64_t)first_row * rowbytes, left > 0xffffffffLL ? 0xffffffffu : (uint32_t)left);
+    };
+
+    // lane -> (row lr of an 8-row group, slot ls): LDS slot ls of row r holds chunk ls ^ lds_swz<8>(r)
+    const int lr = lane >> 3, ls = lane & 7;
+    const int lane_off[2] = {lr * (int)rowbytes + ((ls ^ lds_swz<8>(lr)) << 4), lr * (int)rowbytes + ((ls ^ lds_swz<8>(8 + lr)) << 4)};
+    rsrc_words curA, curW, curW2, nextA, nextW, nextW2;
+    int cur_k = 0, gstep = 0;                                // the cursor: byte of the row that is fetched next; steps done by this workgroup
+    // this wave's two transfers of one half of the cursor's step into stage st: 16 rows, 2 KiB that no other wave fills
+    auto issue_half = [&](auto ihalf, int st) {
+        constexpr int h = decltype(ihalf)::value;
+        constexpr bool isA = h < 2;
+        constexpr int q = h & 1;
+        const int row = isA ? wm * 128 + q * 64 + wn * 16 : DUAL ? wave * 16 : (wave >> 1) * 64 + q * 32 + (wave & 1) * 16;
+        const rsrc_words rs = isA ? curA : DUAL && q ? curW2 : curW;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int dst = (int)lds0 + (st & 1) * STAGE + h * HALFB + (wave * 16 + j * 8) * 128;
+            dma16(rs, __builtin_amdgcn_readfirstlane(dst), lane_off[j], cur_k, (row + j * 8) * (int)rowbytes);
+        }
+    };
+    using H_A0 = std::integral_constant<int, 0>; using H_A1 = std::integral_constant<int, 1>; using H_B0 = std::integral_constant<int, 2>; using H_B1 = std::integral_constant<int, 3>;
+    auto advance = [&]() {
+        cur_k += 128;
+        if (cur_k == (int)rowbytes) { cur_k = 0; curA = nextA; curW = nextW; if constexpr (DUAL) curW2 = nextW2; }
+    };
+    // a tile's vectors: up to 1 KiB of `src` from a wave (columns and rows past the end read zero)
+    auto fetch_vec = [&](const float* src, int left, int at, int bytes) {
+        rsrc_words rs = make_rsrc_words(src, left > 0 ? (uint32_t)left : 0u);
+        asm volatile("s_nop 4" : "+s"(rs));             // the wait states behind a vector write of the words, where the compiler kept them in vector registers
+        if (bytes >= 1024 || lane < bytes / 16) dma16(rs, __builtin_amdgcn_readfirstlane((int)lds0 + at), lane * 16, 0, 0);
+    };
+    auto issue_vectors = [&](int m0t, int n0t, int buf) {
+        const int at = VECS + buf * BIASB, cols = (p.N - n0t) * 4, rows = (p.M - m0t) * 8;
+        if (wave == 0 && p.bias) fetch_vec(p.bias + n0t, cols, at, BNO * 4);
+        if (DUAL && wave == 4 && p.bias2) fetch_vec(p.bias2 + n0t, cols, at + BNO * 4, BNO * 4);
+        if constexpr (ROWS) {
+            if (wave == 1) fetch_vec((RL ? p.res_beta : p.ln_c) + n0t, cols, at + COLB, BNO * 4);
+            if (DUAL && wave == 5) fetch_vec(p.ln_c2 + n0t, cols, at + COLB + BNO * 4, BNO * 4);
+            if (p.nparts) {
+                if (wave < p.nparts) {
+                    const float* src = p.parts + 2 * ((int64_t)wave * p.M + m0t);
+                    fetch_vec(src, rows, PARTS_AT + wave * BM * 8, 1024);
+                    fetch_vec(src + 256, rows - 1024, PARTS_AT + wave * BM * 8 + 1024, 1024);
+                }
+            } else if (wave == 7) {
+                const float* src = (RL ? p.res_stats : p.ln_stats) + 2 * (int64_t)m0t;
+                fetch_vec(src, rows, at + 2 * COLB, 1024);
+                fetch_vec(src + 256, rows - 1024, at + 2 * COLB + 1024, 1024);
+            }
+        }
+    };
+    static_assert(GRL_MAX_PARTS <= 8, "a wave per partial");
+
+    OutT* C = (OutT*)p.C;
+    const int rowB = p.N * OES;                             // bytes of an output row
+    const bool staged = ((int64_t)p.N * OES) % 16 == 0 && !p.cache1 && !p.cache2 && (RL || (int64_t)p.N * OES * BM < (1LL << 31));
+    constexpr int UB = WNO * OES >= 128 ? 128 : WNO * OES;  // bytes of a staged row
+    constexpr int UC = UB / OES, GROUPS = WNO / UC, CB = UB / 16, PER = 16 * CB / 64;
+    constexpr int UNITS = 8 * GROUPS, STORES = UNITS * PER; // of a wave per tile
+    static_assert(STORES + 8 < 64, "the memory counter's range");
+
+    int pid = blockIdx.x, m0, n0, bbuf = 0;
+    tile_of(pid, m0, n0);
+    issue_vectors(m0, n0, bbuf);
+    curA = rsrc_of(p.A, m0, p.M); curW = rsrc_of(p.W, n0, p.N);
+    curW2 = DUAL ? rsrc_of(p.W2, n0, p.N) : curW;
+    issue_half(H_B0{}, 0); issue_half(H_A0{}, 0); issue_half(H_B1{}, 0); issue_half(H_A1{}, 0);
+    cur_k = 128;
+    issue_half(H_B0{}, 1); issue_half(H_A0{}, 1); issue_half(H_B1{}, 1);
+    wait_vmcnt<6>();
+    asm volatile("s_barrier" ::: "memory");
+    if (behind) asm volatile("s_barrier" ::: "memory");
+    bool stores_behind = false;                              // the previous tile's stores are behind the transfers that are due next
+    int m0p = 0, n0p = 0;                                    // RL: the previous tile, whose row sums are still to be added
+    bool sums_due = false;
+
+    // RL: {sum, sum of squares} of a tile's rows from those of the four wave columns
+    auto finish_rows = [&](int m0t, int n0t) {
+        if constexpr (RL) {
+            if (wave < 4) {
+                f32x2_t t[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) t[j] = *(const f32x2_t*)(lds + SUMS_AT + (j * BM + tid) * 8);
+                const f32x2_t s = {(t[0][0] + t[1][0]) + (t[2][0] + t[3][0]), (t[0][1] + t[1][1]) + (t[2][1] + t[3][1])};
+                if (m0t + tid < p.M) *(f32x2_t*)(p.part_out + ((int64_t)(n0t / BNO) * p.M + m0t + tid) * 2) = s;
+            }
+        }
+    };
+    // partials of the row statistics, merged in the first step: the same sums in the same order as ln_stats_merge_kernel
+    auto merge_parts = [&] {
+        if constexpr (ROWS) {
+            if (p.nparts && wave < 4) {
+                f32x2_t t[GRL_MAX_PARTS];
+#pragma unroll
+                for (int j = 0; j < GRL_MAX_PARTS; ++j) t[j] = *(const f32x2_t*)(lds + PARTS_AT + (j * BM + tid) * 8);
+                float sum = 0.f, sq = 0.f;
+#pragma unroll
+                for (int j = 0; j < GRL_MAX_PARTS; ++j)
+                    if (j < p.nparts) { sum += t[j][0]; sq += t[j][1]; }
+                const float width = (float)(RL ? p.N : p.K), mean = sum / width;
+                const float sd = sqrtf(fmaxf(sq / width - mean * mean, 0.f) + p.eps);
+                *(f32x2_t*)(lds + VECS + bbuf * BIASB + 2 * COLB + 8 * tid) = f32x2_t{1.0f / sd, mean / sd};
+            }
+        }
+    };
+
+    for (;;) {
+        const int npid = pid + (int)gridDim.x;
+        const bool has_next = npid < ntiles;
+        int m0n = 0, n0n = 0;
+        if (has_next) {
+            tile_of(npid, m0n, n0n);
+            nextA = rsrc_of(p.A, m0n, p.M); nextW = rsrc_of(p.W, n0n, p.N);
+            nextW2 = DUAL ? rsrc_of(p.W2, n0n, p.N) : nextW;
+        } else nextA = nextW = nextW2 = make_rsrc_words(p.A, 0);      // transfers of a next tile that is not there: zeros, nothing is read
+
+        // what every accumulator block starts from: the bias of its columns (and the beta of the norm that the epilogue re-forms on the residual) when
+        // the staged epilogue follows, else zeros (the direct epilogue adds the bias itself; the folded LayerNorm scales the sum before its bias)
+        f32x4 c4[4];
+        static_for<4>([&](auto ic) {
+            constexpr int b = decltype(ic)::value / 2, half = decltype(ic)::value % 2;
+            constexpr bool up = DUAL && b >= TNO;
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+            if (!LN && staged) {
+                const char* bl = lds + VECS + bbuf * BIASB + (wn * WNO + (b % TNO) * 32 + 16 * half + 4 * lq) * 4;
+                if (up ? p.bias2 : p.bias) v = *(const f32x4*)(bl + (up ? BNO * 4 : 0));
+                if constexpr (RL) v += *(const f32x4*)(bl + COLB);
+            }
+            c4[decltype(ic)::value] = v;
+        });
+
+        Acc16<4, 2> blocks;
+        auto& acc = blocks.v;
+        u32x4 fa[4][2], fb[2][2][2];
+        auto step = [&](auto ifirst, int kt) {
+            constexpr bool FIRST = decltype(ifirst)::value;
+            const char* s = lds + (gstep & 1) * STAGE;
+            int lch[2];
+#pragma unroll
+            for (int sl = 0; sl < 2; ++sl) lch[sl] = l4 * 128 + (((4 * sl + lq) ^ lds_swz<8>(l4)) << 4);
+            auto read_a = [&](int q) {
+#pragma unroll
+                for (int sl = 0; sl < 2; ++sl)
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) fa[a][sl] = *(const u32x4*)(s + wm * 8192 + lch[sl] + q * HALFB + a * 2048);
+            };
+            auto read_b = [&](int q) {
+#pragma unroll
+                for (int sl = 0; sl < 2; ++sl)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) fb[q][b][sl] = *(const u32x4*)(s + wn * 4096 + lch[sl] + (2 + q) * HALFB + b * 2048);
+            };
+            auto mfmas = [&](auto iqa) {
+                constexpr int qa = decltype(iqa)::value;
+                __builtin_amdgcn_s_setprio(1);
+                // (in serpentine order: from one instruction to the next an operand stays, 0.5 to 1 % of the products that the power limit bounds)
+                static_for<32>([&](auto it) {
+                    constexpr int t = decltype(it)::value, sl = t / 16, a = t / 4 % 4, b = a & 1 ? 3 - t % 4 : t % 4;
+                    f32x4& to = acc[4 * qa + a][b];
+                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fb[b / 2][b % 2][sl]), __builtin_bit_cast(bf16x8, fa[a][sl]), FIRST && sl == 0 ? c4[b] : to, 0, 0, 0);
+                });
+                __builtin_amdgcn_s_setprio(0);
+            };
+            auto reads_back = [&] {          // the reads of a memory part are back, everybody's behind the barrier
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto meet = [&] {
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto due = [&] {                 // everything but the last eight transfers (and the stores in front of them) has landed
+                if (FIRST && stores_behind) wait_vmcnt<8 + STORES>();
+                else wait_vmcnt<8>();
+            };
+            read_b(0); read_a(0); read_b(1);
+            if (!FIRST && kt == 1 && has_next) issue_vectors(m0n, n0n, bbuf ^ 1);
+            issue_half(H_A1{}, gstep + 1);
+            advance();
+            due();                           // A1 of this step
+            reads_back(); mfmas(std::integral_constant<int, 0>{}); meet();
+            read_a(1);
+            issue_half(H_B0{}, gstep); issue_half(H_A0{}, gstep); issue_half(H_B1{}, gstep);
+            due();                           // B0, A0 and B1 of the next step
+            if constexpr (FIRST) {
+                merge_parts();
+                if (RL && sums_due) finish_rows(m0p, n0p);
+            }
+            reads_back(); mfmas(std::integral_constant<int, 1>{});
+            ++gstep;
+        };
+        step(std::true_type{}, 0);
+        for (int kt = 1; kt < KT; ++kt) {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            step(std::false_type{}, kt);
+        }
+        // the waves in front meet the others' last matrix part here and run their epilogue beside it; the others meet them behind theirs
+        __builtin_amdgcn_sched_barrier(0);
+        if (!behind) asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+
+        if (staged) {
+            char* own = lds + ((gstep - 1) & 1) * STAGE + HALFB + wave * 2048;
+            const char* vec = lds + VECS + bbuf * BIASB;
+            // this lane's 16-byte piece of a staged row: chunk cc of row rr (+ 2 per further read: a read's 8 rows are such that its turns meet no bank twice)
+            const int cc = lane & (CB - 1), rr = CB == 8 ? ((lane >> 4) << 2) + ((lane >> 3) & 1) : lane >> 2;
+            auto tile_rsrc = [&](const void* base) {
+                const int64_t left = ((int64_t)(p.M - m0) * p.N - n0) * OES;
+                return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)base + ((int64_t)m0 * p.N + n0) * OES), 0, left > 0x7fffffff ? 0x7fffffff : (int)left, 0x00020000);
+            };
+            const __amdgpu_buffer_rsrc_t rsC = tile_rsrc(p.C), rsR = tile_rsrc(HASRES ? p.residual : p.C);
+            constexpr int NONTEMPORAL = 2;
+            int coff[GROUPS];
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) {
+                const int col = wn * WNO + g * UC + cc * EPCO;
+                coff[g] = n0 + col < p.N ? (wm * 128 + rr) * rowB + col * OES : (int)0x80000000;
+            }
+            // residual pieces: the memory counter retires in order, so all of them (bf16) are requested in front of the first store
+            constexpr int AHEAD = OES == 2 ? UNITS : 1;
+            u32x4 res[HASRES ? AHEAD : 1][PER];
+            auto fetch_res = [&](auto iu) {
+                constexpr int u = decltype(iu)::value, i = u / GROUPS, g = u % GROUPS;
+                if constexpr (HASRES) {
+#pragma unroll
+                    for (int j = 0; j < PER; ++j) res[u % AHEAD][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsR, coff[g], (16 * i + 2 * j) * rowB, NONTEMPORAL));
+                }
+            };
+            float gq[RL ? EPCO : 1];
+            if constexpr (RL) {
+                const int nq = n0 + wn * WNO + cc * EPCO;          // N is a multiple of the piece here
+#pragma unroll
+                for (int e = 0; e < EPCO; e += 4) {
+                    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+                    const f32x4 gv = nq + e < p.N ? *(const f32x4*)(p.res_gamma + nq + e) : zero;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) gq[e + k] = gv[k];
+                }
+            }
+            if constexpr (AHEAD > 1) static_for<UNITS>([&](auto iu) { fetch_res(iu); });
+            // folded LayerNorm: sum_k LN(x)[m,k] W0[n,k] = rstd_m * acc[m,n] + (b'[n] - rstd_m * mean_m * c[n]), the vectors in registers
+            f32x4 bv[LN ? 4 : 1], cv[LN ? 4 : 1];
+            if constexpr (LN) static_for<4>([&](auto ic) {
+                constexpr int b = decltype(ic)::value / 2, half = decltype(ic)::value % 2;
+                constexpr bool up = DUAL && b >= TNO;
+                const char* bl = vec + (wn * WNO + (b % TNO) * 32 + 16 * half + 4 * lq) * 4 + (up ? BNO * 4 : 0);
+                bv[decltype(ic)::value] = (up ? p.bias2 : p.bias) ? *(const f32x4*)bl : f32x4{0.f, 0.f, 0.f, 0.f};
+                cv[decltype(ic)::value] = *(const f32x4*)(bl + COLB);
+            });
+            static_assert(EPI != EPI_ROPE || (!DUAL && !LN && OES == 2), "a wave's 64 columns are one head");
+            const bool rotated = EPI == EPI_ROPE && n0 + wn * WNO < p.rope_cols;
+            // EPI_ROPE: the two halves of a pair, columns d and d + 32 of a head, are the same register of blocks b and b + 2, so the rotation
+            // stays in registers: four multiply-adds a pair, on the sums before they are rounded.  cos and sin are requested a band ahead.
+            f32x4 cs[EPI == EPI_ROPE ? 2 : 1][2][2];
+            auto fetch_rope = [&](auto ii) {
+                constexpr int i = decltype(ii)::value;
+                if constexpr (EPI == EPI_ROPE) if (rotated) {
+                    const int m = m0 + wm * 128 + 16 * i + l4, mc = m < p.M ? m : p.M - 1;
+                    const float* t = (const float*)p.rope + rope_position(p, mc) * 64 + 8 * lq;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        cs[i & 1][b][0] = *(const f32x4*)(t + 32 * b);
+                        cs[i & 1][b][1] = *(const f32x4*)(t + 32 * b + 4);
+                    }
+                }
+            };
+            fetch_rope(std::integral_constant<int, 0>{});
+            // a unit: 16 rows of 64 or 128 bytes.  convert() writes it to this wave's place, collect() asks for it back, emit() stores it one unit later
+            u32x4 val[2][PER];
+            f32x2_t rst[2][RL ? PER : 1];
+            auto convert = [&](auto iu) {
+                constexpr int u = decltype(iu)::value, i = u / GROUPS, g = u % GROUPS;
+                if constexpr (g == 0 && i + 1 < 8) fetch_rope(std::integral_constant<int, i + 1>{});
+                if constexpr (AHEAD == 1) fetch_res(iu);
+                float rs = 1.f, rm = 0.f;
+                if constexpr (LN) {
+                    const f32x2_t st = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * 128 + 16 * i + l4));
+                    rs = st[0]; rm = st[1];
+                }
+                auto put = [&](int b, const float (&v)[4]) {          // four columns of block b of the unit
+                    const int byte = (16 * b + 4 * lq) * OES;
+                    store4<OutT>((OutT*)(own + l4 * UB + (((byte >> 4) ^ lds_swz<CB>(l4)) << 4) + (byte & 15)), v[0], v[1], v[2], v[3]);
+                };
+                if constexpr (EPI == EPI_ROPE) {
+                    static_for<2>([&](auto ib) {
+                        constexpr int b = decltype(ib)::value;
+                        float v[4], w[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) { v[e] = acc[i][b][e]; w[e] = acc[i][b + 2][e]; }
+                        if (rotated) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float co = cs[i & 1][b][e >> 1][2 * (e & 1)], si = cs[i & 1][b][e >> 1][2 * (e & 1) + 1], x = v[e], y = w[e];
+                                v[e] = x * co - y * si;
+                                w[e] = y * co + x * si;
+                            }
+                        }
+                        put(b, v);
+                        put(b + 2, w);
+                    });
+                } else
+                static_for<UC / 16>([&](auto ib) {
+                    constexpr int b = g * (UC / 16) + decltype(ib)::value, b2 = DUAL ? b + 2 : b;
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = LN ? fmaf(acc[i][b][e], rs, fmaf(-rm, cv[LN ? b : 0][e], bv[LN ? b : 0][e])) : acc[i][b][e];
+                    if constexpr (DUAL) {
+                        float up[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) up[e] = LN ? fmaf(acc[i][b2][e], rs, fmaf(-rm, cv[LN ? b2 : 0][e], bv[LN ? b2 : 0][e])) : acc[i][b2][e];
+                        glu_apply4(v, up, p);
+                    } else if constexpr (EPI == EPI_GELU) gelu_fast4(v);
+                    else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = epi_apply<EPI>(v[e], p);
+                    }
+                    put(decltype(ib)::value, v);
+                });
+            };
+            // (a wave's LDS accesses are done in order: these reads see the unit's writes, and the next unit's writes come behind them)
+            auto collect = [&](auto iu) {
+                constexpr int u = decltype(iu)::value, i = u / GROUPS;
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    const int r = rr + 2 * j;
+                    val[u & 1][j] = *(const u32x4*)(own + r * UB + ((cc ^ lds_swz<CB>(r)) << 4));
+                    if constexpr (RL) rst[u & 1][j] = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * 128 + 16 * i + r));
+                }
+                asm volatile("" ::: "memory");
+            };
+            auto emit = [&](auto iu) {
+                constexpr int u = decltype(iu)::value, i = u / GROUPS, g = u % GROUPS;
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    u32x4 out = val[u & 1][j];
+                    if constexpr (EPI == EPI_RES) out = add_chunk<OutT>(out, res[u % AHEAD][j]);
+                    if constexpr (RL) {
+                        float xr[EPCO], o[EPCO];
+                        Chunk<OutT>::unpack(res[u % AHEAD][j], xr);
+                        Chunk<OutT>::unpack(out, o);
+                        float sum = 0.f, sq = 0.f;
+#pragma unroll
+                        for (int e = 0; e < EPCO; ++e) o[e] = fmaf(fmaf(xr[e], rst[u & 1][j][0], -rst[u & 1][j][1]), gq[e], o[e]);
+                        out = Chunk<OutT>::pack(o);
+                        // (columns past N contribute 0: gamma, beta, bias and the products are 0 there)
+                        Chunk<OutT>::moments(out, o, sum, sq);
+                        sum += dpp_move<0xb1>(sum); sq += dpp_move<0xb1>(sq);            // quad_perm 1,0,3,2
+                        sum += dpp_move<0x4e>(sum); sq += dpp_move<0x4e>(sq);            // quad_perm 2,3,0,1
+                        sum += dpp_move<0x141>(sum); sq += dpp_move<0x141>(sq);          // row_half_mirror
+                        if (cc == 0) *(f32x2_t*)(lds + SUMS_AT + wn * BM * 8 + 8 * (wm * 128 + 16 * i + rr + 2 * j)) = f32x2_t{sum, sq};
+                    }
+                    // (the row's offset is added to the lane's, not passed as the scalar one: a VALU instruction right behind a four-word store may
+                    // overwrite its data before the last lanes' is read; the compiler puts a wait state between them only where the scalar offset is
+                    // zero, and without one elements came out wrong)
+                    // written once, read by another kernel: keep it from displacing the operand panels in L2
+                    __builtin_amdgcn_raw_buffer_store_b128(out, rsC, coff[g] + (16 * i + 2 * j) * rowB, 0, NONTEMPORAL);
+                }
+            };
+            convert(std::integral_constant<int, 0>{});
+            collect(std::integral_constant<int, 0>{});
+            static_for<UNITS>([&](auto iu) {
+                constexpr int u = decltype(iu)::value;
+                if constexpr (u + 1 < UNITS) {
+                    convert(std::integral_constant<int, u + 1>{});
+                    collect(std::integral_constant<int, u + 1>{});
+                }
+                emit(iu);
+            });
+        } else if constexpr (!RL && EPI != EPI_ROPE) {        // EPI_RESLN and EPI_ROPE exist in the staged form only: the host launches them for nothing else
+            epilogue_direct<OutT, 4, 2, TNO, 128, WNO, EPI, DUAL, LN>(blocks, p, m0, n0, wm, wn, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (behind) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        stores_behind = staged;
+        m0p = m0; n0p = n0; sums_due = true;
+        if (!has_next) break;
+        pid = npid; m0 = m0n; n0 = n0n; bbuf ^= 1;
+    }
+    if (!behind) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    finish_rows(m0p, n0p);
+    wait_vmcnt<0>();                     // no transfer may be on its way to LDS that is somebody else's
+}
