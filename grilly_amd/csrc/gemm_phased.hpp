@@ -10,6 +10,8 @@
 //   memory part 0: reads B0, A0, B1 of step t;  requests A1 of step t + 1;          matrix part 0: rows of A0
 //   memory part 1: reads A1 of step t;          requests B0, A0, B1 of step t + 2;  matrix part 1: rows of A1
 //
+// (X and Y below: Y is the operand whose halves are multiplied in turn, A, and X the other; with EPI_RESLN they change places.)
+//
 // A memory part ends when its reads are back, so a half is requested again one part after its last read, and is due six parts later: 64 to
 // 96 KiB are in flight all the time.  The cursor runs on into the next tile, so nothing drains between tiles: the epilogue stands between
 // the last matrix part and the next tile's first memory part, and only A1 of the last step's stage is not being refilled then.  There,
@@ -28,7 +30,11 @@
 
 template <typename OutT, int EPI, bool DUAL, bool LN = false>
 __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
-    constexpr int BM = 256, BN = 256, BNO = DUAL ? BN / 2 : BN, WNO = BNO / 4, TNO = WNO / 32;
+    // A wave's share of the tile: 128 rows x 64 columns.  The row sums of EPI_RESLN are added chunk by chunk in the order of the 32 lanes that hold
+    // a row of 256 columns elsewhere (c with c + 8, + 4, + 2, + 1, the halves last), which needs 128 columns of a row in one wave: 64 rows x
+    // 128 columns there, weights and activations in each other's part.
+    constexpr bool TR = EPI == EPI_RESLN;
+    constexpr int BM = 256, BN = 256, BNO = DUAL ? BN / 2 : BN, WM = TR ? 64 : 128, WNO = TR ? 128 : BNO / 4, TNO = WNO / 32;
     constexpr int HALFB = 128 * 128, STAGE = 4 * HALFB;
     constexpr int OES = (int)sizeof(OutT), EPCO = 16 / OES;
     constexpr bool RL = EPI == EPI_RESLN;                   // LayerNorm(residual) formed in the epilogue + row statistics out
@@ -37,11 +43,11 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     // tile's 256 row-statistics pairs.  Two buffers, alternating per tile.
     constexpr int VECS = 2 * STAGE, COLB = BN * 4, BIASB = ROWS ? 2 * COLB + BM * 8 : COLB;
     constexpr int PARTS_AT = VECS + 2 * BIASB, SUMS_AT = PARTS_AT + (ROWS ? GRL_MAX_PARTS * BM * 8 : 0);
-    __shared__ __attribute__((aligned(1024))) char lds[SUMS_AT + (RL ? 4 * BM * 8 : 0)];
+    __shared__ __attribute__((aligned(1024))) char lds[SUMS_AT + (RL ? 2 * BM * 8 : 0)];
     static_assert(!(LN && RL) && !(RL && DUAL) && !(HASRES && DUAL), "one set of row statistics per tile");
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 2, wn = wave & 3, l4 = lane & 15, lq = lane >> 4;
+    const int wm = TR ? wave >> 1 : wave >> 2, wn = TR ? wave & 1 : wave & 3, l4 = lane & 15, lq = lane >> 4;
     const bool behind = wave >= 4;                           // the waves that run one part behind
     const int ntiles = p.tiles_m * p.tiles_n;
     const int64_t rowbytes = (int64_t)p.K * 2;
@@ -71,9 +77,9 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     // this wave's two transfers of one half of the cursor's step into stage st: 16 rows, 2 KiB that no other wave fills
     auto issue_half = [&](auto ihalf, int st) {
         constexpr int h = decltype(ihalf)::value;
-        constexpr bool isA = h < 2;
+        constexpr bool isA = (h < 2) != TR;
         constexpr int q = h & 1;
-        const int row = isA ? wm * 128 + q * 64 + wn * 16 : DUAL ? wave * 16 : (wave >> 1) * 64 + q * 32 + (wave & 1) * 16;
+        const int row = h < 2 ? (wave >> 2) * 128 + q * 64 + (wave & 3) * 16 : DUAL ? wave * 16 : (wave >> 1) * 64 + q * 32 + (wave & 1) * 16;
         const rsrc_words rs = isA ? curA : DUAL && q ? curW2 : curW;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -81,7 +87,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
             dma16(rs, __builtin_amdgcn_readfirstlane(dst), lane_off[j], cur_k, (row + j * 8) * (int)rowbytes);
         }
     };
-    using H_A0 = std::integral_constant<int, 0>; using H_A1 = std::integral_constant<int, 1>; using H_B0 = std::integral_constant<int, 2>; using H_B1 = std::integral_constant<int, 3>;
+    using H_Y0 = std::integral_constant<int, 0>; using H_Y1 = std::integral_constant<int, 1>; using H_X0 = std::integral_constant<int, 2>; using H_X1 = std::integral_constant<int, 3>;
     auto advance = [&]() {
         cur_k += 128;
         if (cur_k == (int)rowbytes) { cur_k = 0; curA = nextA; curW = nextW; if constexpr (DUAL) curW2 = nextW2; }
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     const bool staged = ((int64_t)p.N * OES) % 16 == 0 && !p.cache1 && !p.cache2 && (RL || (int64_t)p.N * OES * BM < (1LL << 31));
     constexpr int UB = WNO * OES >= 128 ? 128 : WNO * OES;  // bytes of a staged row
     constexpr int UC = UB / OES, GROUPS = WNO / UC, CB = UB / 16, PER = 16 * CB / 64;
-    constexpr int UNITS = 8 * GROUPS, STORES = UNITS * PER; // of a wave per tile
+    constexpr int UNITS = WM / 16 * GROUPS, STORES = UNITS * PER; // of a wave per tile
     static_assert(STORES + 8 < 64, "the memory counter's range");
 
     int pid = blockIdx.x, m0, n0, bbuf = 0;
@@ -127,9 +133,9 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     issue_vectors(m0, n0, bbuf);
     curA = rsrc_of(p.A, m0, p.M); curW = rsrc_of(p.W, n0, p.N);
     curW2 = DUAL ? rsrc_of(p.W2, n0, p.N) : curW;
-    issue_half(H_B0{}, 0); issue_half(H_A0{}, 0); issue_half(H_B1{}, 0); issue_half(H_A1{}, 0);
+    issue_half(H_X0{}, 0); issue_half(H_Y0{}, 0); issue_half(H_X1{}, 0); issue_half(H_Y1{}, 0);
     cur_k = 128;
-    issue_half(H_B0{}, 1); issue_half(H_A0{}, 1); issue_half(H_B1{}, 1);
+    issue_half(H_X0{}, 1); issue_half(H_Y0{}, 1); issue_half(H_X1{}, 1);
     wait_vmcnt<6>();
     asm volatile("s_barrier" ::: "memory");
     if (behind) asm volatile("s_barrier" ::: "memory");
@@ -137,15 +143,12 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     int m0p = 0, n0p = 0;                                    // RL: the previous tile, whose row sums are still to be added
     bool sums_due = false;
 
-    // RL: {sum, sum of squares} of a tile's rows from those of the four wave columns
+    // RL: {sum, sum of squares} of a tile's rows from those of the two wave columns
     auto finish_rows = [&](int m0t, int n0t) {
         if constexpr (RL) {
             if (wave < 4) {
-                f32x2_t t[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) t[j] = *(const f32x2_t*)(lds + SUMS_AT + (j * BM + tid) * 8);
-                const f32x2_t s = {(t[0][0] + t[1][0]) + (t[2][0] + t[3][0]), (t[0][1] + t[1][1]) + (t[2][1] + t[3][1])};
-                if (m0t + tid < p.M) *(f32x2_t*)(p.part_out + ((int64_t)(n0t / BNO) * p.M + m0t + tid) * 2) = s;
+                const f32x2_t t = *(const f32x2_t*)(lds + SUMS_AT + tid * 8), u = *(const f32x2_t*)(lds + SUMS_AT + (BM + tid) * 8);
+                if (m0t + tid < p.M) *(f32x2_t*)(p.part_out + ((int64_t)(n0t / BNO) * p.M + m0t + tid) * 2) = f32x2_t{t[0] + u[0], t[1] + u[1]};
             }
         }
     };
@@ -180,47 +183,51 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
         // what every accumulator block starts from: the bias of its columns (and the beta of the norm that the epilogue re-forms on the residual) when
         // the staged epilogue follows, else zeros (the direct epilogue adds the bias itself; the folded LayerNorm scales the sum before its bias)
         f32x4 c4[4];
-        static_for<4>([&](auto ic) {
-            constexpr int b = decltype(ic)::value / 2, half = decltype(ic)::value % 2;
-            constexpr bool up = DUAL && b >= TNO;
-            f32x4 v = {0.f, 0.f, 0.f, 0.f};
-            if (!LN && staged) {
-                const char* bl = lds + VECS + bbuf * BIASB + (wn * WNO + (b % TNO) * 32 + 16 * half + 4 * lq) * 4;
-                if (up ? p.bias2 : p.bias) v = *(const f32x4*)(bl + (up ? BNO * 4 : 0));
-                if constexpr (RL) v += *(const f32x4*)(bl + COLB);
-            }
-            c4[decltype(ic)::value] = v;
-        });
+        auto start_values = [&](auto iq) {                   // (TR: a phase has columns of its own)
+            static_for<4>([&](auto ic) {
+                constexpr int c = decltype(ic)::value + (TR ? 4 * decltype(iq)::value : 0), b = c / 2, half = c % 2;
+                constexpr bool up = DUAL && b >= TNO;
+                f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                if (!LN && staged) {
+                    const char* bl = lds + VECS + bbuf * BIASB + (wn * WNO + (b % TNO) * 32 + 16 * half + 4 * lq) * 4;
+                    if (up ? p.bias2 : p.bias) v = *(const f32x4*)(bl + (up ? BNO * 4 : 0));
+                    if constexpr (RL) v += *(const f32x4*)(bl + COLB);
+                }
+                c4[decltype(ic)::value] = v;
+            });
+        };
+        start_values(std::integral_constant<int, 0>{});
 
-        Acc16<4, 2> blocks;
+        Acc16<WM / 32, TR ? 4 : 2> blocks;
         auto& acc = blocks.v;
-        u32x4 fa[4][2], fb[2][2][2];
+        u32x4 fy[4][2], fx[2][2][2];
         auto step = [&](auto ifirst, int kt) {
             constexpr bool FIRST = decltype(ifirst)::value;
             const char* s = lds + (gstep & 1) * STAGE;
             int lch[2];
 #pragma unroll
             for (int sl = 0; sl < 2; ++sl) lch[sl] = l4 * 128 + (((4 * sl + lq) ^ lds_swz<8>(l4)) << 4);
-            auto read_a = [&](int q) {
+            auto read_y = [&](int q) {
 #pragma unroll
                 for (int sl = 0; sl < 2; ++sl)
 #pragma unroll
-                    for (int a = 0; a < 4; ++a) fa[a][sl] = *(const u32x4*)(s + wm * 8192 + lch[sl] + q * HALFB + a * 2048);
+                    for (int y = 0; y < 4; ++y) fy[y][sl] = *(const u32x4*)(s + (TR ? wn : wm) * 8192 + lch[sl] + q * HALFB + y * 2048);
             };
-            auto read_b = [&](int q) {
+            auto read_x = [&](int q) {
 #pragma unroll
                 for (int sl = 0; sl < 2; ++sl)
 #pragma unroll
-                    for (int b = 0; b < 2; ++b) fb[q][b][sl] = *(const u32x4*)(s + wn * 4096 + lch[sl] + (2 + q) * HALFB + b * 2048);
+                    for (int x = 0; x < 2; ++x) fx[q][x][sl] = *(const u32x4*)(s + (TR ? wm : wn) * 4096 + lch[sl] + (2 + q) * HALFB + x * 2048);
             };
-            auto mfmas = [&](auto iqa) {
-                constexpr int qa = decltype(iqa)::value;
+            auto mfmas = [&](auto iq) {
+                constexpr int q = decltype(iq)::value;
                 __builtin_amdgcn_s_setprio(1);
                 // (in serpentine order: from one instruction to the next an operand stays, 0.5 to 1 % of the products that the power limit bounds)
                 static_for<32>([&](auto it) {
-                    constexpr int t = decltype(it)::value, sl = t / 16, a = t / 4 % 4, b = a & 1 ? 3 - t % 4 : t % 4;
-                    f32x4& to = acc[4 * qa + a][b];
-                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fb[b / 2][b % 2][sl]), __builtin_bit_cast(bf16x8, fa[a][sl]), FIRST && sl == 0 ? c4[b] : to, 0, 0, 0);
+                    constexpr int t = decltype(it)::value, sl = t / 16, y = t / 4 % 4, x = y & 1 ? 3 - t % 4 : t % 4;
+                    f32x4& to = acc[TR ? x : 4 * q + y][TR ? 4 * q + y : x];
+                    const u32x4 &weights = TR ? fy[y][sl] : fx[x / 2][x % 2][sl], &rows = TR ? fx[x / 2][x % 2][sl] : fy[y][sl];
+                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, weights), __builtin_bit_cast(bf16x8, rows), FIRST && sl == 0 ? c4[TR ? y : x] : to, 0, 0, 0);
                 });
                 __builtin_amdgcn_s_setprio(0);
             };
@@ -238,14 +245,15 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                 if (FIRST && stores_behind) wait_vmcnt<8 + STORES>();
                 else wait_vmcnt<8>();
             };
-            read_b(0); read_a(0); read_b(1);
+            read_x(0); read_y(0); read_x(1);
             if (!FIRST && kt == 1 && has_next) issue_vectors(m0n, n0n, bbuf ^ 1);
-            issue_half(H_A1{}, gstep + 1);
+            issue_half(H_Y1{}, gstep + 1);
             advance();
             due();                           // A1 of this step
             reads_back(); mfmas(std::integral_constant<int, 0>{}); meet();
-            read_a(1);
-            issue_half(H_B0{}, gstep); issue_half(H_A0{}, gstep); issue_half(H_B1{}, gstep);
+            read_y(1);
+            if constexpr (TR && FIRST) start_values(std::integral_constant<int, 1>{});
+            issue_half(H_X0{}, gstep); issue_half(H_Y0{}, gstep); issue_half(H_X1{}, gstep);
             due();                           // B0, A0 and B1 of the next step
             if constexpr (FIRST) {
                 merge_parts();
@@ -281,7 +289,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
 #pragma unroll
             for (int g = 0; g < GROUPS; ++g) {
                 const int col = wn * WNO + g * UC + cc * EPCO;
-                coff[g] = n0 + col < p.N ? (wm * 128 + rr) * rowB + col * OES : (int)0x80000000;
+                coff[g] = n0 + col < p.N ? (wm * WM + rr) * rowB + col * OES : (int)0x80000000;
             }
             // residual pieces: the memory counter retires in order, so all of them (bf16) are requested in front of the first store
             constexpr int AHEAD = OES == 2 ? UNITS : 1;
@@ -293,18 +301,21 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                     for (int j = 0; j < PER; ++j) res[u % AHEAD][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsR, coff[g], (16 * i + 2 * j) * rowB, NONTEMPORAL));
                 }
             };
-            float gq[RL ? EPCO : 1];
-            if constexpr (RL) {
-                const int nq = n0 + wn * WNO + cc * EPCO;          // N is a multiple of the piece here
+            float gq[RL ? GROUPS : 1][RL ? EPCO : 1];
+            if constexpr (RL) static_for<GROUPS>([&](auto ig) {
+                constexpr int g = decltype(ig)::value;
+                const int nq = n0 + wn * WNO + g * UC + cc * EPCO;          // N is a multiple of the piece here
 #pragma unroll
                 for (int e = 0; e < EPCO; e += 4) {
                     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
                     const f32x4 gv = nq + e < p.N ? *(const f32x4*)(p.res_gamma + nq + e) : zero;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) gq[e + k] = gv[k];
+                    for (int k = 0; k < 4; ++k) gq[g][e + k] = gv[k];
                 }
-            }
+            });
             if constexpr (AHEAD > 1) static_for<UNITS>([&](auto iu) { fetch_res(iu); });
+            static_assert(!RL || (GROUPS == 2 && CB == 8), "a row's 16 pieces: 8 lanes, two units");
+            float held[RL ? PER : 1][2];                      // RL: the sums of the first unit's pieces of a row
             // folded LayerNorm: sum_k LN(x)[m,k] W0[n,k] = rstd_m * acc[m,n] + (b'[n] - rstd_m * mean_m * c[n]), the vectors in registers
             f32x4 bv[LN ? 4 : 1], cv[LN ? 4 : 1];
             if constexpr (LN) static_for<4>([&](auto ic) {
@@ -322,7 +333,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
             auto fetch_rope = [&](auto ii) {
                 constexpr int i = decltype(ii)::value;
                 if constexpr (EPI == EPI_ROPE) if (rotated) {
-                    const int m = m0 + wm * 128 + 16 * i + l4, mc = m < p.M ? m : p.M - 1;
+                    const int m = m0 + wm * WM + 16 * i + l4, mc = m < p.M ? m : p.M - 1;
                     const float* t = (const float*)p.rope + rope_position(p, mc) * 64 + 8 * lq;
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
@@ -341,7 +352,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                 if constexpr (AHEAD == 1) fetch_res(iu);
                 float rs = 1.f, rm = 0.f;
                 if constexpr (LN) {
-                    const f32x2_t st = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * 128 + 16 * i + l4));
+                    const f32x2_t st = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * WM + 16 * i + l4));
                     rs = st[0]; rm = st[1];
                 }
                 auto put = [&](int b, const float (&v)[4]) {          // four columns of block b of the unit
@@ -392,7 +403,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                 for (int j = 0; j < PER; ++j) {
                     const int r = rr + 2 * j;
                     val[u & 1][j] = *(const u32x4*)(own + r * UB + ((cc ^ lds_swz<CB>(r)) << 4));
-                    if constexpr (RL) rst[u & 1][j] = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * 128 + 16 * i + r));
+                    if constexpr (RL) rst[u & 1][j] = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * WM + 16 * i + r));
                 }
                 asm volatile("" ::: "memory");
             };
@@ -408,14 +419,21 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                         Chunk<OutT>::unpack(out, o);
                         float sum = 0.f, sq = 0.f;
 #pragma unroll
-                        for (int e = 0; e < EPCO; ++e) o[e] = fmaf(fmaf(xr[e], rst[u & 1][j][0], -rst[u & 1][j][1]), gq[e], o[e]);
+                        for (int e = 0; e < EPCO; ++e) o[e] = fmaf(fmaf(xr[e], rst[u & 1][j][0], -rst[u & 1][j][1]), gq[g][e], o[e]);
                         out = Chunk<OutT>::pack(o);
                         // (columns past N contribute 0: gamma, beta, bias and the products are 0 there)
                         Chunk<OutT>::moments(out, o, sum, sq);
-                        sum += dpp_move<0xb1>(sum); sq += dpp_move<0xb1>(sq);            // quad_perm 1,0,3,2
-                        sum += dpp_move<0x4e>(sum); sq += dpp_move<0x4e>(sq);            // quad_perm 2,3,0,1
-                        sum += dpp_move<0x141>(sum); sq += dpp_move<0x141>(sq);          // row_half_mirror
-                        if (cc == 0) *(f32x2_t*)(lds + SUMS_AT + wn * BM * 8 + 8 * (wm * 128 + 16 * i + rr + 2 * j)) = f32x2_t{sum, sq};
+                        if constexpr (g == 0) { held[j][0] = sum; held[j][1] = sq; }
+                        else {
+                            auto over_row = [](float a, float b) {          // piece c with c + 8, then + 4, + 2, + 1
+                                float v = a + b;
+                                v += dpp_move<0x1b>(dpp_move<0x141>(v));     // row_half_mirror, quad_perm 3,2,1,0: lane ^ 4
+                                v += dpp_move<0x4e>(v);                      // quad_perm 2,3,0,1
+                                return v + dpp_move<0xb1>(v);                // quad_perm 1,0,3,2
+                            };
+                            sum = over_row(held[j][0], sum); sq = over_row(held[j][1], sq);
+                            if (cc == 0) *(f32x2_t*)(lds + SUMS_AT + wn * BM * 8 + 8 * (wm * WM + 16 * i + rr + 2 * j)) = f32x2_t{sum, sq};
+                        }
                     }
                     // (the row's offset is added to the lane's, not passed as the scalar one: a VALU instruction right behind a four-word store may
                     // overwrite its data before the last lanes' is read; the compiler puts a wait state between them only where the scalar offset is
@@ -435,7 +453,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                 emit(iu);
             });
         } else if constexpr (!RL && EPI != EPI_ROPE) {        // EPI_RESLN and EPI_ROPE exist in the staged form only: the host launches them for nothing else
-            epilogue_direct<OutT, 4, 2, TNO, 128, WNO, EPI, DUAL, LN>(blocks, p, m0, n0, wm, wn, lane);
+            epilogue_direct<OutT, 4, 2, TNO, WM, WNO, EPI, DUAL, LN>(blocks, p, m0, n0, wm, wn, lane);
         }
         __builtin_amdgcn_sched_barrier(0);
         if (behind) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
