@@ -291,8 +291,9 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                 const int col = wn * WNO + g * UC + cc * EPCO;
                 coff[g] = n0 + col < p.N ? (wm * WM + rr) * rowB + col * OES : (int)0x80000000;
             }
-            // residual pieces: the memory counter retires in order, so all of them (bf16) are requested in front of the first store
-            constexpr int AHEAD = OES == 2 ? UNITS : 1;
+            // residual pieces: the memory counter retires in order, so all of them (bf16; fp32: a unit's, a unit ahead) are requested in front of the first store
+            constexpr bool AT_ONCE = OES == 2;
+            constexpr int AHEAD = AT_ONCE ? UNITS : 2;
             u32x4 res[HASRES ? AHEAD : 1][PER];
             auto fetch_res = [&](auto iu) {
                 constexpr int u = decltype(iu)::value, i = u / GROUPS, g = u % GROUPS;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
                     for (int k = 0; k < 4; ++k) gq[g][e + k] = gv[k];
                 }
             });
-            if constexpr (AHEAD > 1) static_for<UNITS>([&](auto iu) { fetch_res(iu); });
+            if constexpr (AT_ONCE) static_for<UNITS>([&](auto iu) { fetch_res(iu); });
             static_assert(!RL || (GROUPS == 2 && CB == 8), "a row's 16 pieces: 8 lanes, two units");
             float held[RL ? PER : 1][2];                      // RL: the sums of the first unit's pieces of a row
             // folded LayerNorm: sum_k LN(x)[m,k] W0[n,k] = rstd_m * acc[m,n] + (b'[n] - rstd_m * mean_m * c[n]), the vectors in registers
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
             auto convert = [&](auto iu) {
                 constexpr int u = decltype(iu)::value, i = u / GROUPS, g = u % GROUPS;
                 if constexpr (g == 0 && i + 1 < 8) fetch_rope(std::integral_constant<int, i + 1>{});
-                if constexpr (AHEAD == 1) fetch_res(iu);
+                if constexpr (!AT_ONCE) fetch_res(iu);
                 float rs = 1.f, rm = 0.f;
                 if constexpr (LN) {
                     const f32x2_t st = *(const f32x2_t*)(vec + 2 * COLB + 8 * (wm * WM + 16 * i + l4));

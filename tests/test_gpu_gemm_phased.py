@@ -134,3 +134,22 @@ def test_folded_rows_far_from_zero(backend):
     y = lnl.ln_linear(backend, "bf16", x, g, bt, W, b, 1e-5)[0]
     assert np.isfinite(y).all()
     assert O.max_rel(y[r], O.truth_linear(O.truth_layernorm(x[r], g, bt, 1e-5), W, b)) < TOL_BF16
+
+
+@pytest.mark.parametrize("slabs", [2, 5])
+def test_residual_of_fp32_results(backend, slabs):
+    """bf16 operands, an fp32 residual and fp32 results (in place): every unit of a tile's output gets its own residual.  Tolerance: fp32 sums
+    of K products, 2^-23 * K of the largest."""
+    c, B, K = backend.core, L.GRL_BF16, 64 * slabs
+    rng = np.random.default_rng(slabs)
+    x, w = O.bf16_round(rng.standard_normal((M, K), dtype=np.float32)), O.bf16_round((rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32))
+    b, res, r = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N), dtype=np.float32), rows_of(rng)
+    bufs = [c.upload(x, B), c.upload(w, B), c.upload(b), c.upload(res)]
+    try:
+        dx, dw, db, dy = bufs
+        L.check(c.lib.grl_gemm_nt_res(c.ctx, B, L.GRL_F32, M, N, K, dx.ptr, dw.ptr, db.ptr, dy.ptr, dy.ptr), "gemm_nt_res")
+        ref = O.truth_linear(x[r], w, b) + res[r].astype(np.float64)
+        assert O.max_rel(c.download(dy, (M, N))[r], ref) < K * 2.0 ** -23
+    finally:
+        for t in bufs:
+            t.free()
