@@ -155,11 +155,16 @@ __global__ __launch_bounds__(NW * 64, OCC) void fa2_bf16_kernel(Fa16Args p) {
     else if (p.causal) { bh = lin / nqb; qb = nqb - 1 - lin % nqb; }
     else { qb = lin % nqb; bh = lin / nqb; }
     qb = uni(qb); bh = uni(bh);
-    const int b = uni(bh / p.H), h = uni(bh % p.H);
+    int b = uni(bh / p.H);
+    const int h = uni(bh % p.H);
+    static_assert(ROPE_Q != 0 || HAS_MASK || (TILE >= 4 * (FA_MOST_RANKED + 4) && NT >= FA_MOST_RANKED), "room to rank the sequences");
     const int q0 = qb * QB;
     const int qw0 = q0 + wave * QW;
     int64_t row0; int S;
-    fa_sequence(p.offsets, b, p.S, row0, S);
+    bool ranked = false;
+    if constexpr (ROPE_Q == 0 && !HAS_MASK) ranked = (p.order & 8) && p.offsets && p.B <= FA_MOST_RANKED && p.S <= 65536;
+    if (ranked) fa_ranked<NT>(p.offsets, p.B, b, (int*)(lds + OFF_V + (NSTG - 1) * TILE), b, row0, S);
+    else fa_sequence(p.offsets, b, p.S, row0, S);
     if (q0 >= S) return;
     const uint16_t* Qg = p.Q + row0 * p.q_stride + h * D;
 
@@ -705,7 +710,7 @@ static int launch_fa16(grl_ctx* c, const FaArgs& a, int rope_q) {
     f.mask = a.mask; f.O = (uint16_t*)a.O; f.rope = a.rope; f.offsets = a.offsets;
     f.B = a.B; f.S = a.S; f.H = a.H; f.scale = a.scale; f.causal = a.causal;
     static const int order_env = [] { const char* e = getenv("GRL_FA_ORDER"); return e ? atoi(e) : -1; }();
-    f.order = order_env >= 0 ? fa_order_checked(order_env) : fa_order(a.causal, a.S, a.offsets && !a.mask && rope_q == 0, (int64_t)a.B * a.H, D);
+    f.order = order_env >= 0 ? fa_order_checked(order_env) : fa_order_ranked(fa_order(a.causal, a.S, a.offsets && !a.mask && rope_q == 0, (int64_t)a.B * a.H, D), a.S, a.B, (int64_t)a.B * a.H * ((a.S + 127) / 128));
     f.q_stride = a.q_stride; f.k_stride = a.k_stride; f.v_stride = a.v_stride; f.o_stride = a.o_stride;
     // GRL_FA_CFG forces a configuration, for tuning runs:
     //   1: 8 waves, 64-key tiles, deep ring   2: 8 waves, 128-key tiles   3: 4 waves, 64-key tiles, 4 stages (head dims up to 64)

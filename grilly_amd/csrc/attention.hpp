@@ -17,8 +17,10 @@ struct FaArgs {
 };
 
 // Workgroup numbering of the bf16 kernel, bits: 1 XCD-contiguous runs of ids, 2 the heaviest query blocks of all heads first, 4 heads dealt out to
-// the XCDs in turn (in place of 1: mixed, some heads would be computed twice and others never).
-static inline int fa_order_checked(int order) { return order & 4 ? order & 6 : order & 3; }
+// the XCDs in turn (in place of 1: mixed, some heads would be computed twice and others never), 8 (ragged batches, on top of 4) the longest
+// sequences first.
+static inline int fa_order_checked(int order) { return order & 4 ? order & 14 : order & 3; }
+constexpr int FA_MOST_RANKED = 32;        // sequences of a batch that a workgroup ranks by length
 // Measured: causal and short sequences do best head by head on XCD-contiguous runs; long dense sequences with the plain id order (32 CUs of
 // an XCD streaming the same K/V tiles in lockstep miss L2 together).
 // Ragged batches (without mask and rotation: see the kernel): heads dealt out.  A contiguous run per XCD gives an XCD six sequences of a
@@ -30,6 +32,16 @@ static inline int fa_order(bool causal, int64_t S, bool ragged, int64_t heads, i
     if (ragged && D >= 64 && heads >= 64 && S <= 1024) return 4;
     return causal || S <= 1024 ? 1 : 0;
 }
+// Dealt-out ragged batches of few long sequences: the longest first.  Their workgroups (`blocks`, empty ones counted) are all resident at
+// once, so a launch lasts as long as the CU that was dealt the most work; by falling length the deal comes out nearly even.  Every
+// workgroup ranks the sequences for itself, 0.3 to 0.5 us.  us, in batch order -> ranked, lengths uniform from an eighth to all of S:
+// 32 x 300 x 12 heads of 64 17.7 -> 14.2, 16 x 512 x 12 17.3 -> 16.2, 24 x 900 x 8 42.5 -> 39.7, 32 x 400 x 8 heads of 128 36.7 -> 33.5; over 30
+// batches of 300 to 900 5 % on the mean (0.80 to 1.02).  Where the line leaves off: fewer blocks than 2.5 per CU are no deal
+// (10 x 512 x 8 12.1 -> 13.1), short sequences lose the ranking's time (24 x 200 x 12 11.3 -> 11.5), and of many blocks or sequences
+// the later ones fill the gaps as they come (64 x 512 x 12 49.9 -> 52.6, 32 x 900 x 16 73.2 -> 74.5).
+static inline int fa_order_ranked(int order, int64_t S, int64_t B, int64_t blocks) {
+    return order == 4 && S > 256 && B > 1 && B <= FA_MOST_RANKED && blocks >= 640 && blocks <= 3072 ? 12 : order;
+}
 // Where workgroup `id` of nwg = nqb * nbh stands in the walk.  DEAL: the heads that make whole turns of eight are dealt out, the query blocks
 // of one head next to each other on one XCD; the rest keep their ids.
 template <bool DEAL> __host__ __device__ __forceinline__ int fa_place(int order, int id, int nwg, int nqb, int nbh) {
@@ -39,6 +51,8 @@ template <bool DEAL> __host__ __device__ __forceinline__ int fa_place(int order,
         if ((order & 4) && id < (nbh & ~7) * nqb) lin = (loc / nqb * 8 + xcd) * nqb + loc % nqb;
     return lin;
 }
+
+typedef __attribute__((ext_vector_type(4))) int i32x4_t;
 
 // Sequence b of the batch: its first row and its length.  In a ragged batch the sequences stand back to back and every one
 // has its own length (queries and keys alike); the grid is laid out for the longest, and a workgroup whose queries lie past
@@ -50,6 +64,35 @@ __device__ __forceinline__ void fa_sequence(const int32_t* offsets, int b, int S
     } else {
         row0 = (int64_t)b * S; len = S;
     }
+}
+
+// The sequence of the given rank by length, longest first (of equal ones the first in the batch first): b, its first row and its length.
+// `scratch`: LDS of at least FA_MOST_RANKED + 4 ints that nobody else writes before the workgroup meets again behind this.
+template <int NT> __device__ __forceinline__ void fa_ranked(const int32_t* offsets, int B, int rank, int* scratch, int& b, int64_t& row0, int& len) {
+    const int tid = threadIdx.x, B4 = (B + 3) & ~3;
+    int mine = 0, first = 0;
+    if (tid < B4) {
+        if (tid < B) {
+            first = offsets[tid];
+            mine = (offsets[tid + 1] - first) * FA_MOST_RANKED + FA_MOST_RANKED - 1 - tid;      // distinct; 0 behind the batch
+        }
+        scratch[tid] = mine;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tid < B) {
+        int longer = 0;
+        for (int u = 0; u < B4; u += 4) {
+            const i32x4_t v = *(const i32x4_t*)(scratch + u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) longer += v[e] > mine;
+        }
+        if (longer == rank) *(i32x4_t*)(scratch + FA_MOST_RANKED) = i32x4_t{tid, first, mine / FA_MOST_RANKED, 0};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const i32x4_t found = *(const i32x4_t*)(scratch + FA_MOST_RANKED);
+    b = __builtin_amdgcn_readfirstlane(found[0]);
+    row0 = __builtin_amdgcn_readfirstlane(found[1]);
+    len = __builtin_amdgcn_readfirstlane(found[2]);
 }
 
 template <int N, typename F> __device__ __forceinline__ void sfor(F&& f) {

@@ -90,6 +90,37 @@ def test_fa2_ragged(backend, dtype, lengths, D, causal, rope):
             assert O.max_rel(o[None, s], ref) < (TOL_F32 if dtype == "fp32" else TOL_BF16), (b, n)
 
 
+# just inside and just outside the rule that ranks the sequences by length: 640 blocks of 128 queries at least, 32 sequences at most, longer than 256
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,H,causal,lens", [
+    (64, 8, False, [257] + [1] * 30 + [256]), (64, 9, False, [0, 300, 300, 17, 0] + [300] * 20), (64, 12, True, [500] + list(range(3, 500, 29))),
+    (128, 8, False, [400 - 9 * i for i in range(32)]), (64, 8, False, [300 - 9 * i for i in range(33)]), (64, 40, False, [900, 1, 899])])
+def test_order_of_sequences(backend, D, H, causal, lens):
+    """Where a sequence stands in the batch changes nothing but where its result stands: bit for bit, and against the oracle."""
+    c, rng, scale = backend.core, np.random.default_rng(D + len(lens)), 1.0 / float(np.sqrt(D))
+    parts = [[O.bf16_round(rng.standard_normal((n, H, D)).astype(np.float32)) for _ in range(3)] for n in lens]
+
+    def run(order):
+        off = np.concatenate([[0], np.cumsum([lens[i] for i in order])]).astype(np.int32)
+        pos = np.concatenate([np.arange(lens[i]) for i in order]).astype(np.int32)
+        bufs = [c.upload(np.concatenate([parts[i][j] for i in order]), L.GRL_BF16) for j in range(3)] + [c.upload_raw(off), c.upload_raw(pos), c.alloc(int(off[-1]) * H * D * 2)]
+        try:
+            rg = L.Ragged(bufs[3].ptr, bufs[4].ptr, len(lens), int(off[-1]), max(lens))
+            L.check(c.lib.grl_fa2_fwd_ragged(c.ctx, L.GRL_BF16, ctypes.byref(rg), H, D, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, bufs[5].ptr, H * D, H * D, H * D, H * D,
+                                             scale, int(causal), L.ROPE_NONE, 10000.0, 1.0), "fa2_ragged")
+            o = c.download(bufs[5], (int(off[-1]), H, D), L.GRL_BF16)
+        finally:
+            for t in bufs:
+                t.free()
+        return {i: o[off[k]:off[k + 1]] for k, i in enumerate(order)}
+
+    one, other = run(list(range(len(lens)))), run([int(i) for i in rng.permutation(len(lens))])
+    for i, n in enumerate(lens):
+        np.testing.assert_array_equal(one[i], other[i])
+        if n:
+            assert O.max_rel(one[i][None], O.truth_attention(*(t[None] for t in parts[i]), causal=causal)) < TOL_BF16, (i, n)
+
+
 def _masks(rng, B, S):
     n = rng.integers(1, S + 1, B)
     n[0] = S
