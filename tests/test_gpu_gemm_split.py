@@ -203,6 +203,14 @@ def test_shares_of_k_take_nothing_from_the_pool_under_capture(backend, M, K, N, 
             t.free()
 
 
+@pytest.mark.parametrize("M,K,N", [(300, 3072, 768), (351, 3072, 768), (639, 3072, 768), (449, 4096, 1024), (1201, 2048, 512), (1999, 1152, 764)])
+def test_shares_in_place_of_two_small_tiles_a_unit(backend, M, K, N):
+    """In shares of K where a compute unit would get two 32 x 32 tiles or more of a long K (the first size: one, no shares); under capture without."""
+    rng = np.random.default_rng(M + K + N)
+    x, W, b = rng.standard_normal((M, K)).astype(np.float32), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    assert rel(run(backend, x, W, b), x.astype(np.float64) @ W.T.astype(np.float64) + b) < 2.0 ** -24 * (1 + np.sqrt(6 * K / 16))
+    test_shares_of_k_take_nothing_from_the_pool_under_capture(backend, M, K, N, "fp32")
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("M,K,N", [(1499, 384, 1152), (3001, 384, 1152), (9793, 384, 1536), (9791, 64, 1528), (257, 128, 264)])
 def test_every_element_of_the_staged_epilogues(backend, dtype, M, K, N):
