@@ -11,6 +11,7 @@ SOURCE = r"""
 #include "attention.hpp"
 extern "C" int kernel_run(int variant, int elem_size, int dual) { return gemm_kernel_run(variant, elem_size, dual); }
 extern "C" int kernel(long long M, long long N, long long K, int elem_size, int dual) { return gemm_kernel(M, N, K, elem_size, dual, 256); }
+extern "C" int product(long long M, long long N, long long K, int shares) { return gemm_kernel(M, N, K, 4, false, 256, 0, (Shares)shares); }
 extern "C" int rope_kernel(long long M, long long N, long long K, int elem_size) { return gemm_rope_kernel(M, N, K, 2 * N / 3, elem_size, 256); }
 extern "C" int resln_kernel(long long M, long long N, long long K, int elem_size) { return gemm_resln_kernel(M, N, K, elem_size, 256); }
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
@@ -30,6 +31,7 @@ def rules(tmp_path_factory):
                     "-o", str(at / "rules.so"), str(at / "rules.hip")], check=True, timeout=100)
     lib = ctypes.CDLL(str(at / "rules.so"))
     lib.kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
+    lib.product.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     lib.rope_kernel.argtypes = lib.resln_kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     return lib
 
@@ -90,3 +92,20 @@ def test_sizes_of_the_row_partials_tests(rules):
     assert {g[3] for g in GATED} == {3, 4, 6, 7} and {k for l in LAYERS for k in l[4]} >= {3, 4, 6, 7, 8}
     odd = [(M, d, w) for M, d, _, w, _ in GATED if M % 2 and 128 < d <= (1536 if w == 3 else 768)]      # two to six partials
     assert {w for _, _, w in odd} == {3, 4, 6, 7}
+
+
+NEVER, NOT_NOW, YES = 0, 1, 2          # enum class Shares
+
+
+def test_recorded_products_are_no_less_accurate(rules):
+    """fp32 under capture: what is far better off in shares of K takes kernel 6, whose four chains the shares are, not the fastest kernel
+    without shares (3 or 4: one chain; 9 on the fp32 instruction).  Kernel 9 stays where it is no more than somewhat behind the shares."""
+    far = [(4128, 2304, 8192), (4419, 2048, 6144), (2091, 8192, 8192), (5971, 1152, 6144), (230, 1536, 10400), (8, 1536, 7136), (1500, 768, 3072)]
+    assert [rules.product(*s, YES) for s in far] == [11] * 7 and [rules.product(*s, NOT_NOW) for s in far] == [6] * 7
+    assert {3, 4, 9} == {rules.product(*s, NEVER) for s in far[:-1]}
+    near = [(450, 768, 3072), (350, 768, 3072), (1200, 512, 2048)]
+    assert [rules.product(*s, YES) for s in near] == [11] * 3 and [rules.product(*s, NOT_NOW) for s in near] == [9] * 3
+    for M in range(8, 6000, 83):
+        for N in (128, 384, 768, 1152, 2304, 4096):
+            for K in (480, 512, 1152, 3072, 8192):
+                assert rules.product(M, N, K, NOT_NOW) in (6, rules.product(M, N, K, NEVER))
