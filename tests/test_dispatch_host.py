@@ -109,3 +109,11 @@ def test_recorded_products_are_no_less_accurate(rules):
         for N in (128, 384, 768, 1152, 2304, 4096):
             for K in (480, 512, 1152, 3072, 8192):
                 assert rules.product(M, N, K, NOT_NOW) in (6, rules.product(M, N, K, NEVER))
+
+
+def test_shares_of_k_in_place_of_two_small_tiles_a_unit(rules):
+    """(M, N, K): 11 only where a unit gets two 32 x 32 tiles or more of 1024 k at least, each line from both sides"""
+    sizes = [(300, 768, 3072), (351, 768, 3072), (639, 768, 3072), (449, 1024, 4096), (1201, 512, 2048),
+             (1999, 764, 1152), (1753, 764, 1152), (1688, 764, 1024), (1688, 764, 992), (566, 1800, 896), (563, 2048, 896), (349, 3072, 960)]
+    assert [rules.product(*s, YES) for s in sizes] == [9, 11, 11, 11, 11, 9, 11, 11, 9, 9, 9, 9]
+    assert {rules.product(*s, NEVER) for s in sizes} == {9}
