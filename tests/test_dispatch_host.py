@@ -116,4 +116,4 @@ def test_shares_of_k_in_place_of_two_small_tiles_a_unit(rules):
     sizes = [(300, 768, 3072), (351, 768, 3072), (639, 768, 3072), (449, 1024, 4096), (1201, 512, 2048),
              (1999, 764, 1152), (1753, 764, 1152), (1688, 764, 1024), (1688, 764, 992), (566, 1800, 896), (563, 2048, 896), (349, 3072, 960)]
     assert [rules.product(*s, YES) for s in sizes] == [9, 11, 11, 11, 11, 9, 11, 11, 9, 9, 9, 9]
-    assert {rules.product(*s, NEVER) for s in sizes} == {9}
+    assert {rules.product(*s, NEVER) for s in sizes} == {9} and rules.product(33, 388, 2080, YES) == 9

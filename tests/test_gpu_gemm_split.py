@@ -211,6 +211,15 @@ def test_shares_in_place_of_two_small_tiles_a_unit(backend, M, K, N):
     assert rel(run(backend, x, W, b), x.astype(np.float64) @ W.T.astype(np.float64) + b) < 2.0 ** -24 * (1 + np.sqrt(6 * K / 16))
     test_shares_of_k_take_nothing_from_the_pool_under_capture(backend, M, K, N, "fp32")
 
+
+@pytest.mark.parametrize("M,K,N", [(1999, 1152, 764), (1688, 992, 764), (300, 3072, 768), (33, 2080, 388),      # one workgroup a tile: split operands, then the fp32 instruction
+                                   (1753, 1152, 764), (1688, 1024, 764)])                                      # shares
+@pytest.mark.parametrize("positive", [False, True])
+def test_small_tiles_of_a_long_sum(backend, M, K, N, positive):
+    """32 x 32 tiles (test_dispatch_host pins which of these sizes take them) and the shares that stand in for them, K of 31 slabs and more"""
+    test_error_against_float64(backend, M, K, N, positive)
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("M,K,N", [(1499, 384, 1152), (3001, 384, 1152), (9793, 384, 1536), (9791, 64, 1528), (257, 128, 264)])
 def test_every_element_of_the_staged_epilogues(backend, dtype, M, K, N):
