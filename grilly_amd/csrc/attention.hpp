@@ -66,17 +66,23 @@ __device__ __forceinline__ void fa_sequence(const int32_t* offsets, int b, int S
     }
 }
 
-// The sequence of the given rank by length, longest first (of equal ones the first in the batch first): b, its first row and its length.
+// Where a sequence of `len` rows stands among those of its batch, larger keys first: the longest first, of equal ones the first in the batch.
+// Distinct and not negative whatever `len` is (offsets that fall count as empty sequences): every rank below B has its owner.
+__host__ __device__ __forceinline__ int fa_rank_key(int len, int b) {
+    return (len < 0 ? 0 : len < 65536 ? len : 65536) * FA_MOST_RANKED + FA_MOST_RANKED - 1 - b;
+}
+// The sequence of the given rank: b, its first row and its length.
 // `scratch`: LDS of at least FA_MOST_RANKED + 4 ints that nobody else writes before the workgroup meets again behind this.
 template <int NT> __device__ __forceinline__ void fa_ranked(const int32_t* offsets, int B, int rank, int* scratch, int& b, int64_t& row0, int& len) {
     const int tid = threadIdx.x, B4 = (B + 3) & ~3;
-    int mine = 0, first = 0;
+    int mine = 0, first = 0, own = 0;
     if (tid < B4) {
         if (tid < B) {
             first = offsets[tid];
-            mine = (offsets[tid + 1] - first) * FA_MOST_RANKED + FA_MOST_RANKED - 1 - tid;      // distinct; 0 behind the batch
+            own = offsets[tid + 1] - first;
+            mine = fa_rank_key(own, tid);
         }
-        scratch[tid] = mine;
+        scratch[tid] = mine;             // 0 behind the batch
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (tid < B) {
@@ -86,7 +92,7 @@ template <int NT> __device__ __forceinline__ void fa_ranked(const int32_t* offse
 #pragma unroll
             for (int e = 0; e < 4; ++e) longer += v[e] > mine;
         }
-        if (longer == rank) *(i32x4_t*)(scratch + FA_MOST_RANKED) = i32x4_t{tid, first, mine / FA_MOST_RANKED, 0};
+        if (longer == rank) *(i32x4_t*)(scratch + FA_MOST_RANKED) = i32x4_t{tid, first, own, 0};
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const i32x4_t found = *(const i32x4_t*)(scratch + FA_MOST_RANKED);

@@ -17,6 +17,7 @@ extern "C" int resln_kernel(long long M, long long N, long long K, int elem_size
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
 extern "C" int order_checked(int order) { return fa_order_checked(order); }
 extern "C" int order(int causal, int S, int ragged, int heads, int D) { return fa_order(causal, S, ragged, heads, D); }
+extern "C" int rank_key(int len, int b) { return fa_rank_key(len, b); }
 extern "C" int place(int deal, int order, int id, int nwg, int nqb, int nbh) {
     return deal ? fa_place<true>(order, id, nwg, nqb, nbh) : fa_place<false>(order, id, nwg, nqb, nbh);
 }
@@ -117,3 +118,14 @@ def test_shares_of_k_in_place_of_two_small_tiles_a_unit(rules):
              (1999, 764, 1152), (1753, 764, 1152), (1688, 764, 1024), (1688, 764, 992), (566, 1800, 896), (563, 2048, 896), (349, 3072, 960)]
     assert [rules.product(*s, YES) for s in sizes] == [9, 11, 11, 11, 11, 9, 11, 11, 9, 9, 9, 9]
     assert {rules.product(*s, NEVER) for s in sizes} == {9} and rules.product(33, 388, 2080, YES) == 9
+
+
+@pytest.mark.parametrize("lens", [[5, 0, 900, 5, 900, 1, 0], [-7, 3, -2 ** 31, 0, 3, -1], [2 ** 31 - 1, 65536, 65537, 1, 2 ** 26], [300] * 32, [-1] * 31 + [0], list(range(32, 0, -1))])
+def test_every_rank_has_one_sequence(rules, lens):
+    """as fa_ranked counts: the longer ones among the batch and the zeros that fill its last four.  Lengths as any offsets give them, also falling ones."""
+    keys = [rules.rank_key(n, b) for b, n in enumerate(lens)]
+    padded = keys + [0] * (-len(keys) % 4)
+    ranks = [sum(k > mine for k in padded) for mine in keys]
+    assert sorted(ranks) == list(range(len(lens)))
+    length = lambda b: min(max(lens[b], 0), 65536)
+    assert sorted(range(len(lens)), key=lambda b: ranks[b]) == sorted(range(len(lens)), key=lambda b: (-length(b), b))
