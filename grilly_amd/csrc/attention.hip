@@ -704,13 +704,14 @@ static int launch_fa16_cfg(grl_ctx* c, const Fa16Args& f, int rope_q) {
 }
 
 template <int D>
-static int launch_fa16(grl_ctx* c, const FaArgs& a, int rope_q) {
+static int launch_fa16(grl_ctx* c, const FaArgs& a, int rope_q, int64_t rows) {
     Fa16Args f{};
     f.Q = (const uint16_t*)a.Q; f.K = (const uint16_t*)a.K; f.V = (const uint16_t*)a.V;
     f.mask = a.mask; f.O = (uint16_t*)a.O; f.rope = a.rope; f.offsets = a.offsets;
     f.B = a.B; f.S = a.S; f.H = a.H; f.scale = a.scale; f.causal = a.causal;
     static const int order_env = [] { const char* e = getenv("GRL_FA_ORDER"); return e ? atoi(e) : -1; }();
-    f.order = order_env >= 0 ? fa_order_checked(order_env) : fa_order_ranked(fa_order(a.causal, a.S, a.offsets && !a.mask && rope_q == 0, (int64_t)a.B * a.H, D), a.S, a.B, (int64_t)a.B * a.H * ((a.S + 127) / 128));
+    const int order = fa_order(a.causal, a.S, a.offsets && !a.mask && rope_q == 0, (int64_t)a.B * a.H, D);
+    f.order = order_env >= 0 ? fa_order_checked(order_env) : fa_order_ranked(order, a.causal, a.S, a.B, a.H, rows, c->prop.multiProcessorCount);
     f.q_stride = a.q_stride; f.k_stride = a.k_stride; f.v_stride = a.v_stride; f.o_stride = a.o_stride;
     // GRL_FA_CFG forces a configuration, for tuning runs:
     //   1: 8 waves, 64-key tiles, deep ring   2: 8 waves, 128-key tiles   3: 4 waves, 64-key tiles, 4 stages (head dims up to 64)
@@ -955,7 +956,7 @@ static int fa2_common(grl_ctx* c, const char* who, int dtype, int64_t B, int64_t
         if (dtype == GRL_F32) {
             rc = launch_fa32(c, a, (int)D, fused);
         } else {
-            rc = D == 32 ? launch_fa16<32>(c, a, rope_q) : D == 64 ? launch_fa16<64>(c, a, rope_q) : launch_fa16<128>(c, a, rope_q);
+            rc = D == 32 ? launch_fa16<32>(c, a, rope_q, nrows) : D == 64 ? launch_fa16<64>(c, a, rope_q, nrows) : launch_fa16<128>(c, a, rope_q, nrows);
         }
     }
     if (own) grl_free(c, own);   // stream order keeps the blocks alive until the kernel has finished

@@ -32,15 +32,20 @@ static inline int fa_order(bool causal, int64_t S, bool ragged, int64_t heads, i
     if (ragged && D >= 64 && heads >= 64 && S <= 1024) return 4;
     return causal || S <= 1024 ? 1 : 0;
 }
-// Dealt-out ragged batches of few long sequences: the longest first.  Their workgroups (`blocks`, empty ones counted) are all resident at
-// once, so a launch lasts as long as the CU that was dealt the most work; by falling length the deal comes out nearly even.  Every
-// workgroup ranks the sequences for itself, 0.3 to 0.5 us.  us, in batch order -> ranked, lengths uniform from an eighth to all of S:
-// 32 x 300 x 12 heads of 64 17.7 -> 14.2, 16 x 512 x 12 17.3 -> 16.2, 24 x 900 x 8 42.5 -> 39.7, 32 x 400 x 8 heads of 128 36.7 -> 33.5; over 30
-// batches of 300 to 900 5 % on the mean (0.80 to 1.02).  Where the line leaves off: fewer blocks than 2.5 per CU are no deal
-// (10 x 512 x 8 12.1 -> 13.1), short sequences lose the ranking's time (24 x 200 x 12 11.3 -> 11.5), and of many blocks or sequences
-// the later ones fill the gaps as they come (64 x 512 x 12 49.9 -> 52.6, 32 x 900 x 16 73.2 -> 74.5).
-static inline int fa_order_ranked(int order, int64_t S, int64_t B, int64_t blocks) {
-    return order == 4 && S > 256 && B > 1 && B <= FA_MOST_RANKED && blocks >= 640 && blocks <= 3072 ? 12 : order;
+// Dealt-out ragged batches of few long sequences of unequal length: the longest first.  Their workgroups (`blocks` of 128 queries, empty ones
+// counted) are all resident at once or nearly, so a launch lasts as long as the CU that was dealt the most work; by falling length the deal
+// comes out nearly even.  Every workgroup ranks the sequences for itself, which costs a launch 0.5 to 1.5 us.  In batch order / ranked, mean
+// of 26 sizes (8 .. 32 sequences, longest 260 .. 1024, 8 .. 16 heads of 64 and 128), by how full the rectangle B x S is: 0.43 0.93, 0.58 0.94,
+// 0.76 0.99, 0.86 1.003, 0.93 1.02, 1.0 1.03.  us, lengths uniform from an eighth to all of S: 32 x 300 x 12 heads of 64 18.2 -> 17.0, 24 x 300 x 12
+// 16.7 -> 13.7, 16 x 512 x 12 18.4 -> 17.4, 13 x 749 x 12 28.4 -> 19.5, 24 x 900 x 8 39.3 -> 36.6, 32 x 400 x 8 heads of 128 35.0 -> 32.5.
+// Where the line leaves off: rectangles more than three quarters full (32 x 300 x 12 all of 300: 24.3 -> 25.7), fewer blocks than 2.5 per CU are no
+// deal (10 x 512 x 8 12.1 -> 13.1), short sequences lose the ranking's time (24 x 200 x 12 11.3 -> 11.5), so do causal ones up to 512, whose
+// work falls off with the square of the length (30 x 465 x 12 heads of 128 36.5 -> 39.4), sequences of four blocks gain nothing once they are more
+// than four blocks per CU (24 x 512 x 12 1.02, 21 x 476 x 16 1.03, 28 x 512 x 16 0.995; of three blocks 32 x 384 x 12 0.89, of six and more 0.93),
+// and of many blocks or sequences the later ones fill the gaps as they come (64 x 512 x 12 49.9 -> 52.6, 32 x 900 x 16 73.2 -> 74.5).
+static inline int fa_order_ranked(int order, bool causal, int64_t S, int64_t B, int64_t H, int64_t rows, int64_t cus) {
+    const int64_t each = (S + 127) / 128, blocks = B * H * each;
+    return order == 4 && S > (causal ? 512 : 256) && B > 1 && B <= FA_MOST_RANKED && 4 * rows <= 3 * B * S && 2 * blocks >= 5 * cus && blocks <= (each == 4 ? 4 : 12) * cus ? 12 : order;
 }
 // Where workgroup `id` of nwg = nqb * nbh stands in the walk.  DEAL: the heads that make whole turns of eight are dealt out, the query blocks
 // of one head next to each other on one XCD; the rest keep their ids.

@@ -17,6 +17,7 @@ extern "C" int resln_kernel(long long M, long long N, long long K, int elem_size
 extern "C" int takes_partials(int kernel) { return gemm_kernel_takes_partials(kernel); }
 extern "C" int order_checked(int order) { return fa_order_checked(order); }
 extern "C" int order(int causal, int S, int ragged, int heads, int D) { return fa_order(causal, S, ragged, heads, D); }
+extern "C" int ranked(int order, int causal, int S, int B, int H, long long rows, int cus) { return fa_order_ranked(order, causal, S, B, H, rows, cus); }
 extern "C" int rank_key(int len, int b) { return fa_rank_key(len, b); }
 extern "C" int place(int deal, int order, int id, int nwg, int nqb, int nbh) {
     return deal ? fa_place<true>(order, id, nwg, nqb, nbh) : fa_place<false>(order, id, nwg, nqb, nbh);
@@ -32,6 +33,7 @@ def rules(tmp_path_factory):
                     "-o", str(at / "rules.so"), str(at / "rules.hip")], check=True, timeout=100)
     lib = ctypes.CDLL(str(at / "rules.so"))
     lib.kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
+    lib.ranked.argtypes = [ctypes.c_int] * 5 + [ctypes.c_longlong, ctypes.c_int]
     lib.product.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     lib.rope_kernel.argtypes = lib.resln_kernel.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     return lib
@@ -129,3 +131,24 @@ def test_every_rank_has_one_sequence(rules, lens):
     assert sorted(ranks) == list(range(len(lens)))
     length = lambda b: min(max(lens[b], 0), 65536)
     assert sorted(range(len(lens)), key=lambda b: ranks[b]) == sorted(range(len(lens)), key=lambda b: (-length(b), b))
+
+
+@pytest.mark.parametrize("order", range(8, 16))
+def test_every_block_is_computed_once_by_ranked_orders(rules, order):
+    """GRL_FA_ORDER with the ranking's bit, which stands for nothing without dealt-out heads"""
+    checked = rules.order_checked(order)
+    assert checked & 8 == (8 if order & 4 else 0)
+    test_every_attention_block_is_computed_once(rules, order)
+
+
+def test_which_batches_are_ranked(rules):
+    """both sides of each line: longest sequence, sequences, how full the rectangle is, blocks per compute unit, the order it stands on"""
+    ranked = lambda S, B, H, fill=0.5, causal=0, order=4, cus=256: rules.ranked(order, causal, S, B, H, int(fill * B * S), cus) == 12
+    assert ranked(300, 32, 12) and [ranked(S, 32, 12) for S in (256, 257)] == [False, True]
+    assert [ranked(S, 16, 16, causal=1) for S in (512, 513)] == [False, True]
+    assert [ranked(300, B, 16) for B in (32, 33)] == [True, False] and not ranked(1000, 1, 512)
+    assert [ranked(600, 32, 12, fill) for fill in (0.75, 0.7501, 1.0)] == [True, False, False]
+    assert [ranked(S, 32, H) for S, H in ((512, 8), (512, 9), (384, 9), (385, 9), (513, 9))] == [True, False, True, False, True]      # 1024 blocks, 1152, 864, 1152, 1440
+    assert [ranked(384, B, H) for B, H in ((15, 14), (16, 14), (32, 8))] == [False, True, True]              # 630, 672, 768 blocks
+    assert [ranked(512, 20, 8, cus=cus) for cus in (256, 257)] == [True, False] and [ranked(1024, 32, 12, cus=cus) for cus in (256, 255)] == [True, False]
+    assert not any(ranked(300, 32, 12, order=order) for order in (0, 1, 2))

@@ -121,6 +121,15 @@ def test_order_of_sequences(backend, D, H, causal, lens):
             assert O.max_rel(one[i][None], O.truth_attention(*(t[None] for t in parts[i]), causal=causal)) < TOL_BF16, (i, n)
 
 
+# batches that the rule ranks, with empty sequences, equal lengths and causal ones; the last just past its line for full rectangles
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,H,causal,lens", [
+    (64, 9, False, [0, 300, 300, 17, 0] + [300] * 10 + [100] * 12), (64, 12, True, [600] + list(range(3, 600, 35))), (128, 8, True, [0, 700, 699, 1] + [350] * 12),
+    (64, 10, False, [400] * 17 + [0] * 6), (64, 10, False, [400] * 17 + [0] * 5)])
+def test_order_of_unequal_sequences(backend, D, H, causal, lens):
+    test_order_of_sequences(backend, D, H, causal, lens)
+
+
 def _masks(rng, B, S):
     n = rng.integers(1, S + 1, B)
     n[0] = S
