@@ -28,7 +28,8 @@
 // do not meet (65536 x 2304 x 768 184 -> 185; x 384 109 -> 106), stores that stay in the caches (188.7 -> 199.8), no wave priorities (level).
 #pragma once
 
-template <typename OutT, int EPI, bool DUAL, bool LN = false>
+// ASKS: for launches of no more tiles than workgroups, see ask_for_residual
+template <typename OutT, int EPI, bool DUAL, bool LN = false, bool ASKS = false>
 __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     // A wave's share of the tile: 128 rows x 64 columns.  The row sums of EPI_RESLN are added chunk by chunk in the order of the 32 lanes that hold
     // a row of 256 columns elsewhere (c with c + 8, + 4, + 2, + 1, the halves last), which needs 128 columns of a row in one wave: 64 rows x
@@ -43,7 +44,9 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     // tile's 256 row-statistics pairs.  Two buffers, alternating per tile.
     constexpr int VECS = 2 * STAGE, COLB = BN * 4, BIASB = ROWS ? 2 * COLB + BM * 8 : COLB;
     constexpr int PARTS_AT = VECS + 2 * BIASB, SUMS_AT = PARTS_AT + (ROWS ? GRL_MAX_PARTS * BM * 8 : 0);
-    __shared__ __attribute__((aligned(1024))) char lds[SUMS_AT + (RL ? 2 * BM * 8 : 0)];
+    constexpr int ASKED_AT = SUMS_AT + (RL ? 2 * BM * 8 : 0);
+    __shared__ __attribute__((aligned(1024))) char lds[ASKED_AT + (ASKS ? 1024 : 0)];
+    static_assert(!ASKS || (HASRES && OES == 2), "what is asked for");
     static_assert(!(LN && RL) && !(RL && DUAL) && !(HASRES && DUAL), "one set of row statistics per tile");
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -130,6 +133,20 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
 
     int pid = blockIdx.x, m0, n0, bbuf = 0;
     tile_of(pid, m0, n0);
+    // A workgroup with one tile would do nothing but wait while its residual comes: the tile's lines are brought to L2 two steps before the end,
+    // by transfers of 16 bytes of each (32 rows of four lines from a wave) into 1 KiB that nobody reads.  us, without -> with, no operand of
+    // a launch touched by the one before: 16384 x 1024 x 1024 39.8 -> 36.5, with LayerNormed residual 44.3 -> 40.7, 18000 x 768 x 384 22.2 -> 21.1 and
+    // 26.6 -> 25.6, 21000 x 768 x 768 32.1 -> 30.5 and 36.8 -> 34.7 (an epilogue staged by the whole workgroup: 37.1, 40.5, 20.8, 25.6, 31.1, 35.1).
+    // A kernel of its own: with several tiles the lines push operands out of L2 (65536 x 2304 x 768 226 -> 241), and the test for it alone
+    // spills scalars (1 % of 65536 x 768 x 768 with LayerNormed residual).  Six steps ahead is too early to find the lines there.
+    auto ask_for_residual = [&] {
+        const int64_t left = ((int64_t)(p.M - m0) * p.N - n0) * OES;
+        rsrc_words rs = make_rsrc_words((const char*)p.residual + ((int64_t)m0 * p.N + n0) * OES, left > 0x7fffffff ? 0x7fffffffu : (uint32_t)left);
+        asm volatile("s_nop 4" : "+s"(rs));                  // as in fetch_vec
+        const int at = (wave * 32 + (lane >> 2)) * rowB + (lane & 3) * 128;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) dma16(rs, __builtin_amdgcn_readfirstlane((int)lds0 + ASKED_AT), at, 0, 16 * j * rowB);
+    };
     issue_vectors(m0, n0, bbuf);
     curA = rsrc_of(p.A, m0, p.M); curW = rsrc_of(p.W, n0, p.N);
     curW2 = DUAL ? rsrc_of(p.W2, n0, p.N) : curW;
@@ -247,6 +264,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
             };
             read_x(0); read_y(0); read_x(1);
             if (!FIRST && kt == 1 && has_next) issue_vectors(m0n, n0n, bbuf ^ 1);
+            if constexpr (ASKS) if (kt == KT - 2 && staged) ask_for_residual();
             issue_half(H_Y1{}, gstep + 1);
             advance();
             due();                           // A1 of this step

@@ -152,3 +152,9 @@ def test_which_batches_are_ranked(rules):
     assert [ranked(384, B, H) for B, H in ((15, 14), (16, 14), (32, 8))] == [False, True, True]              # 630, 672, 768 blocks
     assert [ranked(512, 20, 8, cus=cus) for cus in (256, 257)] == [True, False] and [ranked(1024, 32, 12, cus=cus) for cus in (256, 255)] == [True, False]
     assert not any(ranked(300, 32, 12, order=order) for order in (0, 1, 2))
+
+
+def test_one_phased_tile_for_each_unit(rules):
+    """the size of the test of that name in test_gpu_gemm_phased: 256 x 256 tiles, fewer than compute units"""
+    M, N = 71 * 256 - 37, 3 * 256 - 8
+    assert all(rules.kernel(M, N, 64 * slabs, 2, 0) == 3 == rules.resln_kernel(M, N, 64 * slabs, 2) for slabs in (2, 3, 7))

@@ -153,3 +153,12 @@ def test_residual_of_fp32_results(backend, slabs):
     finally:
         for t in bufs:
             t.free()
+
+
+@pytest.mark.parametrize("slabs", [2, 3, 7])
+@pytest.mark.parametrize("kind", ["residual", "normed_residual"])
+def test_one_tile_for_each_unit(backend, monkeypatch, kind, slabs):
+    """213 tiles: the residual's lines are asked for under the last steps, also where those are the first"""
+    monkeypatch.setitem(globals(), "M", 71 * 256 - 37)
+    monkeypatch.setitem(globals(), "N", 3 * 256 - 8)
+    test_phased_tiles(backend, kind, slabs)
