@@ -97,6 +97,7 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
     };
     // a tile's vectors: up to 1 KiB of `src` from a wave (columns and rows past the end read zero)
     auto fetch_vec = [&](const float* src, int left, int at, int bytes) {
+        const int lane = EPI == EPI_ROPE ? fresh_lane() : (int)threadIdx.x & 63;
         rsrc_words rs = make_rsrc_words(src, left > 0 ? (uint32_t)left : 0u);
         asm volatile("s_nop 4" : "+s"(rs));             // the wait states behind a vector write of the words, where the compiler kept them in vector registers
         if (bytes >= 1024 || lane < bytes / 16) dma16(rs, __builtin_amdgcn_readfirstlane((int)lds0 + at), lane * 16, 0, 0);
@@ -293,6 +294,8 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
         __builtin_amdgcn_sched_barrier(0);
 
         if (staged) {
+            // EPI_ROPE: the lane's coordinates are formed anew; addresses kept over the tile loop spilled, and their reloads drained the transfers
+            const int lane = EPI == EPI_ROPE ? fresh_lane() : tid & 63, l4 = lane & 15, lq = lane >> 4;
             char* own = lds + ((gstep - 1) & 1) * STAGE + HALFB + wave * 2048;
             const char* vec = lds + VECS + bbuf * BIASB;
             // this lane's 16-byte piece of a staged row: chunk cc of row rr (+ 2 per further read: a read's 8 rows are such that its turns meet no bank twice)
@@ -347,13 +350,30 @@ __global__ __launch_bounds__(512) void gemm_nt_phased_kernel(GemmArgs p) {
             static_assert(EPI != EPI_ROPE || (!DUAL && !LN && OES == 2), "a wave's 64 columns are one head");
             const bool rotated = EPI == EPI_ROPE && n0 + wn * WNO < p.rope_cols;
             // EPI_ROPE: the two halves of a pair, columns d and d + 32 of a head, are the same register of blocks b and b + 2, so the rotation
-            // stays in registers: four multiply-adds a pair, on the sums before they are rounded.  cos and sin are requested a band ahead.
+            // stays in registers: four multiply-adds a pair, on the sums before they are rounded.  cos and sin are requested a band ahead, the
+            // bands' positions all at once (one by one, each waited for everything in flight).
             f32x4 cs[EPI == EPI_ROPE ? 2 : 1][2][2];
+            int rope_at[EPI == EPI_ROPE ? WM / 16 : 1];           // where a row's values start in the table
+            if constexpr (EPI == EPI_ROPE) if (rotated) {
+                const int first = m0 + wm * WM + l4, last = p.M - 1;
+                if (p.rope_pos) {
+#pragma unroll
+                    for (int i = 0; i < WM / 16; ++i) rope_at[i] = p.rope_pos[min(first + 16 * i, last)];
+#pragma unroll
+                    for (int i = 0; i < WM / 16; ++i) rope_at[i] = (int)min((uint32_t)rope_at[i], (uint32_t)(p.rope_S - 1));
+                } else {
+                    int turn = p.rope_S;
+                    asm volatile("" : "+s"(turn));           // the divisor's reciprocal is formed here, not kept over the tile loop
+#pragma unroll
+                    for (int i = 0; i < WM / 16; ++i) rope_at[i] = min(first + 16 * i, last) % turn;
+                }
+#pragma unroll
+                for (int i = 0; i < WM / 16; ++i) rope_at[i] = rope_at[i] * 64 + 8 * lq;
+            }
             auto fetch_rope = [&](auto ii) {
                 constexpr int i = decltype(ii)::value;
                 if constexpr (EPI == EPI_ROPE) if (rotated) {
-                    const int m = m0 + wm * WM + 16 * i + l4, mc = m < p.M ? m : p.M - 1;
-                    const float* t = (const float*)p.rope + rope_position(p, mc) * 64 + 8 * lq;
+                    const float* t = (const float*)p.rope + rope_at[i];
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
                         cs[i & 1][b][0] = *(const f32x4*)(t + 32 * b);

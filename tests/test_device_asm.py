@@ -128,3 +128,20 @@ def test_every_transfer_of_the_library_has_its_waits(tmp_path):
                 assert not bad, bad[:3]
                 transfers += n
     assert transfers > 1000
+
+
+def test_phased_kernels_keep_nothing_in_scratch(tmp_path):
+    """A reload from scratch waits for the wave's memory counter to run out, the transfers of two steps with it."""
+    llvm, lib = "/opt/rocm/llvm/bin", os.path.join(os.path.dirname(CSRC), "lib", "libgrilly_hip.so")
+    if not os.path.exists(lib):
+        pytest.skip("library not built")
+    shutil.copy(lib, tmp_path / "l.so")
+    subprocess.run([os.path.join(llvm, "llvm-objdump"), "--offloading", "l.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL, timeout=60)
+    scratch = {}
+    for f in glob.glob(str(tmp_path / "*gfx950")):
+        notes = subprocess.run([os.path.join(llvm, "llvm-readelf"), "--notes", f], check=True, capture_output=True, text=True, timeout=60).stdout
+        for k in re.split(r"\n  - ", notes):
+            name, size = re.search(r"\.name:\s+(\S+)", k), re.search(r"\.private_segment_fixed_size:\s+(\d+)", k)
+            if name and size and "gemm_nt_phased_kernel" in name[1]:
+                scratch[name[1]] = int(size[1])
+    assert len(scratch) > 10 and not any(scratch.values()), scratch
