@@ -751,8 +751,8 @@ def main():
         # timed back to back in a table of their own are reported next to it.
         fused = getattr(enc, "fused_now", False)
         names = ("gemm_out_resln", "gemm_ffn2_resln") if fused else ("gemm_qkv", "gemm_out", "gemm_ffn2")
-        tname = "float" if a.dtype == "fp32" else "bf16"
-        kname = f"gemm_nt_dma_kernel<{tname},{tname},256,256,2,4,{'EPI_RESLN' if fused else 'EPI_NONE'}>"
+        big_tiles = lambda epi: f"gemm_nt_phased_kernel<bf16,{epi}>" if a.dtype == "bf16" else f"gemm_nt_dma_kernel<float,float,256,256,2,4,{epi}>"
+        kname = big_tiles("EPI_RESLN" if fused else "EPI_NONE")
         g = [kt[k] for k in names]
         avg_flops = sum(r["flops"] for r in g) / len(g)
         fwd_ms = sum(fk[k]["ms"] for k in names) / len(names)
@@ -789,7 +789,7 @@ def main():
             # layer and of earlier measurements of this benchmark), same definition: mean FLOPs over mean duration
             gp = [kt[k] for k in ("gemm_qkv", "gemm_out", "gemm_ffn2")]
             fl, ms3 = sum(r["flops"] for r in gp) / 3, sum(r["ms"] for r in gp) / 3
-            out["roofline_plain_gemm"] = {"kernel": f"gemm_nt_dma_kernel<{tname},{tname},256,256,2,4,EPI_NONE>", "launches": ["gemm_qkv", "gemm_out", "gemm_ffn2"],
+            out["roofline_plain_gemm"] = {"kernel": big_tiles("EPI_NONE"), "launches": ["gemm_qkv", "gemm_out", "gemm_ffn2"],
                                           "achieved": round(fl / (ms3 * 1e-3) / 1e12, 1), "peak": peak / 1e12, "unit": "TFLOP/s",
                                           "frac": round(fl / (ms3 * 1e-3) / peak, 4), "avg_launch_ms": round(ms3, 4),
                                           "shader_clock_ghz": round(sum(r["shader_clock_ghz"] for r in gp) / 3, 3),

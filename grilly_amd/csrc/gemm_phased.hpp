@@ -12,18 +12,22 @@
 //
 // (X and Y below: Y is the operand whose halves are multiplied in turn, A, and X the other; with EPI_RESLN they change places.)
 //
-// A memory part ends when its reads are back, so a half is requested again one part after its last read, and is due six parts later: 64 to
-// 96 KiB are in flight all the time.  The cursor runs on into the next tile, so nothing drains between tiles: the epilogue stands between
-// the last matrix part and the next tile's first memory part, and only A1 of the last step's stage is not being refilled then.  There,
-// in the 2 KiB that its own transfers will fill, every wave turns 16 output rows at a time into 16-byte pieces of 128-byte rows: no barrier
-// in the epilogue, and the stores stand behind the transfers of two steps in the memory counter.
+// A memory part ends when its reads are back, so a half is requested again one part after the waves behind have read it; the counted wait
+// asks for it four parts later, and it is read six parts later.  64 to 96 KiB are in flight all the time.  The cursor runs on into the next tile,
+// and the epilogue stands between the last matrix part and the next tile's first memory part; only A1 of the last step's stage is not
+// being refilled then.  There, in the 2 KiB that its own transfers will fill, every wave turns 16 output rows at a time into 16-byte pieces of
+// 128-byte rows: no barrier in the epilogue, and the stores stand behind the transfers of two steps in the memory counter.  An epilogue
+// that only stores waits for none of them.  One that loads (residual, cos and sin) waits once for all that is in flight, because the
+// counter retires in order.
 //
 // Bound: the board's power limit on real operands (with all-zero ones the same launches are 20 to 25 % faster: a step of 2048 matrix cycles
 // takes 2340 at 2.4 GHz), then the output stores, which all CUs issue at once: without them 65536 x 2304 x 768 takes 163 us instead of
 // 184, 65536 x 768 x 768 with LayerNormed residual 75 instead of 88.
-// us, four phases of 16 instructions with an epilogue staged by the whole workgroup (four barriers, the stages drained for it) -> this:
-// 65536 x 2304 x 768 195.6 -> 187.6, 65536 x 2304 x 384 112.6 -> 105.7, folded 65536 x 3072 x 768 with GELU 301 -> 292, 65536 x 768 x 768 with
-// LayerNormed residual 93.1 -> 90.3, 8192 x 8192 x 8192 764 -> 739, gated 16384 x 11008 x 4096 2115 -> 2066; 65536 x 768 x 3072 level.
+// us, four phases of 16 instructions with an epilogue staged by the whole workgroup (four barriers, the stages drained for it) and the same LDS
+// swizzle -> this, in turn on one box: 65536 x 2304 x 768 191.5 -> 183.7, folded 200.1 -> 190.3, 65536 x 1152 x 384 64.2 -> 61.2, folded 65536 x 3072 x
+// 768 with GELU 297.4 -> 285.2, 65536 x 768 x 768 with LayerNormed residual 92.1 -> 91.3, 8192 x 8192 x 8192 747 -> 725, gated 16384 x 11008 x 4096
+// 2050 -> 2023; 65536 x 768 x 3072 level.  Slower: bf16 residuals of short sums in several tiles (65536 x 768 x 128 44.0 -> 45.5, 33000 x 768 x 384
+// 37.1 -> 37.7), whose epilogue that wait is most of.
 // Without the stagger 27 % slower (four phases).  Tried and dropped: workgroups that start up to 3 us apart, so that their stores
 // do not meet (65536 x 2304 x 768 184 -> 185; x 384 109 -> 106), stores that stay in the caches (188.7 -> 199.8), no wave priorities (level).
 #pragma once
